@@ -324,6 +324,41 @@ def grouped_gemm_gathered_wgrad_cuda(
     _lib.check(rc, "grouped_gemm_gathered_wgrad_cuda")
 
 
+@custom_op(f"{LIBRARY_NAME}::grouped_gemm_thin_cuda", mutates_args={"output"})
+def grouped_gemm_thin_cuda(
+    x: torch.Tensor,
+    row_index: torch.Tensor | None,
+    divisor: int,
+    weight: torch.Tensor,
+    bias: torch.Tensor | None,
+    counts: torch.Tensor,
+    offsets: torch.Tensor,
+    output: torch.Tensor,
+    swiglu: bool,
+) -> None:
+    """The forward product of an expert projection for groups of a few rows: output [R, N] = rows @ W^T (+ bias), or with
+    swiglu [R, N / 2] = swiglu_packed of it; rows packed in x, or x[row_index[i] // divisor] (fma_grouped_gemm_thin)."""
+    _lib.require_gpu(x, row_index, weight, bias, counts, offsets, output)
+    E, N, K = weight.shape
+    R = output.size(0)
+    assert x.dim() == 2 and x.size(1) == K and x.dtype == weight.dtype == output.dtype
+    assert output.shape == (R, N // 2 if swiglu else N)
+    assert (row_index is None and x.size(0) == R) or (row_index.dtype == torch.int32 and row_index.numel() == R)
+    assert counts.dtype == offsets.dtype == torch.uint32 and counts.numel() == offsets.numel() == E
+    assert bias is None or (bias.shape == (E, N) and bias.dtype == x.dtype)
+    for t in (x, row_index, weight, bias, counts, offsets, output):
+        assert t is None or t.is_contiguous()
+    if output.numel() == 0:
+        return
+    with torch.cuda.device(x.device):
+        rc = _lib.load().fma_grouped_gemm_thin(
+            x.data_ptr(), x.size(0), _lib.ptr(row_index), divisor, weight.data_ptr(), _lib.ptr(bias), output.data_ptr(),
+            counts.data_ptr(), offsets.data_ptr(), R, E, N, K, int(swiglu), _lib.dtype_code(x.dtype),
+            _lib.current_stream(x.device),
+        )
+    _lib.check(rc, "grouped_gemm_thin_cuda")
+
+
 @custom_op(f"{LIBRARY_NAME}::expert_bias_add_cuda", mutates_args={"y"})
 def expert_bias_add_cuda(y: torch.Tensor, bias: torch.Tensor, M_array: torch.Tensor) -> None:
     _lib.require_gpu(y, bias, M_array)
@@ -900,6 +935,20 @@ def gathered_up_projection_experts(
     return _GatheredUpProjection.apply(
         x, weight, bias, perm, inv, M_array, N_array, K_array, top_k, swiglu, torch.is_grad_enabled()
     )
+
+
+@torch.no_grad()
+def thin_swiglu_experts(
+    x: torch.Tensor, weight1: torch.Tensor, bias1: torch.Tensor | None, weight2: torch.Tensor, bias2: torch.Tensor | None,
+    perm: torch.Tensor, counts: torch.Tensor, offsets: torch.Tensor, top_k: int,
+) -> torch.Tensor:  # fmt: skip
+    """gathered_swiglu_experts without a backward, for a few rows per expert: same values, bit for bit"""
+    R = perm.numel()
+    act = torch.empty(R, weight2.size(2), device=x.device, dtype=x.dtype)
+    output = torch.empty(R, weight2.size(1), device=x.device, dtype=x.dtype)
+    grouped_gemm_thin_cuda(x, perm, top_k, weight1, bias1, counts, offsets, act, True)
+    grouped_gemm_thin_cuda(act, None, 1, weight2, bias2, counts, offsets, output, False)
+    return output
 
 
 def can_gather_inside_gemm(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> bool:

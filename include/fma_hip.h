@@ -253,6 +253,15 @@ int fma_grouped_gemm_gathered(const void* x, int64_t x_rows, const int32_t* row_
                               const void* bias, void* out, void* act, const uint32_t* M_arr, int64_t E, int64_t N,
                               int64_t K, int swiglu, int dtype, void* stream);
 
+/* The forward product for groups of a few rows each (a decode step): out_e = x_e W_e^T (+ bias_e), with swiglu (N = 2 I)
+ * out = swiglu_packed of it, [R, I]. Rows packed (row_index NULL) or picked as x[row_index[i] / divisor]. counts and offsets
+ * (inclusive) as fma_moe_build_index returns them, R their total. Same results, bit for bit, as fma_grouped_gemm_ragged,
+ * fma_grouped_gemm_swiglu and fma_grouped_gemm_gathered; any group size is computed, groups of more than 64 rows stream
+ * their weights once per 64 rows. Same references as fma_grouped_gemm_gathered. */
+int fma_grouped_gemm_thin(const void* x, int64_t x_rows, const int32_t* row_index, int32_t divisor, const void* W,
+                          const void* bias, void* out, const uint32_t* counts, const uint32_t* offsets, int64_t R,
+                          int64_t E, int64_t N, int64_t K, int swiglu, int dtype, void* stream);
+
 /* The weight gradient of an expert projection with the gather of the routed rows inside the operand load: for each
  * expert e with K_e rows (packed rows i of all experts back to back, R = sum K_e)
  *   dW_e[M, N] = alpha * dy_e[K_e, M]^T * xg_e[K_e, N],   xg[i, :] = x[row_index[i] / divisor, :]
