@@ -98,6 +98,31 @@ __device__ __forceinline__ void buffer_load_lds_quiet(u32x4 rsrc, uint32_t voff,
                  : "=&s"(saved_m0)
                  : "v"(voff), "s"(uniform(rsrc)), "s"(uniform(soff)), "s"(uniform(lds_addr)));
 }
+// The same load as a compiler fence, for kernels that read what it fills with ordinary LDS reads: nothing moves across it, and the
+// wait for it is wait_vm. STREAM: with the non-temporal hint.
+template <bool STREAM>
+__device__ __forceinline__ void load_lds(u32x4 rsrc, uint32_t voff, uint32_t soff, uint32_t lds_addr) {
+    uint32_t saved_m0;
+    if constexpr (STREAM)
+        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %4\n\ts_nop 2\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds\n\t"
+                     "s_mov_b32 m0, %0"
+                     : "=&s"(saved_m0)
+                     : "v"(voff), "s"(uniform(rsrc)), "s"(uniform(soff)), "s"(uniform(lds_addr))
+                     : "memory");
+    else
+        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %4\n\ts_nop 2\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds\n\t"
+                     "s_mov_b32 m0, %0"
+                     : "=&s"(saved_m0)
+                     : "v"(voff), "s"(uniform(rsrc)), "s"(uniform(soff)), "s"(uniform(lds_addr))
+                     : "memory");
+}
+// at most N of this wavefront's vector-memory operations are outstanding afterwards (they complete in issue order)
+template <int N>
+__device__ __forceinline__ void wait_vm() {
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
+}
+// all LDS reads of this wavefront have returned
+__device__ __forceinline__ void wait_lds() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 // the 4-byte form of the same load (64 lanes x 4 bytes = 256 bytes of LDS per instruction)
 __device__ __forceinline__ void buffer_load_lds_quiet_b32(u32x4 rsrc, uint32_t voff, uint32_t soff, uint32_t lds_addr) {
     uint32_t saved_m0;

@@ -46,28 +46,6 @@ constexpr uint32_t kRPI = 8;   // rows per load instruction
 __device__ __forceinline__ uint32_t flip(uint32_t row) { return (row >> 1) & 7u; }
 __device__ __forceinline__ uint32_t lds_off(uint32_t row, uint32_t chunk) { return row * kKB + ((chunk ^ flip(row)) << 4); }
 
-template <int N>
-__device__ __forceinline__ void wait_vm() {
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory");
-}
-// buffer_load_lds_quiet as a compiler fence (the stage it fills is read by ordinary loads), STREAM: non-temporal
-template <bool STREAM>
-__device__ __forceinline__ void load_lds(u32x4 rsrc, uint32_t voff, uint32_t soff, uint32_t lds_addr) {
-    uint32_t saved_m0;
-    if constexpr (STREAM)
-        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %4\n\ts_nop 2\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds\n\t"
-                     "s_mov_b32 m0, %0"
-                     : "=&s"(saved_m0)
-                     : "v"(voff), "s"(uniform(rsrc)), "s"(uniform(soff)), "s"(uniform(lds_addr))
-                     : "memory");
-    else
-        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %4\n\ts_nop 2\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds\n\t"
-                     "s_mov_b32 m0, %0"
-                     : "=&s"(saved_m0)
-                     : "v"(voff), "s"(uniform(rsrc)), "s"(uniform(soff)), "s"(uniform(lds_addr))
-                     : "memory");
-}
-
 template <int ROWS>
 struct Config;
 template <>
@@ -147,7 +125,7 @@ __device__ __forceinline__ void unit(const Args& a, uint8_t* lds, uint32_t e, ui
     const uint32_t r16 = lane & 15u, q = lane >> 4;
     uint32_t slot = 0, fill = kD - 1;
     for (uint32_t s = 0; s < nsteps; ++s) {
-        // the stage filled here was read in the previous iteration; those reads have returned (the products used them)
+        wait_lds();  // the stage filled here was read in the previous iteration
         issue(s + kD - 1, fill);
         fill = fill == kD - 1 ? 0 : fill + 1;
         wait_vm<kIPS*(kD - 1)>();

@@ -13,6 +13,7 @@ import torch
 from torch.library import custom_op
 
 from ... import _lib
+from ..._ops import hip_op
 from ...constants import LIBRARY_NAME
 from ...ops import grouped_gemm
 from ...utils import ensure_contiguous
@@ -357,6 +358,41 @@ def grouped_gemm_thin_cuda(
             _lib.current_stream(x.device),
         )
     _lib.check(rc, "grouped_gemm_thin_cuda")
+
+
+@hip_op("moe_decode_cuda", mutates_args={"output", "logits", "workspace"})
+def moe_decode_cuda(
+    x: torch.Tensor,
+    gate_weight: torch.Tensor,
+    weight1: torch.Tensor,
+    bias1: torch.Tensor | None,
+    weight2: torch.Tensor,
+    bias2: torch.Tensor | None,
+    top_k: int,
+    output: torch.Tensor,
+    logits: torch.Tensor,
+    workspace: torch.Tensor,
+) -> None:
+    """MoE.forward of a SwiGLU layer for a few tokens without a backward: output [T, H], router logits [T, E]
+    (fma_moe_decode)."""
+    _lib.require_gpu(x, gate_weight, weight1, bias1, weight2, bias2, output, logits, workspace)
+    T, H = x.shape
+    E, N, K = weight1.shape
+    I = N // 2
+    assert N % 2 == 0 and K == H and gate_weight.shape == (E, H) and weight2.shape == (E, H, I)
+    assert output.shape == (T, H) and logits.shape == (T, E)
+    assert x.dtype == gate_weight.dtype == weight1.dtype == weight2.dtype == output.dtype == logits.dtype
+    assert bias1 is None or (bias1.shape == (E, N) and bias1.dtype == x.dtype)
+    assert bias2 is None or (bias2.shape == (E, H) and bias2.dtype == x.dtype)
+    for t in (x, gate_weight, weight1, bias1, weight2, bias2, output, logits, workspace):
+        assert t is None or t.is_contiguous()
+    with torch.cuda.device(x.device):
+        rc = _lib.load().fma_moe_decode(
+            x.data_ptr(), gate_weight.data_ptr(), weight1.data_ptr(), _lib.ptr(bias1), weight2.data_ptr(), _lib.ptr(bias2),
+            T, H, I, E, top_k, output.data_ptr(), logits.data_ptr(), workspace.data_ptr(), workspace.numel(),
+            _lib.dtype_code(x.dtype), _lib.current_stream(x.device),
+        )
+    _lib.check(rc, "moe_decode_cuda")
 
 
 @custom_op(f"{LIBRARY_NAME}::expert_bias_add_cuda", mutates_args={"y"})
@@ -949,6 +985,24 @@ def thin_swiglu_experts(
     grouped_gemm_thin_cuda(x, perm, top_k, weight1, bias1, counts, offsets, act, True)
     grouped_gemm_thin_cuda(act, None, 1, weight2, bias2, counts, offsets, output, False)
     return output
+
+
+MAX_DECODE_ROWS, MAX_DECODE_EXPERTS = 1024, 256  # limits of fma_moe_decode
+
+
+@torch.no_grad()
+def moe_decode(
+    x: torch.Tensor, gate_weight: torch.Tensor, weight1: torch.Tensor, bias1: torch.Tensor | None, weight2: torch.Tensor,
+    bias2: torch.Tensor | None, top_k: int,
+) -> tuple[torch.Tensor, torch.Tensor]:  # fmt: skip
+    """(output, router logits) of the layer for a few tokens"""
+    T, H = x.shape
+    E = weight1.size(0)
+    output, logits = torch.empty_like(x), x.new_empty(T, E)
+    nbytes = _lib.load().fma_moe_decode_workspace_bytes(T, H, weight2.size(2), E, top_k)
+    workspace = x.new_empty(nbytes, dtype=torch.uint8)
+    moe_decode_cuda(x, gate_weight, weight1, bias1, weight2, bias2, top_k, output, logits, workspace)
+    return output, logits
 
 
 def can_gather_inside_gemm(x: torch.Tensor, weight: torch.Tensor, bias: torch.Tensor | None) -> bool:

@@ -43,6 +43,9 @@ extern "C" {
 #define FMA_MAX_GROUPS 1024
 /* largest top_k of the fused router */
 #define FMA_MAX_ROUTER_TOP_K 64
+/* limits of the one-call forward for a few tokens: (token, choice) slots and experts */
+#define FMA_MAX_DECODE_ROWS 1024
+#define FMA_MAX_DECODE_EXPERTS 256
 /* longest row of the normalisation kernels (the reference's MAX_TRITON_BLOCK_SIZE, fma/constants.py:17) */
 #define FMA_MAX_NORM_HIDDEN 65536
 
@@ -261,6 +264,22 @@ int fma_grouped_gemm_gathered(const void* x, int64_t x_rows, const int32_t* row_
 int fma_grouped_gemm_thin(const void* x, int64_t x_rows, const int32_t* row_index, int32_t divisor, const void* W,
                           const void* bias, void* out, const uint32_t* counts, const uint32_t* offsets, int64_t R,
                           int64_t E, int64_t N, int64_t K, int swiglu, int dtype, void* stream);
+
+/* Router and routing index of a few tokens in two launches: logits [T, E] and weights [T, k] as fma_router_topk, counts,
+ * offsets, perm and inv as fma_moe_build_index of its choice (same bits). T * top_k <= FMA_MAX_DECODE_ROWS,
+ * E <= FMA_MAX_DECODE_EXPERTS. */
+int fma_router_topk_index(const void* x, const void* gate_weight, int64_t T, int64_t H, int64_t E, int64_t top_k,
+                          void* logits, void* weights, uint32_t* counts, uint32_t* offsets, int32_t* perm, int32_t* inv,
+                          int dtype, void* stream);
+
+/* MoE.forward (fma/modules/moe/__init__.py:165-298) of a SwiGLU layer for a few tokens without a backward, enqueued by one
+ * call: fma_router_topk_index, fma_grouped_gemm_thin for both projections, fma_combine. W1 [E, 2 I, H], W2 [E, H, I], biases
+ * [E, 2 I] / [E, H] or NULL; y [T, H] and logits [T, E] are written. The limits of fma_router_topk_index; the workspace needs no
+ * initialisation. */
+int64_t fma_moe_decode_workspace_bytes(int64_t T, int64_t H, int64_t I, int64_t E, int64_t top_k);
+int fma_moe_decode(const void* x, const void* gate_weight, const void* W1, const void* bias1, const void* W2,
+                   const void* bias2, int64_t T, int64_t H, int64_t I, int64_t E, int64_t top_k, void* y, void* logits,
+                   void* workspace, int64_t workspace_bytes, int dtype, void* stream);
 
 /* The weight gradient of an expert projection with the gather of the routed rows inside the operand load: for each
  * expert e with K_e rows (packed rows i of all experts back to back, R = sum K_e)

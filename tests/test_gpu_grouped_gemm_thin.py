@@ -62,3 +62,37 @@ def test_layer_without_backward_equals_the_training_forward(T, k, E, bias):
     with torch.no_grad():
         y, logits = moe(x, kernel_backend=KernelBackend.cuda)
     assert torch.equal(logits, expect_logits) and torch.equal(y, expect)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize(
+    "T,H,E,k",
+    # one and several workgroups, partial blocks of 16 tokens and experts, the split reduction (E <= 16), one to many steps of
+    # 128 with a remainder, the most slots and experts
+    [(1, 2048, 64, 8), (1, 8, 1, 1), (16, 4096, 8, 2), (17, 136, 17, 3), (65, 512, 16, 2), (128, 4096, 128, 8), (15, 1048, 256, 64),
+     (1024, 128, 250, 1)],
+)
+def test_router_and_index_in_two_launches(T, H, E, k, dtype):
+    from fma import _lib
+
+    g = torch.Generator().manual_seed(T + H)
+    x = torch.randn(T, H, generator=g).to(dtype).to(DEV)
+    # two halves with the same experts: ties among the logits
+    w = (torch.randn(E, H, generator=g) * 0.05).to(dtype)
+    w[E // 2 :] = w[: E - E // 2].clone()
+    w = w.to(DEV)
+    expect_logits, expect_weights, selected, _ = ci.fused_router_with_histogram(x, w, k)
+    expect = ci.build_routing_index(selected, E)
+    logits, weights = torch.empty_like(expect_logits), torch.empty_like(expect_weights)
+    counts, offsets = (torch.empty(E, dtype=torch.uint32, device=DEV) for _ in range(2))
+    perm, inv = (torch.empty(T * k, dtype=torch.int32, device=DEV) for _ in range(2))
+    rc = _lib.load().fma_router_topk_index(
+        x.data_ptr(), w.data_ptr(), T, H, E, k, logits.data_ptr(), weights.data_ptr(), counts.data_ptr(), offsets.data_ptr(),
+        perm.data_ptr(), inv.data_ptr(), _lib.dtype_code(dtype), _lib.current_stream(x.device),
+    )
+    _lib.check(rc, "router_topk_index")
+    for got, want, name in zip((logits, weights, counts, offsets, perm, inv),
+                               (expect_logits, expect_weights, expect[0], expect[1], expect[2], expect[4]),
+                               ("logits", "weights", "counts", "offsets", "perm", "inv")):
+        assert torch.equal(got.view(torch.int32) if got.dtype == torch.uint32 else got,
+                           want.view(torch.int32) if want.dtype == torch.uint32 else want), name
