@@ -5,11 +5,11 @@
 // ramp-up, and the kernels for many tokens put a small batch on one or two compute units. The router's product (router.hip)
 // gives every 16 to 64 tokens ONE workgroup, which then fetches the whole router matrix through one compute unit's address path
 // (64 x 2048: 16 us, 128 x 4096: 46 us), and the index build behind it is two more launches of 4 to 8 us.
-//  * router_logits_kernel: a workgroup per 16 tokens x 16 experts, operands by direct global -> LDS loads of whole lines into a
-//    ring that keeps up to 56 KB in flight; the same sums in the same order as router.hip (for up to 16 experts: four wavefronts
+//  * router_logits_kernel: a workgroup per 16 tokens x 16 experts, operands by direct global -> LDS loads of whole lines, 128 KB
+//    in flight; the same sums in the same order as router.hip (for up to 16 experts: four wavefronts
 //    with every fourth step each, partial sums added in that order), so logits and choice have the same bits.
 //  * topk_index_kernel: ONE workgroup turns the logits of up to 1024 (token, choice) slots into weights, choice, counts, offsets
-//    and both permutations: keys, choices, histograms and ranks never leave LDS. It replaces the top-k tail of the router, the
+//    and both permutations: keys stay in registers, choices, histograms and ranks in LDS. It replaces the top-k tail of the router, the
 //    scan and the placement.
 #include "gemm_parts.h"
 #include "router_parts.h"
@@ -18,21 +18,21 @@ namespace fmahip {
 namespace {
 
 constexpr uint32_t kRowBytes = kStepK * 2;  // bytes of a row per step
-constexpr uint32_t kStageBytes = 32 * kRowBytes;
-constexpr int kLoads = 8;  // load instructions per stage: four rows each
+constexpr uint32_t kStepBytes = 32 * kRowBytes;
+constexpr int kBatch = 8;  // steps per batch; two batches (128 KB) in LDS
 
 // LDS position of 16-byte chunk c of row r (16 chunks per row): the sixteen rows of a fragment read take sixteen columns
 __device__ __forceinline__ uint32_t chunk_off(uint32_t r, uint32_t c) { return r * kRowBytes + ((c ^ (r & 15u)) << 4); }
 
-// SPLIT: four wavefronts share the reduction (step s belongs to wavefront s % 4); otherwise one wavefront runs all of it
+// One workgroup per 16 tokens x 16 experts. Four wavefronts fetch, 16 of the 64 load instructions of a batch each (a step: 16
+// token rows and 16 expert rows of 256 bytes, four rows per instruction), two batches in flight: up to a row of 2048 elements is
+// one trip to memory, however cold. SPLIT: step s is multiplied by wavefront s % 4; otherwise by the first, in order.
 template <typename EL, bool SPLIT>
-__global__ __launch_bounds__(SPLIT ? 256 : 64) void router_logits_kernel(const RouterArgs a) {
+__global__ __launch_bounds__(256) void router_logits_kernel(const RouterArgs a) {
     using frag = typename EL::frag;
-    constexpr int kWaves = SPLIT ? 4 : 1;
-    constexpr int kD = SPLIT ? 4 : 8;  // stages per wavefront: 128 KB, 64 KB
-    __shared__ __attribute__((aligned(1024))) uint8_t s_ring[kWaves][kD * kStageBytes];
+    __shared__ __attribute__((aligned(1024))) uint8_t s_steps[2][kBatch * kStepBytes];
     __shared__ float s_part[SPLIT ? 4 : 1][kTok][16];
-    const uint32_t lane = threadIdx.x & 63u, wave = SPLIT ? threadIdx.x >> 6 : 0u;
+    const uint32_t lane = threadIdx.x & 63u, wave = gemm::uniform(threadIdx.x >> 6);
     const uint32_t tok0 = blockIdx.x * kTok, e0 = blockIdx.y * 16u;
     const uint32_t H2 = (uint32_t)a.H * 2u;
     const uint32_t toks = (uint32_t)a.T - tok0 < 16u ? (uint32_t)a.T - tok0 : 16u;
@@ -41,38 +41,47 @@ __global__ __launch_bounds__(SPLIT ? 256 : 64) void router_logits_kernel(const R
     const gemm::u32x4 rx = gemm::make_rsrc_words(a.x + (uint64_t)tok0 * a.H, toks * H2);
     const gemm::u32x4 rw = gemm::make_rsrc_words(a.w + (uint64_t)e0 * a.H, exps * H2);
     const uint32_t lr = lane >> 4, lp = lane & 15u;
-    uint8_t* ring = s_ring[wave];
-    const uint32_t ring0 = gemm::lds_address(ring);
-    const uint32_t nsteps = (H2 + kRowBytes - 1) / kRowBytes;
-    const uint32_t mine = (nsteps + kWaves - 1 - wave) / kWaves;  // steps of this wavefront
+    const uint32_t nbatch = (H2 + kBatch * kRowBytes - 1) / (kBatch * kRowBytes);
 
-    auto issue = [&](uint32_t i, uint32_t slot) {
-        const uint32_t kb = (wave + kWaves * i) * kRowBytes;
-        const bool last = kb + kRowBytes > H2;
+    // wavefronts 0 and 1 fetch the token rows, 2 and 3 the expert rows, eight rows of every step each
+    const gemm::u32x4 src = wave < 2 ? rx : rw;
+    const uint32_t half = (wave & 1u) * 8u;
+    auto issue = [&](uint32_t b) {
+        const uint32_t lds0 = gemm::lds_address(s_steps[b & 1u]) + wave * (kStepBytes / 4);
 #pragma unroll
-        for (uint32_t l = 0; l < kLoads; ++l) {
-            const uint32_t row = (l & 3u) * 4u;
-            const uint32_t chunk = lp ^ ((row + lr) & 15u);
-            uint32_t v = lr * H2 + chunk * 16u;
-            if (last && kb + chunk * 16u >= H2) v = gemm::kOutOfRange;
-            gemm::load_lds<false>(l < 4 ? rx : rw, v, row * H2 + kb, ring0 + slot * kStageBytes + l * 1024u);
+        for (uint32_t s = 0; s < kBatch; ++s) {
+            const uint32_t kb = (b * kBatch + s) * kRowBytes;
+#pragma unroll
+            for (uint32_t l = 0; l < 2; ++l) {
+                const uint32_t row = half + l * 4u;
+                const uint32_t chunk = lp ^ ((row + lr) & 15u);
+                const uint32_t v = kb + chunk * 16u < H2 ? lr * H2 + chunk * 16u : gemm::kOutOfRange;
+                gemm::load_lds<false>(src, v, row * H2 + kb, lds0 + s * kStepBytes + l * 1024u);
+            }
         }
     };
     f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int d = 0; d < kD - 1; ++d) issue((uint32_t)d, (uint32_t)d);
     const uint32_t r = lane & 15u, q = lane >> 4;
-    for (uint32_t i = 0; i < mine; ++i) {
-        gemm::wait_lds();  // the stage filled here was read in the previous iteration
-        issue(i + kD - 1, (i + kD - 1) % kD);
-        gemm::wait_vm<kLoads*(kD - 1)>();
-        const uint8_t* stage = ring + (i % kD) * kStageBytes;
+    issue(0);
+    issue(1);
+    for (uint32_t b = 0; b < nbatch; ++b) {
+        gemm::wait_vm<2 * kBatch>();
+        __syncthreads();
+        const uint8_t* steps = s_steps[b & 1u];
 #pragma unroll
-        for (uint32_t j = 0; j < 4; ++j) {
-            const frag xf = load_frag<frag>(reinterpret_cast<const uint16_t*>(stage + chunk_off(r, q * 4u + j)));
-            const frag wf = load_frag<frag>(reinterpret_cast<const uint16_t*>(stage + 16 * kRowBytes + chunk_off(r, q * 4u + j)));
-            acc = EL::mfma(xf, wf, acc);
+        for (uint32_t s = 0; s < kBatch; ++s) {
+            if (SPLIT ? (s & 3u) != wave : wave != 0) continue;
+            const uint8_t* stage = steps + s * kStepBytes;
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) {
+                const frag xf = load_frag<frag>(reinterpret_cast<const uint16_t*>(stage + chunk_off(r, q * 4u + j)));
+                const frag wf = load_frag<frag>(reinterpret_cast<const uint16_t*>(stage + 16 * kRowBytes + chunk_off(r, q * 4u + j)));
+                acc = EL::mfma(xf, wf, acc);
+            }
         }
+        gemm::wait_lds();
+        __syncthreads();
+        issue(b + 2);  // past the end of the rows: zeros, so that the count above holds
     }
     gemm::wait_vm<0>();
     // a lane holds tokens 4 q .. 4 q + 3 of expert r
@@ -83,7 +92,7 @@ __global__ __launch_bounds__(SPLIT ? 256 : 64) void router_logits_kernel(const R
         const uint32_t tok = threadIdx.x >> 4, c = threadIdx.x & 15u;
         const float v = (s_part[0][tok][c] + s_part[1][tok][c]) + (s_part[2][tok][c] + s_part[3][tok][c]);
         if (tok < toks && c < exps) a.logits[(uint64_t)(tok0 + tok) * a.E + e0 + c] = EL::bits(v);
-    } else {
+    } else if (wave == 0) {
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const uint32_t tok = q * 4 + i;
@@ -97,12 +106,12 @@ constexpr int kIndexWaves = kIndexThreads / kWave;
 constexpr int kIndexTokens = kIndexThreads / 16;  // tokens whose top-k runs at the same time
 static_assert(FMA_MAX_DECODE_ROWS == kIndexThreads, "a thread per (token, choice) slot");
 
-template <typename EL>
+// NK = ceil(E / 16), rounded up to a power of two: keys per lane
+template <typename EL, int NK>
 __global__ __launch_bounds__(kIndexThreads) void topk_index_kernel(RouterArgs a, uint32_t nbits, uint32_t* __restrict__ counts,
                                                                    uint32_t* __restrict__ offsets, int32_t* __restrict__ perm,
                                                                    int32_t* __restrict__ inv) {
     constexpr int kEMax = FMA_MAX_DECODE_EXPERTS;
-    __shared__ uint32_t s_key[kIndexTokens][kEMax + kRowPad];
     __shared__ int32_t s_sel[kIndexThreads];
     __shared__ uint32_t s_cnt[kIndexWaves][kEMax];  // slots of each wavefront per expert, then where they start
     __shared__ uint32_t s_tot[kEMax / kWave];
@@ -116,11 +125,13 @@ __global__ __launch_bounds__(kIndexThreads) void topk_index_kernel(RouterArgs a,
         if (t0 + (tid >> 6) * 4u >= (uint32_t)a.T) break;  // no token for this wavefront
         const uint32_t token = t0 + (tid >> 4);
         const uint32_t from = token < (uint32_t)a.T ? token : (uint32_t)a.T - 1u;  // (real keys; nothing is stored for it)
-        uint32_t* const row = s_key[tid >> 4];
-        for (uint32_t n = c; n < E; n += 16) row[n] = make_key<EL>(a.logits[(uint64_t)from * E + n], (int)n);
-        uint32_t* const rows[1] = {row};
-        const int64_t tokens[1] = {(int64_t)token};
-        topk_softmax_tokens<EL, 1>(rows, (int)c, tokens, 0, a, nullptr);
+        uint32_t keys[NK];
+#pragma unroll
+        for (int i = 0; i < NK; ++i) {
+            const uint32_t n = c + 16u * i;
+            keys[i] = n < E ? make_key<EL>(a.logits[(uint64_t)from * E + n], (int)n) : 0u;
+        }
+        topk_softmax_in_registers<EL, NK>(keys, (int)c, (int64_t)token, a);
     }
     for (uint32_t i = tid; i < (uint32_t)kIndexWaves * E; i += kIndexThreads) s_cnt[i / E][i % E] = 0;
     __syncthreads();
@@ -168,12 +179,19 @@ template <typename EL>
 int launch_router_index(const RouterArgs& a, uint32_t* counts, uint32_t* offsets, int32_t* perm, int32_t* inv, hipStream_t st) {
     const dim3 grid((uint32_t)((a.T + kTok - 1) / kTok), (uint32_t)((a.E + 15) / 16));
     if (a.E <= 16) hipLaunchKernelGGL((router_logits_kernel<EL, true>), grid, dim3(256), 0, st, a);
-    else hipLaunchKernelGGL((router_logits_kernel<EL, false>), grid, dim3(64), 0, st, a);
+    else hipLaunchKernelGGL((router_logits_kernel<EL, false>), grid, dim3(256), 0, st, a);
     int rc = launch_status("router_topk_index (logits)");
     if (rc) return rc;
     uint32_t nbits = 0;
     while ((1u << nbits) < (uint32_t)a.E) ++nbits;
-    hipLaunchKernelGGL(topk_index_kernel<EL>, dim3(1), dim3(kIndexThreads), 0, st, a, nbits, counts, offsets, perm, inv);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(1), dim3(kIndexThreads), 0, st, a, nbits, counts, offsets, perm, inv);
+    };
+    if (a.E <= 16) launch(topk_index_kernel<EL, 1>);
+    else if (a.E <= 32) launch(topk_index_kernel<EL, 2>);
+    else if (a.E <= 64) launch(topk_index_kernel<EL, 4>);
+    else if (a.E <= 128) launch(topk_index_kernel<EL, 8>);
+    else launch(topk_index_kernel<EL, 16>);
     return launch_status("router_topk_index (top-k and index)");
 }
 

@@ -101,6 +101,40 @@ __device__ __forceinline__ float row16_sum(float v) {
     return v;
 }
 
+// Weights of NR tokens by the 16 lanes of a DPP row from their sorted choices: choice j is the key mine[t][j / 16] of lane j % 16,
+// first[t] the first of them (the largest logit) in every lane.
+template <typename EL, int NR>
+__device__ __forceinline__ void softmax_tokens(const uint32_t (&mine)[NR][kMaxTopK / 16], const uint32_t (&first)[NR], int c,
+                                               const int64_t (&token)[NR], const int64_t tok0, const RouterArgs& a,
+                                               uint32_t* s_hist) {
+    const int E = a.E, k = a.k;
+#pragma unroll
+    for (int t = 0; t < NR; ++t) {
+        const float vmax = key_value<EL>(first[t]);
+        float e[kMaxTopK / 16];
+        float sum = 0.f;
+#pragma unroll
+        for (int i = 0; i < kMaxTopK / 16; ++i) {
+            e[i] = c + 16 * i < k ? expf(key_value<EL>(mine[t][i]) - vmax) : 0.f;
+            sum += e[i];
+        }
+        sum = row16_sum(sum);
+        if (token[t] < a.T) {
+#pragma unroll
+            for (int i = 0; i < kMaxTopK / 16; ++i) {
+                const int j = c + 16 * i;
+                if (j < k) {
+                    const int col = key_column(mine[t][i]);
+                    a.selected[token[t] * k + j] = col;
+                    a.weights[token[t] * k + j] = EL::bits(e[i] / sum);
+                    if (a.counts || a.hist) atomicAdd(&s_hist[(int)((token[t] - tok0) >> 4) * E + col], 1u);
+                }
+            }
+        }
+    }
+}
+
+
 // Top-k and softmax of NR tokens at once by the 16 lanes of a DPP row (the NR chains of dependent reductions are
 // independent of each other, which is what hides their latency); keys[t] is token t's row of sort keys in LDS, of which
 // lane c owns (reads, and clears when chosen) the columns congruent to c mod 16. Choice j is remembered by lane
@@ -136,30 +170,29 @@ __device__ __forceinline__ void topk_softmax_tokens(uint32_t* const (&keys)[NR],
                 if (c == (j & 15) && (j >> 4) == i) mine[t][i] = best[t];
         }
     }
+    softmax_tokens<EL, NR>(mine, first, c, token, tok0, a, s_hist);
+}
+
+// The same for one token whose keys are in registers: lane c holds the keys of the columns congruent to c mod 16 (0 where there
+// is none), NK = ceil(E / 16) of them.
+template <typename EL, int NK>
+__device__ __forceinline__ void topk_softmax_in_registers(uint32_t (&keys)[NK], int c, int64_t token, const RouterArgs& a) {
+    uint32_t mine[1][kMaxTopK / 16] = {};
+    uint32_t first[1] = {0};
+    for (int j = 0; j < a.k; ++j) {
+        uint32_t best = keys[0];
 #pragma unroll
-    for (int t = 0; t < NR; ++t) {
-        const float vmax = key_value<EL>(first[t]);
-        float e[kMaxTopK / 16];
-        float sum = 0.f;
+        for (int i = 1; i < NK; ++i) best = max(best, keys[i]);
+        best = row16_max(best);  // top_k <= E: a real key, and no two keys are equal
 #pragma unroll
-        for (int i = 0; i < kMaxTopK / 16; ++i) {
-            e[i] = c + 16 * i < k ? expf(key_value<EL>(mine[t][i]) - vmax) : 0.f;
-            sum += e[i];
-        }
-        sum = row16_sum(sum);
-        if (token[t] < a.T) {
+        for (int i = 0; i < NK; ++i) keys[i] = keys[i] == best ? 0u : keys[i];
+        if (j == 0) first[0] = best;
 #pragma unroll
-            for (int i = 0; i < kMaxTopK / 16; ++i) {
-                const int j = c + 16 * i;
-                if (j < k) {
-                    const int col = key_column(mine[t][i]);
-                    a.selected[token[t] * k + j] = col;
-                    a.weights[token[t] * k + j] = EL::bits(e[i] / sum);
-                    if (a.counts || a.hist) atomicAdd(&s_hist[(int)((token[t] - tok0) >> 4) * E + col], 1u);
-                }
-            }
-        }
+        for (int i = 0; i < kMaxTopK / 16; ++i)
+            if (c == (j & 15) && (j >> 4) == i) mine[0][i] = best;
     }
+    const int64_t tokens[1] = {token};
+    softmax_tokens<EL, 1>(mine, first, c, tokens, 0, a, nullptr);
 }
 
 }  // namespace
