@@ -6,6 +6,7 @@ pointers, sizes and the current HIP stream. There is no fallback: if the library
 a RuntimeError is raised.
 """
 
+import contextlib
 import ctypes
 import os
 import threading
@@ -124,5 +125,14 @@ def require_gpu(*tensors: torch.Tensor) -> None:
             raise RuntimeError("this op runs on the GPU only: got a tensor on " + str(t.device))
 
 
+_STAY = contextlib.nullcontext()
+
+
+def on_device(device: torch.device):
+    """torch.cuda.device(device), without its cost (2 us) where that is the current device already"""
+    return _STAY if torch.cuda.current_device() == device.index else torch.cuda.device(device)
+
+
 def current_stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    # the handle of torch.cuda.current_stream(device) without the Stream object around it
+    return torch._C._cuda_getCurrentRawStream(device.index)

@@ -10,11 +10,9 @@ ungroup row movement) and for the row kernels of fma/modules/moe/triton_implemen
 """
 
 import torch
-from torch.library import custom_op
 
 from ... import _lib
 from ..._ops import hip_op
-from ...constants import LIBRARY_NAME
 from ...ops import grouped_gemm
 from ...utils import ensure_contiguous
 
@@ -22,7 +20,7 @@ from ...utils import ensure_contiguous
 # ---- custom ops ---------------------------------------------------------------------------------
 
 
-@custom_op(f"{LIBRARY_NAME}::moe_build_index_cuda", mutates_args={"counts", "offsets", "perm", "eid", "inv"})
+@hip_op("moe_build_index_cuda", mutates_args={"counts", "offsets", "perm", "eid", "inv"})
 def moe_build_index_cuda(
     ids: torch.Tensor,
     counts: torch.Tensor,
@@ -38,7 +36,7 @@ def moe_build_index_cuda(
     R, E = ids.numel(), counts.numel()
     assert perm.numel() == eid.numel() == inv.numel() == R and offsets.numel() == E
     lib = _lib.load()
-    with torch.cuda.device(ids.device):
+    with _lib.on_device(ids.device):
         # per-chunk histograms; scratch owned by this call (the op body is opaque to tracing, so the size query
         # and the allocation may live here)
         nbytes = max(lib.fma_moe_build_index_workspace_bytes(R, E), 4)
@@ -50,10 +48,7 @@ def moe_build_index_cuda(
     _lib.check(rc, "moe_build_index_cuda")
 
 
-@custom_op(
-    f"{LIBRARY_NAME}::moe_build_index_from_hist_cuda",
-    mutates_args={"token_block_hist", "counts", "offsets", "perm", "eid", "inv"},
-)
+@hip_op("moe_build_index_from_hist_cuda", mutates_args={"token_block_hist", "counts", "offsets", "perm", "eid", "inv"})
 def moe_build_index_from_hist_cuda(
     ids: torch.Tensor,
     top_k: int,
@@ -74,7 +69,7 @@ def moe_build_index_from_hist_cuda(
     assert perm.numel() == eid.numel() == inv.numel() == R and offsets.numel() == E and R % top_k == 0
     assert token_block_hist.dtype == torch.uint32 and token_block_hist.is_contiguous()
     assert token_block_hist.shape == ((R // top_k + 15) // 16, E)
-    with torch.cuda.device(ids.device):
+    with _lib.on_device(ids.device):
         rc = _lib.load().fma_moe_build_index_from_hist(
             ids.data_ptr(), R, E, top_k, _lib.ptr(token_block_hist), counts.data_ptr(), offsets.data_ptr(),
             perm.data_ptr(), eid.data_ptr(), inv.data_ptr(), _lib.current_stream(ids.device),
@@ -82,13 +77,13 @@ def moe_build_index_from_hist_cuda(
     _lib.check(rc, "moe_build_index_from_hist_cuda")
 
 
-@custom_op(f"{LIBRARY_NAME}::gather_rows_cuda", mutates_args={"output"})
+@hip_op("gather_rows_cuda", mutates_args={"output"})
 def gather_rows_cuda(x: torch.Tensor, idx: torch.Tensor, divisor: int, output: torch.Tensor) -> None:
     _lib.require_gpu(x, idx, output)
     assert x.dim() == 2 and output.dim() == 2 and x.size(1) == output.size(1) and x.dtype == output.dtype
     assert idx.dtype == torch.int32 and idx.numel() == output.size(0)  # x may have more rows than are gathered
     assert x.is_contiguous() and output.is_contiguous() and idx.is_contiguous()
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         rc = _lib.load().fma_gather_rows(
             x.data_ptr(), idx.data_ptr(), output.size(0), x.size(1), divisor, output.data_ptr(),
             _lib.dtype_code(x.dtype), _lib.current_stream(x.device),
@@ -96,7 +91,7 @@ def gather_rows_cuda(x: torch.Tensor, idx: torch.Tensor, divisor: int, output: t
     _lib.check(rc, "gather_rows_cuda")
 
 
-@custom_op(f"{LIBRARY_NAME}::dispatch_rows_cuda", mutates_args={"output"})
+@hip_op("dispatch_rows_cuda", mutates_args={"output"})
 def dispatch_rows_cuda(x: torch.Tensor, inv: torch.Tensor, top_k: int, output: torch.Tensor) -> None:
     _lib.require_gpu(x, inv, output)
     T, H = x.shape
@@ -104,7 +99,7 @@ def dispatch_rows_cuda(x: torch.Tensor, inv: torch.Tensor, top_k: int, output: t
     assert output.dim() == 2 and output.size(0) >= T * top_k and output.size(1) == H and x.dtype == output.dtype
     assert inv.dtype == torch.int32 and inv.numel() == T * top_k
     assert x.is_contiguous() and output.is_contiguous() and inv.is_contiguous()
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         rc = _lib.load().fma_dispatch_rows(
             x.data_ptr(), inv.data_ptr(), T, top_k, H, output.data_ptr(), _lib.dtype_code(x.dtype),
             _lib.current_stream(x.device),
@@ -112,7 +107,7 @@ def dispatch_rows_cuda(x: torch.Tensor, inv: torch.Tensor, top_k: int, output: t
     _lib.check(rc, "dispatch_rows_cuda")
 
 
-@custom_op(f"{LIBRARY_NAME}::combine_cuda", mutates_args={"output"})
+@hip_op("combine_cuda", mutates_args={"output"})
 def combine_cuda(
     o: torch.Tensor, inv: torch.Tensor, gates: torch.Tensor | None, top_k: int, output: torch.Tensor
 ) -> None:
@@ -122,7 +117,7 @@ def combine_cuda(
     assert inv.dtype == torch.int32 and inv.numel() == T * top_k
     assert gates is None or (gates.dtype == o.dtype and gates.numel() == T * top_k and gates.is_contiguous())
     assert o.is_contiguous() and output.is_contiguous() and inv.is_contiguous()
-    with torch.cuda.device(o.device):
+    with _lib.on_device(o.device):
         rc = _lib.load().fma_combine(
             o.data_ptr(), inv.data_ptr(), _lib.ptr(gates), T, top_k, H, output.data_ptr(), _lib.dtype_code(o.dtype),
             _lib.current_stream(o.device),
@@ -130,7 +125,7 @@ def combine_cuda(
     _lib.check(rc, "combine_cuda")
 
 
-@custom_op(f"{LIBRARY_NAME}::combine_backward_cuda", mutates_args={"o_grad", "gates_grad"})
+@hip_op("combine_backward_cuda", mutates_args={"o_grad", "gates_grad"})
 def combine_backward_cuda(
     output_grad: torch.Tensor,
     o: torch.Tensor,
@@ -149,7 +144,7 @@ def combine_backward_cuda(
         assert t is None or t.is_contiguous()
     assert gates is None or gates.dtype == o.dtype
     assert gates_grad is None or (gates_grad.dtype == o.dtype and gates_grad.numel() == T * top_k)
-    with torch.cuda.device(o.device):
+    with _lib.on_device(o.device):
         rc = _lib.load().fma_combine_bwd(
             output_grad.data_ptr(), o.data_ptr(), inv.data_ptr(), _lib.ptr(gates), T, top_k, H, o_grad.data_ptr(),
             _lib.ptr(gates_grad), _lib.dtype_code(o.dtype), _lib.current_stream(o.device),
@@ -157,7 +152,7 @@ def combine_backward_cuda(
     _lib.check(rc, "combine_backward_cuda")
 
 
-@custom_op(f"{LIBRARY_NAME}::grouped_gemm_ragged_cuda", mutates_args={"output"})
+@hip_op("grouped_gemm_ragged_cuda", mutates_args={"output"})
 def grouped_gemm_ragged_cuda(
     A: torch.Tensor, B: torch.Tensor, output: torch.Tensor, sizes: torch.Tensor, vary_k: bool, M: int, N: int, K: int,
     is_A_transposed: bool, is_B_transposed: bool, bias: torch.Tensor | None = None,
@@ -175,7 +170,7 @@ def grouped_gemm_ragged_cuda(
     # an operand without elements is never read, but the entry point rejects NULL: any valid device address stands in
     a_ptr = A.data_ptr() if A.numel() else output.data_ptr()
     b_ptr = B.data_ptr() if B.numel() else output.data_ptr()
-    with torch.cuda.device(A.device):
+    with _lib.on_device(A.device):
         rc = _lib.load().fma_grouped_gemm_ragged(
             a_ptr, b_ptr, output.data_ptr(), sizes.data_ptr(), _lib.ptr(bias), sizes.numel(),
             _lib.FMA_VARY_K if vary_k else _lib.FMA_VARY_M, M, N, K, int(is_A_transposed), int(is_B_transposed), 1.0,
@@ -204,7 +199,7 @@ def _expert_gemm(
     )
 
 
-@custom_op(f"{LIBRARY_NAME}::grouped_gemm_swiglu_cuda", mutates_args={"h", "act"})
+@hip_op("grouped_gemm_swiglu_cuda", mutates_args={"h", "act"})
 def grouped_gemm_swiglu_cuda(
     x: torch.Tensor, weight: torch.Tensor, M_array: torch.Tensor, h: torch.Tensor | None, act: torch.Tensor,
     bias: torch.Tensor | None = None,
@@ -222,7 +217,7 @@ def grouped_gemm_swiglu_cuda(
         assert t is None or t.is_contiguous()
     if act.numel() == 0:
         return  # no rows routed anywhere (or no output columns): nothing to compute, and empty tensors have no address
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         rc = _lib.load().fma_grouped_gemm_swiglu(
             x.data_ptr(), weight.data_ptr(), _lib.ptr(bias), _lib.ptr(h), act.data_ptr(), M_array.data_ptr(), E, inter, K,
             _lib.dtype_code(x.dtype), _lib.current_stream(x.device),
@@ -230,7 +225,7 @@ def grouped_gemm_swiglu_cuda(
     _lib.check(rc, "grouped_gemm_swiglu_cuda")
 
 
-@custom_op(f"{LIBRARY_NAME}::grouped_gemm_swiglu_bwd_cuda", mutates_args={"h_grad"})
+@hip_op("grouped_gemm_swiglu_bwd_cuda", mutates_args={"h_grad"})
 def grouped_gemm_swiglu_bwd_cuda(
     output_grad: torch.Tensor, weight: torch.Tensor, h: torch.Tensor, M_array: torch.Tensor, h_grad: torch.Tensor
 ) -> None:
@@ -247,7 +242,7 @@ def grouped_gemm_swiglu_bwd_cuda(
         assert t.is_contiguous()
     if R == 0 or inter == 0:
         return
-    with torch.cuda.device(h.device):
+    with _lib.on_device(h.device):
         rc = _lib.load().fma_grouped_gemm_swiglu_bwd(
             output_grad.data_ptr(), weight.data_ptr(), h.data_ptr(), h_grad.data_ptr(), M_array.data_ptr(), E, inter, K,
             _lib.dtype_code(h.dtype), _lib.current_stream(h.device),
@@ -255,7 +250,7 @@ def grouped_gemm_swiglu_bwd_cuda(
     _lib.check(rc, "grouped_gemm_swiglu_bwd_cuda")
 
 
-@custom_op(f"{LIBRARY_NAME}::grouped_gemm_gathered_cuda", mutates_args={"out", "act"})
+@hip_op("grouped_gemm_gathered_cuda", mutates_args={"out", "act"})
 def grouped_gemm_gathered_cuda(
     x: torch.Tensor,
     row_index: torch.Tensor,
@@ -283,7 +278,7 @@ def grouped_gemm_gathered_cuda(
         assert t is None or t.is_contiguous()
     if R == 0 or N == 0:
         return
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         rc = _lib.load().fma_grouped_gemm_gathered(
             x.data_ptr(), x.size(0), row_index.data_ptr(), divisor, weight.data_ptr(), _lib.ptr(bias), _lib.ptr(out),
             _lib.ptr(act), M_array.data_ptr(), E, N, K, int(act is not None), _lib.dtype_code(x.dtype),
@@ -292,7 +287,7 @@ def grouped_gemm_gathered_cuda(
     _lib.check(rc, "grouped_gemm_gathered_cuda")
 
 
-@custom_op(f"{LIBRARY_NAME}::grouped_gemm_gathered_wgrad_cuda", mutates_args={"weight_grad"})
+@hip_op("grouped_gemm_gathered_wgrad_cuda", mutates_args={"weight_grad"})
 def grouped_gemm_gathered_wgrad_cuda(
     output_grad: torch.Tensor,
     x: torch.Tensor,
@@ -317,7 +312,7 @@ def grouped_gemm_gathered_wgrad_cuda(
     if R == 0:
         weight_grad.zero_()
         return
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         rc = _lib.load().fma_grouped_gemm_gathered_wgrad(
             output_grad.data_ptr(), x.data_ptr(), x.size(0), row_index.data_ptr(), divisor, weight_grad.data_ptr(),
             K_array.data_ptr(), E, N, K, 1.0, _lib.dtype_code(x.dtype), _lib.current_stream(x.device),
@@ -325,7 +320,7 @@ def grouped_gemm_gathered_wgrad_cuda(
     _lib.check(rc, "grouped_gemm_gathered_wgrad_cuda")
 
 
-@custom_op(f"{LIBRARY_NAME}::grouped_gemm_thin_cuda", mutates_args={"output"})
+@hip_op("grouped_gemm_thin_cuda", mutates_args={"output"})
 def grouped_gemm_thin_cuda(
     x: torch.Tensor,
     row_index: torch.Tensor | None,
@@ -351,7 +346,7 @@ def grouped_gemm_thin_cuda(
         assert t is None or t.is_contiguous()
     if output.numel() == 0:
         return
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         rc = _lib.load().fma_grouped_gemm_thin(
             x.data_ptr(), x.size(0), _lib.ptr(row_index), divisor, weight.data_ptr(), _lib.ptr(bias), output.data_ptr(),
             counts.data_ptr(), offsets.data_ptr(), R, E, N, K, int(swiglu), _lib.dtype_code(x.dtype),
@@ -386,7 +381,7 @@ def moe_decode_cuda(
     assert bias2 is None or (bias2.shape == (E, H) and bias2.dtype == x.dtype)
     for t in (x, gate_weight, weight1, bias1, weight2, bias2, output, logits, workspace):
         assert t is None or t.is_contiguous()
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         rc = _lib.load().fma_moe_decode(
             x.data_ptr(), gate_weight.data_ptr(), weight1.data_ptr(), _lib.ptr(bias1), weight2.data_ptr(), _lib.ptr(bias2),
             T, H, I, E, top_k, output.data_ptr(), logits.data_ptr(), workspace.data_ptr(), workspace.numel(),
@@ -395,14 +390,14 @@ def moe_decode_cuda(
     _lib.check(rc, "moe_decode_cuda")
 
 
-@custom_op(f"{LIBRARY_NAME}::expert_bias_add_cuda", mutates_args={"y"})
+@hip_op("expert_bias_add_cuda", mutates_args={"y"})
 def expert_bias_add_cuda(y: torch.Tensor, bias: torch.Tensor, M_array: torch.Tensor) -> None:
     _lib.require_gpu(y, bias, M_array)
     E, N = bias.shape
     assert y.dim() == 2 and y.size(1) == N and y.dtype == bias.dtype
     assert M_array.dtype == torch.uint32 and M_array.numel() == E
     assert y.is_contiguous() and bias.is_contiguous() and M_array.is_contiguous()
-    with torch.cuda.device(y.device):
+    with _lib.on_device(y.device):
         rc = _lib.load().fma_expert_bias_add(
             y.data_ptr(), bias.data_ptr(), M_array.data_ptr(), E, y.size(0), N, _lib.dtype_code(y.dtype),
             _lib.current_stream(y.device),
@@ -410,7 +405,7 @@ def expert_bias_add_cuda(y: torch.Tensor, bias: torch.Tensor, M_array: torch.Ten
     _lib.check(rc, "expert_bias_add_cuda")
 
 
-@custom_op(f"{LIBRARY_NAME}::expert_bias_grad_cuda", mutates_args={"bias_grad"})
+@hip_op("expert_bias_grad_cuda", mutates_args={"bias_grad"})
 def expert_bias_grad_cuda(output_grad: torch.Tensor, M_array: torch.Tensor, bias_grad: torch.Tensor) -> None:
     _lib.require_gpu(output_grad, M_array, bias_grad)
     E, N = bias_grad.shape
@@ -419,7 +414,7 @@ def expert_bias_grad_cuda(output_grad: torch.Tensor, M_array: torch.Tensor, bias
     assert output_grad.is_contiguous() and bias_grad.is_contiguous() and M_array.is_contiguous()
     lib = _lib.load()
     code = _lib.dtype_code(output_grad.dtype)
-    with torch.cuda.device(output_grad.device):
+    with _lib.on_device(output_grad.device):
         nbytes = max(lib.fma_expert_bias_grad_workspace_bytes(E, output_grad.size(0), N), 4)
         workspace = torch.empty(nbytes, dtype=torch.uint8, device=output_grad.device)  # per-slice partial sums
         rc = lib.fma_expert_bias_grad(
@@ -429,9 +424,7 @@ def expert_bias_grad_cuda(output_grad: torch.Tensor, M_array: torch.Tensor, bias
     _lib.check(rc, "expert_bias_grad_cuda")
 
 
-@custom_op(
-    f"{LIBRARY_NAME}::router_topk_cuda", mutates_args={"logits", "weights", "selected", "counts", "token_block_hist"}
-)
+@hip_op("router_topk_cuda", mutates_args={"logits", "weights", "selected", "counts", "token_block_hist"})
 def router_topk_cuda(
     x: torch.Tensor,
     gate_weight: torch.Tensor,
@@ -454,7 +447,7 @@ def router_topk_cuda(
     )
     for t in (x, gate_weight, logits, weights, selected, counts, token_block_hist):
         assert t is None or t.is_contiguous()
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         rc = _lib.load().fma_router_topk(
             x.data_ptr(), gate_weight.data_ptr(), T, H, E, top_k, logits.data_ptr(), weights.data_ptr(),
             selected.data_ptr(), _lib.ptr(counts), _lib.ptr(token_block_hist), _lib.dtype_code(x.dtype),
@@ -463,7 +456,7 @@ def router_topk_cuda(
     _lib.check(rc, "router_topk_cuda")
 
 
-@custom_op(f"{LIBRARY_NAME}::router_topk_backward_cuda", mutates_args={"logits_grad"})
+@hip_op("router_topk_backward_cuda", mutates_args={"logits_grad"})
 def router_topk_backward_cuda(
     logits: torch.Tensor,
     selected: torch.Tensor,
@@ -480,7 +473,7 @@ def router_topk_backward_cuda(
     assert logits_output_grad is None or (logits_output_grad.shape == (T, E) and logits_output_grad.dtype == logits.dtype)
     for t in (logits, selected, weights_grad, logits_output_grad, logits_grad):
         assert t is None or t.is_contiguous()
-    with torch.cuda.device(logits.device):
+    with _lib.on_device(logits.device):
         rc = _lib.load().fma_router_topk_bwd(
             logits.data_ptr(), selected.data_ptr(), _lib.ptr(weights_grad), _lib.ptr(logits_output_grad), T, E, top_k,
             logits_grad.data_ptr(), _lib.dtype_code(logits.dtype), _lib.current_stream(logits.device),

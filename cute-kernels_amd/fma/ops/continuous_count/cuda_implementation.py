@@ -2,13 +2,12 @@
 (fma/ops/continuous_count/cuda_implementation/__init__.py:12-16), bound to fma_continuous_count of libfma_hip.so."""
 
 import torch
-from torch.library import custom_op
 
 from ... import _lib
-from ...constants import LIBRARY_NAME
+from ..._ops import hip_op
 
 
-@custom_op(f"{LIBRARY_NAME}::continuous_count_cuda", mutates_args={"output"})
+@hip_op("continuous_count_cuda", mutates_args={"output"})
 def continuous_count_cuda(
     x: torch.Tensor, output: torch.Tensor, E: int, THREAD_BLOCK_CLUSTER_SIZE: int, BLOCK_SIZE: int
 ) -> None:
@@ -20,7 +19,7 @@ def continuous_count_cuda(
     x = x.contiguous()
     lib = _lib.load()
     n = x.numel()
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         # per-workgroup partial histograms; uninitialised memory from the caching allocator, owned by this call
         ws = torch.empty(max(lib.fma_continuous_count_workspace_bytes(n, E), 4), dtype=torch.uint8, device=x.device)
         rc = lib.fma_continuous_count(

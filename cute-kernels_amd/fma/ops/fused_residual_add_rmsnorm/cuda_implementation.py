@@ -3,17 +3,13 @@ reference's fused_residual_add_rmsnorm_forward_triton / fused_residual_add_rmsno
 (fma/ops/fused_residual_add_rmsnorm/triton_implementation/forward.py:64-102, backward.py:101-145)."""
 
 import torch
-from torch.library import custom_op
 
 from ... import _lib
-from ...constants import LIBRARY_NAME
+from ..._ops import hip_op
 from ...utils import get_num_elements_and_hidden_size
 
 
-@custom_op(
-    f"{LIBRARY_NAME}::fused_residual_add_rmsnorm_forward_cuda",
-    mutates_args={"output", "added_x_residual", "rmsnorm_denominator"},
-)
+@hip_op("fused_residual_add_rmsnorm_forward_cuda", mutates_args={"output", "added_x_residual", "rmsnorm_denominator"})
 def fused_residual_add_rmsnorm_forward_cuda(
     x: torch.Tensor,
     residual: torch.Tensor,
@@ -32,7 +28,7 @@ def fused_residual_add_rmsnorm_forward_cuda(
     assert rmsnorm_denominator is None or (rmsnorm_denominator.dtype == torch.float32 and rmsnorm_denominator.numel() == B)
     for t in (x, residual, weight, output, added_x_residual, rmsnorm_denominator):
         assert t is None or t.is_contiguous()
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         rc = _lib.load().fma_fused_residual_add_rmsnorm_fwd(
             x.data_ptr(), residual.data_ptr(), _lib.ptr(weight), output.data_ptr(), added_x_residual.data_ptr(),
             _lib.ptr(rmsnorm_denominator), B, H, eps, 1.0 if multiplier is None else multiplier,
@@ -41,10 +37,7 @@ def fused_residual_add_rmsnorm_forward_cuda(
     _lib.check(rc, "fused_residual_add_rmsnorm_forward_cuda")
 
 
-@custom_op(
-    f"{LIBRARY_NAME}::fused_residual_add_rmsnorm_backward_cuda",
-    mutates_args={"x_grad", "residual_grad", "weight_grad"},
-)
+@hip_op("fused_residual_add_rmsnorm_backward_cuda", mutates_args={"x_grad", "residual_grad", "weight_grad"})
 def fused_residual_add_rmsnorm_backward_cuda(
     added_x_residual: torch.Tensor,
     weight: torch.Tensor | None,
@@ -70,7 +63,7 @@ def fused_residual_add_rmsnorm_backward_cuda(
     for t in (added_x_residual, weight, output_grad, added_x_residual_grad, rmsnorm_denominator, x_grad, residual_grad, weight_grad):
         assert t is None or t.is_contiguous()
     lib = _lib.load()
-    with torch.cuda.device(added_x_residual.device):
+    with _lib.on_device(added_x_residual.device):
         # per-workgroup partial weight gradients; scratch owned by this call
         nbytes = lib.fma_fused_residual_add_rmsnorm_bwd_workspace_bytes(B, H) if weight is not None else 0
         workspace = torch.empty(max(nbytes, 4), dtype=torch.uint8, device=added_x_residual.device)

@@ -2,10 +2,9 @@
 (fma/ops/grouped_gemm/cuda_implementation/__init__.py:15-30), bound to fma_grouped_gemm of libfma_hip.so."""
 
 import torch
-from torch.library import custom_op
 
 from ... import _lib
-from ...constants import LIBRARY_NAME
+from ..._ops import hip_op
 
 
 def _launch(A, B, output, M_array, N_array, K_array, is_A_transposed, is_B_transposed, alpha) -> None:
@@ -16,7 +15,7 @@ def _launch(A, B, output, M_array, N_array, K_array, is_A_transposed, is_B_trans
     # rejects NULL: any valid device address stands in for it.
     a_ptr = A.data_ptr() if A.numel() else output.data_ptr()
     b_ptr = B.data_ptr() if B.numel() else output.data_ptr()
-    with torch.cuda.device(A.device):
+    with _lib.on_device(A.device):
         rc = lib.fma_grouped_gemm(
             a_ptr, b_ptr, output.data_ptr(), M_array.data_ptr(), N_array.data_ptr(), K_array.data_ptr(),
             M_array.numel(), int(is_A_transposed), int(is_B_transposed), float(alpha), _lib.dtype_code(A.dtype),
@@ -25,7 +24,7 @@ def _launch(A, B, output, M_array, N_array, K_array, is_A_transposed, is_B_trans
     _lib.check(rc, "grouped_gemm_cuda")
 
 
-@custom_op(f"{LIBRARY_NAME}::grouped_gemm_cuda", mutates_args={"output"})
+@hip_op("grouped_gemm_cuda", mutates_args={"output"})
 def grouped_gemm_cuda(
     A: torch.Tensor,
     B: torch.Tensor,

@@ -4,10 +4,9 @@ fma_swiglu_backward of libfma_hip.so. Unlike the reference's CUDA kernels they a
 reference needs its Triton kernels for that, fma/ops/swiglu/triton_implementation/forward.py:49-66)."""
 
 import torch
-from torch.library import custom_op
 
 from ... import _lib
-from ...constants import LIBRARY_NAME
+from ..._ops import hip_op
 
 
 def _rows_view(t: torch.Tensor) -> tuple[int, int, int] | None:
@@ -46,7 +45,7 @@ def _as_rows(t: torch.Tensor, writable: bool) -> tuple[torch.Tensor, int, int, i
     return (t,) + view
 
 
-@custom_op(f"{LIBRARY_NAME}::swiglu_forward_cuda", mutates_args={"output"})
+@hip_op("swiglu_forward_cuda", mutates_args={"output"})
 def swiglu_forward_cuda(gate: torch.Tensor, up: torch.Tensor, output: torch.Tensor, BLOCK_SIZE: int) -> None:
     _lib.require_gpu(gate, up, output)
     assert gate.shape == up.shape == output.shape
@@ -54,7 +53,7 @@ def swiglu_forward_cuda(gate: torch.Tensor, up: torch.Tensor, output: torch.Tens
     gate, rows, cols, gs = _as_rows(gate, False)
     up, _, _, us = _as_rows(up, False)
     output, _, _, os_ = _as_rows(output, True)
-    with torch.cuda.device(gate.device):
+    with _lib.on_device(gate.device):
         rc = _lib.load().fma_swiglu_forward(
             gate.data_ptr(), up.data_ptr(), output.data_ptr(), rows, cols, gs, us, os_, _lib.dtype_code(gate.dtype),
             _lib.current_stream(gate.device),
@@ -62,7 +61,7 @@ def swiglu_forward_cuda(gate: torch.Tensor, up: torch.Tensor, output: torch.Tens
     _lib.check(rc, "swiglu_forward_cuda")
 
 
-@custom_op(f"{LIBRARY_NAME}::swiglu_backward_cuda", mutates_args={"gate_grad", "up_grad"})
+@hip_op("swiglu_backward_cuda", mutates_args={"gate_grad", "up_grad"})
 def swiglu_backward_cuda(
     gate: torch.Tensor,
     up: torch.Tensor,
@@ -79,7 +78,7 @@ def swiglu_backward_cuda(
     output_grad, _, _, ds = _as_rows(output_grad, False)
     gate_grad, _, _, ggs = _as_rows(gate_grad, True)
     up_grad, _, _, ugs = _as_rows(up_grad, True)
-    with torch.cuda.device(gate.device):
+    with _lib.on_device(gate.device):
         rc = _lib.load().fma_swiglu_backward(
             gate.data_ptr(), up.data_ptr(), output_grad.data_ptr(), gate_grad.data_ptr(), up_grad.data_ptr(), rows,
             cols, gs, us, ds, ggs, ugs, _lib.dtype_code(gate.dtype), _lib.current_stream(gate.device),
