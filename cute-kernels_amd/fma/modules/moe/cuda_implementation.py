@@ -355,7 +355,7 @@ def grouped_gemm_thin_cuda(
     _lib.check(rc, "grouped_gemm_thin_cuda")
 
 
-@hip_op("moe_decode_cuda", mutates_args={"output", "logits", "workspace"})
+@hip_op("moe_decode_cuda", mutates_args={"output", "logits"})
 def moe_decode_cuda(
     x: torch.Tensor,
     gate_weight: torch.Tensor,
@@ -366,11 +366,10 @@ def moe_decode_cuda(
     top_k: int,
     output: torch.Tensor,
     logits: torch.Tensor,
-    workspace: torch.Tensor,
 ) -> None:
     """MoE.forward of a SwiGLU layer for a few tokens without a backward: output [T, H], router logits [T, E]
     (fma_moe_decode)."""
-    _lib.require_gpu(x, gate_weight, weight1, bias1, weight2, bias2, output, logits, workspace)
+    _lib.require_gpu(x, gate_weight, weight1, bias1, weight2, bias2, output, logits)
     T, H = x.shape
     E, N, K = weight1.shape
     I = N // 2
@@ -379,10 +378,13 @@ def moe_decode_cuda(
     assert x.dtype == gate_weight.dtype == weight1.dtype == weight2.dtype == output.dtype == logits.dtype
     assert bias1 is None or (bias1.shape == (E, N) and bias1.dtype == x.dtype)
     assert bias2 is None or (bias2.shape == (E, H) and bias2.dtype == x.dtype)
-    for t in (x, gate_weight, weight1, bias1, weight2, bias2, output, logits, workspace):
+    for t in (x, gate_weight, weight1, bias1, weight2, bias2, output, logits):
         assert t is None or t.is_contiguous()
+    lib = _lib.load()
     with _lib.on_device(x.device):
-        rc = _lib.load().fma_moe_decode(
+        # scratch owned by this call; the op body is opaque to tracing, so the size query and the allocation live here
+        workspace = x.new_empty(lib.fma_moe_decode_workspace_bytes(T, H, I, E, top_k), dtype=torch.uint8)
+        rc = lib.fma_moe_decode(
             x.data_ptr(), gate_weight.data_ptr(), weight1.data_ptr(), _lib.ptr(bias1), weight2.data_ptr(), _lib.ptr(bias2),
             T, H, I, E, top_k, output.data_ptr(), logits.data_ptr(), workspace.data_ptr(), workspace.numel(),
             _lib.dtype_code(x.dtype), _lib.current_stream(x.device),
@@ -967,6 +969,7 @@ def gathered_up_projection_experts(
 
 
 @torch.no_grad()
+@ensure_contiguous
 def thin_swiglu_experts(
     x: torch.Tensor, weight1: torch.Tensor, bias1: torch.Tensor | None, weight2: torch.Tensor, bias2: torch.Tensor | None,
     perm: torch.Tensor, counts: torch.Tensor, offsets: torch.Tensor, top_k: int,
@@ -989,12 +992,8 @@ def moe_decode(
     bias2: torch.Tensor | None, top_k: int,
 ) -> tuple[torch.Tensor, torch.Tensor]:  # fmt: skip
     """(output, router logits) of the layer for a few tokens"""
-    T, H = x.shape
-    E = weight1.size(0)
-    output, logits = torch.empty_like(x), x.new_empty(T, E)
-    nbytes = _lib.load().fma_moe_decode_workspace_bytes(T, H, weight2.size(2), E, top_k)
-    workspace = x.new_empty(nbytes, dtype=torch.uint8)
-    moe_decode_cuda(x, gate_weight, weight1, bias1, weight2, bias2, top_k, output, logits, workspace)
+    output, logits = torch.empty_like(x), x.new_empty(x.size(0), weight1.size(0))
+    moe_decode_cuda(x, gate_weight, weight1, bias1, weight2, bias2, top_k, output, logits)
     return output, logits
 
 

@@ -4,6 +4,7 @@ of a pass, 32 / 64 weight rows of a wavefront, 64 reduction elements of a step, 
 
 import pytest
 import torch
+from torch.autograd import forward_ad
 
 from fma.modules.moe import cuda_implementation as ci
 
@@ -62,6 +63,42 @@ def test_layer_without_backward_equals_the_training_forward(T, k, E, bias):
     with torch.no_grad():
         y, logits = moe(x, kernel_backend=KernelBackend.cuda)
     assert torch.equal(logits, expect_logits) and torch.equal(y, expect)
+
+
+@pytest.mark.parametrize("T", [7, 100, 300])  # one native call; more than 64 and than 1024 (token, choice) slots
+def test_layer_without_backward_in_other_forms(T):
+    """what the general path takes or refuses is taken or refused on the kernels for a few rows as well: tracing without a
+    graph break, weights of any strides, forward-mode AD (refused), a subclass's own expert computation"""
+    from fma import KernelBackend, MoE, swiglu_packed
+
+    torch.manual_seed(T)
+    E, k, H, I = 16, 4, 128, 64
+    moe = MoE(E, k, H, I, swiglu_packed, True, True, 0.05).to(torch.bfloat16).to(DEV)
+    x = torch.randn(T, H, device=DEV).bfloat16()
+    run = lambda m, x: m(x, kernel_backend=KernelBackend.cuda)
+    with torch.no_grad():
+        y, logits = run(moe, x)
+        for got in (torch.compile(lambda x: run(moe, x), fullgraph=True)(x),
+                    torch.compile(lambda x: run(moe, x), fullgraph=True, dynamic=True)(x)):
+            assert torch.equal(got[0], y) and torch.equal(got[1], logits)
+
+        with forward_ad.dual_level():
+            with pytest.raises(NotImplementedError):
+                run(moe, forward_ad.make_dual(x, torch.ones_like(x)))
+
+        class Doubled(MoE):
+            def _compute_experts(self, *args, **kwargs):
+                return 2 * super()._compute_experts(*args, **kwargs)
+
+        moe.__class__ = Doubled
+        assert torch.equal(run(moe, x)[0], 2 * y)  # (a power of two: exact)
+        moe.__class__ = MoE
+
+        for p in moe.parameters():
+            p.data = p.data.transpose(-1, -2).contiguous().transpose(-1, -2)
+        assert not moe.c_fc.weight.is_contiguous()
+        got = run(moe, x.t().contiguous().t().view(T, H))
+        assert torch.equal(got[0], y) and torch.equal(got[1], logits)
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
