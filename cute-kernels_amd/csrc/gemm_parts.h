@@ -28,6 +28,7 @@ constexpr int EPI_SWIGLU_ACT = 2;  // the activation only (a forward pass that n
 // the product is the gradient of a SwiGLU activation: the gradient of the packed pre-activation h is written instead
 // (columns c and I + c of a row from column c of the product), with h read in the epilogue
 constexpr int EPI_SWIGLU_BWD = 3;
+constexpr int EPI_SPLIT = 4;  // fp32 sums over a part of the reduction
 
 // ---- the two 16-bit element types: conversions and the matrix instruction ------------------------------------------
 typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;

@@ -30,6 +30,9 @@
 //    the rows of A as rows row_index[i] / divisor of the token matrix (a table of the tile's 256 entries in LDS, four
 //    per-lane offsets per K step), the weight gradient takes the reduction rows of B the same way (eight entries per
 //    wavefront and K step, requested two steps ahead). Both give the bits of the packed kernel on a gathered copy.
+#include <algorithm>
+#include <cmath>
+
 #include "gemm_parts.h"
 
 namespace fmahip {
@@ -66,6 +69,10 @@ struct Args {
     const uint32_t* m_dev;
     const uint32_t* n_dev;
     const uint32_t* k_dev;
+    // EPI_SPLIT: every tile is computed `splits` times, each time over split_steps K steps (an even number, so that only the
+    // last part can end inside a step or on an odd one); part s of packed row r goes to partial[(s * rows + r) * n ..]
+    float* partial;
+    uint32_t splits, split_steps, rows;
 };
 
 // s_waitcnt immediate: vmcnt(vm), and lgkmcnt(0) too if lgkm0 (expcnt untouched)
@@ -97,6 +104,9 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
     static_assert(!kGlu || (A_KC && B_KC && !VARY_K), "the SwiGLU epilogue exists for the NT layout only");
     static_assert(EPI != EPI_SWIGLU_BWD || (A_KC && !B_KC && !VARY_K && !BIAS && !GATHER_ANY),
                   "the SwiGLU-gradient epilogue exists for the input-gradient (NN) layout only");
+    // kSplit: fp32 sums over a part of the reduction, added up by split_reduce_kernel
+    constexpr bool kSplit = EPI == EPI_SPLIT;
+    static_assert(!kSplit || (A_KC && !VARY_K && !BIAS && !GATHER_ANY), "the reduction is split in the NT and NN layouts only");
     static_assert(!BIAS || (A_KC && B_KC && !VARY_K), "the bias term exists for the forward (NT) layout only");
     static_assert(!GATHER || (A_KC && B_KC), "rows are gathered in the forward (NT) layout only");
     static_assert(!kGatherK || (!A_KC && !B_KC && EPI == EPI_PLAIN), "reduction rows are gathered in the weight-gradient (TN) layout only");
@@ -172,7 +182,7 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
     auto group_m = [&](uint32_t e) { return VARY_K ? dim_m : sizes[e]; };
     auto group_k = [&](uint32_t e) { return VARY_K ? sizes[e] : dim_k; };
     const uint32_t Ne = dim_n;
-    constexpr bool kCanNarrow = A_KC && B_KC;
+    constexpr bool kCanNarrow = A_KC && B_KC && !kSplit;
     constexpr uint32_t kTileN = kGlu ? BN / 2 : BN;  // columns of the tile grid one tile covers
     const uint32_t n_span = kGlu ? Ne / 2 : Ne;      // columns the tile grid runs over
     bool narrow = false;
@@ -296,11 +306,19 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
         uint32_t row0;                   // first packed row (reduction row, if the reduction varies) of the group
         uint64_t off_a, off_b, off_d;
         uint32_t pf_r, pf_c;  // position of the tile in its XCD's 8 x 4 block of tiles (row, column)
+        uint32_t ks, part;    // kSplit: first K element of the tile's part of the reduction, and which part
     };
     auto lookup = [&](uint32_t round) -> Tile {
         Tile t{};
-        const uint32_t v = round * grid + ((round & 1u) ? grid - 1u - slot : slot);
-        if ((uint64_t)round * grid >= total_tiles || v >= total_tiles) return t;
+        uint32_t v = round * grid + ((round & 1u) ? grid - 1u - slot : slot);
+        const uint32_t total_units = kSplit ? total_tiles * args.splits : total_tiles;
+        if ((uint64_t)round * grid >= total_units || v >= total_units) return t;
+        if constexpr (kSplit) {
+            // part by part: neighbours in the sequence share operand panels as they do without a split
+            t.part = v / total_tiles;
+            t.ks = t.part * args.split_steps * (uint32_t)BK;
+            v -= t.part * total_tiles;
+        }
         // position of the group that holds tile v: the number of groups whose tiles end at or before v. Every lane
         // compares one table entry per 64 groups and a ballot counts them (a binary search would be ten dependent LDS
         // round trips for 1024 groups; this is one per 64 groups, issued back to back).
@@ -351,7 +369,12 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
         t.fast = fast;
         return t;
     };
-    auto k_steps = [&](const Tile& t) { return (t.Ke + BK - 1) / BK; };
+    auto k_steps = [&](const Tile& t) {
+        const uint32_t all = (t.Ke + BK - 1) / BK;
+        if constexpr (!kSplit) return all;
+        const uint32_t left = all - t.part * args.split_steps;
+        return left < args.split_steps ? left : args.split_steps;
+    };
     // groups of at most 64 rows run a K loop of their own with a third LDS stage (grouped_gemm.hip); they start cold
     auto is_thin = [&](const Tile& t) { return A_KC && t.Me <= 64u && k_steps(t) >= 3u; };
     // a tile whose first two K steps can be fetched by the tile before it, and which can fetch the next tile's
@@ -521,13 +544,14 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
     constexpr bool kPrefetch = A_KC == B_KC;
     uint32_t pf_voff = kOutOfRange;
     const uint16_t* pf_base = nullptr;
-    uint32_t pf_bytes = 0, pf_ldb = 0, pf_col_bytes = 0, pf_kdim = 0, pf_steps = 0;
+    uint32_t pf_bytes = 0, pf_ldb = 0, pf_col_bytes = 0, pf_kdim = 0, pf_steps = 0, pf_k0 = 0;
     const bool pf_is_b = (wave & 1u) != 0;
     const bool pf_t = pf_is_b ? !B_KC : !A_KC;
     auto setup_prefetch = [&](const Tile& t) {
         if constexpr (!kPrefetch) return;
         const uint32_t p = wave >> 1;
         pf_steps = k_steps(t);
+        if constexpr (kSplit) pf_k0 = t.ks;
         if (!pf_is_b) {
             const uint32_t i = p * 16u + lane;
             if constexpr (GATHER) {
@@ -563,7 +587,7 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
     // requests this wavefront's lines of K step `kstep` of the current tile (nothing past its last step)
     auto issue_prefetch = [&](uint32_t kstep) {
         if constexpr (!kPrefetch) return;
-        const uint32_t k0 = kstep * (uint32_t)BK;
+        const uint32_t k0 = kstep * (uint32_t)BK + pf_k0;
         const bool inside = kstep < pf_steps;
         const uint32_t rows = k0 >= pf_kdim ? 0u : (pf_kdim - k0 < (uint32_t)BK ? pf_kdim - k0 : (uint32_t)BK);
         const uint16_t* base = pf_t ? pf_base + (uint64_t)k0 * (pf_ldb / 2u) : pf_base;
@@ -582,6 +606,7 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
     // store instructions per wavefront and tile (the epilogue issues a fixed number)
     constexpr uint32_t kTileStores = EPI == EPI_PLAIN        ? WM * WN * 2 / 1024
                                      : EPI == EPI_SWIGLU_BWD ? 2 * (WM * WN * 2 / 1024)  // two columns written per column
+                                     : kSplit                ? WM * WN * 4 / 1024
                                                              : (EPI == EPI_SWIGLU ? WM * WN * 2 / 1024 : 0) + WM * WN / 1024;
 
     // loads of one K step of the CURRENT loaders' aim into `stage` (compiler-visible: placed by the scheduling hints)
@@ -675,7 +700,7 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
             asm volatile("" ::: "memory");
         }
         setup_prefetch(cur);
-        const uint32_t KT = (Ke + BK - 1) / BK;
+        const uint32_t KT = k_steps(cur);
         const uint32_t KT2 = (KT + 1u) & ~1u;  // steps of the K loop: an odd count gets a step of zeros
         const bool thin = is_thin(cur);
         // kGatherK: where in row_index the entries of this wavefront for K step `abs_step` of the load stream begin: a step
@@ -818,11 +843,14 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
                 uint32_t k0;
                 if constexpr (SRC == 0) {
                     k0 = (kt + 2u) * (uint32_t)BK;
+                    if constexpr (kSplit) k0 += cur.ks;
                 } else if constexpr (SRC == 1) {
                     k0 = (kt + 2u - KT2) * (uint32_t)BK;
+                    if constexpr (kSplit) k0 += nxt.ks;
                 } else {
                     const bool of_next = kt + 2u >= KT2;
                     k0 = (of_next ? kt + 2u - KT2 : kt + 2u) * (uint32_t)BK;
+                    if constexpr (kSplit) k0 += of_next ? nxt.ks : cur.ks;
                     if constexpr (!GATHER)
                         aim_a(Feed<A_KC>{of_next ? fa_nxt.base0 : fa_cur.base0, nullptr, of_next ? fa_nxt.extent : fa_cur.extent,
                                          of_next ? fa_nxt.ldb : fa_cur.ldb, of_next ? fa_nxt.col_bytes : fa_cur.col_bytes},
@@ -996,12 +1024,13 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
                 else lt_b.issue_quiet_halves(lds_address(b_lo[st]), lds_address(b_hi[st]), k0);
             };
             issue_bias();
-            issue_thin(0, 0);
-            issue_thin(1, BK);
+            const uint32_t k_first = kSplit ? cur.ks : 0u;
+            issue_thin(0, k_first);
+            issue_thin(1, k_first + BK);
             __builtin_amdgcn_s_waitcnt(waitcnt_imm((int)kThinLoads, false));
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
-            issue_thin(2, 2 * BK);
+            issue_thin(2, k_first + 2 * BK);
             auto thin_loop = [&](auto fa_c) {
                 constexpr int FA = decltype(fa_c)::value;
                 auto thin_step = [&](int st, uint32_t kt) {
@@ -1031,7 +1060,7 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
                     __builtin_amdgcn_s_waitcnt(waitcnt_imm((int)kThinLoads, false));
                     __builtin_amdgcn_s_barrier();
                     asm volatile("" ::: "memory");
-                    issue_thin(st, (kt + 3) * BK);
+                    issue_thin(st, k_first + (kt + 3) * BK);
                 };
                 uint32_t kt = 0;
                 for (; kt + 2 < KT; kt += 3) {
@@ -1058,8 +1087,8 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
                     gk_request_lds(gk_first(2u), 0, false);
                     gk_request_lds(gk_first(3u), 1, false);
                 }
-                issue_quiet(0, 0);
-                issue_quiet(1, BK);
+                issue_quiet(0, kSplit ? cur.ks : 0u);
+                issue_quiet(1, (kSplit ? cur.ks : 0u) + BK);
                 const __amdgpu_buffer_rsrc_t nowhere = make_rsrc(args.D, 0u);
 #pragma unroll
                 for (uint32_t i = 0; i < kTileStores; ++i)  // (distinct offsets: identical stores would be merged into one)
@@ -1244,7 +1273,21 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
         for (int i = 0; i < RB; ++i) {
             const uint32_t r0 = m0 + wm * WM + i * 16;  // first output row of this block
             const uint32_t rows_valid = r0 < Me ? (Me - r0 < 16u ? Me - r0 : 16u) : 0u;
-            if constexpr (EPI == EPI_PLAIN || EPI == EPI_SWIGLU_BWD) {
+            if constexpr (kSplit) {
+                // the sums as they are: a lane's four consecutive columns of every 16 x 16 block, 64 bytes per row and block
+                const uint32_t col0 = n0 + wn * WN;
+                const uint32_t cols_valid = col0 < n_lim ? n_lim - col0 : 0u;
+                float* const origin = args.partial + ((uint64_t)cur.part * args.rows + cur.row0 + r0) * Ne + col0;
+                const __amdgpu_buffer_rsrc_t rs = make_rsrc(reinterpret_cast<const uint16_t*>(origin), rows_valid * (Ne * 4u));
+#pragma unroll
+                for (int j = 0; j < CB; ++j) {
+                    const uint32_t col = j * 16 + put_col;
+                    const uint32_t off = col < cols_valid ? put_row * (Ne * 4u) + col * 4u : kOutOfRange + (uint32_t)j * 16u;
+                    const f32x16& c = acc[i];
+                    store_tile16<false>(rs, off, uint4{__float_as_uint(c[4 * j]), __float_as_uint(c[4 * j + 1]),
+                                                       __float_as_uint(c[4 * j + 2]), __float_as_uint(c[4 * j + 3])});
+                }
+            } else if constexpr (EPI == EPI_PLAIN || EPI == EPI_SWIGLU_BWD) {
                 const uint32_t col0 = n0 + wn * WN;
                 const uint32_t cols_valid = col0 < n_lim ? n_lim - col0 : 0u;
                 uint2 w[CB];
@@ -1364,7 +1407,9 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
     template __global__ void ragged_gemm_kernel<EL, true, true, EPI_PLAIN, false, true, true>(const Args);      \
     template __global__ void ragged_gemm_kernel<EL, true, true, EPI_SWIGLU, false, true, true>(const Args);     \
     template __global__ void ragged_gemm_kernel<EL, true, true, EPI_SWIGLU_ACT, false, true, true>(const Args); \
-    template __global__ void ragged_gemm_kernel<EL, false, false, EPI_PLAIN, true, false, true>(const Args);
+    template __global__ void ragged_gemm_kernel<EL, false, false, EPI_PLAIN, true, false, true>(const Args);    \
+    template __global__ void ragged_gemm_kernel<EL, true, true, EPI_SPLIT, false, false, false>(const Args);    \
+    template __global__ void ragged_gemm_kernel<EL, true, false, EPI_SPLIT, false, false, false>(const Args);
 FMA_RAGGED_INSTANTIATE(ElemBf16)
 FMA_RAGGED_INSTANTIATE(ElemF16)
 #undef FMA_RAGGED_INSTANTIATE
@@ -1394,6 +1439,126 @@ int launch_plain(const Args& args, bool a_kc, bool b_kc, hipStream_t st) {
     if (a_kc && !b_kc) return launch<EL, true, false, EPI_PLAIN, VARY_K>(args, st);
     if (!a_kc && b_kc) return launch<EL, false, true, EPI_PLAIN, VARY_K>(args, st);
     return launch<EL, false, false, EPI_PLAIN, VARY_K>(args, st);
+}
+
+// ---- split reduction ---------------------------------------------------------------------------------------------
+// A launch with fewer tiles than compute units leaves the others idle for the whole reduction: the second projection of
+// 1021 tokens on 8 experts (2048 x 8192) is 96 tiles of 128 K steps, 205 us. With the reduction in two parts (192 tiles of
+// 64 steps, fp32 sums to memory and one pass over them) it takes 130 us. More of the same (parts; before -> now):
+//   NT 2048 x 8192, 8 groups of 64 / 128 rows (4)            167 -> 69 us, 180 -> 84 us
+//   NT 4096 x 14336, 8 groups of 128 / 512 rows (2 / 3)      357 -> 234 us, 690 -> 570 us
+//   NN 2048 x 16384, 8 groups of 128 / 512 / 1024 rows       339 -> 133 us (4), 380 -> 317 us (3), 700 -> 580 us (3)
+//   NN 4096 x 28672, 8 groups of 32 / 64 / 512 rows          496 -> 310 us (2), 633 -> 371 us (2), 1330 -> 1015 us (4)
+//
+// How many parts: the number with the least predicted time, rounds of tiles times (K steps + a tile's fixed cost) or the
+// weights at the rate they stream, plus the traffic of the sums. The row counts lie in device memory, so the number of tiles
+// is the expected one for evenly loaded groups. Parts have at least kSplitMinSteps steps, the sums at most kSplitMaxBytes (they
+// stay in the last-level cache), and a split has to promise a tenth less than none. Groups of few rows run the three-stage
+// loop, whose steps are shorter, without a split on half-width tiles in the NT layout: NT 4096 x 14336 on 8 groups of 32 rows
+// streams its weights in 176 us as it is and would take 184 us in two parts.
+constexpr double kStepUs = 1.45, kThinStepUs[2] = {1.1, 0.75}, kTileSteps = 6.0, kThinRows = 48.0, kWeightBytesPerUs = 5.5e6;
+constexpr double kReduceUs = 4.0, kReduceBytesPerUs = 4.5e6, kSplitGain = 0.9;
+constexpr uint32_t kSplitMinSteps = 24;
+constexpr int64_t kSplitMaxBytes = 256ll << 20;
+struct SplitPlan {
+    uint32_t splits, steps;  // parts and K steps of each (even; the last part takes what is left); splits 1: no split
+};
+SplitPlan plan_split(int64_t R, int64_t E, int64_t N, int64_t K, bool b_kc) {
+    const uint32_t all = (uint32_t)((K + BK - 1) / BK);
+    SplitPlan best{1u, all};
+    // (the sizes for which every tile takes the matrix-instruction path)
+    if (R < 1 || E < 1 || N < 8 || N % 8 || N >= (1 << 23) || K % 8 || K >= (1 << 21) || R > 0x7fffffffll) return best;
+    if (all < 2 * kSplitMinSteps) return best;
+    const int cus = num_compute_units() > 0 ? num_compute_units() : 256;
+    const double active = (double)(R < E ? R : E), mean = (double)R / active;
+    const double row_tiles = active * (mean < BM / 2 ? 1.0 : mean / BM + 0.5);
+    const double tiles = row_tiles * (double)((N + BN - 1) / BN);
+    const bool thin = mean <= kThinRows, narrow = thin && b_kc && 2.0 * tiles <= cus;
+    const double step_us = thin ? kThinStepUs[b_kc] : kStepUs;
+    const double weights_us = active * N * K * 2.0 / kWeightBytesPerUs;
+    auto us = [&](uint32_t parts, uint32_t steps) {
+        const double units = tiles * parts * (parts == 1 && narrow ? 2.0 : 1.0);
+        const double products = std::ceil(units / cus - 1e-9) * (steps + kTileSteps) * step_us;
+        const double sums = parts > 1 ? kReduceUs + (double)R * N * (8.0 * parts + 2.0) / kReduceBytesPerUs : 0.0;
+        return std::max(products, weights_us) + sums;
+    };
+    double best_us = us(1, all) * kSplitGain;
+    for (uint32_t parts = 2; parts * kSplitMinSteps <= all && parts <= 32; ++parts) {
+        const uint32_t steps = ((all + parts - 1) / parts + 1u) & ~1u;
+        const uint32_t used = (all + steps - 1) / steps;
+        if (used != parts || R * N * 4 * (int64_t)parts > kSplitMaxBytes) continue;
+        const double t = us(parts, steps);
+        if (t < best_us) {
+            best_us = t;
+            best = SplitPlan{parts, steps};
+        }
+    }
+    return best;
+}
+
+// out[r, :] = round(alpha * (sum over the parts, in order)), plus the bias of the row's group as the kernels' epilogue adds it.
+// Bound by memory (parts * 4 + 2 bytes per element). A workgroup takes kReduceRows rows; which group a row belongs to is
+// read off a prefix of the sizes (built per workgroup: E values, one scan), and rows past the last group are left alone.
+constexpr int kReduceThreads = 256, kReduceRows = 4;
+template <typename EL, bool BIAS>
+__global__ __launch_bounds__(kReduceThreads) void split_reduce_kernel(const Args args) {
+    __shared__ uint32_t s_end[FMA_MAX_GROUPS];
+    const uint32_t tid = threadIdx.x, E = args.E, N = args.n;
+    if (tid < 64u) {
+        uint32_t carry = 0;
+        for (uint32_t base = 0; base < E; base += 64u) {
+            const uint32_t e = base + tid;
+            const uint32_t incl = wave_inclusive_scan<uint32_t>(e < E ? args.sizes[e] : 0u);
+            if (e < E) s_end[e] = carry + incl;
+            carry += __shfl(incl, 63, 64);
+        }
+    }
+    __syncthreads();
+    const uint32_t vecs = N / 8u;  // of 8 columns
+    const uint64_t part = (uint64_t)args.rows * N;
+    const uint32_t first = blockIdx.x * (uint32_t)kReduceRows;
+    for (uint32_t i = tid; i < (uint32_t)kReduceRows * vecs; i += kReduceThreads) {
+        const uint32_t r = first + i / vecs, col = (i % vecs) * 8u;
+        if (r >= args.rows || r >= s_end[E - 1u]) return;
+        const float* src = args.partial + (uint64_t)r * N + col;
+        float sum[8];
+#pragma unroll
+        for (int x = 0; x < 8; ++x) sum[x] = 0.0f;
+        for (uint32_t s = 0; s < args.splits; ++s, src += part) {
+            const float4 lo = reinterpret_cast<const float4*>(src)[0], hi = reinterpret_cast<const float4*>(src)[1];
+            sum[0] += lo.x; sum[1] += lo.y; sum[2] += lo.z; sum[3] += lo.w;
+            sum[4] += hi.x; sum[5] += hi.y; sum[6] += hi.z; sum[7] += hi.w;
+        }
+#pragma unroll
+        for (int x = 0; x < 8; ++x) sum[x] *= args.alpha;
+        if constexpr (BIAS) {
+            uint32_t lo = 0, hi = E - 1u;  // the first group that ends past row r
+            while (lo < hi) {
+                const uint32_t mid = (lo + hi) >> 1;
+                if (s_end[mid] > r) hi = mid;
+                else lo = mid + 1u;
+            }
+            const uint16_t* b = args.bias + (uint64_t)lo * N + col;
+#pragma unroll
+            for (int x = 0; x < 8; ++x) sum[x] = EL::round(sum[x]) + EL::from_bits(b[x]);
+        }
+        uint4 packed;
+        packed.x = EL::pack2(sum[0], sum[1]);
+        packed.y = EL::pack2(sum[2], sum[3]);
+        packed.z = EL::pack2(sum[4], sum[5]);
+        packed.w = EL::pack2(sum[6], sum[7]);
+        *reinterpret_cast<uint4*>(args.D + (uint64_t)r * N + col) = packed;
+    }
+}
+
+template <typename EL>
+int launch_split(const Args& args, bool b_kc, hipStream_t st) {
+    const int rc = b_kc ? launch<EL, true, true, EPI_SPLIT, false>(args, st) : launch<EL, true, false, EPI_SPLIT, false>(args, st);
+    if (rc != FMA_OK) return rc;
+    const dim3 grid((args.rows + kReduceRows - 1) / kReduceRows), block(kReduceThreads);
+    if (args.bias) hipLaunchKernelGGL((split_reduce_kernel<EL, true>), grid, block, 0, st, args);
+    else hipLaunchKernelGGL((split_reduce_kernel<EL, false>), grid, block, 0, st, args);
+    return launch_status("grouped_gemm_ragged(reduce)");
 }
 
 // The forward product of an expert projection, out_e = x_e W_e^T (+ bias_e), with the rows of x_e packed (row_index
@@ -1474,9 +1639,21 @@ int launch_ragged_from_arrays(const void* A, const void* B, void* D, const uint3
 extern "C" {
 
 
+int64_t fma_grouped_gemm_ragged_workspace_bytes(int64_t R, int64_t E, int64_t N, int64_t K, int trans_b) {
+    const fmahip::gemm::ragged::SplitPlan plan = fmahip::gemm::ragged::plan_split(R, E, N, K, trans_b != 0);
+    return plan.splits > 1 ? R * N * 4 * (int64_t)plan.splits : 0;
+}
+
 int fma_grouped_gemm_ragged(const void* A, const void* B, void* D, const uint32_t* sizes, const void* bias, int64_t E,
                             int vary, int64_t M, int64_t N, int64_t K, int trans_a, int trans_b, float alpha, int dtype,
                             void* stream) {
+    return fma_grouped_gemm_ragged_split(A, B, D, sizes, bias, E, vary, M, N, K, trans_a, trans_b, alpha, 0, nullptr, 0, dtype,
+                                         stream);
+}
+
+int fma_grouped_gemm_ragged_split(const void* A, const void* B, void* D, const uint32_t* sizes, const void* bias, int64_t E,
+                                  int vary, int64_t M, int64_t N, int64_t K, int trans_a, int trans_b, float alpha,
+                                  int64_t rows, void* workspace, int64_t workspace_bytes, int dtype, void* stream) {
     using namespace fmahip;
     using namespace fmahip::gemm;
     FMA_REQUIRE(dtype == FMA_BF16 || dtype == FMA_F16, dtype_bytes(dtype) ? FMA_ERR_UNSUPPORTED : FMA_ERR_BAD_DTYPE,
@@ -1518,6 +1695,20 @@ int fma_grouped_gemm_ragged(const void* A, const void* B, void* D, const uint32_
     args.n = (uint32_t)N;
     args.k = (uint32_t)K;
     args.alpha = alpha;
+    const ragged::SplitPlan plan =
+        workspace && vary == FMA_VARY_M && a_kc ? ragged::plan_split(rows, E, N, K, b_kc) : ragged::SplitPlan{1u, 0u};
+    if (plan.splits > 1) {
+        FMA_REQUIRE(aligned16(workspace), FMA_ERR_MISALIGNED, "grouped_gemm_ragged: the workspace must be 16-byte aligned");
+        const int64_t need = rows * N * 4 * (int64_t)plan.splits;
+        FMA_REQUIRE(workspace_bytes >= need, FMA_ERR_WORKSPACE_TOO_SMALL,
+                    "grouped_gemm_ragged: workspace of %lld bytes is smaller than the %lld needed", (long long)workspace_bytes,
+                    (long long)need);
+        args.partial = (float*)workspace;
+        args.splits = plan.splits;
+        args.split_steps = plan.steps;
+        args.rows = (uint32_t)rows;
+        return dtype == FMA_BF16 ? ragged::launch_split<ElemBf16>(args, b_kc, st) : ragged::launch_split<ElemF16>(args, b_kc, st);
+    }
     if (bias)
         return dtype == FMA_BF16 ? ragged::launch_forward<ElemBf16, EPI_PLAIN>(args, st)
                                  : ragged::launch_forward<ElemF16, EPI_PLAIN>(args, st);

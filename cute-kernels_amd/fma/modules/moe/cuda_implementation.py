@@ -170,11 +170,18 @@ def grouped_gemm_ragged_cuda(
     # an operand without elements is never read, but the entry point rejects NULL: any valid device address stands in
     a_ptr = A.data_ptr() if A.numel() else output.data_ptr()
     b_ptr = B.data_ptr() if B.numel() else output.data_ptr()
+    lib = _lib.load()
+    rows = output.numel() // N
     with _lib.on_device(A.device):
-        rc = _lib.load().fma_grouped_gemm_ragged(
+        # sums of a split reduction, where the launch has too few tiles for the compute units; owned by this call
+        nbytes = 0
+        if not vary_k and not is_A_transposed and A.numel() >= rows * K:
+            nbytes = lib.fma_grouped_gemm_ragged_workspace_bytes(rows, sizes.numel(), N, K, int(is_B_transposed))
+        workspace = torch.empty(nbytes, dtype=torch.uint8, device=A.device) if nbytes else None
+        rc = lib.fma_grouped_gemm_ragged_split(
             a_ptr, b_ptr, output.data_ptr(), sizes.data_ptr(), _lib.ptr(bias), sizes.numel(),
             _lib.FMA_VARY_K if vary_k else _lib.FMA_VARY_M, M, N, K, int(is_A_transposed), int(is_B_transposed), 1.0,
-            _lib.dtype_code(A.dtype), _lib.current_stream(A.device),
+            rows, _lib.ptr(workspace), nbytes, _lib.dtype_code(A.dtype), _lib.current_stream(A.device),
         )
     _lib.check(rc, "grouped_gemm_ragged_cuda")
 
@@ -974,7 +981,8 @@ def thin_swiglu_experts(
     x: torch.Tensor, weight1: torch.Tensor, bias1: torch.Tensor | None, weight2: torch.Tensor, bias2: torch.Tensor | None,
     perm: torch.Tensor, counts: torch.Tensor, offsets: torch.Tensor, top_k: int,
 ) -> torch.Tensor:  # fmt: skip
-    """gathered_swiglu_experts without a backward, for a few rows per expert: same values, bit for bit"""
+    """gathered_swiglu_experts without a backward, for a few rows per expert: same values, bit for bit, where the second
+    projection's reduction is not split there (grouped_gemm_ragged_cuda), up to the order of its fp32 sums where it is"""
     R = perm.numel()
     act = torch.empty(R, weight2.size(2), device=x.device, dtype=x.dtype)
     output = torch.empty(R, weight2.size(1), device=x.device, dtype=x.dtype)

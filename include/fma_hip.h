@@ -214,6 +214,17 @@ int fma_grouped_gemm_ragged(const void* A, const void* B, void* D, const uint32_
                             int vary, int64_t M, int64_t N, int64_t K, int trans_a, int trans_b, float alpha, int dtype,
                             void* stream);
 
+/* fma_grouped_gemm_ragged for launches whose tiles are too few for the compute units: with a workspace (16-byte aligned, of
+ * fma_grouped_gemm_ragged_workspace_bytes(rows, E, N, K, trans_b) bytes; that query returns 0 where no split pays), vary == FMA_VARY_M
+ * and trans_a == 0, the reduction is computed in several parts whose fp32 sums are added in order. rows: the number of packed
+ * rows, at least the sum of sizes. Same result as without a split up to the order of the fp32 sum, and the same from call to
+ * call; workspace NULL, a workspace query of 0 or another form: exactly fma_grouped_gemm_ragged. Rows past the groups are
+ * left as they are. */
+int64_t fma_grouped_gemm_ragged_workspace_bytes(int64_t rows, int64_t E, int64_t N, int64_t K, int trans_b);
+int fma_grouped_gemm_ragged_split(const void* A, const void* B, void* D, const uint32_t* sizes, const void* bias, int64_t E,
+                                  int vary, int64_t M, int64_t N, int64_t K, int trans_a, int trans_b, float alpha,
+                                  int64_t rows, void* workspace, int64_t workspace_bytes, int dtype, void* stream);
+
 /* Up-projection with SwiGLU fused into the epilogue. For each expert e with M_e rows (rows of all experts
  * packed back to back, sum M_e = R):
  *   h_e   = x_e[M_e, K] * W_e[2I, K]^T            (rounded to dtype; written to h if h != NULL)

@@ -1,0 +1,67 @@
+"""GPU parity of fma_grouped_gemm_ragged_split: launches with few tiles, whose reduction is computed in parts. Operands are
+small integers, so that every fp32 sum is exact in any order (|sum| <= 9 K < 2^24) and the result has to equal the unsplit
+one, and the float64 product rounded once, bit for bit."""
+
+import pytest
+import torch
+
+from fma import _lib
+
+from gpu_util import DEV
+
+pytestmark = pytest.mark.gpu
+
+
+def _call(A, B, sizes, rows, N, K, tB, bias, alpha, workspace_bytes):
+    lib = _lib.load()
+    out = torch.full((rows, N), 7.0, dtype=A.dtype, device=DEV)
+    s = torch.tensor(sizes, dtype=torch.int64).to(torch.uint32).to(DEV)
+    # never read before it is written: NaN would show
+    workspace = torch.full((max(workspace_bytes // 4, 1),), float("nan"), device=DEV)
+    rc = lib.fma_grouped_gemm_ragged_split(
+        A.data_ptr(), B.data_ptr(), out.data_ptr(), s.data_ptr(), _lib.ptr(bias), len(sizes), _lib.FMA_VARY_M, 0, N, K, 0,
+        int(tB), alpha, rows, workspace.data_ptr() if workspace_bytes else None, workspace_bytes, _lib.dtype_code(A.dtype),
+        torch.cuda.current_stream().cuda_stream,
+    )
+    assert rc == 0, lib.fma_last_error_string()
+    torch.cuda.synchronize()
+    return out
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("tB", [True, False])
+@pytest.mark.parametrize(
+    "sizes,N,K,bias,alpha",
+    [
+        ([250, 257, 0, 3, 64, 65, 512, 130], 2048, 8192, True, 1.0),  # ragged, empty, thin groups; whole K steps
+        ([128] * 8, 2048, 4104, False, 1.0),  # 65 K steps, the last of 8 elements: an odd and partial last part
+        ([1], 264, 3080, False, 0.5),  # the shortest split reduction, one row, a partial column tile
+        ([600, 30], 520, 5000, True, 1.0),  # partial column tile of 8, K a multiple of 8 only
+        ([16] * 40, 8, 16384, False, 1.0),  # one narrow column tile, many parts
+    ],
+)
+def test_split_equals_unsplit(dtype, tB, sizes, N, K, bias, alpha):
+    bias = bias and tB  # (added in the forward form only)
+    E, R = len(sizes), sum(sizes)
+    rows = R + 5  # rows past the groups stay as they are
+    g = torch.Generator(device=DEV).manual_seed(K + N)
+    A = torch.randint(-3, 4, (rows, K), device=DEV, generator=g).to(dtype)
+    B = torch.randint(-3, 4, (E, N, K) if tB else (E, K, N), device=DEV, generator=g).to(dtype)
+    b = torch.randint(-64, 65, (E, N), device=DEV, generator=g).to(dtype) if bias else None
+    nbytes = _lib.load().fma_grouped_gemm_ragged_workspace_bytes(rows, E, N, K, int(tB))
+    assert nbytes >= 2 * rows * N * 4, "the sizes are chosen to be split"
+    got = _call(A, B, sizes, rows, N, K, tB, b, alpha, nbytes)
+    assert torch.equal(got, _call(A, B, sizes, rows, N, K, tB, b, alpha, 0))
+    assert (got[R:] == 7.0).all()
+    at = 0
+    for e, m in enumerate(sizes):
+        expect = (alpha * (A[at : at + m].double() @ (B[e].T if tB else B[e]).double())).to(dtype)
+        if bias:
+            expect = (expect.float() + b[e].float()).to(dtype)
+        assert torch.equal(got[at : at + m], expect), f"group {e}"
+        at += m
+
+
+@pytest.mark.parametrize("rows,E,N,K", [(65536, 128, 4096, 1536), (16, 8, 2048, 3000), (2042, 8, 2047, 8192), (0, 8, 2048, 8192)])
+def test_no_split_where_it_cannot_pay_or_run(rows, E, N, K):
+    assert _lib.load().fma_grouped_gemm_ragged_workspace_bytes(rows, E, N, K, 1) == 0
