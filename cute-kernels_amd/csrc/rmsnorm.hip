@@ -7,10 +7,12 @@
 //
 // One workgroup of 256 threads per row at a time, each thread holding up to VPT 16-byte vectors of the row in
 // registers; rows that are longer than that, or whose length in bytes is not a multiple of 16, take a two-pass
-// element-wise kernel that reads its inputs twice (the second time from the L2). The backward gives every workgroup a
-// contiguous chunk of rows so that it can keep the weight gradient of its chunk in registers across rows; the chunks'
-// partial gradients go to a workspace and a second launch adds them up in a fixed order (the reference adds them with
-// atomics, in arrival order).
+// element-wise kernel that reads its inputs twice (the second time from the L2). In the backward a workgroup keeps the weight
+// gradient of its rows in registers; the partial gradients go to a workspace and a second launch adds them up in a fixed
+// order (the reference adds them with atomics, in arrival order). The rows of a workgroup are a grid apart, so that the
+// rows in flight are neighbours in memory: against a contiguous chunk of rows per workgroup, whose concurrent streams are
+// equal power-of-two distances apart, [16384, 4096] bf16 took 131 instead of 139 us and [32768, 4096] 249 instead of 272 us
+// (both with two workgroups per compute unit).
 #include "common.h"
 
 namespace fmahip {
@@ -18,9 +20,18 @@ namespace {
 
 constexpr int kNormThreads = 256;
 constexpr int kNormWaves = kNormThreads / kWave;
-// chunks of rows (= rows of the weight-gradient workspace) per compute unit; measured on [16384, 4096] bf16: 1 -> 214 us,
-// 2 -> 143 us, 3 -> 151 us, 4 -> 173 us, 8 -> 162 us for both launches
-constexpr int kBwdWorkgroupsPerCU = 2;
+// Workgroups of the backward pass per compute unit. A workgroup handles its rows one after the other, one row ahead in
+// flight, so more of them keep more bytes in flight until the registers of a compute unit run out (a second, short round of
+// workgroups) or the sum over their partial weight gradients weighs more than it saves. Both launches, bf16, cold buffers,
+// us for 2 / 3 / 4 / 6 workgroups:
+//   [16384, 4096] 131 / 128 / 158 / -      [32768, 2880] 222 / 189 / 236 / -      [4096, 2880] 40.4 / 38.2 / 48.8 / -
+//   [32768, 2048] 155 / 128 / 131 / 161    [8192, 2048] 49.2 / 45.6 / 47.7 / 60.6  [3000, 2880] 33.6 / 34.1 / 42.0 / -
+//   [32768, 1024] 141 / 104 / 89 / 112     [8192, 1024] 43.7 / 38.4 / 37.2 / 46.4  [4096, 1024] 26.9 / 26.0 / 27.9 / 34.6
+// fp16 gains less and later, 2 / now: [32768, 2880] 192 -> 170, [32768, 1024] 105 -> 75, [8192, 4096] 73.9 -> 73.8, while three
+// cost [4096, 1024] 22.4 -> 23.3. Hence three from six rows each on, four from eight rows each on where a row fills at most half
+// of the threads, and two otherwise (few rows; more than two vectors per thread, whose registers leave room for no more).
+constexpr int kBwdPerCU = 3, kBwdPerCUHalfRows = 4, kBwdPerCUFew = 2;
+constexpr int kBwdMinRows = 6, kBwdMinHalfRows = 8;
 
 struct Sum2 {
     float a, b;
@@ -161,8 +172,8 @@ template <typename T, int VPT, bool HAS_W>
 __global__ __launch_bounds__(kNormThreads) void rmsnorm_bwd_kernel(
     const Vec16<T>* __restrict__ added, const Vec16<T>* __restrict__ weight, const Vec16<T>* __restrict__ dy,
     const Vec16<T>* __restrict__ d_added_in, const float* __restrict__ denom, Vec16<T>* __restrict__ dx,
-    Vec16<T>* __restrict__ d_residual, float* __restrict__ dw_partial, int64_t B, int64_t rows_per_workgroup, int nvec,
-    float inv_H, float eps, float multiplier) {
+    Vec16<T>* __restrict__ d_residual, float* __restrict__ dw_partial, int64_t B, int nvec, float inv_H, float eps,
+    float multiplier) {
     constexpr int N = Vec16<T>::N;
     __shared__ float s_red[2][kNormWaves][2];
     const int tid = threadIdx.x;
@@ -176,8 +187,6 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_bwd_kernel(
 #pragma unroll
         for (int e = 0; e < N; ++e) dw[i][e] = 0.f;
     }
-    const int64_t row0 = (int64_t)blockIdx.x * rows_per_workgroup;
-    const int64_t row1 = row0 + rows_per_workgroup < B ? row0 + rows_per_workgroup : B;
     // the vectors of the next row are requested before this row is worked on, so that their latency runs under this row's
     // arithmetic, barrier and stores (a workgroup handles its rows one after the other)
     Vec16<T> rv[VPT], gv[VPT], av[VPT];
@@ -193,12 +202,12 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_bwd_kernel(
             }
         }
     };
-    if (row0 < row1) fetch(rv, gv, av, row0);
+    if (blockIdx.x < B) fetch(rv, gv, av, blockIdx.x);
     int parity = 0;
-    for (int64_t row = row0; row < row1; ++row, parity ^= 1) {
+    for (int64_t row = blockIdx.x; row < B; row += gridDim.x, parity ^= 1) {
         const int64_t base = row * nvec;
         Vec16<T> rn[VPT], gn[VPT], an[VPT];
-        fetch(rn, gn, an, row + 1 < row1 ? row + 1 : row);  // after the last row: this row again, unused
+        fetch(rn, gn, an, row + gridDim.x < B ? row + gridDim.x : row);  // after the last row: this row again, unused
         float dot = 0.f, ss = 0.f;
 #pragma unroll
         for (int i = 0; i < VPT; ++i) {
@@ -342,10 +351,23 @@ int vectors_per_thread(int64_t row_bytes, bool all_aligned) {
     return 0;
 }
 
-int64_t backward_workgroups(int64_t B) {
+// workgroups of the backward pass (= rows of the weight-gradient workspace) for rows of nvec vectors, vpt per thread
+int64_t backward_workgroups(int64_t B, int vpt, int64_t nvec) {
     const int64_t cus = num_compute_units() > 0 ? num_compute_units() : 256;
-    const int64_t want = cus * kBwdWorkgroupsPerCU;
+    int64_t want = cus * kBwdPerCUFew;
+    if (vpt == 1 && nvec <= kNormThreads / 2 && B >= cus * kBwdPerCUHalfRows * kBwdMinHalfRows)
+        want = cus * kBwdPerCUHalfRows;
+    else if ((vpt == 1 || vpt == 2) && B >= cus * kBwdPerCU * kBwdMinRows)
+        want = cus * kBwdPerCU;
     return B < want ? (B > 0 ? B : 1) : want;
+}
+
+// enough for every element type and alignment of [B, H]
+int64_t backward_workspace_bytes(int64_t B, int64_t H) {
+    const int64_t few = backward_workgroups(B, 0, 0), full = backward_workgroups(B, 2, kNormThreads),
+                  half = backward_workgroups(B, 1, 1);
+    const int64_t most = full > half ? full : half;
+    return (few > most ? few : most) * H * 4;
 }
 
 template <typename T, int VPT>
@@ -385,34 +407,34 @@ int launch_fwd(const void* x, const void* residual, const void* weight, void* ou
 template <typename T, int VPT>
 void launch_bwd_vec(bool has_w, dim3 grid, hipStream_t st, const void* added, const void* weight, const void* dy,
                     const void* d_added_in, const float* denom, void* dx, void* d_residual, float* partial, int64_t B,
-                    int64_t rows_per, int nvec, float inv_H, float eps, float mult) {
+                    int nvec, float inv_H, float eps, float mult) {
     using V = Vec16<T>;
     if (has_w)
         hipLaunchKernelGGL((rmsnorm_bwd_kernel<T, VPT, true>), grid, dim3(kNormThreads), 0, st, (const V*)added,
                            (const V*)weight, (const V*)dy, (const V*)d_added_in, denom, (V*)dx, (V*)d_residual, partial, B,
-                           rows_per, nvec, inv_H, eps, mult);
+                           nvec, inv_H, eps, mult);
     else
         hipLaunchKernelGGL((rmsnorm_bwd_kernel<T, VPT, false>), grid, dim3(kNormThreads), 0, st, (const V*)added,
                            (const V*)weight, (const V*)dy, (const V*)d_added_in, denom, (V*)dx, (V*)d_residual, partial, B,
-                           rows_per, nvec, inv_H, eps, mult);
+                           nvec, inv_H, eps, mult);
 }
 
 template <typename T>
 int launch_bwd(const void* added, const void* weight, const void* dy, const void* d_added_in, const float* denom, void* dx,
-               void* d_residual, float* d_weight, float* partial, int64_t G, int64_t B, int64_t H, float eps, float mult,
-               hipStream_t st) {
+               void* d_residual, float* d_weight, float* partial, int64_t B, int64_t H, float eps, float mult, hipStream_t st) {
     const bool aligned = aligned16(added) && aligned16(dy) && aligned16(dx) && aligned16(d_residual) &&
                          (!weight || aligned16(weight)) && (!d_added_in || aligned16(d_added_in));
     const int vpt = vectors_per_thread(H * (int64_t)sizeof(T), aligned);
+    const int nvec = (int)(H * (int64_t)sizeof(T) / 16);
+    const int64_t G = backward_workgroups(B, vpt, nvec);
     const int64_t rows_per = (B + G - 1) / G;
     const dim3 grid((uint32_t)G);
     const float inv_H = 1.0f / (float)H;
-    const int nvec = (int)(H * (int64_t)sizeof(T) / 16);
     switch (vpt) {
-        case 1: launch_bwd_vec<T, 1>(weight, grid, st, added, weight, dy, d_added_in, denom, dx, d_residual, partial, B, rows_per, nvec, inv_H, eps, mult); break;
-        case 2: launch_bwd_vec<T, 2>(weight, grid, st, added, weight, dy, d_added_in, denom, dx, d_residual, partial, B, rows_per, nvec, inv_H, eps, mult); break;
-        case 4: launch_bwd_vec<T, 4>(weight, grid, st, added, weight, dy, d_added_in, denom, dx, d_residual, partial, B, rows_per, nvec, inv_H, eps, mult); break;
-        case 8: launch_bwd_vec<T, 8>(weight, grid, st, added, weight, dy, d_added_in, denom, dx, d_residual, partial, B, rows_per, nvec, inv_H, eps, mult); break;
+        case 1: launch_bwd_vec<T, 1>(weight, grid, st, added, weight, dy, d_added_in, denom, dx, d_residual, partial, B, nvec, inv_H, eps, mult); break;
+        case 2: launch_bwd_vec<T, 2>(weight, grid, st, added, weight, dy, d_added_in, denom, dx, d_residual, partial, B, nvec, inv_H, eps, mult); break;
+        case 4: launch_bwd_vec<T, 4>(weight, grid, st, added, weight, dy, d_added_in, denom, dx, d_residual, partial, B, nvec, inv_H, eps, mult); break;
+        case 8: launch_bwd_vec<T, 8>(weight, grid, st, added, weight, dy, d_added_in, denom, dx, d_residual, partial, B, nvec, inv_H, eps, mult); break;
         default:
             hipLaunchKernelGGL(rmsnorm_bwd_generic_kernel<T>, grid, dim3(kNormThreads), 0, st, (const T*)added,
                                (const T*)weight, (const T*)dy, (const T*)d_added_in, denom, (T*)dx, (T*)d_residual, partial,
@@ -463,7 +485,7 @@ int fma_fused_residual_add_rmsnorm_fwd(const void* x, const void* residual, cons
 
 int64_t fma_fused_residual_add_rmsnorm_bwd_workspace_bytes(int64_t B, int64_t H) {
     if (B <= 0 || H <= 0) return 0;
-    return fmahip::backward_workgroups(B) * H * 4;
+    return fmahip::backward_workspace_bytes(B, H);
 }
 
 int fma_fused_residual_add_rmsnorm_bwd(const void* added_x_residual, const void* weight, const void* output_grad,
@@ -487,12 +509,12 @@ int fma_fused_residual_add_rmsnorm_bwd(const void* added_x_residual, const void*
     }
     FMA_REQUIRE(added_x_residual && output_grad && x_grad && residual_grad, FMA_ERR_NULL_POINTER,
                 "fused_residual_add_rmsnorm_bwd: NULL pointer");
-    int64_t G = backward_workgroups(B);
     if (weight) {
+        const int64_t need = backward_workspace_bytes(B, H);
         FMA_REQUIRE(workspace != nullptr, FMA_ERR_NULL_POINTER, "fused_residual_add_rmsnorm_bwd: NULL workspace");
-        FMA_REQUIRE(workspace_bytes >= G * H * 4, FMA_ERR_WORKSPACE_TOO_SMALL,
+        FMA_REQUIRE(workspace_bytes >= need, FMA_ERR_WORKSPACE_TOO_SMALL,
                     "fused_residual_add_rmsnorm_bwd: workspace of %lld bytes, %lld needed", (long long)workspace_bytes,
-                    (long long)(G * H * 4));
+                    (long long)need);
         FMA_REQUIRE((reinterpret_cast<uintptr_t>(workspace) & 3u) == 0, FMA_ERR_MISALIGNED,
                     "fused_residual_add_rmsnorm_bwd: workspace must be 4-byte aligned");
     }
@@ -500,13 +522,13 @@ int fma_fused_residual_add_rmsnorm_bwd(const void* added_x_residual, const void*
     switch (dtype) {
         case FMA_F32:
             return launch_bwd<float>(added_x_residual, weight, output_grad, added_x_residual_grad, rmsnorm_denominator,
-                                     x_grad, residual_grad, weight_grad, partial, G, B, H, eps, multiplier, st);
+                                     x_grad, residual_grad, weight_grad, partial, B, H, eps, multiplier, st);
         case FMA_F16:
             return launch_bwd<f16_t>(added_x_residual, weight, output_grad, added_x_residual_grad, rmsnorm_denominator,
-                                     x_grad, residual_grad, weight_grad, partial, G, B, H, eps, multiplier, st);
+                                     x_grad, residual_grad, weight_grad, partial, B, H, eps, multiplier, st);
         default:
             return launch_bwd<bf16_t>(added_x_residual, weight, output_grad, added_x_residual_grad,
-                                      rmsnorm_denominator, x_grad, residual_grad, weight_grad, partial, G, B, H, eps,
+                                      rmsnorm_denominator, x_grad, residual_grad, weight_grad, partial, B, H, eps,
                                       multiplier, st);
     }
 }

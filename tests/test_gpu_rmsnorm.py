@@ -159,3 +159,26 @@ def test_rejects_what_it_does_not_implement():
     a = fused_residual_add_rmsnorm(x, x, None, None)[0]
     b = fused_residual_add_rmsnorm(x, x, None, torch.finfo(torch.float32).eps)[0]
     assert torch.equal(a, b)
+
+
+# around the row counts at which the backward takes more workgroups (4608 rows; 8192 where a row fills half of the threads),
+# one to two vectors per thread, counts that leave some workgroups one row less
+@pytest.mark.parametrize(
+    "B,H", [(4607, 2048), (4608, 2048), (4609, 2048), (4608, 1024), (5001, 720), (8191, 512), (8192, 512), (8197, 512), (9001, 64)]
+)
+def test_backward_row_split_against_fp64(B, H):
+    g = torch.Generator(device=DEV).manual_seed(B + H)
+    x, residual, dy, dr = (torch.randn(B, H, generator=g, device=DEV) for _ in range(4))
+    weight = torch.randn(H, generator=g, device=DEV)
+    leaves = [t.clone().requires_grad_() for t in (x, residual, weight)]
+    z, r = fused_residual_add_rmsnorm(*leaves, _EPSILON)
+    torch.autograd.backward((z, r), (dy, dr))
+    exact = [t.double().requires_grad_() for t in (x, residual, weight)]
+    s = exact[0] + exact[1]
+    unit = s * torch.rsqrt(s.square().mean(-1, keepdim=True) + _EPSILON)
+    torch.autograd.backward((unit * exact[2], s), (dy.double(), dr.double()))
+    for got, want in zip(leaves[:2], exact[:2]):
+        assert float((got.grad - want.grad).abs().max()) <= 1.5e-4  # the bar of the cases above
+    # a sum of at most B / 512 + 1 rows in fp32, then fp64; 16 more roundings for the terms themselves
+    bound = (B // 512 + 17) * 2.0**-24 * (dy.double() * unit.detach()).abs().sum(0)
+    assert bool(((leaves[2].grad - exact[2].grad).abs() <= bound).all())
