@@ -159,3 +159,29 @@ def test_build_refuses_gemm_kernels_with_register_spills():
     with pytest.raises(RuntimeError, match="names no"):
         build._check_no_scratch("grouped_gemm.hip", "remark: Function Name: other\n", "grouped_gemm_kernel")
     assert "grouped_gemm.hip" in build.NO_SCRATCH_SOURCES
+
+
+def test_ensure_contiguous_inside_containers():
+    """tensors inside containers of every kind that torch's pytree knows, registered ones among them"""
+    from collections import OrderedDict, deque, namedtuple
+    from torch.utils import _pytree
+
+    class Pair:
+        def __init__(self, a, b):
+            self.a, self.b = a, b
+
+    _pytree.register_pytree_node(Pair, lambda p: ([p.a, p.b], None), lambda leaves, _: Pair(*leaves))
+    Named = namedtuple("Named", "a b")
+    t = torch.zeros(3, 4).t()
+    plain = (1, 2.0, "s", None, True, torch.float32, KernelBackend.cuda, len)
+
+    @fma.ensure_contiguous
+    def leaves(*args, **kwargs):
+        return _pytree.tree_leaves((args, kwargs))
+
+    containers = [t, [t], (t, 1), {"t": t}, OrderedDict(t=t), deque([t]), Named(t, 2), Pair(t, [t]), [Pair(1, deque([t]))]]
+    for c in containers:
+        for got in (leaves(c, *plain), leaves(*plain, keyword=c)):
+            tensors = [x for x in got if isinstance(x, torch.Tensor)]
+            assert tensors and all(x.is_contiguous() and x.shape == t.shape for x in tensors)
+            assert all(any(x is p for x in got) for p in plain if p is not None)
