@@ -94,6 +94,11 @@ def test_layer_without_backward_in_other_forms(T):
         assert torch.equal(run(moe, x)[0], 2 * y)  # (a power of two: exact)
         moe.__class__ = MoE
 
+        moe._compute_experts = lambda *args, **kwargs: 2 * MoE._compute_experts(moe, *args, **kwargs)
+        for call in (run, torch.compile(run, fullgraph=True)):
+            assert torch.equal(call(moe, x)[0], 2 * y)
+        del moe._compute_experts
+
         for p in moe.parameters():
             p.data = p.data.transpose(-1, -2).contiguous().transpose(-1, -2)
         assert not moe.c_fc.weight.is_contiguous()
