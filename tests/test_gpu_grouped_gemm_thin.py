@@ -99,6 +99,13 @@ def test_layer_without_backward_in_other_forms(T):
             assert torch.equal(call(moe, x)[0], 2 * y)
         del moe._compute_experts
 
+        moe.fuse_swiglu_backward = False
+        moe.c_proj.cuda_forward = lambda **kwargs: 2 * type(moe.c_proj).cuda_forward(moe.c_proj, **kwargs)
+        assert torch.equal(run(moe, x)[0], 2 * y)
+        moe.fuse_swiglu_backward = True
+        assert torch.equal(run(moe, x)[0], y)
+        del moe.c_proj.cuda_forward
+
         for p in moe.parameters():
             p.data = p.data.transpose(-1, -2).contiguous().transpose(-1, -2)
         assert not moe.c_fc.weight.is_contiguous()
