@@ -65,10 +65,15 @@ def test_layer_without_backward_equals_the_training_forward(T, k, E, bias):
     assert torch.equal(logits, expect_logits) and torch.equal(y, expect)
 
 
+def no_grad_sum(run, moe, x):
+    with torch.no_grad():  # (inside the transform, where the grad mode outside does not count)
+        return run(moe, x)[0].float().sum()
+
+
 @pytest.mark.parametrize("T", [7, 100, 300])  # one native call; more than 64 and than 1024 (token, choice) slots
 def test_layer_without_backward_in_other_forms(T):
     """what the general path takes or refuses is taken or refused on the kernels for a few rows as well: tracing without a
-    graph break, weights of any strides, forward-mode AD (refused), a subclass's own expert computation"""
+    graph break, weights of any strides, forward-mode AD and functorch transforms (refused), a subclass's own expert computation"""
     from fma import KernelBackend, MoE, swiglu_packed
 
     torch.manual_seed(T)
@@ -85,6 +90,9 @@ def test_layer_without_backward_in_other_forms(T):
         with forward_ad.dual_level():
             with pytest.raises(NotImplementedError):
                 run(moe, forward_ad.make_dual(x, torch.ones_like(x)))
+        for transform in (torch.func.grad, torch.vmap):
+            with pytest.raises(RuntimeError):
+                transform(lambda x: no_grad_sum(run, moe, x))(x[None] if transform is torch.vmap else x)
 
         class Doubled(MoE):
             def _compute_experts(self, *args, **kwargs):
