@@ -9,7 +9,7 @@
 //  * no workgroup barrier anywhere: a wavefront fills a private ring of LDS stages by direct global -> LDS loads, each
 //    instruction 8 rows x 128 bytes (whole cache lines), waits with a counted vmcnt and multiplies; 6 such wavefronts (3 of the
 //    64-row kind) fit a compute unit's LDS and keep 70 to 90 KB in flight there;
-//  * the weight loads carry the non-temporal hint: every line is used by one wavefront only. A plain read kernel over 1.9 GB
+//  * the weight loads carry the non-temporal hint where every line is used by one wavefront only. A plain read kernel over 1.9 GB
 //    measures 6.3 TB/s without and 7.1 to 7.5 TB/s with it; this kernel 5.7 and 6.3 TB/s (up), 6.0 and 6.9 TB/s (down). The
 //    tokens, which every wavefront of an expert reads, are loaded without it (with it: +5 % time at 13 rows per expert).
 // Measured, bf16, up / down projection, weights from HBM (three sets in turn), against the tile kernel:
@@ -19,6 +19,16 @@
 //   hidden 4096, I 1536, E 128, k 8, 100 tokens: 611 / 290 us -> 506 / 244 us
 // Tried: 256 bytes per row and instruction (-0 to +8 % time), deeper rings with fewer wavefronts (0 to +10 %), rings of three
 // stages with eight wavefronts (+3 % on the large shapes, -2 % on the small).
+// An expert with more rows than a pass holds (32, or 64 of the other kind) streams its weights once per pass. The passes run
+// side by side, eight workgroups apart, in step (all with the token blocks of a full pass) and without the non-temporal hint, so that
+// the second pass finds the lines in the XCD's L2. Whole layer, us: the tile kernel / one wavefront taking the passes one after
+// the other / this, at uneven routing:
+//   hidden 2048, I 768, E 128, k 8, 512 tokens, one expert in every token's choice: 355 / 440 / 303
+//   hidden 2048, I 768, E 256, k 8, 1024 tokens, two experts in every choice:       619 / 963 / 567
+//   hidden 4096, I 14336, E 8, k 2, 64 tokens, all with the same two experts:        255 / 361 / 243
+//   hidden 4096, I 1536, E 128, k 8, 128 tokens, all with the same eight experts:    223 / 271 / 190
+// With the hint the last two take 269 and 215 us; with the smaller token blocks of a short last pass, which then runs ahead of the
+// others, 48 tokens of the third take 286 instead of 230 us.
 #include "gemm_parts.h"
 
 namespace fmahip {
@@ -35,7 +45,8 @@ struct Args {
     const uint32_t* offsets;   // [E] inclusive prefix of counts
     uint32_t E, N, K;
     uint32_t divisor, x_rows;
-    uint32_t units;  // wavefronts per expert
+    uint32_t units;  // wavefronts per pass of an expert
+    uint32_t slots;  // passes of an expert that run side by side
 };
 
 constexpr uint32_t kKB = 128;  // bytes of a row per step: one cache line
@@ -59,8 +70,9 @@ struct Config<64> {  // more: a token fragment feeds twice as many instructions
     static constexpr uint32_t kMaxTokens = 64;
 };
 
-// ROWS weight rows from column n0 on (swiglu: half of them "up", half "gate") times `rows` <= 16 TB rows from grouped row row0
-template <typename EL, int ROWS, bool GLU, bool BIAS, int TB>
+// ROWS weight rows from column n0 on (swiglu: half of them "up", half "gate") times `rows` <= 16 TB rows from grouped row row0.
+// STREAM: weights with the non-temporal hint, for lines that no other wavefront reads.
+template <typename EL, int ROWS, bool GLU, bool BIAS, int TB, bool STREAM>
 __device__ __forceinline__ void unit(const Args& a, uint8_t* lds, uint32_t e, uint32_t row0, uint32_t rows, uint32_t n0) {
     using frag = typename EL::frag;
     constexpr int WB = ROWS / 16;
@@ -103,7 +115,7 @@ __device__ __forceinline__ void unit(const Args& a, uint8_t* lds, uint32_t e, ui
             const uint32_t rel = GLU ? (uint32_t)(i % (kWI / 2)) * kRPI : (uint32_t)i * kRPI;
             uint32_t v = lr * K2 + chunk * 16u;
             if (last && kb + chunk * 16u >= K2) v = kOutOfRange;
-            load_lds<true>(GLU && i >= kWI / 2 ? rw1 : rw0, v, rel * K2 + kb, stage + (uint32_t)i * 1024u);
+            load_lds<STREAM>(GLU && i >= kWI / 2 ? rw1 : rw0, v, rel * K2 + kb, stage + (uint32_t)i * 1024u);
         }
 #pragma unroll
         for (int i = 0; i < kTI; ++i) {
@@ -181,53 +193,78 @@ __device__ __forceinline__ void unit(const Args& a, uint8_t* lds, uint32_t e, ui
     }
 }
 
-// Workgroup = one wavefront: unit blockIdx.x % units of the (blockIdx.x / units)-th expert that has rows. The host does not know
-// how many experts have rows; workgroups beyond them end at once.
+// Workgroup = one wavefront: one unit of one pass of an expert, of which up to a.slots run side by side. The host does not know
+// how many experts have rows, nor how many passes they take: workgroups beyond the last end at once.
 template <typename EL, int ROWS, bool GLU, bool BIAS>
 __global__ __launch_bounds__(64) void thin_gemm_kernel(const Args a) {
     __shared__ __attribute__((aligned(1024))) uint8_t lds[Config<ROWS>::kLds];
+    constexpr uint32_t kMax = Config<ROWS>::kMaxTokens;
     const uint32_t lane = threadIdx.x;
-    const uint32_t j = blockIdx.x / a.units, u = blockIdx.x % a.units;
-    uint32_t e = a.E, seen = 0;
+    const uint32_t j = blockIdx.x / a.units;  // slot, counted over all experts
+    uint32_t e = a.E, seen = 0, slots = 1;
     for (uint32_t base = 0; base < a.E; base += 64) {
         const uint32_t m = base + lane < a.E ? a.counts[base + lane] : 0u;
-        const uint64_t mask = __ballot(m != 0);
-        const uint32_t here = (uint32_t)__popcll(mask);
+        uint32_t before, here, mine = m != 0 ? 1u : 0u;  // slots of the experts before this lane's, of all 64, of this lane's
+        if (__ballot(m > kMax) == 0) {
+            const uint64_t mask = __ballot(m != 0);
+            before = (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
+            here = (uint32_t)__popcll(mask);
+        } else {
+            mine = (m + kMax - 1) / kMax;
+            mine = mine < a.slots ? mine : a.slots;
+            before = wave_inclusive_scan<uint32_t>(mine);
+            here = (uint32_t)__builtin_amdgcn_readlane((int)before, 63);
+            before -= mine;
+        }
         if (seen + here > j) {
-            const uint32_t rank = (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
-            e = base + (uint32_t)__builtin_ctzll(__ballot(m != 0 && rank == j - seen));
+            const uint32_t src = (uint32_t)__builtin_ctzll(__ballot(before <= j - seen && j - seen < before + mine));
+            e = base + src;
+            slots = (uint32_t)__builtin_amdgcn_readlane((int)mine, (int)src);
+            seen += (uint32_t)__builtin_amdgcn_readlane((int)before, (int)src);
             break;
         }
         seen += here;
     }
     e = uniform(e);
     if (e >= a.E) return;
-    uint32_t left = uniform(a.counts[e]);
-    uint32_t row0 = uniform(a.offsets[e]) - left;
+    uint32_t slot = 0, u = blockIdx.x - seen * a.units;
+    if (__builtin_expect(slots > 1, 0)) {
+        const uint32_t whole = a.units & ~7u;  // the last units of an expert, fewer than eight, lie that many apart
+        if (u < whole * slots) {
+            slot = u / 8u % slots;
+            u = u / (8u * slots) * 8u + u % 8u;
+        } else {
+            u -= whole * slots;
+            slot = u / (a.units - whole);
+            u = whole + u % (a.units - whole);
+        }
+    }
+    const uint32_t rows = uniform(a.counts[e]);
+    const uint32_t first = uniform(a.offsets[e]) - rows;
     const uint32_t n0 = u * (GLU ? ROWS / 2 : ROWS);
-    // an expert with more rows than a pass holds streams its weights once per pass
-    while (left) {
-        constexpr uint32_t kMax = Config<ROWS>::kMaxTokens;
-        if (left <= 16) {
-            unit<EL, ROWS, GLU, BIAS, 1>(a, lds, e, row0, left, n0);
-            break;
-        }
-        if (kMax > 32 && left <= 32) {
-            unit<EL, ROWS, GLU, BIAS, 2>(a, lds, e, row0, left, n0);
-            break;
-        }
-        const uint32_t take = left < kMax ? left : kMax;
-        unit<EL, ROWS, GLU, BIAS, kMax / 16>(a, lds, e, row0, take, n0);
-        row0 += take;
-        left -= take;
+    if (__builtin_expect(slots > 1, 0)) {
+        for (uint32_t at = slot * kMax; at < rows; at += slots * kMax)
+            unit<EL, ROWS, GLU, BIAS, kMax / 16, false>(a, lds, e, first + at, rows - at < kMax ? rows - at : kMax, n0);
+    } else if (rows <= 16) {
+        unit<EL, ROWS, GLU, BIAS, 1, true>(a, lds, e, first, rows, n0);
+    } else if (kMax > 32 && rows <= 32) {
+        unit<EL, ROWS, GLU, BIAS, 2, true>(a, lds, e, first, rows, n0);
+    } else {
+        unit<EL, ROWS, GLU, BIAS, kMax / 16, true>(a, lds, e, first, rows, n0);
     }
 }
 
 template <typename EL, int ROWS>
-int launch(Args a, bool glu, int64_t groups, hipStream_t st) {
+int launch(Args a, bool glu, int64_t R, int64_t groups, hipStream_t st) {
     const uint32_t cols = glu ? a.N / 2 : a.N, per = glu ? ROWS / 2 : ROWS;
     a.units = (cols + per - 1) / per;
-    const dim3 grid((uint32_t)(groups * a.units)), block(64);
+    // slots: one for every expert with rows, and one more for every kMaxTokens rows beyond its first; the grid stays far below the
+    // launch limit of 2^32 threads
+    constexpr int64_t kMaxSlots = 16, kMaxGrid = 1 << 25;
+    const int64_t most = kMaxGrid / (groups * a.units);
+    a.slots = (uint32_t)(most < 1 ? 1 : (most < kMaxSlots ? most : kMaxSlots));
+    const int64_t extra = (R - groups) / Config<ROWS>::kMaxTokens, spare = groups * (a.slots - 1);
+    const dim3 grid((uint32_t)((groups + (extra < spare ? extra : spare)) * a.units)), block(64);
     if (glu) {
         if (a.bias) hipLaunchKernelGGL((thin_gemm_kernel<EL, ROWS, true, true>), grid, block, 0, st, a);
         else hipLaunchKernelGGL((thin_gemm_kernel<EL, ROWS, true, false>), grid, block, 0, st, a);
@@ -287,6 +324,6 @@ extern "C" int fma_grouped_gemm_thin(const void* x, int64_t x_rows, const int32_
     // with E 128 at 6 rows 506 / 244 against 531 / 250 us, E 64 at one row 16.8 / 9.3 against 18.6 / 11.6 us.
     const bool wide = R > 16 * groups;
     if (dtype == FMA_BF16)
-        return wide ? thin::launch<ElemBf16, 64>(a, swiglu != 0, groups, st) : thin::launch<ElemBf16, 32>(a, swiglu != 0, groups, st);
-    return wide ? thin::launch<ElemF16, 64>(a, swiglu != 0, groups, st) : thin::launch<ElemF16, 32>(a, swiglu != 0, groups, st);
+        return wide ? thin::launch<ElemBf16, 64>(a, swiglu != 0, R, groups, st) : thin::launch<ElemBf16, 32>(a, swiglu != 0, R, groups, st);
+    return wide ? thin::launch<ElemF16, 64>(a, swiglu != 0, R, groups, st) : thin::launch<ElemF16, 32>(a, swiglu != 0, R, groups, st);
 }

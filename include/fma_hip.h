@@ -270,8 +270,8 @@ int fma_grouped_gemm_gathered(const void* x, int64_t x_rows, const int32_t* row_
 /* The forward product for groups of a few rows each (a decode step): out_e = x_e W_e^T (+ bias_e), with swiglu (N = 2 I)
  * out = swiglu_packed of it, [R, I]. Rows packed (row_index NULL) or picked as x[row_index[i] / divisor]. counts and offsets
  * (inclusive) as fma_moe_build_index returns them, R their total. Same results, bit for bit, as fma_grouped_gemm_ragged,
- * fma_grouped_gemm_swiglu and fma_grouped_gemm_gathered; any group size is computed, groups of more than 64 rows stream
- * their weights once per 64 rows. Same references as fma_grouped_gemm_gathered. */
+ * fma_grouped_gemm_swiglu and fma_grouped_gemm_gathered; any group size is computed, a group streams its
+ * weights once per 32 rows (per 64 rows where R is more than 16 rows per group, the groups counted as min(R, E)). Same references as fma_grouped_gemm_gathered. */
 int fma_grouped_gemm_thin(const void* x, int64_t x_rows, const int32_t* row_index, int32_t divisor, const void* W,
                           const void* bias, void* out, const uint32_t* counts, const uint32_t* offsets, int64_t R,
                           int64_t E, int64_t N, int64_t K, int swiglu, int dtype, void* stream);

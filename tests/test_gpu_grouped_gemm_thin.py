@@ -25,6 +25,9 @@ pytestmark = pytest.mark.gpu
         ([64, 65, 0, 130, 16, 17], 144, 2056),
         ([7, 31, 64], 4096, 1408),
         ([1] * 70 + [0] * 20 + [3] * 7, 64, 192),
+        # several passes of an expert, side by side and more of them than that (16): 32 rows each, then 64
+        ([1] * 70 + [600, 0, 33, 2, 64], 336, 136),
+        ([1100, 0, 65, 3], 336, 136),
     ],
 )
 def test_thin_product_equals_the_tile_kernel(sizes, N, K, swiglu, bias, dtype):
