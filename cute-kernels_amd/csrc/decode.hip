@@ -237,7 +237,8 @@ int64_t fma_moe_decode_workspace_bytes(int64_t T, int64_t H, int64_t I, int64_t 
     if (T < 0 || H < 0 || I < 0 || E < 0 || top_k < 0) return 0;
     using fmahip::round_up;
     const int64_t R = T * top_k;
-    return 2 * round_up(4 * E) + 2 * round_up(4 * R) + round_up(2 * R) + round_up(2 * R * I) + round_up(2 * R * H);
+    return 2 * round_up(4 * E) + 2 * round_up(4 * R) + round_up(2 * R) + round_up(2 * R * H) +
+           round_up(fma_thin_swiglu_experts_workspace_bytes(R, I));
 }
 
 int fma_moe_decode(const void* x, const void* gate_weight, const void* W1, const void* bias1, const void* W2, const void* bias2,
@@ -260,13 +261,14 @@ int fma_moe_decode(const void* x, const void* gate_weight, const void* W1, const
     int32_t* perm = (int32_t*)take(4 * R);
     int32_t* inv = (int32_t*)take(4 * R);
     void* weights = take(2 * R);
-    void* act = take(2 * R * I);
     void* out = take(2 * R * H);
+    const int64_t experts_bytes = fma_thin_swiglu_experts_workspace_bytes(R, I);
+    void* experts = take(experts_bytes);
     int rc = fma_router_topk_index(x, gate_weight, T, H, E, top_k, logits, weights, counts, offsets, perm, inv, dtype, stream);
     if (rc) return rc;
-    rc = fma_grouped_gemm_thin(x, T, perm, (int32_t)top_k, W1, bias1, act, counts, offsets, R, E, 2 * I, H, 1, dtype, stream);
-    if (rc) return rc;
-    rc = fma_grouped_gemm_thin(act, R, nullptr, 1, W2, bias2, out, counts, offsets, R, E, H, I, 0, dtype, stream);
+    // (a token's choices are distinct: no expert has more than T rows)
+    rc = fma_thin_swiglu_experts(x, T, perm, (int32_t)top_k, W1, bias1, W2, bias2, out, counts, offsets, R, T, E, H, I, experts,
+                                 experts_bytes, dtype, stream);
     if (rc) return rc;
     return fma_combine(out, inv, weights, T, top_k, H, y, dtype, stream);
 }

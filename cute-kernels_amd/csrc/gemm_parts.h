@@ -166,6 +166,19 @@ __device__ __forceinline__ u32x4 make_rsrc_words(const uint16_t* p, uint32_t byt
 __device__ __forceinline__ uint64_t uniform(uint64_t x) {
     return ((uint64_t)uniform((uint32_t)(x >> 32)) << 32) | uniform((uint32_t)x);
 }
+// Whether groups take so many passes of 2^pass_bits rows that the streaming kernel of thin_experts.hip leaves the product to the
+// tile kernel: 1.75 and more per group with rows, on average (measured in thin_experts.hip). All lanes call; the same in every lane.
+__device__ __forceinline__ bool takes_many_passes(const uint32_t* sizes, uint32_t E, uint32_t pass_bits, uint32_t lane) {
+    uint32_t passes = 0, groups = 0;
+    for (uint32_t base = 0; base < E; base += 64) {
+        const uint32_t m = base + lane < E ? sizes[base + lane] : 0u;
+        passes += (m >> pass_bits) + ((m & ((1u << pass_bits) - 1u)) != 0 ? 1u : 0u);
+        groups += (uint32_t)__popcll(__ballot(m != 0));
+    }
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) passes += (uint32_t)__shfl_xor((int)passes, d, 64);
+    return uniform(passes) * 4u >= groups * 7u;
+}
 constexpr uint32_t kOutOfRange = 0x80000000u;  // lane offset no descriptor of this kernel reaches (sizes stay < 2^31)
 
 

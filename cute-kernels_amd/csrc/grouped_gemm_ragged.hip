@@ -73,6 +73,10 @@ struct Args {
     // last part can end inside a step or on an odd one); part s of packed row r goes to partial[(s * rows + r) * n ..]
     float* partial;
     uint32_t splits, split_steps, rows;
+    // not NULL: the kernel runs only if *taken, which it decides (takes_many_passes) and writes first if pass_bits is not 0;
+    // otherwise the streaming kernel behind it computes the product (thin_experts.hip)
+    uint32_t* taken;
+    uint32_t pass_bits;
 };
 
 // s_waitcnt immediate: vmcnt(vm), and lgkmcnt(0) too if lgkm0 (expcnt untouched)
@@ -141,6 +145,19 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
     const uint32_t wm = wave / NWN;
     const uint32_t wn = wave % NWN;
     const uint32_t E = args.E;
+
+    if constexpr (A_KC && B_KC && !VARY_K && (EPI == EPI_PLAIN || EPI == EPI_SWIGLU_ACT)) {
+        if (args.taken) {
+            uint32_t take;
+            if (args.pass_bits) {
+                take = takes_many_passes(args.sizes, E, args.pass_bits, lane) ? 1u : 0u;
+                if (blockIdx.x == 0 && tid == 0) *args.taken = take;
+            } else {
+                take = *args.taken;
+            }
+            if (!take) return;
+        }
+    }
 
     // The dimensions all groups share. Called with per-group arrays of all three dimensions (fma_grouped_gemm), the kernel
     // first looks whether the launch has its form: rows vary -> N and K the same for every group; reduction varies -> M and
@@ -1563,9 +1580,10 @@ int launch_split(const Args& args, bool b_kc, hipStream_t st) {
 
 // The forward product of an expert projection, out_e = x_e W_e^T (+ bias_e), with the rows of x_e packed (row_index
 // NULL) or picked through row_index; swiglu: N = 2 I, out is the pre-activation (may be NULL) and act its activation.
+// taken, pass_bits: see Args.
 int up_projection(const char* who, const void* x, int64_t x_rows, const int32_t* row_index, int32_t divisor, const void* W,
                   const void* bias, void* out, void* act, const uint32_t* M_arr, int64_t E, int64_t N, int64_t K, int swiglu,
-                  int dtype, hipStream_t st) {
+                  int dtype, hipStream_t st, uint32_t* taken = nullptr, uint32_t pass_bits = 0) {
     FMA_REQUIRE(dtype == FMA_BF16 || dtype == FMA_F16, dtype_bytes(dtype) ? FMA_ERR_UNSUPPORTED : FMA_ERR_BAD_DTYPE,
                 "%s: bf16 and fp16 operands are implemented (dtype code %d)", who, dtype);
     FMA_REQUIRE(E >= 0, FMA_ERR_BAD_SIZE, "%s: negative group count %lld", who, (long long)E);
@@ -1602,6 +1620,8 @@ int up_projection(const char* who, const void* x, int64_t x_rows, const int32_t*
     args.n = (uint32_t)N;
     args.k = (uint32_t)K;
     args.alpha = 1.0f;
+    args.taken = taken;
+    args.pass_bits = pass_bits;
     // whether the pre-activation is stored is a compile-time property of the kernel: the epilogue is then one
     // straight-line block
     if (!swiglu) return dtype == FMA_BF16 ? launch_forward<ElemBf16, EPI_PLAIN>(args, st) : launch_forward<ElemF16, EPI_PLAIN>(args, st);

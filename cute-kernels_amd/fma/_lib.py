@@ -58,6 +58,10 @@ SIGNATURES = {
     "fma_moe_decode_workspace_bytes": (_i64, [_i64, _i64, _i64, _i64, _i64]),
     "fma_moe_decode": (_i32, [_p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _p, _p, _p, _i64, _i32, _p]),
     "fma_grouped_gemm_thin": (_i32, [_p, _i64, _p, _i32, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i32, _i32, _p]),
+    "fma_thin_swiglu_experts_workspace_bytes": (_i64, [_i64, _i64]),
+    "fma_thin_swiglu_experts": (
+        _i32, [_p, _i64, _p, _i32, _p, _p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i64, _i64, _p, _i64, _i32, _p],
+    ),
     "fma_grouped_gemm_swiglu": (_i32, [_p, _p, _p, _p, _p, _p, _i64, _i64, _i64, _i32, _p]),
     "fma_expert_bias_add": (_i32, [_p, _p, _p, _i64, _i64, _i64, _i32, _p]),
     "fma_expert_bias_grad_workspace_bytes": (_i64, [_i64, _i64, _i64]),

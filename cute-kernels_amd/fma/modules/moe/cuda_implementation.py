@@ -362,6 +362,47 @@ def grouped_gemm_thin_cuda(
     _lib.check(rc, "grouped_gemm_thin_cuda")
 
 
+@hip_op("thin_swiglu_experts_cuda", mutates_args={"output"})
+def thin_swiglu_experts_cuda(
+    x: torch.Tensor,
+    row_index: torch.Tensor,
+    divisor: int,
+    weight1: torch.Tensor,
+    bias1: torch.Tensor | None,
+    weight2: torch.Tensor,
+    bias2: torch.Tensor | None,
+    counts: torch.Tensor,
+    offsets: torch.Tensor,
+    max_rows: int,
+    output: torch.Tensor,
+) -> None:
+    """Both projections of a SwiGLU layer's experts for a few rows each: output [R, H] from the rows x[row_index[i] // divisor], of
+    which no expert has more than max_rows (fma_thin_swiglu_experts)."""
+    _lib.require_gpu(x, row_index, weight1, bias1, weight2, bias2, counts, offsets, output)
+    E, N, H = weight1.shape
+    I, R = N // 2, output.size(0)
+    assert N % 2 == 0 and x.dim() == 2 and x.size(1) == H and weight2.shape == (E, H, I) and output.shape == (R, H)
+    assert x.dtype == weight1.dtype == weight2.dtype == output.dtype
+    assert row_index.dtype == torch.int32 and row_index.numel() == R
+    assert counts.dtype == offsets.dtype == torch.uint32 and counts.numel() == offsets.numel() == E
+    assert bias1 is None or (bias1.shape == (E, N) and bias1.dtype == x.dtype)
+    assert bias2 is None or (bias2.shape == (E, H) and bias2.dtype == x.dtype)
+    for t in (x, row_index, weight1, bias1, weight2, bias2, counts, offsets, output):
+        assert t is None or t.is_contiguous()
+    if output.numel() == 0:
+        return
+    lib = _lib.load()
+    with _lib.on_device(x.device):
+        # the activation and the kernels' word to each other; owned by this call
+        workspace = x.new_empty(lib.fma_thin_swiglu_experts_workspace_bytes(R, I), dtype=torch.uint8)
+        rc = lib.fma_thin_swiglu_experts(
+            x.data_ptr(), x.size(0), row_index.data_ptr(), divisor, weight1.data_ptr(), _lib.ptr(bias1), weight2.data_ptr(),
+            _lib.ptr(bias2), output.data_ptr(), counts.data_ptr(), offsets.data_ptr(), R, max_rows, E, H, I,
+            workspace.data_ptr(), workspace.numel(), _lib.dtype_code(x.dtype), _lib.current_stream(x.device),
+        )
+    _lib.check(rc, "thin_swiglu_experts_cuda")
+
+
 @hip_op("moe_decode_cuda", mutates_args={"output", "logits"})
 def moe_decode_cuda(
     x: torch.Tensor,
@@ -983,11 +1024,9 @@ def thin_swiglu_experts(
 ) -> torch.Tensor:  # fmt: skip
     """gathered_swiglu_experts without a backward, for a few rows per expert: same values, bit for bit, where the second
     projection's reduction is not split there (grouped_gemm_ragged_cuda), up to the order of its fp32 sums where it is"""
-    R = perm.numel()
-    act = torch.empty(R, weight2.size(2), device=x.device, dtype=x.dtype)
-    output = torch.empty(R, weight2.size(1), device=x.device, dtype=x.dtype)
-    grouped_gemm_thin_cuda(x, perm, top_k, weight1, bias1, counts, offsets, act, True)
-    grouped_gemm_thin_cuda(act, None, 1, weight2, bias2, counts, offsets, output, False)
+    output = torch.empty(perm.numel(), weight2.size(1), device=x.device, dtype=x.dtype)
+    # (a token's choices are distinct: no expert has more rows than there are tokens)
+    thin_swiglu_experts_cuda(x, perm, top_k, weight1, bias1, weight2, bias2, counts, offsets, x.size(0), output)
     return output
 
 

@@ -276,6 +276,17 @@ int fma_grouped_gemm_thin(const void* x, int64_t x_rows, const int32_t* row_inde
                           const void* bias, void* out, const uint32_t* counts, const uint32_t* offsets, int64_t R,
                           int64_t E, int64_t N, int64_t K, int swiglu, int dtype, void* stream);
 
+/* Both projections of a SwiGLU layer's experts for a few rows each, without a backward: out [R, H] =
+ * swiglu_packed(x_e W1_e^T + bias1_e) W2_e^T + bias2_e, W1 [E, 2 I, H], W2 [E, H, I], biases or NULL; rows as for
+ * fma_grouped_gemm_thin, which computes it, in the same bits. No expert may have more than max_rows rows; where that leaves room
+ * for experts of more than four passes the tile kernels are enqueued in front and take both products if the experts with rows need
+ * 1.75 passes and more on average. The workspace needs no initialisation. */
+int64_t fma_thin_swiglu_experts_workspace_bytes(int64_t R, int64_t I);
+int fma_thin_swiglu_experts(const void* x, int64_t x_rows, const int32_t* row_index, int32_t divisor, const void* W1,
+                            const void* bias1, const void* W2, const void* bias2, void* out, const uint32_t* counts,
+                            const uint32_t* offsets, int64_t R, int64_t max_rows, int64_t E, int64_t H, int64_t I,
+                            void* workspace, int64_t workspace_bytes, int dtype, void* stream);
+
 /* Router and routing index of a few tokens in two launches: logits [T, E] and weights [T, k] as fma_router_topk, counts,
  * offsets, perm and inv as fma_moe_build_index of its choice (same bits). T * top_k <= FMA_MAX_DECODE_ROWS,
  * E <= FMA_MAX_DECODE_EXPERTS. */
@@ -284,7 +295,7 @@ int fma_router_topk_index(const void* x, const void* gate_weight, int64_t T, int
                           int dtype, void* stream);
 
 /* MoE.forward (fma/modules/moe/__init__.py:165-298) of a SwiGLU layer for a few tokens without a backward, enqueued by one
- * call: fma_router_topk_index, fma_grouped_gemm_thin for both projections, fma_combine. W1 [E, 2 I, H], W2 [E, H, I], biases
+ * call: fma_router_topk_index, fma_thin_swiglu_experts, fma_combine. W1 [E, 2 I, H], W2 [E, H, I], biases
  * [E, 2 I] / [E, H] or NULL; y [T, H] and logits [T, E] are written. The limits of fma_router_topk_index; the workspace needs no
  * initialisation. */
 int64_t fma_moe_decode_workspace_bytes(int64_t T, int64_t H, int64_t I, int64_t E, int64_t top_k);

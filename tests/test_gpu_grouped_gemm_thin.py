@@ -68,6 +68,27 @@ def test_layer_without_backward_equals_the_training_forward(T, k, E, bias):
     assert torch.equal(logits, expect_logits) and torch.equal(y, expect)
 
 
+# Routing on which the streaming kernel keeps the products, and on which it leaves them to the tile kernel (the choice is made on
+# the device where an expert can take more than four passes): passes of 32 rows, of 64 rows, the one-call forward pass.
+@pytest.mark.parametrize("hot", [0, 1, 4, 8])
+@pytest.mark.parametrize("T,k,E", [(129, 8, 128), (192, 8, 128), (333, 8, 128), (300, 2, 128), (1030, 8, 256)])
+@pytest.mark.parametrize("bias", [False, True])
+def test_layer_without_backward_under_uneven_routing(T, k, E, hot, bias):
+    from fma import KernelBackend, MoE, swiglu_packed
+
+    torch.manual_seed(T + hot)
+    moe = MoE(E, k, 136, 72, swiglu_packed, True, bias, 0.05).to(torch.bfloat16).to(DEV)
+    x = torch.randn(T, 136, device=DEV).bfloat16()
+    x[:, 0] = 8.0
+    with torch.no_grad():  # these experts are in every token's choice
+        moe.gate.weight[torch.randperm(E)[: min(hot, k)], 0] = 4.0
+    expect, expect_logits = moe(x, kernel_backend=KernelBackend.cuda)
+    with torch.no_grad():
+        for _ in range(2):  # (the second finds what the first left in the workspace)
+            y, logits = moe(x, kernel_backend=KernelBackend.cuda)
+            assert torch.equal(logits, expect_logits) and torch.equal(y, expect)
+
+
 def no_grad_sum(run, moe, x):
     with torch.no_grad():  # (inside the transform, where the grad mode outside does not count)
         return run(moe, x)[0].float().sum()
