@@ -185,3 +185,18 @@ def test_ensure_contiguous_inside_containers():
             tensors = [x for x in got if isinstance(x, torch.Tensor)]
             assert tensors and all(x.is_contiguous() and x.shape == t.shape for x in tensors)
             assert all(any(x is p for x in got) for p in plain if p is not None)
+
+
+def test_audit_knows_every_epilogue():
+    """isa_audit.py stops at a kernel instantiated with an epilogue whose stores it cannot count"""
+    import os
+    import re
+    import sys
+
+    root = os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "cute-kernels_amd")
+    sys.path.insert(0, root)
+    import isa_audit
+
+    with open(os.path.join(root, "csrc", "gemm_parts.h")) as f:
+        epilogues = dict(re.findall(r"constexpr int (EPI_\w+) = (\d+);", f.read()))
+    assert len(epilogues) >= 5 and {int(v) for v in epilogues.values()} == set(isa_audit.EPI_STORES)
