@@ -200,3 +200,21 @@ def test_audit_knows_every_epilogue():
     with open(os.path.join(root, "csrc", "gemm_parts.h")) as f:
         epilogues = dict(re.findall(r"constexpr int (EPI_\w+) = (\d+);", f.read()))
     assert len(epilogues) >= 5 and {int(v) for v in epilogues.values()} == set(isa_audit.EPI_STORES)
+
+
+def test_build_refuses_scratch_where_waits_are_counted():
+    """every source whose kernels wait with a hand-counted vmcnt is built under the check for register spills"""
+    import os
+    import re
+    import sys
+
+    root = os.path.join(os.path.dirname(os.path.abspath(__file__)), "..", "cute-kernels_amd")
+    sys.path.insert(0, root)
+    import build
+
+    for name in os.listdir(os.path.join(root, "csrc")):
+        with open(os.path.join(root, "csrc", name)) as f:
+            # (the definition in the header is wait_vm() itself; a wait for everything needs no count)
+            counts = re.findall(r"(?:wait_vm<|waitcnt_imm\(\(int\)|vmcnt\()([^>)\n]+)", f.read())
+        if name.endswith(".hip") and any(c.strip() != "0" for c in counts):
+            assert name in build.NO_SCRATCH_SOURCES, name
