@@ -261,9 +261,9 @@ int fma_moe_decode(const void* x, const void* gate_weight, const void* W1, const
     int32_t* perm = (int32_t*)take(4 * R);
     int32_t* inv = (int32_t*)take(4 * R);
     void* weights = take(2 * R);
-    void* out = take(2 * R * H);
     const int64_t experts_bytes = fma_thin_swiglu_experts_workspace_bytes(R, I);
     void* experts = take(experts_bytes);
+    void* out = take(2 * R * H);
     int rc = fma_router_topk_index(x, gate_weight, T, H, E, top_k, logits, weights, counts, offsets, perm, inv, dtype, stream);
     if (rc) return rc;
     // (a token's choices are distinct: no expert has more than T rows)

@@ -200,20 +200,27 @@ __device__ __forceinline__ void unit(const Args& a, uint8_t* lds, uint32_t e, ui
     }
 }
 
+// What a launch has to reckon with. One kernel for all three takes 1 % longer at one to eight tokens.
+constexpr int ONE_PASS = 0;     // no expert has more rows than a pass (if one has, its passes follow one another)
+constexpr int MANY_PASSES = 1;  // some may have
+constexpr int MAY_YIELD = 2;    // and the tile kernel in front may have computed the product
+
 // Workgroup = one wavefront: one unit of one pass of an expert, of which up to a.slots run side by side. The host does not know
 // how many experts have rows, nor how many passes they take: workgroups beyond the last end at once.
-template <typename EL, int ROWS, bool GLU, bool BIAS>
+template <typename EL, int ROWS, bool GLU, bool BIAS, int PASSES>
 __global__ __launch_bounds__(64) void thin_gemm_kernel(const Args a) {
     __shared__ __attribute__((aligned(1024))) uint8_t lds[Config<ROWS>::kLds];
     constexpr uint32_t kMax = Config<ROWS>::kMaxTokens;
     const uint32_t lane = threadIdx.x;
-    if (a.taken && *a.taken) return;
+    if constexpr (PASSES == MAY_YIELD) {
+        if (*a.taken) return;
+    }
     const uint32_t j = blockIdx.x / a.units;  // slot, counted over all experts
     uint32_t e = a.E, seen = 0, slots = 1;
     for (uint32_t base = 0; base < a.E; base += 64) {
         const uint32_t m = base + lane < a.E ? a.counts[base + lane] : 0u;
         uint32_t before, here, mine = m != 0 ? 1u : 0u;  // slots of the experts before this lane's, of all 64, of this lane's
-        if (__ballot(m > kMax) == 0) {
+        if (PASSES == ONE_PASS || __ballot(m > kMax) == 0) {
             const uint64_t mask = __ballot(m != 0);
             before = (uint32_t)__popcll(mask & ((1ull << lane) - 1ull));
             here = (uint32_t)__popcll(mask);
@@ -236,7 +243,7 @@ __global__ __launch_bounds__(64) void thin_gemm_kernel(const Args a) {
     e = uniform(e);
     if (e >= a.E) return;
     uint32_t slot = 0, u = blockIdx.x - seen * a.units;
-    if (__builtin_expect(slots > 1, 0)) {
+    if (PASSES != ONE_PASS && __builtin_expect(slots > 1, 0)) {
         const uint32_t whole = a.units & ~7u;  // the last units of an expert, fewer than eight, lie that many apart
         if (u < whole * slots) {
             slot = u / 8u % slots;
@@ -247,40 +254,54 @@ __global__ __launch_bounds__(64) void thin_gemm_kernel(const Args a) {
             u = whole + u % (a.units - whole);
         }
     }
-    const uint32_t rows = uniform(a.counts[e]);
-    const uint32_t first = uniform(a.offsets[e]) - rows;
+    uint32_t rows = uniform(a.counts[e]);
+    uint32_t first = uniform(a.offsets[e]) - rows;
     const uint32_t n0 = u * (GLU ? ROWS / 2 : ROWS);
-    if (__builtin_expect(slots > 1, 0)) {
-        for (uint32_t at = slot * kMax; at < rows; at += slots * kMax)
-            unit<EL, ROWS, GLU, BIAS, kMax / 16, false>(a, lds, e, first + at, rows - at < kMax ? rows - at : kMax, n0);
-    } else if (rows <= 16) {
-        unit<EL, ROWS, GLU, BIAS, 1, true>(a, lds, e, first, rows, n0);
-    } else if (kMax > 32 && rows <= 32) {
-        unit<EL, ROWS, GLU, BIAS, 2, true>(a, lds, e, first, rows, n0);
-    } else {
-        unit<EL, ROWS, GLU, BIAS, kMax / 16, true>(a, lds, e, first, rows, n0);
+    if constexpr (PASSES != ONE_PASS) {
+        if (__builtin_expect(slots > 1, 0)) {
+            for (uint32_t at = slot * kMax; at < rows; at += slots * kMax)
+                unit<EL, ROWS, GLU, BIAS, kMax / 16, false>(a, lds, e, first + at, rows - at < kMax ? rows - at : kMax, n0);
+            return;
+        }
+    }
+    while (rows) {
+        if (rows <= 16) {
+            unit<EL, ROWS, GLU, BIAS, 1, true>(a, lds, e, first, rows, n0);
+            break;
+        }
+        if (kMax > 32 && rows <= 32) {
+            unit<EL, ROWS, GLU, BIAS, 2, true>(a, lds, e, first, rows, n0);
+            break;
+        }
+        const uint32_t take = rows < kMax ? rows : kMax;
+        unit<EL, ROWS, GLU, BIAS, kMax / 16, true>(a, lds, e, first, take, n0);
+        first += take;
+        rows -= take;
     }
 }
 
-template <typename EL, int ROWS>
+template <typename EL, int ROWS, int PASSES>
 int launch(Args a, bool glu, int64_t R, int64_t groups, hipStream_t st) {
     const uint32_t cols = glu ? a.N / 2 : a.N, per = glu ? ROWS / 2 : ROWS;
     a.units = (cols + per - 1) / per;
     // slots: one for every expert with rows, and one more for every kMaxTokens rows beyond its first; the grid stays far below the
     // launch limit of 2^32 threads
-    constexpr int64_t kMaxSlots = 16, kMaxGrid = 1 << 25;
+    constexpr int64_t kMaxSlots = PASSES == ONE_PASS ? 1 : 16, kMaxGrid = 1 << 25;
     const int64_t most = kMaxGrid / (groups * a.units);
     a.slots = (uint32_t)(most < 1 ? 1 : (most < kMaxSlots ? most : kMaxSlots));
     const int64_t extra = (R - groups) / Config<ROWS>::kMaxTokens, spare = groups * (a.slots - 1);
     const dim3 grid((uint32_t)((groups + (extra < spare ? extra : spare)) * a.units)), block(64);
-    if (glu) {
-        if (a.bias) hipLaunchKernelGGL((thin_gemm_kernel<EL, ROWS, true, true>), grid, block, 0, st, a);
-        else hipLaunchKernelGGL((thin_gemm_kernel<EL, ROWS, true, false>), grid, block, 0, st, a);
-    } else {
-        if (a.bias) hipLaunchKernelGGL((thin_gemm_kernel<EL, ROWS, false, true>), grid, block, 0, st, a);
-        else hipLaunchKernelGGL((thin_gemm_kernel<EL, ROWS, false, false>), grid, block, 0, st, a);
-    }
+    auto run = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, block, 0, st, a); };
+    if (glu) a.bias ? run(thin_gemm_kernel<EL, ROWS, true, true, PASSES>) : run(thin_gemm_kernel<EL, ROWS, true, false, PASSES>);
+    else a.bias ? run(thin_gemm_kernel<EL, ROWS, false, true, PASSES>) : run(thin_gemm_kernel<EL, ROWS, false, false, PASSES>);
     return launch_status("grouped_gemm_thin");
+}
+// max_rows: as in fma_thin_swiglu_experts, or 0 (not known)
+template <typename EL, int ROWS>
+int launch(const Args& a, bool glu, int64_t R, int64_t groups, int64_t max_rows, hipStream_t st) {
+    if (a.taken) return launch<EL, ROWS, MAY_YIELD>(a, glu, R, groups, st);
+    if (max_rows >= 1 && max_rows <= Config<ROWS>::kMaxTokens) return launch<EL, ROWS, ONE_PASS>(a, glu, R, groups, st);
+    return launch<EL, ROWS, MANY_PASSES>(a, glu, R, groups, st);
 }
 
 }  // namespace thin
@@ -323,8 +344,8 @@ int check(const char* who, const void* x, int64_t x_rows, const int32_t* row_ind
 
 // a product whose arguments check() has passed
 int product(const void* x, int64_t x_rows, const int32_t* row_index, int32_t divisor, const void* W, const void* bias, void* out,
-            const uint32_t* counts, const uint32_t* offsets, int64_t R, int64_t E, int64_t N, int64_t K, int swiglu,
-            const uint32_t* taken, int dtype, hipStream_t st) {
+            const uint32_t* counts, const uint32_t* offsets, int64_t R, int64_t max_rows, int64_t E, int64_t N, int64_t K,
+            int swiglu, const uint32_t* taken, int dtype, hipStream_t st) {
     if (E == 0 || R == 0) return FMA_OK;
     Args a{};
     a.x = (const uint16_t*)x;
@@ -341,9 +362,9 @@ int product(const void* x, int64_t x_rows, const int32_t* row_index, int32_t div
     a.x_rows = row_index ? (uint32_t)x_rows : 0u;
     a.taken = taken;
     const int64_t groups = R < E ? R : E;  // no more experts than rows can have rows
-    if (dtype == FMA_BF16)
-        return wide(R, E) ? launch<ElemBf16, 64>(a, swiglu != 0, R, groups, st) : launch<ElemBf16, 32>(a, swiglu != 0, R, groups, st);
-    return wide(R, E) ? launch<ElemF16, 64>(a, swiglu != 0, R, groups, st) : launch<ElemF16, 32>(a, swiglu != 0, R, groups, st);
+    const bool w = wide(R, E), glu = swiglu != 0;
+    if (dtype == FMA_BF16) return w ? launch<ElemBf16, 64>(a, glu, R, groups, max_rows, st) : launch<ElemBf16, 32>(a, glu, R, groups, max_rows, st);
+    return w ? launch<ElemF16, 64>(a, glu, R, groups, max_rows, st) : launch<ElemF16, 32>(a, glu, R, groups, max_rows, st);
 }
 
 }  // namespace thin
@@ -358,12 +379,12 @@ int fma_grouped_gemm_thin(const void* x, int64_t x_rows, const int32_t* row_inde
     using namespace fmahip::gemm;
     const int rc = thin::check("grouped_gemm_thin", x, x_rows, row_index, divisor, W, out, counts, offsets, R, E, N, K, swiglu, dtype);
     if (rc) return rc;
-    return thin::product(x, x_rows, row_index, divisor, W, bias, out, counts, offsets, R, E, N, K, swiglu, nullptr, dtype,
+    return thin::product(x, x_rows, row_index, divisor, W, bias, out, counts, offsets, R, 0, E, N, K, swiglu, nullptr, dtype,
                          (hipStream_t)stream);
 }
 
 int64_t fma_thin_swiglu_experts_workspace_bytes(int64_t R, int64_t I) {
-    return R < 0 || I < 0 ? 0 : 256 + 2 * R * I;
+    return R < 0 || I < 0 ? 0 : (2 * R * I + 255) / 256 * 256 + 16;  // the activation, the tile kernel's word
 }
 
 int fma_thin_swiglu_experts(const void* x, int64_t x_rows, const int32_t* row_index, int32_t divisor, const void* W1,
@@ -378,8 +399,8 @@ int fma_thin_swiglu_experts(const void* x, int64_t x_rows, const int32_t* row_in
     FMA_REQUIRE(workspace_bytes >= fma_thin_swiglu_experts_workspace_bytes(R, I) || E == 0 || R == 0, FMA_ERR_WORKSPACE_TOO_SMALL,
                 "%s: workspace of %lld bytes is smaller than the %lld needed", who, (long long)workspace_bytes,
                 (long long)fma_thin_swiglu_experts_workspace_bytes(R, I));
-    uint32_t* taken = (uint32_t*)workspace;
-    void* act = (uint8_t*)workspace + 256;
+    void* act = workspace;
+    uint32_t* taken = (uint32_t*)((uint8_t*)workspace + (2 * R * I + 255) / 256 * 256);
     int rc = thin::check(who, x, x_rows, row_index, divisor, W1, act, counts, offsets, R, E, 2 * I, H, 1, dtype);
     if (!rc) rc = thin::check(who, act, R, nullptr, 1, W2, out, counts, offsets, R, E, H, I, 0, dtype);
     if (rc || E == 0 || R == 0) return rc;
@@ -401,10 +422,11 @@ int fma_thin_swiglu_experts(const void* x, int64_t x_rows, const int32_t* row_in
     if (taken)
         rc = ragged::up_projection(who, x, x_rows, row_index, divisor, W1, bias1, nullptr, act, counts, E, 2 * I, H, 1, dtype, st,
                                    taken, pass_bits);
-    if (!rc) rc = thin::product(x, x_rows, row_index, divisor, W1, bias1, act, counts, offsets, R, E, 2 * I, H, 1, taken, dtype, st);
+    if (!rc) rc = thin::product(x, x_rows, row_index, divisor, W1, bias1, act, counts, offsets, R, max_rows, E, 2 * I, H, 1, taken, dtype,
+                               st);
     if (!rc && taken)
         rc = ragged::up_projection(who, act, R, nullptr, 1, W2, bias2, out, nullptr, counts, E, H, I, 0, dtype, st, taken, 0);
-    return rc ? rc : thin::product(act, R, nullptr, 1, W2, bias2, out, counts, offsets, R, E, H, I, 0, taken, dtype, st);
+    return rc ? rc : thin::product(act, R, nullptr, 1, W2, bias2, out, counts, offsets, R, max_rows, E, H, I, 0, taken, dtype, st);
 }
 
 }  // extern "C"
