@@ -29,10 +29,8 @@ def hip_op(name: str, mutates_args: Iterable[str]) -> Callable:
         mutated = [i for i, p in enumerate(inspect.signature(fn).parameters) if p in mutates_args]
 
         def body(*args) -> None:
-            for i in mutated:
-                # (an inference tensor has no version)
-                if i < len(args) and args[i] is not None and not args[i].is_inference():
-                    increment_version(args[i])
+            # (inference tensors have no version and are passed over)
+            increment_version([args[i] for i in mutated if i < len(args) and args[i] is not None])
             if not torch.is_grad_enabled():
                 return fn(*args)
             torch._C._set_grad_enabled(False)  # (torch.no_grad() would take 1.9 us)
