@@ -65,3 +65,24 @@ def test_split_equals_unsplit(dtype, tB, sizes, N, K, bias, alpha):
 @pytest.mark.parametrize("rows,E,N,K", [(65536, 128, 4096, 1536), (16, 8, 2048, 3000), (2042, 8, 2047, 8192), (0, 8, 2048, 8192)])
 def test_no_split_where_it_cannot_pay_or_run(rows, E, N, K):
     assert _lib.load().fma_grouped_gemm_ragged_workspace_bytes(rows, E, N, K, 1) == 0
+
+
+@pytest.mark.parametrize("tB", [True, False])
+@pytest.mark.parametrize("values", [[float("inf")], [float("inf"), float("-inf")], [float("nan"), 1.0]])
+def test_split_of_infinities_and_nan(values, tB):
+    """in different parts of the reduction, and against each other"""
+    sizes, N, K = [3, 130, 64], 264, 4104
+    E, R = len(sizes), sum(sizes)
+    g = torch.Generator(device=DEV).manual_seed(K)
+    A = torch.randint(-3, 4, (R, K), device=DEV, generator=g).bfloat16()
+    B = torch.randint(1, 4, (E, N, K) if tB else (E, K, N), device=DEV, generator=g).bfloat16()
+    for row in (1, 60, 196):
+        for i, v in enumerate(values):
+            A[row, [5, K - 3][i]] = v  # the first and the last part
+    nbytes = _lib.load().fma_grouped_gemm_ragged_workspace_bytes(R, E, N, K, int(tB))
+    assert nbytes >= 2 * R * N * 4
+    got, want = (_call(A, B, sizes, R, N, K, tB, None, 1.0, n) for n in (nbytes, 0))
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(got.nan_to_num(nan=0.0), want.nan_to_num(nan=0.0))
+    special = torch.zeros(R, dtype=torch.bool, device=DEV)
+    special[[1, 60, 196]] = True
+    assert torch.equal(torch.isfinite(got).all(1), ~special) and not torch.isfinite(got[special]).any()

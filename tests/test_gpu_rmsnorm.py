@@ -182,3 +182,39 @@ def test_backward_row_split_against_fp64(B, H):
     # a sum of at most B / 512 + 1 rows in fp32, then fp64; 16 more roundings for the terms themselves
     bound = (B // 512 + 17) * 2.0**-24 * (dy.double() * unit.detach()).abs().sum(0)
     assert bool(((leaves[2].grad - exact[2].grad).abs() <= bound).all())
+
+
+# more rows than workgroups, so that every workgroup takes several and the last ones one less: each number of vectors per thread
+# (1, 2, 4, 8), each type, without a weight too
+@pytest.mark.parametrize("has_weight", [True, False])
+@pytest.mark.parametrize(
+    "B,H,dtype",
+    [(1031, 4096, torch.float32), (1031, 8192, torch.float32), (1031, 8192, torch.bfloat16), (1031, 16384, torch.bfloat16),
+     (1031, 16384, torch.float16), (4609, 2048, torch.float16), (8197, 1024, torch.float16), (2000, 2880, torch.bfloat16)],
+)  # fmt: skip
+def test_backward_of_many_rows_against_fp64(B, H, dtype, has_weight):
+    from fma.ops.fused_residual_add_rmsnorm.cuda_implementation import fused_residual_add_rmsnorm_backward_cuda
+
+    g = torch.Generator(device=DEV).manual_seed(B + H)
+    s, dy, dr = (torch.randn(B, H, generator=g, device=DEV).to(dtype) for _ in range(3))
+    w = torch.randn(H, generator=g, device=DEV).to(dtype) if has_weight else None
+    dx, dres = torch.empty_like(s), torch.empty_like(s)
+    dw = torch.empty(H, device=DEV) if has_weight else None
+    fused_residual_add_rmsnorm_backward_cuda(s, w, dy, dr, None, dx, dres, dw, _EPSILON, 0.5)
+    rstd = torch.rsqrt(s.double().square().mean(-1, keepdim=True) + _EPSILON)
+    unit = s.double() * rstd
+    scaled = dy.double() * (w.double() if has_weight else 1.0)
+    want = (scaled - unit * (unit * scaled).mean(-1, keepdim=True)) * rstd + dr.double()
+    # one rounding to the type, and fp32 arithmetic on the terms: a thread adds up to 64 of a row's products one after the other, ten
+    # more levels join the threads, and some ten roundings make up a term
+    size = (scaled.abs() + unit.abs() * (unit * scaled).abs().mean(-1, keepdim=True)) * rstd + dr.double().abs()
+    unit_roundoff = {torch.float32: 2.0**-24, torch.float16: 2.0**-11, torch.bfloat16: 2.0**-8}[dtype]
+    bound = unit_roundoff * want.abs() + 84 * 2.0**-24 * size
+    assert bool(((dres.double() - want).abs() <= bound).all())
+    assert bool(((dx.double() - 0.5 * want).abs() <= 0.5 * bound + 2.0**-24).all())  # (fp16: below the smallest normal number)
+    if has_weight:
+        # at most B / 512 + 1 rows in fp32, then fp64; 16 more roundings for the terms and 74 for the mean square of a row, halved
+        # by the root; in a 16-bit type the normalised element of a term is the one that the forward hands on, rounded to the type
+        term = (B // 512 + 17 + 37) * 2.0**-24 + (unit_roundoff if dtype != torch.float32 else 0.0)
+        bound = term * (dy.double() * unit).abs().sum(0)
+        assert bool(((dw.double() - (dy.double() * unit).sum(0)).abs() <= bound).all())
