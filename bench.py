@@ -8,8 +8,9 @@ A step is one forward + backward of the expert path (index construction, gather,
 down-projection, router-weighted combine, and all their gradients) on synthetic, seeded inputs that are resident in HBM
 before the timed region. The router (gate linear, top-k, softmax) is upstream of the path and is not timed. Prints ONE
 JSON line: whole-layer tokens/s plus, measured in the same process with events on the launch stream, the duration of
-every kernel of the path against its roofline (bf16 MFMA peak for the grouped GEMMs, HBM peak for the row kernels and
-continuous_count), and the CPU oracle timed on this machine's host cores on a bounded sample.
+every kernel of the path and its fraction of its roofline (bf16 MFMA peak for the grouped GEMMs, HBM peak for the row kernels
+and continuous_count), and the CPU oracle timed on this machine's host cores on a bounded sample. The kernels' full records
+(spread, rates, bytes, operations) go to stderr, one JSON line per workload: the line on stdout stays within a few KB.
 """
 
 import argparse
@@ -369,17 +370,32 @@ def measure_workload(name, args, full):
                                                stream)), n=3, peak=PEAK_F32_TFLOPS)
         del a32, w32, o32
 
-    # the same two forward GEMMs on a batch of a few rows per expert (16 each, e.g. 64 tokens at top-2 of 8): there
-    # the kernels are a stream of the expert weights, so the roof is the HBM one and the bytes are the weights' (plus
-    # the few activation rows)
+    # a few rows per expert (16 each, e.g. 64 tokens at top-2 of 8) without a backward: the two projections on the streaming
+    # kernel, and the whole forward pass as one call with its router (evenly routed by chance, not by construction). A stream of the
+    # expert weights, so the roof is the HBM one and the bytes are the weights' (plus the few activation rows)
     M_dec = max(1, min(64, 128 // E))
     R_dec = M_dec * E
     counts_dec = torch.full((E,), M_dec, dtype=torch.int32, device=dev).view(torch.uint32)
-    hbm(f"small_batch_up_fwd(NT + SwiGLU, {M_dec} rows per expert, h not stored)", w1_b + R_dec * (H + I) * s,
-        lambda i: ok(lib.fma_grouped_gemm_swiglu(xg.data_ptr(), w1.data_ptr(), None, None, a.data_ptr(),
-                                                 counts_dec.data_ptr(), E, I, H, BF16, stream)), n=30, gemm_kernel=True)
-    hbm(f"small_batch_down_fwd(NT, {M_dec} rows per expert)", w2_b + R_dec * (H + I) * s,
-        lambda i: gemm(a, w2, o, counts_dec, VARY_M, 0, H, I, 0, 1), n=30, gemm_kernel=True)
+    offsets_dec = (torch.arange(1, E + 1, dtype=torch.int32, device=dev) * M_dec).view(torch.uint32)
+    hbm(f"small_batch_up_fwd(streaming, SwiGLU, {M_dec} rows per expert)", w1_b + R_dec * (H + I) * s,
+        lambda i: ok(lib.fma_grouped_gemm_thin(xg.data_ptr(), R_dec, None, 1, w1.data_ptr(), None, a.data_ptr(),
+                                               counts_dec.data_ptr(), offsets_dec.data_ptr(), R_dec, E, 2 * I, H, 1, BF16,
+                                               stream)), n=30, gemm_kernel=True)
+    hbm(f"small_batch_down_fwd(streaming, {M_dec} rows per expert)", w2_b + R_dec * (H + I) * s,
+        lambda i: ok(lib.fma_grouped_gemm_thin(a.data_ptr(), R_dec, None, 1, w2.data_ptr(), None, o.data_ptr(),
+                                               counts_dec.data_ptr(), offsets_dec.data_ptr(), R_dec, E, H, I, 0, BF16,
+                                               stream)), n=30, gemm_kernel=True)
+    T_dec = max(1, R_dec // k)
+    chosen = 1.0 - (1.0 - k / E) ** T_dec  # share of the experts that some token is expected to choose
+    if want(f"moe_decode({T_dec} tokens)", True):
+        gate = (torch.randn(E, H, device=dev) * 0.02).bfloat16()
+        y_dec, logits_dec = torch.empty(T_dec, H, **bf), torch.empty(T_dec, E, **bf)
+        ws_dec = torch.empty(lib.fma_moe_decode_workspace_bytes(T_dec, H, I, E, k), dtype=torch.uint8, device=dev)
+        hbm(f"moe_decode({T_dec} tokens)", int(chosen * (w1_b + w2_b)) + gate.numel() * s + 2 * T_dec * H * s,
+            lambda i: ok(lib.fma_moe_decode(x.data_ptr(), gate.data_ptr(), w1.data_ptr(), None, w2.data_ptr(), None, T_dec, H, I,
+                                            E, k, y_dec.data_ptr(), logits_dec.data_ptr(), ws_dec.data_ptr(), ws_dec.numel(),
+                                            BF16, stream)), n=30, gemm_kernel=True)
+        del gate, ws_dec
 
     # calibration for the profiler's FETCH_SIZE / WRITE_SIZE counters: a plain device copy of known size (ATen's
     # elementwise copy kernel): reads 1 GiB, writes 1 GiB
@@ -632,6 +648,12 @@ def cpu_baseline(context, name):
     return out
 
 
+def report_kernels(workload, kernels):
+    """{name: [median ms, fraction of the kernel's roofline if it has one]} for the line on stdout; the full records go to stderr"""
+    print(json.dumps({"workload": workload, "kernels": kernels}), file=sys.stderr, flush=True)
+    return {name: [round(k["ms"], 5)] + ([round(k["frac"], 4)] if "frac" in k else []) for name, k in kernels.items()}
+
+
 def main():
     args = parse_args()
     if args.gpus != 1:
@@ -674,7 +696,7 @@ def main():
         "layer_gemm_frac_of_peak": layer["layer_gemm_frac_of_peak"],
     }
     if kernels:
-        result["kernels"] = kernels
+        result["kernels_ms_and_frac"] = report_kernels(args.workload, kernels)
         dominant = kernels.get("up_projection_swiglu_fwd(NT)") or next(iter(kernels.values()))
         result["roofline"] = {
             "kernel": "ragged_gemm_kernel<NT, SwiGLU epilogue> (up-projection forward)",
@@ -702,7 +724,7 @@ def main():
         del context
         entry = {key: layer[key] for key in ("workload", "ms_per_step", "tokens_per_s", "ms_per_step_with_router",
                                              "ms_per_step_by_row_movement", "ms_forward_no_grad", "layer_gemm_tflops", "layer_gemm_frac_of_peak")}
-        entry["kernels"] = kernels
+        entry["kernels_ms_and_frac"] = report_kernels(name, kernels)
         result["workloads"][name] = entry
         torch.cuda.empty_cache()
 
