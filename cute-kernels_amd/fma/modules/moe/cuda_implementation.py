@@ -177,7 +177,12 @@ def grouped_gemm_ragged_cuda(
         nbytes = 0
         if not vary_k and not is_A_transposed and A.numel() >= rows * K:
             nbytes = lib.fma_grouped_gemm_ragged_workspace_bytes(rows, sizes.numel(), N, K, int(is_B_transposed))
-        workspace = torch.empty(nbytes, dtype=torch.uint8, device=A.device) if nbytes else None
+        workspace = None
+        if nbytes:
+            try:
+                workspace = torch.empty(nbytes, dtype=torch.uint8, device=A.device)
+            except torch.OutOfMemoryError:  # up to 256 MiB that the product can do without
+                nbytes = 0
         rc = lib.fma_grouped_gemm_ragged_split(
             a_ptr, b_ptr, output.data_ptr(), sizes.data_ptr(), _lib.ptr(bias), sizes.numel(),
             _lib.FMA_VARY_K if vary_k else _lib.FMA_VARY_M, M, N, K, int(is_A_transposed), int(is_B_transposed), 1.0,

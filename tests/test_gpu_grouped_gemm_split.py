@@ -86,3 +86,29 @@ def test_split_of_infinities_and_nan(values, tB):
     special = torch.zeros(R, dtype=torch.bool, device=DEV)
     special[[1, 60, 196]] = True
     assert torch.equal(torch.isfinite(got).all(1), ~special) and not torch.isfinite(got[special]).any()
+
+
+def test_product_runs_unsplit_where_the_sums_find_no_memory():
+    from fma.modules.moe import cuda_implementation as ci
+
+    sizes, N, K = [512] * 8, 4096, 14336
+    E, R = len(sizes), sum(sizes)
+    nbytes = _lib.load().fma_grouped_gemm_ragged_workspace_bytes(R, E, N, K, 1)
+    assert nbytes >= 64 << 20
+    g = torch.Generator(device=DEV).manual_seed(1)
+    A = torch.randint(-3, 4, (R, K), device=DEV, generator=g).bfloat16()
+    B = torch.randint(-3, 4, (E, N, K), device=DEV, generator=g).bfloat16()
+    s = torch.tensor(sizes, dtype=torch.int32, device=DEV).view(torch.uint32)
+    outputs = [torch.empty(R, N, device=DEV, dtype=torch.bfloat16) for _ in range(2)]
+    ci.grouped_gemm_ragged_cuda(A, B, outputs[0], s, False, 0, N, K, False, True)
+    torch.cuda.empty_cache()
+    try:  # a limit of this process's allocator that is below what it holds already: nothing more is to be had
+        torch.cuda.set_per_process_memory_fraction(1e-4)
+        held = []
+        with pytest.raises(torch.OutOfMemoryError):  # what is free inside of it is used up
+            for _ in range(200):
+                held.append(torch.empty(nbytes, dtype=torch.uint8, device=DEV))
+        ci.grouped_gemm_ragged_cuda(A, B, outputs[1], s, False, 0, N, K, False, True)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    assert torch.equal(*outputs)
