@@ -12,7 +12,7 @@
 // order (the reference adds them with atomics, in arrival order). The rows of a workgroup are a grid apart, so that the
 // rows in flight are neighbours in memory: against a contiguous chunk of rows per workgroup, whose concurrent streams are
 // equal power-of-two distances apart, [16384, 4096] bf16 took 131 instead of 139 us and [32768, 4096] 249 instead of 272 us
-// (both with two workgroups per compute unit).
+// (both with two workgroups per compute unit); few short rows are the exception (rows_together).
 #include "common.h"
 
 namespace fmahip {
@@ -172,8 +172,8 @@ template <typename T, int VPT, bool HAS_W>
 __global__ __launch_bounds__(kNormThreads) void rmsnorm_bwd_kernel(
     const Vec16<T>* __restrict__ added, const Vec16<T>* __restrict__ weight, const Vec16<T>* __restrict__ dy,
     const Vec16<T>* __restrict__ d_added_in, const float* __restrict__ denom, Vec16<T>* __restrict__ dx,
-    Vec16<T>* __restrict__ d_residual, float* __restrict__ dw_partial, int64_t B, int nvec, float inv_H, float eps,
-    float multiplier) {
+    Vec16<T>* __restrict__ d_residual, float* __restrict__ dw_partial, int64_t B, int64_t chunk, int nvec, float inv_H,
+    float eps, float multiplier) {
     constexpr int N = Vec16<T>::N;
     __shared__ float s_red[2][kNormWaves][2];
     const int tid = threadIdx.x;
@@ -202,12 +202,15 @@ __global__ __launch_bounds__(kNormThreads) void rmsnorm_bwd_kernel(
             }
         }
     };
-    if (blockIdx.x < B) fetch(rv, gv, av, blockIdx.x);
+    // chunk consecutive rows, or rows a grid apart (0)
+    const int64_t row0 = chunk ? (int64_t)blockIdx.x * chunk : blockIdx.x, step = chunk ? 1 : gridDim.x;
+    const int64_t row1 = chunk && row0 + chunk < B ? row0 + chunk : B;
+    if (row0 < row1) fetch(rv, gv, av, row0);
     int parity = 0;
-    for (int64_t row = blockIdx.x; row < B; row += gridDim.x, parity ^= 1) {
+    for (int64_t row = row0; row < row1; row += step, parity ^= 1) {
         const int64_t base = row * nvec;
         Vec16<T> rn[VPT], gn[VPT], an[VPT];
-        fetch(rn, gn, an, row + gridDim.x < B ? row + gridDim.x : row);  // after the last row: this row again, unused
+        fetch(rn, gn, an, row + step < row1 ? row + step : row);  // after the last row: this row again, unused
         float dot = 0.f, ss = 0.f;
 #pragma unroll
         for (int i = 0; i < VPT; ++i) {
@@ -362,6 +365,15 @@ int64_t backward_workgroups(int64_t B, int vpt, int64_t nvec) {
     return B < want ? (B > 0 ? B : 1) : want;
 }
 
+// Rows of a workgroup next to each other instead of a grid apart (see the top): for few rows of one vector per thread, where it
+// is the faster of the two. us apart / together: [4096, 2048] bf16 32.1 / 31.4, fp16 28.6 / 27.4, [4096, 1024] bf16 27.1 / 26.8, fp16
+// 23.5 / 22.5, fp32 27.1 / 25.6. With more vectors it gains nothing in bf16 ([8192, 8192] 208 / 210, [1200, 8192] 51 / 55) and costs
+// 4 to 8 % in fp16 and fp32.
+bool rows_together(int64_t B, int vpt, int64_t G) {
+    const int64_t cus = num_compute_units() > 0 ? num_compute_units() : 256;
+    return vpt == 1 && G == cus * kBwdPerCUFew && B >= 4 * G;  // (with fewer, whole workgroups would have no row)
+}
+
 // enough for every element type and alignment of [B, H]
 int64_t backward_workspace_bytes(int64_t B, int64_t H) {
     const int64_t few = backward_workgroups(B, 0, 0), full = backward_workgroups(B, 2, kNormThreads),
@@ -407,16 +419,16 @@ int launch_fwd(const void* x, const void* residual, const void* weight, void* ou
 template <typename T, int VPT>
 void launch_bwd_vec(bool has_w, dim3 grid, hipStream_t st, const void* added, const void* weight, const void* dy,
                     const void* d_added_in, const float* denom, void* dx, void* d_residual, float* partial, int64_t B,
-                    int nvec, float inv_H, float eps, float mult) {
+                    int64_t chunk, int nvec, float inv_H, float eps, float mult) {
     using V = Vec16<T>;
     if (has_w)
         hipLaunchKernelGGL((rmsnorm_bwd_kernel<T, VPT, true>), grid, dim3(kNormThreads), 0, st, (const V*)added,
                            (const V*)weight, (const V*)dy, (const V*)d_added_in, denom, (V*)dx, (V*)d_residual, partial, B,
-                           nvec, inv_H, eps, mult);
+                           chunk, nvec, inv_H, eps, mult);
     else
         hipLaunchKernelGGL((rmsnorm_bwd_kernel<T, VPT, false>), grid, dim3(kNormThreads), 0, st, (const V*)added,
                            (const V*)weight, (const V*)dy, (const V*)d_added_in, denom, (V*)dx, (V*)d_residual, partial, B,
-                           nvec, inv_H, eps, mult);
+                           chunk, nvec, inv_H, eps, mult);
 }
 
 template <typename T>
@@ -428,13 +440,14 @@ int launch_bwd(const void* added, const void* weight, const void* dy, const void
     const int nvec = (int)(H * (int64_t)sizeof(T) / 16);
     const int64_t G = backward_workgroups(B, vpt, nvec);
     const int64_t rows_per = (B + G - 1) / G;
+    const int64_t chunk = rows_together(B, vpt, G) ? rows_per : 0;
     const dim3 grid((uint32_t)G);
     const float inv_H = 1.0f / (float)H;
     switch (vpt) {
-        case 1: launch_bwd_vec<T, 1>(weight, grid, st, added, weight, dy, d_added_in, denom, dx, d_residual, partial, B, nvec, inv_H, eps, mult); break;
-        case 2: launch_bwd_vec<T, 2>(weight, grid, st, added, weight, dy, d_added_in, denom, dx, d_residual, partial, B, nvec, inv_H, eps, mult); break;
-        case 4: launch_bwd_vec<T, 4>(weight, grid, st, added, weight, dy, d_added_in, denom, dx, d_residual, partial, B, nvec, inv_H, eps, mult); break;
-        case 8: launch_bwd_vec<T, 8>(weight, grid, st, added, weight, dy, d_added_in, denom, dx, d_residual, partial, B, nvec, inv_H, eps, mult); break;
+        case 1: launch_bwd_vec<T, 1>(weight, grid, st, added, weight, dy, d_added_in, denom, dx, d_residual, partial, B, chunk, nvec, inv_H, eps, mult); break;
+        case 2: launch_bwd_vec<T, 2>(weight, grid, st, added, weight, dy, d_added_in, denom, dx, d_residual, partial, B, chunk, nvec, inv_H, eps, mult); break;
+        case 4: launch_bwd_vec<T, 4>(weight, grid, st, added, weight, dy, d_added_in, denom, dx, d_residual, partial, B, chunk, nvec, inv_H, eps, mult); break;
+        case 8: launch_bwd_vec<T, 8>(weight, grid, st, added, weight, dy, d_added_in, denom, dx, d_residual, partial, B, chunk, nvec, inv_H, eps, mult); break;
         default:
             hipLaunchKernelGGL(rmsnorm_bwd_generic_kernel<T>, grid, dim3(kNormThreads), 0, st, (const T*)added,
                                (const T*)weight, (const T*)dy, (const T*)d_added_in, denom, (T*)dx, (T*)d_residual, partial,

@@ -190,7 +190,9 @@ def test_backward_row_split_against_fp64(B, H):
 @pytest.mark.parametrize(
     "B,H,dtype",
     [(1031, 4096, torch.float32), (1031, 8192, torch.float32), (1031, 8192, torch.bfloat16), (1031, 16384, torch.bfloat16),
-     (1031, 16384, torch.float16), (4609, 2048, torch.float16), (8197, 1024, torch.float16), (2000, 2880, torch.bfloat16)],
+     (1031, 16384, torch.float16), (4609, 2048, torch.float16), (8197, 1024, torch.float16), (2000, 2880, torch.bfloat16),
+     # rows of one vector per thread, few of them: each workgroup takes neighbours from four each on; remainders, workgroups without a row
+     (513, 2048, torch.bfloat16), (2049, 2048, torch.bfloat16), (4001, 1024, torch.float32), (4097, 720, torch.float16)],
 )  # fmt: skip
 def test_backward_of_many_rows_against_fp64(B, H, dtype, has_weight):
     from fma.ops.fused_residual_add_rmsnorm.cuda_implementation import fused_residual_add_rmsnorm_backward_cuda
