@@ -1473,6 +1473,10 @@ int launch_plain(const Args& args, bool a_kc, bool b_kc, hipStream_t st) {
 // stay in the last-level cache), and a split has to promise a tenth less than none. Groups of few rows run the three-stage
 // loop, whose steps are shorter, without a split on half-width tiles in the NT layout: NT 4096 x 14336 on 8 groups of 32 rows
 // streams its weights in 176 us as it is and would take 184 us in two parts.
+// Uneven loads make fewer tiles, which a split helps the more; where they happen to fill the compute units exactly once as they are, the
+// sums are the price. Training steps without -> with splits: 2048 tokens, hidden 4096, I 14336, E 8, k 2, evenly 5100 -> 4630 us, all
+// on two experts 3870 -> 3990 us; 4000 tokens, hidden 2048, I 8192: 2775 -> 2627 and 2157 -> 2225 us; 512 and 1021 tokens gain either way
+// (2219 -> 1779 and 2727 -> 2478 us, 886 -> 565 us at 256 tokens of the second shape).
 constexpr double kStepUs = 1.45, kThinStepUs[2] = {1.1, 0.75}, kTileSteps = 6.0, kThinRows = 48.0, kWeightBytesPerUs = 5.5e6;
 constexpr double kReduceUs = 4.0, kReduceBytesPerUs = 4.5e6, kSplitGain = 0.9;
 constexpr uint32_t kSplitMinSteps = 24;

@@ -89,6 +89,37 @@ def test_layer_without_backward_under_uneven_routing(T, k, E, hot, bias):
             assert torch.equal(logits, expect_logits) and torch.equal(y, expect)
 
 
+def test_replays_take_either_kernel():
+    """a captured pass in which the device chooses between the two kernels: even and collapsed routing in turn"""
+    from fma import KernelBackend, MoE, swiglu_packed
+
+    T, k, E, H = 200, 8, 128, 136
+    torch.manual_seed(3)
+    moe = MoE(E, k, H, 72, swiglu_packed, True, True, 0.05).to(torch.bfloat16).to(DEV)
+    with torch.no_grad():
+        moe.gate.weight[:8, 0] = 4.0
+    x_static = torch.randn(T, H, device=DEV).bfloat16()
+    run = lambda x: moe(x, kernel_backend=KernelBackend.cuda)
+    with torch.no_grad():
+        side = torch.cuda.Stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            for _ in range(2):
+                run(x_static)
+        torch.cuda.current_stream().wait_stream(side)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            y_static, logits_static = run(x_static)
+    for step, common in enumerate((8.0, 0.0, 8.0, 8.0, 0.0, 0.0)):  # 8: every token chooses the first eight experts
+        x = torch.randn(T, H, device=DEV).bfloat16()
+        x[:, 0] = common
+        expect, expect_logits = run(x)  # the training forward, eager, between the replays
+        x_static.copy_(x)
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(y_static, expect) and torch.equal(logits_static, expect_logits), step
+
+
 def no_grad_sum(run, moe, x):
     with torch.no_grad():  # (inside the transform, where the grad mode outside does not count)
         return run(moe, x)[0].float().sum()
