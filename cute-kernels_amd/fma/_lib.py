@@ -138,7 +138,8 @@ _STAY = contextlib.nullcontext()
 
 def on_device(device: torch.device):
     """torch.cuda.device(device), without its cost (2 us) where that is the current device already"""
-    return _STAY if torch.cuda.current_device() == device.index else torch.cuda.device(device)
+    # (torch.cuda.current_device() without its look whether there is a context: tensors are on the GPU)
+    return _STAY if torch._C._cuda_getDevice() == device.index else torch.cuda.device(device)
 
 
 def current_stream(device: torch.device) -> int:

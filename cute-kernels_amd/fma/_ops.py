@@ -6,7 +6,7 @@ wrappers that custom_op puts around every call take 14 us of host time here agai
 dispatcher directly, and a step of this package is a dozen calls.
 
 What the wrappers do beside dispatching is kept:
- * a call advances the version counters of the arguments it declares as mutated (0.6 us; as a kernel of its own in front of
+ * a call advances the version counters of the arguments it declares as mutated (0.5 us; as a kernel of its own in front of
    the body, where custom_op does it, 7 to 10 us), so that autograd still refuses a backward pass through a buffer that an
    operator has overwritten since it was saved;
  * the body runs without recording gradients, whatever the grad mode around the call;
@@ -14,10 +14,11 @@ What the wrappers do beside dispatching is kept:
 """
 
 import inspect
+from operator import itemgetter
 from typing import Callable, Iterable
 
 import torch
-from torch.autograd.graph import increment_version
+from torch._C import _increment_version
 
 from .constants import LIBRARY_NAME
 
@@ -26,11 +27,17 @@ _library = torch.library.Library(LIBRARY_NAME, "FRAGMENT")
 
 def hip_op(name: str, mutates_args: Iterable[str]) -> Callable:
     def register(fn: Callable) -> torch._ops.OpOverload:
-        mutated = [i for i, p in enumerate(inspect.signature(fn).parameters) if p in mutates_args]
+        parameters = inspect.signature(fn).parameters.values()
+        mutated = [i for i, p in enumerate(parameters) if p.name in mutates_args]
+        optional = any(p.annotation is not torch.Tensor for p in parameters if p.name in mutates_args)
+        written = itemgetter(*mutated) if len(mutated) > 1 else itemgetter(slice(mutated[0], mutated[0] + 1))
 
         def body(*args) -> None:
-            # (inference tensors have no version and are passed over)
-            increment_version([args[i] for i in mutated if i < len(args) and args[i] is not None])
+            # (what torch.autograd.graph.increment_version calls; inference tensors have no version and are passed over)
+            if optional:
+                _increment_version([args[i] for i in mutated if i < len(args) and args[i] is not None])
+            else:
+                _increment_version(written(args))
             if not torch.is_grad_enabled():
                 return fn(*args)
             torch._C._set_grad_enabled(False)  # (torch.no_grad() would take 1.9 us)
