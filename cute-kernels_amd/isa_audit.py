@@ -2,7 +2,7 @@
 
 Usage: python cute-kernels_amd/isa_audit.py [file.s]
 
-The kernels of csrc/grouped_gemm_ragged.hip wait for their operand loads with `s_waitcnt vmcnt(N)` where N is a constant
+The kernels of csrc/ragged_kernel.h (instantiated in csrc/grouped_gemm_ragged.hip) wait for their operand loads with `s_waitcnt vmcnt(N)` where N is a constant
 that counts the vector-memory instructions a wavefront has issued after the loads it waits for (loads and stores complete
 in issue order). The constants are derived in the source from the number of loads per K step, the number of stores an
 epilogue issues and whether a prefetch, a bias load or a request for row_index entries follows a step's loads. This script
