@@ -52,6 +52,7 @@ def _headers() -> list[str]:
 # register spill would add loads and stores of its own and shift those counts, so that LDS stages could be read before
 # the operands have landed. Their kernels must use no scratch memory; the build checks the compiler's resource report.
 NO_SCRATCH_SOURCES = {"grouped_gemm.hip": "grouped_gemm_kernel", "grouped_gemm_ragged.hip": "ragged_gemm_kernel",
+                      "grouped_gemm_ragged_tall.hip": "ragged_gemm_kernel",
                       "thin_experts.hip": "thin_gemm_kernel", "decode.hip": "router_logits_kernel"}
 
 

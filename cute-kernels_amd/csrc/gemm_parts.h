@@ -1,4 +1,4 @@
-// Building blocks of the grouped-GEMM kernel for gfx950 (grouped_gemm.hip): the 16-bit
+// Building blocks of the grouped-GEMM kernels for gfx950 (grouped_gemm.hip, ragged_kernel.h): the 16-bit
 // element types with their matrix instruction, buffer-descriptor addressing with direct global -> LDS loads, and the
 // epilogue's transposing trip through LDS.
 #pragma once
@@ -452,6 +452,21 @@ struct LoaderK {
             buffer_load_lds_quiet(second ? r1 : r0, v, k0 * 2u + row * ldb, lds0 + (uint32_t)(i * NW) * 1024u);
         }
     }
+    // rows 256 .. 287 of a tile of 288 rows, into the 4 KB `extra`: one instruction per wavefront, in which wavefronts 4 .. 7 fetch
+    // the rows of 0 .. 3 once more (every wavefront then issues as many loads, and both write the same bytes)
+    __device__ __forceinline__ uint32_t extra_row0() const { return 256u - (wave & ~3u) * 8u; }
+    __device__ __forceinline__ void issue_extra(uint8_t* extra, uint32_t k0) const {
+        static_assert(NW == 8 && !SPLIT);
+        uint32_t v = voff;
+        if (k0 + BK > kdim && k0 + chunk * 8u >= kdim) v = kOutOfRange;
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(make_rsrc(base0, bytes), (lds_void*)(extra + (wave & 3u) * 1024), 16, v,
+                                                 k0 * 2u + extra_row0() * ldb, 0, 0);
+    }
+    __device__ __forceinline__ void issue_quiet_extra(uint8_t* extra, uint32_t k0) const {
+        uint32_t v = voff;
+        if (k0 + BK > kdim && k0 + chunk * 8u >= kdim) v = kOutOfRange;
+        buffer_load_lds_quiet(make_rsrc_words(base0, bytes), v, k0 * 2u + extra_row0() * ldb, lds_address(extra) + (wave & 3u) * 1024u);
+    }
     // only the instruction that covers tile rows 0 .. NW*8-1, to the LDS address lds_base (a tile with few rows)
     __device__ __forceinline__ void issue_quiet_first_rows(uint32_t lds_base, uint32_t k0) const {
         uint32_t v = voff;
@@ -475,7 +490,7 @@ struct LoaderK {
 };
 
 // Operand stored [reduction][out] (out contiguous): tile [64 k][256 out]. A wavefront instruction moves two k rows
-// (2 x 512 B). Rows past the end of the reduction are out of the descriptor's range (zeros); columns past the end of
+// (2 x 512 B; only the first `cols` columns, the others arrive as zeros). Rows past the end of the reduction are out of the descriptor's range (zeros); columns past the end of
 // the operand's rows read whatever follows, which only reaches outputs that are never stored.
 // SWZ16: the chunk positions that mc_frag_off16 reads (otherwise those of mc_frag_off).
 template <int NW, bool SWZ16 = false>
@@ -489,7 +504,7 @@ struct LoaderT {
     uint32_t wave;
 
     __device__ __forceinline__ void setup(const uint16_t* group_base, uint32_t ld, uint32_t kdim_, uint32_t out0,
-                                          uint32_t wave_, uint32_t lane) {
+                                          uint32_t wave_, uint32_t lane, uint32_t cols = BN) {
         base = group_base + out0;
         ldb = ld * 2u;
         col_bytes = out0 * 2u;
@@ -500,7 +515,8 @@ struct LoaderT {
         static_assert(!SWZ16 || NW == 8, "bit 3 of a lane's k row must be the same for every instruction");
         // (an instruction's rows are 16 i + krow: bit 3 of the k row is bit 3 of krow for every instruction i)
         const uint32_t flip = 4u * (krow & 3u) ^ (SWZ16 ? 2u * ((krow >> 3) & 1u) : 0u);
-        voff = khalf * ldb + (((lane & 31u) ^ flip) << 4);
+        const uint32_t piece = (lane & 31u) ^ flip;  // eight columns
+        voff = piece * 8u < cols ? khalf * ldb + (piece << 4) : kOutOfRange;
     }
 
     __device__ __forceinline__ void issue(uint8_t* tile, uint32_t k0) const { issue_range<0, NI>(tile, k0); }

@@ -1,7 +1,5 @@
-// Entry points of the grouped GEMM for launches whose groups differ in one dimension (the kernel: ragged_kernel.h), and the
-// choice and the second pass of a split reduction.
+// Entry points of the grouped GEMM for launches whose groups differ in one dimension (the kernel: ragged_kernel.h).
 #include <algorithm>
-#include <cmath>
 
 #include "ragged_kernel.h"
 
@@ -11,182 +9,58 @@ namespace ragged {
 
 // every instantiation the entry points launch (explicit, so that host stub and device code are both emitted)
 #define FMA_RAGGED_INSTANTIATE(EL)                                                                          \
-    template __global__ void ragged_gemm_kernel<EL, true, true, EPI_PLAIN, false, false, false>(const Args);    \
-    template __global__ void ragged_gemm_kernel<EL, true, false, EPI_PLAIN, false, false, false>(const Args);   \
-    template __global__ void ragged_gemm_kernel<EL, false, true, EPI_PLAIN, false, false, false>(const Args);   \
-    template __global__ void ragged_gemm_kernel<EL, false, false, EPI_PLAIN, false, false, false>(const Args);  \
-    template __global__ void ragged_gemm_kernel<EL, true, true, EPI_PLAIN, true, false, false>(const Args);     \
-    template __global__ void ragged_gemm_kernel<EL, true, false, EPI_PLAIN, true, false, false>(const Args);    \
-    template __global__ void ragged_gemm_kernel<EL, false, true, EPI_PLAIN, true, false, false>(const Args);    \
-    template __global__ void ragged_gemm_kernel<EL, false, false, EPI_PLAIN, true, false, false>(const Args);   \
-    template __global__ void ragged_gemm_kernel<EL, true, true, EPI_SWIGLU, false, false, false>(const Args);   \
-    template __global__ void ragged_gemm_kernel<EL, true, true, EPI_SWIGLU_ACT, false, false, false>(const Args); \
-    template __global__ void ragged_gemm_kernel<EL, true, true, EPI_PLAIN, false, true, false>(const Args);     \
-    template __global__ void ragged_gemm_kernel<EL, true, true, EPI_SWIGLU, false, true, false>(const Args);    \
-    template __global__ void ragged_gemm_kernel<EL, true, true, EPI_SWIGLU_ACT, false, true, false>(const Args); \
-    template __global__ void ragged_gemm_kernel<EL, true, false, EPI_SWIGLU_BWD, false, false, false>(const Args); \
-    template __global__ void ragged_gemm_kernel<EL, true, true, EPI_PLAIN, false, false, true>(const Args);     \
-    template __global__ void ragged_gemm_kernel<EL, true, true, EPI_SWIGLU, false, false, true>(const Args);    \
-    template __global__ void ragged_gemm_kernel<EL, true, true, EPI_SWIGLU_ACT, false, false, true>(const Args); \
-    template __global__ void ragged_gemm_kernel<EL, true, true, EPI_PLAIN, false, true, true>(const Args);      \
-    template __global__ void ragged_gemm_kernel<EL, true, true, EPI_SWIGLU, false, true, true>(const Args);     \
-    template __global__ void ragged_gemm_kernel<EL, true, true, EPI_SWIGLU_ACT, false, true, true>(const Args); \
-    template __global__ void ragged_gemm_kernel<EL, false, false, EPI_PLAIN, true, false, true>(const Args);    \
-    template __global__ void ragged_gemm_kernel<EL, true, true, EPI_SPLIT, false, false, false>(const Args);    \
-    template __global__ void ragged_gemm_kernel<EL, true, false, EPI_SPLIT, false, false, false>(const Args);
+    template __global__ void ragged_gemm_kernel<EL, true, true, EPI_PLAIN, false, false, false, false>(const Args);    \
+    template __global__ void ragged_gemm_kernel<EL, true, false, EPI_PLAIN, false, false, false, false>(const Args);   \
+    template __global__ void ragged_gemm_kernel<EL, false, true, EPI_PLAIN, false, false, false, false>(const Args);   \
+    template __global__ void ragged_gemm_kernel<EL, false, false, EPI_PLAIN, false, false, false, false>(const Args);  \
+    template __global__ void ragged_gemm_kernel<EL, true, true, EPI_PLAIN, true, false, false, false>(const Args);     \
+    template __global__ void ragged_gemm_kernel<EL, true, false, EPI_PLAIN, true, false, false, false>(const Args);    \
+    template __global__ void ragged_gemm_kernel<EL, false, true, EPI_PLAIN, true, false, false, false>(const Args);    \
+    template __global__ void ragged_gemm_kernel<EL, false, false, EPI_PLAIN, true, false, false, false>(const Args);   \
+    template __global__ void ragged_gemm_kernel<EL, true, true, EPI_SWIGLU, false, false, false, false>(const Args);   \
+    template __global__ void ragged_gemm_kernel<EL, true, true, EPI_SWIGLU_ACT, false, false, false, false>(const Args); \
+    template __global__ void ragged_gemm_kernel<EL, true, true, EPI_PLAIN, false, true, false, false>(const Args);     \
+    template __global__ void ragged_gemm_kernel<EL, true, true, EPI_SWIGLU, false, true, false, false>(const Args);    \
+    template __global__ void ragged_gemm_kernel<EL, true, true, EPI_SWIGLU_ACT, false, true, false, false>(const Args); \
+    template __global__ void ragged_gemm_kernel<EL, true, false, EPI_SWIGLU_BWD, false, false, false, false>(const Args); \
+    template __global__ void ragged_gemm_kernel<EL, true, true, EPI_PLAIN, false, false, true, false>(const Args);     \
+    template __global__ void ragged_gemm_kernel<EL, true, true, EPI_SWIGLU, false, false, true, false>(const Args);    \
+    template __global__ void ragged_gemm_kernel<EL, true, true, EPI_SWIGLU_ACT, false, false, true, false>(const Args); \
+    template __global__ void ragged_gemm_kernel<EL, true, true, EPI_PLAIN, false, true, true, false>(const Args);      \
+    template __global__ void ragged_gemm_kernel<EL, true, true, EPI_SWIGLU, false, true, true, false>(const Args);     \
+    template __global__ void ragged_gemm_kernel<EL, true, true, EPI_SWIGLU_ACT, false, true, true, false>(const Args); \
+    template __global__ void ragged_gemm_kernel<EL, false, false, EPI_PLAIN, true, false, true, false>(const Args);    \
+    template __global__ void ragged_gemm_kernel<EL, true, true, EPI_SPLIT, false, false, false, false>(const Args);    \
+    template __global__ void ragged_gemm_kernel<EL, true, false, EPI_SPLIT, false, false, false, false>(const Args);
 FMA_RAGGED_INSTANTIATE(ElemBf16)
 FMA_RAGGED_INSTANTIATE(ElemF16)
 #undef FMA_RAGGED_INSTANTIATE
 
-template <typename EL, bool A_KC, bool B_KC, int EPI, bool VARY_K, bool BIAS = false, bool GATHER = false>
-int launch(const Args& args, hipStream_t st) {
-    int cus = num_compute_units();
-    if (cus <= 0) cus = 256;
-    hipLaunchKernelGGL((ragged_gemm_kernel<EL, A_KC, B_KC, EPI, VARY_K, BIAS, GATHER>), dim3((uint32_t)cus), dim3(NT), 0, st,
-                       args);
-    return launch_status("grouped_gemm_ragged");
-}
-
-// the forward (NT) kernels by epilogue, bias and gather
 template <typename EL, int EPI>
 int launch_forward(const Args& args, hipStream_t st) {
-    const bool bias = args.bias != nullptr, gather = args.row_index != nullptr;
-    if (bias && gather) return launch<EL, true, true, EPI, false, true, true>(args, st);
-    if (bias) return launch<EL, true, true, EPI, false, true, false>(args, st);
-    if (gather) return launch<EL, true, true, EPI, false, false, true>(args, st);
-    return launch<EL, true, true, EPI, false, false, false>(args, st);
+    if (args.E <= kTallGroups) return launch_tall(args, EPI, true, std::is_same<EL, ElemBf16>::value, st);
+    return launch_forward_as<EL, EPI, false>(args, st);
 }
 
 template <typename EL, bool VARY_K>
 int launch_plain(const Args& args, bool a_kc, bool b_kc, hipStream_t st) {
-    if (a_kc && b_kc) return launch<EL, true, true, EPI_PLAIN, VARY_K>(args, st);
-    if (a_kc && !b_kc) return launch<EL, true, false, EPI_PLAIN, VARY_K>(args, st);
-    if (!a_kc && b_kc) return launch<EL, false, true, EPI_PLAIN, VARY_K>(args, st);
-    return launch<EL, false, false, EPI_PLAIN, VARY_K>(args, st);
+    if constexpr (!VARY_K) {
+        if (a_kc && args.E <= kTallGroups) return launch_tall(args, EPI_PLAIN, b_kc, std::is_same<EL, ElemBf16>::value, st);
+    }
+    if (a_kc && b_kc) return launch<EL, true, true, EPI_PLAIN, VARY_K, false, false, false>(args, st);
+    if (a_kc && !b_kc) return launch<EL, true, false, EPI_PLAIN, VARY_K, false, false, false>(args, st);
+    if (!a_kc && b_kc) return launch<EL, false, true, EPI_PLAIN, VARY_K, false, false, false>(args, st);
+    return launch<EL, false, false, EPI_PLAIN, VARY_K, false, false, false>(args, st);
 }
 
-// ---- split reduction ---------------------------------------------------------------------------------------------
-// A launch with fewer tiles than compute units leaves the others idle for the whole reduction: the second projection of
-// 1021 tokens on 8 experts (2048 x 8192) is 96 tiles of 128 K steps, 205 us. With the reduction in two parts (192 tiles of
-// 64 steps, fp32 sums to memory and one pass over them) it takes 130 us. More of the same (parts; before -> now):
-//   NT 2048 x 8192, 8 groups of 64 / 128 rows (4)            167 -> 69 us, 180 -> 84 us
-//   NT 4096 x 14336, 8 groups of 128 / 512 rows (2 / 3)      357 -> 234 us, 690 -> 570 us
-//   NN 2048 x 16384, 8 groups of 128 / 512 / 1024 rows       339 -> 133 us (4), 380 -> 317 us (3), 700 -> 580 us (3)
-//   NN 4096 x 28672, 8 groups of 32 / 64 / 512 rows          496 -> 310 us (2), 633 -> 371 us (2), 1330 -> 1015 us (4)
-//
-// How many parts: the number with the least predicted time, rounds of tiles times (K steps + a tile's fixed cost) or the
-// weights at the rate they stream, plus the traffic of the sums. The row counts lie in device memory, so the number of tiles
-// is the expected one for evenly loaded groups. Parts have at least kSplitMinSteps steps, the sums at most kSplitMaxBytes (they
-// stay in the last-level cache), and a split has to promise a tenth less than none. Groups of few rows run the three-stage
-// loop, whose steps are shorter, without a split on half-width tiles in the NT layout: NT 4096 x 14336 on 8 groups of 32 rows
-// streams its weights in 176 us as it is and would take 184 us in two parts.
-// Uneven loads make fewer tiles, which a split helps the more; where they happen to fill the compute units exactly once as they are, the
-// sums are the price. Training steps without -> with splits: 2048 tokens, hidden 4096, I 14336, E 8, k 2, evenly 5100 -> 4630 us, all
-// on two experts 3870 -> 3990 us; 4000 tokens, hidden 2048, I 8192: 2775 -> 2627 and 2157 -> 2225 us; 512 and 1021 tokens gain either way
-// (2219 -> 1779 and 2727 -> 2478 us, 886 -> 565 us at 256 tokens of the second shape).
-constexpr double kStepUs = 1.45, kThinStepUs[2] = {1.1, 0.75}, kTileSteps = 6.0, kThinRows = 48.0, kWeightBytesPerUs = 5.5e6;
-constexpr double kReduceUs = 4.0, kReduceBytesPerUs = 4.5e6, kSplitGain = 0.9;
-constexpr uint32_t kSplitMinSteps = 24;
-constexpr int64_t kSplitMaxBytes = 256ll << 20;
-struct SplitPlan {
-    uint32_t splits, steps;  // parts and K steps of each (even; the last part takes what is left); splits 1: no split
-};
-SplitPlan plan_split(int64_t R, int64_t E, int64_t N, int64_t K, bool b_kc) {
-    const uint32_t all = (uint32_t)((K + BK - 1) / BK);
-    SplitPlan best{1u, all};
-    // (the sizes for which every tile takes the matrix-instruction path)
-    if (R < 1 || E < 1 || N < 8 || N % 8 || N >= (1 << 23) || K % 8 || K >= (1 << 21) || R > 0x7fffffffll) return best;
-    if (all < 2 * kSplitMinSteps) return best;
-    const int cus = num_compute_units() > 0 ? num_compute_units() : 256;
-    const double active = (double)(R < E ? R : E), mean = (double)R / active;
-    const double row_tiles = active * (mean < BM / 2 ? 1.0 : mean / BM + 0.5);
-    const double tiles = row_tiles * (double)((N + BN - 1) / BN);
-    const bool thin = mean <= kThinRows, narrow = thin && b_kc && 2.0 * tiles <= cus;
-    const double step_us = thin ? kThinStepUs[b_kc] : kStepUs;
-    const double weights_us = active * N * K * 2.0 / kWeightBytesPerUs;
-    auto us = [&](uint32_t parts, uint32_t steps) {
-        const double units = tiles * parts * (parts == 1 && narrow ? 2.0 : 1.0);
-        const double products = std::ceil(units / cus - 1e-9) * (steps + kTileSteps) * step_us;
-        const double sums = parts > 1 ? kReduceUs + (double)R * N * (8.0 * parts + 2.0) / kReduceBytesPerUs : 0.0;
-        return std::max(products, weights_us) + sums;
-    };
-    double best_us = us(1, all) * kSplitGain;
-    for (uint32_t parts = 2; parts * kSplitMinSteps <= all && parts <= 32; ++parts) {
-        const uint32_t steps = ((all + parts - 1) / parts + 1u) & ~1u;
-        const uint32_t used = (all + steps - 1) / steps;
-        if (used != parts || R * N * 4 * (int64_t)parts > kSplitMaxBytes) continue;
-        const double t = us(parts, steps);
-        if (t < best_us) {
-            best_us = t;
-            best = SplitPlan{parts, steps};
-        }
-    }
-    return best;
-}
-
-// out[r, :] = round(alpha * (sum over the parts, in order)), plus the bias of the row's group as the kernels' epilogue adds it.
-// Bound by memory (parts * 4 + 2 bytes per element). A workgroup takes kReduceRows rows; which group a row belongs to is
-// read off a prefix of the sizes (built per workgroup: E values, one scan), and rows past the last group are left alone.
-constexpr int kReduceThreads = 256, kReduceRows = 4;
-template <typename EL, bool BIAS>
-__global__ __launch_bounds__(kReduceThreads) void split_reduce_kernel(const Args args) {
-    __shared__ uint32_t s_end[FMA_MAX_GROUPS];
-    const uint32_t tid = threadIdx.x, E = args.E, N = args.n;
-    if (tid < 64u) {
-        uint32_t carry = 0;
-        for (uint32_t base = 0; base < E; base += 64u) {
-            const uint32_t e = base + tid;
-            const uint32_t incl = wave_inclusive_scan<uint32_t>(e < E ? args.sizes[e] : 0u);
-            if (e < E) s_end[e] = carry + incl;
-            carry += __shfl(incl, 63, 64);
-        }
-    }
-    __syncthreads();
-    const uint32_t vecs = N / 8u;  // of 8 columns
-    const uint64_t part = (uint64_t)args.rows * N;
-    const uint32_t first = blockIdx.x * (uint32_t)kReduceRows;
-    for (uint32_t i = tid; i < (uint32_t)kReduceRows * vecs; i += kReduceThreads) {
-        const uint32_t r = first + i / vecs, col = (i % vecs) * 8u;
-        if (r >= args.rows || r >= s_end[E - 1u]) return;
-        const float* src = args.partial + (uint64_t)r * N + col;
-        float sum[8];
-#pragma unroll
-        for (int x = 0; x < 8; ++x) sum[x] = 0.0f;
-        for (uint32_t s = 0; s < args.splits; ++s, src += part) {
-            const float4 lo = reinterpret_cast<const float4*>(src)[0], hi = reinterpret_cast<const float4*>(src)[1];
-            sum[0] += lo.x; sum[1] += lo.y; sum[2] += lo.z; sum[3] += lo.w;
-            sum[4] += hi.x; sum[5] += hi.y; sum[6] += hi.z; sum[7] += hi.w;
-        }
-#pragma unroll
-        for (int x = 0; x < 8; ++x) sum[x] *= args.alpha;
-        if constexpr (BIAS) {
-            uint32_t lo = 0, hi = E - 1u;  // the first group that ends past row r
-            while (lo < hi) {
-                const uint32_t mid = (lo + hi) >> 1;
-                if (s_end[mid] > r) hi = mid;
-                else lo = mid + 1u;
-            }
-            const uint16_t* b = args.bias + (uint64_t)lo * N + col;
-#pragma unroll
-            for (int x = 0; x < 8; ++x) sum[x] = EL::round(sum[x]) + EL::from_bits(b[x]);
-        }
-        uint4 packed;
-        packed.x = EL::pack2(sum[0], sum[1]);
-        packed.y = EL::pack2(sum[2], sum[3]);
-        packed.z = EL::pack2(sum[4], sum[5]);
-        packed.w = EL::pack2(sum[6], sum[7]);
-        *reinterpret_cast<uint4*>(args.D + (uint64_t)r * N + col) = packed;
-    }
-}
-
-template <typename EL>
-int launch_split(const Args& args, bool b_kc, hipStream_t st) {
-    const int rc = b_kc ? launch<EL, true, true, EPI_SPLIT, false>(args, st) : launch<EL, true, false, EPI_SPLIT, false>(args, st);
-    if (rc != FMA_OK) return rc;
-    const dim3 grid((args.rows + kReduceRows - 1) / kReduceRows), block(kReduceThreads);
-    if (args.bias) hipLaunchKernelGGL((split_reduce_kernel<EL, true>), grid, block, 0, st, args);
-    else hipLaunchKernelGGL((split_reduce_kernel<EL, false>), grid, block, 0, st, args);
-    return launch_status("grouped_gemm_ragged(reduce)");
+// a product with its reduction in args.splits parts: the parts, then their sum
+int launch_split(const Args& args, bool b_kc, bool bf16, hipStream_t st) {
+    const int rc = args.E <= kTallGroups ? launch_tall(args, EPI_SPLIT, b_kc, bf16, st)
+                   : bf16 ? (b_kc ? launch<ElemBf16, true, true, EPI_SPLIT, false, false, false, false>(args, st)
+                                  : launch<ElemBf16, true, false, EPI_SPLIT, false, false, false, false>(args, st))
+                          : (b_kc ? launch<ElemF16, true, true, EPI_SPLIT, false, false, false, false>(args, st)
+                                  : launch<ElemF16, true, false, EPI_SPLIT, false, false, false, false>(args, st));
+    return rc != FMA_OK ? rc : launch_split_reduce(args, bf16, st);
 }
 
 // The forward product of an expert projection, out_e = x_e W_e^T (+ bias_e), with the rows of x_e packed (row_index
@@ -271,8 +145,11 @@ extern "C" {
 
 
 int64_t fma_grouped_gemm_ragged_workspace_bytes(int64_t R, int64_t E, int64_t N, int64_t K, int trans_b) {
-    const fmahip::gemm::ragged::SplitPlan plan = fmahip::gemm::ragged::plan_split(R, E, N, K, trans_b != 0);
-    return plan.splits > 1 ? R * N * 4 * (int64_t)plan.splits : 0;
+    // enough for launches of either tile height, whichever the kernel has for E groups
+    uint32_t parts = 1;
+    for (const bool tall : {false, true})
+        parts = std::max(parts, fmahip::gemm::ragged::plan_split(R, E, N, K, trans_b != 0, tall).splits);
+    return parts > 1 ? R * N * 4 * (int64_t)parts : 0;
 }
 
 int fma_grouped_gemm_ragged(const void* A, const void* B, void* D, const uint32_t* sizes, const void* bias, int64_t E,
@@ -327,7 +204,7 @@ int fma_grouped_gemm_ragged_split(const void* A, const void* B, void* D, const u
     args.k = (uint32_t)K;
     args.alpha = alpha;
     const ragged::SplitPlan plan =
-        workspace && vary == FMA_VARY_M && a_kc ? ragged::plan_split(rows, E, N, K, b_kc) : ragged::SplitPlan{1u, 0u};
+        workspace && vary == FMA_VARY_M && a_kc ? ragged::plan_split(rows, E, N, K, b_kc, E <= ragged::kTallGroups) : ragged::SplitPlan{1u, 0u};
     if (plan.splits > 1) {
         FMA_REQUIRE(aligned16(workspace), FMA_ERR_MISALIGNED, "grouped_gemm_ragged: the workspace must be 16-byte aligned");
         const int64_t need = rows * N * 4 * (int64_t)plan.splits;
@@ -338,7 +215,7 @@ int fma_grouped_gemm_ragged_split(const void* A, const void* B, void* D, const u
         args.splits = plan.splits;
         args.split_steps = plan.steps;
         args.rows = (uint32_t)rows;
-        return dtype == FMA_BF16 ? ragged::launch_split<ElemBf16>(args, b_kc, st) : ragged::launch_split<ElemF16>(args, b_kc, st);
+        return ragged::launch_split(args, b_kc, dtype == FMA_BF16, st);
     }
     if (bias)
         return dtype == FMA_BF16 ? ragged::launch_forward<ElemBf16, EPI_PLAIN>(args, st)
@@ -386,8 +263,9 @@ int fma_grouped_gemm_swiglu_bwd(const void* dy, const void* W, const void* h, vo
     args.k = (uint32_t)K;
     args.alpha = 1.0f;
     hipStream_t st = (hipStream_t)stream;
-    return dtype == FMA_BF16 ? ragged::launch<ElemBf16, true, false, EPI_SWIGLU_BWD, false>(args, st)
-                             : ragged::launch<ElemF16, true, false, EPI_SWIGLU_BWD, false>(args, st);
+    if (args.E <= ragged::kTallGroups) return ragged::launch_tall(args, EPI_SWIGLU_BWD, false, dtype == FMA_BF16, st);
+    return dtype == FMA_BF16 ? ragged::launch<ElemBf16, true, false, EPI_SWIGLU_BWD, false, false, false, false>(args, st)
+                             : ragged::launch<ElemF16, true, false, EPI_SWIGLU_BWD, false, false, false, false>(args, st);
 }
 
 int fma_grouped_gemm_gathered_wgrad(const void* dy, const void* x, int64_t x_rows, const int32_t* row_index, int32_t divisor,
@@ -427,8 +305,8 @@ int fma_grouped_gemm_gathered_wgrad(const void* dy, const void* x, int64_t x_row
     args.k = 0;
     args.alpha = alpha;
     hipStream_t st = (hipStream_t)stream;
-    return dtype == FMA_BF16 ? ragged::launch<ElemBf16, false, false, EPI_PLAIN, true, false, true>(args, st)
-                             : ragged::launch<ElemF16, false, false, EPI_PLAIN, true, false, true>(args, st);
+    return dtype == FMA_BF16 ? ragged::launch<ElemBf16, false, false, EPI_PLAIN, true, false, true, false>(args, st)
+                             : ragged::launch<ElemF16, false, false, EPI_PLAIN, true, false, true, false>(args, st);
 }
 
 int fma_grouped_gemm_gathered(const void* x, int64_t x_rows, const int32_t* row_index, int32_t divisor, const void* W,

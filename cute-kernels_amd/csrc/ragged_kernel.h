@@ -30,6 +30,20 @@
 //    the rows of A as rows row_index[i] / divisor of the token matrix (a table of the tile's 256 entries in LDS, four
 //    per-lane offsets per K step), the weight gradient takes the reduction rows of B the same way (eight entries per
 //    wavefront and K step, requested two steps ahead). Both give the bits of the packed kernel on a gathered copy.
+//  * Tall tiles (TALL; rows vary, A with its reduction contiguous, at most 256 groups, whose shorter table leaves the LDS): a tile may
+//    have 32 rows more, one 16-row block per wavefront in a 4 KB stage of its own. A K step is bound by the delivery of its
+//    operands, above all of B (a tile of 8 rows takes 88 % of a full one's time), so what counts is how many tiles stream a
+//    panel of B: experts of 256 or 512 +- 20 rows, as an even routing makes them, take one or two tiles instead of every other one
+//    a nearly empty one more. A group gets as few tiles as 288 rows allow, of which as few as its rows need are tall (a tall
+//    step costs 6 % more loads and 12 % more matrix instructions). Same sums in the same order: same bits. Products of evenly
+//    routed layers, 256-row tiles -> tall (us): hidden 4096, I 1536, E 128, k 8, 4096 tokens 984 -> 945, 541 -> 500 (up, down), input
+//    gradients 951 -> 852, 595 -> 522; 8192 tokens 1570 -> 1432, 858 -> 801, 1536 -> 1416, 924 -> 806; hidden 4096, I 14336, E 8,
+//    k 2, 4096 tokens 1600 -> 1510, 1004 -> 749, 1996 -> 1460, 900 -> 842; hidden 2048, I 8192, 1021 tokens 228 -> 159 (up); rows that
+//    leave the number of tiles as it is (94 to 156 an expert) 0.99 to 1.01 of the time.
+//  * The last, partial round of tiles of a tall kernel is cut into 2 or 4 parts of their columns where there are workgroups for them: the
+//    loads of B shrink with the columns, and the round takes 0.65 to 0.75 of a whole one's time. Products of 384 tiles (hidden 2880,
+//    I 2880, E 32, k 4, 2000 tokens) 191 -> 179 us (down), 331 -> 314 us (input gradient); of 320 (hidden 2048, I 8192, E 8, k 2, 5000
+//    tokens) 393 -> 364 us.
 #pragma once
 
 #include "gemm_parts.h"
@@ -45,6 +59,10 @@ constexpr uint32_t kStreamOutSteps = 16;  // weight-gradient tiles of at most th
 constexpr int NWM = 2, NWN = 4, NW = NWM * NWN, NT = NW * 64;
 constexpr int WM = BM / NWM, WN = BN / NWN;  // 128 x 64 per wavefront
 constexpr int RB = WM / 16, CB = WN / 16;    // 8 x 4 accumulator blocks of 16 x 16 (the 16x16x32 matrix instruction)
+constexpr int kTallM = 288;                  // rows of a tall tile: 256, and one more 16-row block per wavefront
+constexpr uint32_t kTallGroups = 256;        // groups a launch of the tall kernels may have (their table is that much shorter)
+constexpr int kRowLoads = 5;                 // loads of A rows per wavefront and K step of a tall tile (otherwise four)
+constexpr int kExtraBytes = (kTallM - BM) * kRowBytes;  // LDS of the rows past 256, per stage
 constexpr int kStageBytes = 2048;            // epilogue staging per wavefront: 16 rows of 128 bytes or 32 rows of 64
 
 struct Args {
@@ -94,10 +112,16 @@ struct Feed {
 };
 
 
+// The `rest` tiles left after the whole rounds of `g` workgroups are computed in 1, 2 or 4 (the logarithm is returned) parts of their
+// columns, as many as there are workgroups for.
+__device__ __forceinline__ uint32_t parts_of_tail(uint32_t rest, uint32_t g) {
+    return rest * 4u <= g ? 2u : (rest * 2u <= g ? 1u : 0u);
+}
+
 // Names an accumulator value as one 16-register value (no instruction, no ordering).
 __device__ __forceinline__ void anchor_value(f32x16& c) { asm("" : "+v"(c)); }
 
-template <typename EL, bool A_KC, bool B_KC, int EPI, bool VARY_K, bool BIAS, bool GATHER_ANY>
+template <typename EL, bool A_KC, bool B_KC, int EPI, bool VARY_K, bool BIAS, bool GATHER_ANY, bool TALL>
 __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
     // GATHER: the rows of A are picked through row_index (forward); kGatherK: the reduction rows of B are (weight gradient)
     constexpr bool GATHER = GATHER_ANY && !VARY_K;
@@ -110,6 +134,7 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
     // kSplit: fp32 sums over a part of the reduction, added up by split_reduce_kernel
     constexpr bool kSplit = EPI == EPI_SPLIT;
     static_assert(!kSplit || (A_KC && !VARY_K && !BIAS && !GATHER_ANY), "the reduction is split in the NT and NN layouts only");
+    static_assert(!TALL || (A_KC && !VARY_K), "tall tiles exist where the rows vary and A has its reduction contiguous");
     static_assert(!BIAS || (A_KC && B_KC && !VARY_K), "the bias term exists for the forward (NT) layout only");
     static_assert(!GATHER || (A_KC && B_KC), "rows are gathered in the forward (NT) layout only");
     static_assert(!kGatherK || (!A_KC && !B_KC && EPI == EPI_PLAIN), "reduction rows are gathered in the weight-gradient (TN) layout only");
@@ -120,23 +145,28 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
     __shared__ __attribute__((aligned(1024))) uint8_t s_b0[kTileBytes];
     __shared__ __attribute__((aligned(1024))) uint8_t s_a1[kTileBytes];
     __shared__ __attribute__((aligned(1024))) uint8_t s_b1[kTileBytes];
+    // TALL: rows 256 .. 287 of the A tile, per stage
+    __shared__ __attribute__((aligned(TALL ? 1024 : 16))) uint8_t s_x0[TALL ? kExtraBytes : 16];
+    __shared__ __attribute__((aligned(TALL ? 1024 : 16))) uint8_t s_x1[TALL ? kExtraBytes : 16];
     __shared__ __attribute__((aligned(1024))) uint8_t s_stage[NW * kStageBytes];
     __shared__ uint32_t s_pf[64];  // where the dwords fetched by the L2 prefetch end up (never read)
     // BIAS: per wavefront, the bias values of its own 64 columns (plain) or 32 "up" | 32 "gate" columns
     constexpr int kBiasBytes = 128;
     __shared__ __attribute__((aligned(256))) uint8_t s_bias[BIAS ? NW * kBiasBytes : 16];
-    // GATHER: the row_index entries of the 256 rows of a tile, for the tile of round r in half r % 2. Filled by
+    // GATHER: the row_index entries of the rows of a tile, for the tile of round r in half r % 2. Filled by
     // direct-to-LDS loads and read in assembly: the compiler never sees an access to it.
-    __shared__ __attribute__((aligned(256))) uint32_t s_rows[GATHER ? 512 : 4];
+    constexpr uint32_t kMostRows = TALL ? kTallM : BM;  // of a tile
+    __shared__ __attribute__((aligned(256))) uint32_t s_rows[GATHER ? 2 * kMostRows : 4];
     // kGatherK: row_index entries on their way from one tile's last two steps (or a cold start) to the next tile's first two:
     // per LDS stage and wavefront the 64 dwords of one direct-to-LDS load. Read in assembly only.
     __shared__ __attribute__((aligned(256))) uint32_t s_gk[kGatherK ? 2 * NW * 64 : 4];
     // The group table, one LDS object: first tile of the group at position p of the tile sequence, exclusive prefix of the
     // varying dimension over the groups, and which group is at position p.
-    __shared__ uint32_t s_table[2 * (FMA_MAX_GROUPS + 1) + FMA_MAX_GROUPS / 2];
+    constexpr uint32_t kMostGroups = TALL ? kTallGroups : FMA_MAX_GROUPS;
+    __shared__ uint32_t s_table[2 * (kMostGroups + 1) + kMostGroups / 2];
     uint32_t* const s_tile_start = s_table;
-    uint32_t* const s_prefix = s_table + (FMA_MAX_GROUPS + 1);
-    uint16_t* const s_order = reinterpret_cast<uint16_t*>(s_table + 2 * (FMA_MAX_GROUPS + 1));
+    uint32_t* const s_prefix = s_table + (kMostGroups + 1);
+    uint16_t* const s_order = reinterpret_cast<uint16_t*>(s_table + 2 * (kMostGroups + 1));
 
     const uint32_t tid = threadIdx.x;
     const uint32_t lane = tid & 63u;
@@ -199,13 +229,16 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
     auto group_k = [&](uint32_t e) { return VARY_K ? sizes[e] : dim_k; };
     const uint32_t Ne = dim_n;
     constexpr bool kCanNarrow = A_KC && B_KC && !kSplit;
+    // kTail: the tiles of the last round may be cut into column parts (not those of a split reduction, which fills the round already)
+    constexpr bool kTail = TALL && !kSplit;
     constexpr uint32_t kTileN = kGlu ? BN / 2 : BN;  // columns of the tile grid one tile covers
     const uint32_t n_span = kGlu ? Ne / 2 : Ne;      // columns the tile grid runs over
     bool narrow = false;
+    auto row_tiles = [&](uint32_t m) -> uint32_t { return (m + kMostRows - 1) / kMostRows; };
     auto tiles_of = [&](uint32_t m) -> uint32_t {
         if (m == 0 || Ne == 0) return 0;
         const uint32_t width = (kCanNarrow && narrow && m <= 64u) ? kTileN / 2 : kTileN;
-        return ((m + BM - 1) / BM) * ((n_span + width - 1) / width);
+        return row_tiles(m) * ((n_span + width - 1) / width);
     };
 
     // ---- order of the groups in the tile sequence: by K steps per tile, longest first (see grouped_gemm.hip) ----
@@ -282,6 +315,9 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
     }
     __syncthreads();
     const uint32_t total_tiles = s_tile_start[E];
+    // the last, partial round: its tiles in `tail_parts` parts of their columns
+    const uint32_t tail_first = total_tiles - total_tiles % gridDim.x;
+    const uint32_t tail_shift = kTail && !narrow ? parts_of_tail(total_tiles - tail_first, gridDim.x) : 0u;
 
     // first tile row of B fragment j (16 rows) of this wavefront
     auto b_frag_row = [&](int j) -> uint32_t {
@@ -307,6 +343,7 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
     uint32_t kc_slice[2];
 #pragma unroll
     for (int ks = 0; ks < 2; ++ks) kc_slice[ks] = kc_off(lane & 15u, (uint32_t)ks * 4u + (lane >> 4));
+    const uint32_t x_off = wm * 16 * kRowBytes;    // TALL: this wavefront's row block of the rows past 256
     constexpr uint32_t kSliceT = 32 * kTRowBytes;  // from slice 0 to slice 1 in a [k][out] tile
 
     // workgroup id -> position in the round of gridDim.x tiles: workgroups of one XCD take 32 neighbours
@@ -318,6 +355,7 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
     struct Tile {
         bool valid, fast;
         uint32_t Me, Ke, m0, n0, n_lim;  // n_lim: first column past the tile (kTileN columns wide, or half of that)
+        uint32_t rows;                   // rows of the tile inside the group
         uint32_t e;                      // the group
         uint32_t row0;                   // first packed row (reduction row, if the reduction varies) of the group
         uint64_t off_a, off_b, off_d;
@@ -327,13 +365,21 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
     auto lookup = [&](uint32_t round) -> Tile {
         Tile t{};
         uint32_t v = round * grid + ((round & 1u) ? grid - 1u - slot : slot);
-        const uint32_t total_units = kSplit ? total_tiles * args.splits : total_tiles;
+        const uint32_t total_units = kSplit ? total_tiles * args.splits : tail_first + ((total_tiles - tail_first) << tail_shift);
         if ((uint64_t)round * grid >= total_units || v >= total_units) return t;
         if constexpr (kSplit) {
             // part by part: neighbours in the sequence share operand panels as they do without a split
             t.part = v / total_tiles;
             t.ks = t.part * args.split_steps * (uint32_t)BK;
             v -= t.part * total_tiles;
+        }
+        uint32_t column_part = 0, parts_shift = 0;
+        if constexpr (kTail) {
+            if (v >= tail_first) {
+                parts_shift = tail_shift;
+                column_part = (v - tail_first) & ((1u << tail_shift) - 1u);
+                v = tail_first + ((v - tail_first) >> tail_shift);
+            }
         }
         // position of the group that holds tile v: the number of groups whose tiles end at or before v. Every lane
         // compares one table entry per 64 groups and a ballot counts them (a binary search would be ten dependent LDS
@@ -350,7 +396,7 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
         t.e = e;
         t.Me = group_m(e);
         t.Ke = group_k(e);
-        const uint32_t tiles_m = (t.Me + BM - 1) / BM;
+        const uint32_t tiles_m = row_tiles(t.Me);
         const uint32_t tile_n = (kCanNarrow && narrow && t.Me <= 64u) ? kTileN / 2 : kTileN;
         const uint32_t tiles_n = (n_span + tile_n - 1) / tile_n;
         const uint32_t local = v - uniform(s_tile_start[pos]);
@@ -361,9 +407,19 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
         const uint32_t nt = (local % band) / band_m;
         t.pf_r = (local % band) % band_m;
         t.pf_c = nt & 3u;
-        t.m0 = mt * BM;
+        // TALL: the first tiles of the group are 288 rows high, as many as its rows need; the others 256
+        const uint32_t past = TALL && t.Me > tiles_m * (uint32_t)BM ? (t.Me - tiles_m * (uint32_t)BM + 31u) / 32u : 0u;
+        const uint32_t height = mt < past ? kMostRows : (uint32_t)BM;
+        t.m0 = mt * (uint32_t)BM + (mt < past ? mt : past) * (kMostRows - (uint32_t)BM);
+        t.rows = t.Me - t.m0 < height ? t.Me - t.m0 : height;
         t.n0 = nt * tile_n;
         t.n_lim = n_span - t.n0 < tile_n ? n_span : t.n0 + tile_n;
+        if constexpr (kTail) {
+            // (parts past the last column are tiles without columns)
+            const uint32_t width = tile_n >> parts_shift, end = t.n_lim;
+            t.n0 = t.n0 + column_part * width < end ? t.n0 + column_part * width : end;
+            t.n_lim = end - t.n0 < width ? end : t.n0 + width;
+        }
         // packed element offsets of the group: the varying dimension's prefix times the other dimension of the operand
         const uint64_t before = uniform(s_prefix[e]);
         t.row0 = (uint32_t)before;
@@ -412,7 +468,7 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
         if constexpr (GATHER) return;  // nothing per tile: the rows come from the table in s_rows
         const uint16_t* Ae = args.A + t.off_a;
         if constexpr (A_KC) {
-            lk_a.setup(Ae + (uint64_t)t.m0 * t.Ke, nullptr, t.Me - t.m0 < (uint32_t)BM ? t.Me - t.m0 : (uint32_t)BM, t.Ke, wave, lane);
+            lk_a.setup(Ae + (uint64_t)t.m0 * t.Ke, nullptr, t.rows, t.Ke, wave, lane);
             f = Feed<A_KC>{lk_a.base0, nullptr, lk_a.bytes, lk_a.ldb, 0u};
             v = lk_a.voff;
         } else {
@@ -433,7 +489,7 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
             f = Feed<B_KC>{lk_b.base0, lk_b.base1, lk_b.bytes, lk_b.ldb, 0u};
             v = lk_b.voff;
         } else {
-            lt_b.setup(Be, Ne, t.Ke, t.n0, wave, lane);
+            lt_b.setup(Be, Ne, t.Ke, t.n0, wave, lane, kTail ? t.n_lim - t.n0 : (uint32_t)BN);
             f = Feed<B_KC>{lt_b.base, nullptr, t.Ke, lt_b.ldb, lt_b.col_bytes};
             v = kGatherK ? t.row0 : lt_b.voff;  // gathered: where the group's entries of row_index begin (same in every lane)
         }
@@ -450,9 +506,9 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
     };
 
     // ---- GATHER: the A operand's rows are rows of args.A picked through args.row_index ----
-    // The tile of round r keeps the row_index entries of its 256 rows in half r % 2 of s_rows. A wavefront's four load
-    // instructions of a K step fetch tile rows g_row, g_row + 64, + 128, + 192 of this lane: four table entries, divided by
-    // the divisor, times the row pitch. Entries past the group's rows read as zero (row 0 of A: rows never stored).
+    // The tile of round r keeps the row_index entries of its rows in half r % 2 of s_rows. A wavefront's four load
+    // instructions of a K step fetch tile rows g_row, g_row + 64, + 128, + 192 of this lane (TALL: and a fifth row
+    // 256 + g_row % 32): table entries, divided by the divisor, times the row pitch. Entries past the group's rows read as zero (row 0 of A: rows never stored).
     const uint32_t g_full = GATHER ? args.a_rows * dim_k * 2u : 0u;  // bytes of A (below 2^31)
     const uint32_t g_ldb = dim_k * 2u;
     const uint32_t g_row = logical_row(wave * 8u + (lane >> 3));
@@ -466,38 +522,43 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
         return q | (n & 0x80000000u);
     };
     uint32_t g_bytes_nxt = 0;  // bytes of A the loads for the next tile may read: all of it, or nothing when nothing follows
-    // per-lane offsets of the four loads of a K step of the tile in table half `half` (the step's k0 goes into the
+    // per-lane offsets of the loads of a K step of the tile in table half `half` (the step's k0 goes into the
     // instruction's scalar offset)
-    auto g_tile_offsets = [&](uint32_t half, uint32_t (&v)[4]) {
-        uint32_t n[4];
-        lds_read4_stride64_quiet(lds_address(reinterpret_cast<const uint8_t*>(s_rows)) + half * 1024u + g_row * 4u, n);
+    auto g_tile_offsets = [&](uint32_t half, uint32_t (&v)[kRowLoads]) {
+        uint32_t n4[4], n[kRowLoads];
+        const uint32_t table = lds_address(reinterpret_cast<const uint8_t*>(s_rows)) + half * (kMostRows * 4u);
+        lds_read4_stride64_quiet(table + g_row * 4u, n4);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int i = 0; i < 4; ++i) n[i] = n4[i];
+        if constexpr (TALL) n[4] = lds_read1_quiet(table + (256u + (g_row & 31u)) * 4u);
+#pragma unroll
+        for (int i = 0; i < (TALL ? 5 : 4); ++i) {
             // an entry that names no row of A (negative, or past the last row) reads as a row of zeros
             const uint32_t src = g_source_row(n[i]);
             v[i] = src < args.a_rows ? src * g_ldb + g_chunk * 16u : kOutOfRange;
         }
     };
     // last, partial K step: chunks past the end of K are pushed out of range, which zero-fills them
-    auto g_clip = [&](uint32_t k0, uint32_t (&v)[4]) {
+    auto g_clip = [&](uint32_t k0, uint32_t (&v)[kRowLoads]) {
         const bool past = k0 + (uint32_t)BK > dim_k && k0 + g_chunk * 8u >= dim_k;
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = past ? kOutOfRange : v[i];
+        for (int i = 0; i < (TALL ? 5 : 4); ++i) v[i] = past ? kOutOfRange : v[i];
     };
-    auto g_offsets = [&](uint32_t half, uint32_t k0, uint32_t (&v)[4]) {
+    auto g_offsets = [&](uint32_t half, uint32_t k0, uint32_t (&v)[kRowLoads]) {
         g_tile_offsets(half, v);
         g_clip(k0, v);
     };
-    uint32_t g_kept[4] = {0u, 0u, 0u, 0u};  // g_tile_offsets of the tile the full-tile K loop is loading from
-    // the table of tile t into half `half`: 32 entries per wavefront, in assembly (one load per wavefront)
+    uint32_t g_kept[kRowLoads] = {};  // g_tile_offsets of the tile the full-tile K loop is loading from
+    // the table of tile t into half `half`: 32 (TALL: 36) entries per wavefront, in assembly (one load per wavefront)
     auto g_issue_table = [&](const Tile& t, uint32_t half) {
         if constexpr (GATHER) {
             const bool real = t.valid && t.Me > t.m0;
-            const uint32_t rows = real ? (t.Me - t.m0 < (uint32_t)BM ? t.Me - t.m0 : (uint32_t)BM) : 0u;
+            const uint32_t rows = real ? t.rows : 0u;
+            constexpr uint32_t kEach = kMostRows / NW;
             const u32x4 rs = make_rsrc_words(reinterpret_cast<const uint16_t*>(args.row_index + (real ? (uint64_t)t.row0 + t.m0 : 0u)),
                                              rows * 4u);
-            const uint32_t to = lds_address(reinterpret_cast<const uint8_t*>(s_rows)) + half * 1024u + wave * 128u;
-            if (lane < 32u) buffer_load_lds_quiet_b32(rs, (wave * 32u + lane) * 4u, 0u, to);
+            const uint32_t to = lds_address(reinterpret_cast<const uint8_t*>(s_rows)) + half * (kMostRows * 4u) + wave * (kEach * 4u);
+            if (lane < kEach) buffer_load_lds_quiet_b32(rs, (wave * kEach + lane) * 4u, 0u, to);
         }
     };
     static_assert(!GATHER_ANY || 32 / NW == 4, "four load instructions per wavefront and K step");
@@ -569,16 +630,18 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
         pf_steps = k_steps(t);
         if constexpr (kSplit) pf_k0 = t.ks;
         if (!pf_is_b) {
-            const uint32_t i = p * 16u + lane;
+            // (TALL: lanes 16 and 17 take the rows past 256; those past the tile are out of the descriptor's range or no row)
+            constexpr uint32_t kLanes = TALL ? 18u : 16u;
+            const uint32_t i = lane < 16u ? p * 16u + lane : 64u + p * 2u + (lane - 16u);
             if constexpr (GATHER) {
-                const uint32_t n = lds_read1_quiet(lds_address(reinterpret_cast<const uint8_t*>(s_rows)) + (round & 1u) * 1024u +
-                                                   (lane < 16u ? 4u * i + t.pf_c : 0u) * 4u);
+                const uint32_t n = lds_read1_quiet(lds_address(reinterpret_cast<const uint8_t*>(s_rows)) + (round & 1u) * (kMostRows * 4u) +
+                                                   (lane < kLanes ? 4u * i + t.pf_c : 0u) * 4u);
                 pf_base = args.A; pf_bytes = g_full;
-                const uint32_t src = lane < 16u ? g_source_row(n) : 0xffffffffu;
+                const uint32_t src = lane < kLanes && 4u * i + t.pf_c < t.rows ? g_source_row(n) : 0xffffffffu;
                 pf_voff = src < args.a_rows ? src * g_ldb : kOutOfRange;
             } else if constexpr (A_KC) {
                 pf_base = fa_cur.base0; pf_bytes = fa_cur.extent;
-                pf_voff = lane < 16u ? (4u * i + t.pf_c) * (t.Ke * 2u) : kOutOfRange;
+                pf_voff = lane < kLanes ? (4u * i + t.pf_c) * (t.Ke * 2u) : kOutOfRange;
             } else {
                 pf_base = fa_cur.base0; pf_ldb = fa_cur.ldb; pf_col_bytes = fa_cur.col_bytes; pf_kdim = t.Ke;
                 pf_voff = lane < 16u ? i * fa_cur.ldb + t.pf_c * 128u : kOutOfRange;
@@ -619,7 +682,9 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
 
     constexpr int kLoads = 32 / NW;                // load instructions per wavefront, operand and K step
     constexpr uint32_t kStepLoads = 2 * kLoads;    // per wavefront and K step
-    // store instructions per wavefront and tile (the epilogue issues a fixed number)
+    constexpr uint32_t kColdLoads = kStepLoads + (TALL ? 1 : 0);  // ... of a cold start, which always fetches the rows past 256
+    // store instructions per wavefront and tile (the epilogue issues a fixed number; that of a tile with rows past 256 a few
+    // more, which makes the wait that counts them wait for the oldest few as well)
     constexpr uint32_t kTileStores = EPI == EPI_PLAIN        ? WM * WN * 2 / 1024
                                      : EPI == EPI_SWIGLU_BWD ? 2 * (WM * WN * 2 / 1024)  // two columns written per column
                                      : kSplit                ? WM * WN * 4 / 1024
@@ -634,13 +699,14 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
     };
     // GATHER: the same four loads through the row table in half `half`; `bytes`: how much of A they may read
     // kept: take the offsets from g_kept (the caller has set it for that tile) instead of reading the table
+    // (instruction 4: the rows past 256)
     auto issue_a_gathered = [&](int stage, uint32_t k0, uint32_t half, uint32_t bytes, bool kept, auto i0_c, auto i1_c)
                                 __attribute__((always_inline)) {
         constexpr int I0 = decltype(i0_c)::value, I1 = decltype(i1_c)::value;
-        uint32_t v[4];
+        uint32_t v[kRowLoads];
         if (kept) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) v[i] = g_kept[i];
+            for (int i = 0; i < (TALL ? 5 : 4); ++i) v[i] = g_kept[i];
             g_clip(k0, v);
         } else {
             g_offsets(half, k0, v);
@@ -649,7 +715,12 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
         uint8_t* tile = stage ? s_a1 : s_a0;
 #pragma unroll
         for (int i = I0; i < I1; ++i)
-            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)(tile + (i * NW + wave) * 1024), 16, v[i], k0 * 2u, 0, 0);
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void*)(i < 4 ? tile + (i * NW + wave) * 1024 : (stage ? s_x1 : s_x0) + (wave & 3u) * 1024),
+                                                     16, v[i], k0 * 2u, 0, 0);
+    };
+    // TALL: the rows past 256, one instruction per wavefront (outside the tile's rows: zeros)
+    auto issue_x = [&](int stage, uint32_t k0) __attribute__((always_inline)) {
+        if constexpr (TALL && !GATHER) lk_a.issue_extra(stage ? s_x1 : s_x0, k0);
     };
     auto issue_b = [&](int stage, uint32_t k0, auto i0_c, auto i1_c) __attribute__((always_inline)) {
         constexpr int I0 = decltype(i0_c)::value, I1 = decltype(i1_c)::value;
@@ -666,14 +737,17 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
     // ... and written in assembly, for a cold start
     auto issue_quiet = [&](int stage, uint32_t k0) {
         if constexpr (GATHER) {
-            uint32_t v[4];
+            uint32_t v[kRowLoads];
             g_offsets(round & 1u, k0, v);
             const u32x4 r = make_rsrc_words(args.A, g_full);
             const uint32_t lds0 = lds_address(stage ? s_a1 : s_a0) + wave * 1024u;
 #pragma unroll
             for (int i = 0; i < 4; ++i) buffer_load_lds_quiet(r, v[i], k0 * 2u, lds0 + (uint32_t)(i * NW) * 1024u);
-        } else if constexpr (A_KC) lk_a.issue_quiet(stage ? s_a1 : s_a0, k0);
-        else lt_a.issue_quiet(stage ? s_a1 : s_a0, k0);
+            if constexpr (TALL) buffer_load_lds_quiet(r, v[4], k0 * 2u, lds_address(stage ? s_x1 : s_x0) + (wave & 3u) * 1024u);
+        } else if constexpr (A_KC) {
+            lk_a.issue_quiet(stage ? s_a1 : s_a0, k0);
+            if constexpr (TALL) lk_a.issue_quiet_extra(stage ? s_x1 : s_x0, k0);
+        } else lt_a.issue_quiet(stage ? s_a1 : s_a0, k0);
         if constexpr (kGatherK) {
             uint32_t v[4];
             gk_offsets(k0, lt_b.kdim, gk_request(vb_cur + k0 + wave * 8u, false), v);
@@ -693,12 +767,14 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
     while (cur.valid) {
         const uint32_t Me = cur.Me, Ke = cur.Ke, m0 = cur.m0, n0 = cur.n0, n_lim = cur.n_lim;
         const uint64_t off_d = cur.off_d;
+        const bool has_extra = TALL && cur.rows > (uint32_t)BM;  // rows past 256
 
         if (!streamed) {
             if (!cur.fast) {
                 if constexpr (EPI == EPI_PLAIN && !kGatherK) {  // (the gathered entry point admits only sizes without such tiles)
-                    scalar_tile<EL, A_KC, B_KC, BM, BN>(args.A + cur.off_a, args.B + cur.off_b, args.D + off_d, Me, Ne, Ke, m0, n0,
-                                                        args.alpha, NT);
+                    // (TALL: up to the tile's last row; with A_KC the number of rows is no pitch)
+                    scalar_tile<EL, A_KC, B_KC, TALL ? kTallM : BM, BN>(args.A + cur.off_a, args.B + cur.off_b, args.D + off_d,
+                                                                        TALL ? m0 + cur.rows : Me, Ne, Ke, m0, n0, args.alpha, NT);
                 }
                 cur = nxt;
                 nxt = lookup(round + 2);
@@ -742,6 +818,7 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
             fb_nxt.extent = 0u;
             vb_nxt = vb_cur;
         }
+        const bool extra_near = has_extra || (stream_next && nxt.rows > (uint32_t)BM);
         g_bytes_nxt = stream_next ? g_full : 0u;
         // (the set-ups above left the loader objects aimed at the last tile set up)
         aim_a(fa_cur, va_cur);
@@ -751,9 +828,11 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
         // instruction's result is named as part of that value again (anchor_value): the result then stays in the register
         // quadruple its addend came from. The compiler has no tied-operand form of the 4-register instruction; as 32 separate
         // quadruples the results wandered through the register file and the allocator spilled 3 to 40 registers.
-        f32x16 acc[RB];
+        // (TALL: one more row block, the wavefront's share of the rows past 256)
+        constexpr int RBX = TALL ? RB + 1 : RB;
+        f32x16 acc[RBX];
 #pragma unroll
-        for (int i = 0; i < RB; ++i)
+        for (int i = 0; i < RBX; ++i)
 #pragma unroll
             for (int x = 0; x < 16; ++x) acc[i][x] = 0.0f;
         auto mfma_block = [&](f32x16& c, int j, typename EL::frag b, typename EL::frag a) __attribute__((always_inline)) {
@@ -772,8 +851,9 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
         // column block. In the last phase of a slice every B fragment is replaced by the next slice's as soon as its two
         // matrix instructions have been issued (one set of B registers).
         // The K loop exists in five versions, for wavefronts whose first FA = 8, 4, 2, 1 or 0 row blocks (of 16 rows)
-        // hold rows of the group.
-        typename EL::frag fa[4][2], fb[CB];
+        // hold rows of the group, and TALL in a sixth, FA = 9, for tiles with rows past 256: the ninth block joins the last
+        // pair of each slice.
+        typename EL::frag fa[4][2], fx, fb[CB];
         // A fragments of pair `pair` of slice ks into buffer buf
         auto load_a = [&](auto fa_c, int stage, int ks, int pair, int buf) __attribute__((always_inline)) {
             constexpr int FA = decltype(fa_c)::value;
@@ -785,6 +865,9 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
                 if constexpr (A_KC) fa[buf][i] = __builtin_bit_cast(typename EL::frag, read_kc_frag(ta + a_off[b] + kc_slice[ks]));
                 else fa[buf][i] = __builtin_bit_cast(typename EL::frag, read_tr_frag(ta + a_off[b] + ks * kSliceT));
             }
+        };
+        auto load_x = [&](int stage, int ks) __attribute__((always_inline)) {
+            fx = __builtin_bit_cast(typename EL::frag, read_kc_frag((stage ? s_x1 : s_x0) + x_off + kc_slice[ks]));
         };
         auto load_b = [&](int stage, int ks, int j) __attribute__((always_inline)) {
             const uint8_t* tb = stage ? s_b1 : s_b0;
@@ -802,6 +885,9 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
 #pragma unroll
                     for (int i = 0; i < AB; ++i)
                         mfma_block(acc[pair * 2 + i], j, fb[j], fa[abuf][i]);
+                    if constexpr (FA > RB) {
+                        if (reload) mfma_block(acc[RB], j, fb[j], fx);
+                    }
                     if (reload) load_b(next_stage, next_ks, j);
                 }
             }
@@ -816,7 +902,15 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
             constexpr int FA = decltype(fa_c)::value;
             constexpr int SRC = decltype(src_c)::value;
             constexpr int AB = FA < 2 ? FA : 2;       // row blocks per phase
-            constexpr int PP = FA >= 2 ? FA / 2 : 1;  // phases per k slice
+            constexpr int PP = FA >= RB ? RB / 2 : (FA >= 2 ? FA / 2 : 1);  // phases per k slice
+            constexpr int X = FA > RB ? 1 : 0;        // the ninth row block
+            // The loads of B in front of those of A: in tall tiles of the NN layout, which has no L2 prefetch, 1 to 4 % faster (input
+            // gradients: 1498 -> 1440 us, hidden 4096, I 14336, E 8, k 2, 4096 tokens); in the NT layout 3 to 6 % slower, and in tiles of
+            // few rows up to 6 %.
+            constexpr bool kBFirst = X && !B_KC;
+            // The rows past 256 are fetched where the tile has them and in the steps whose loads may be for the next tile; the versions
+            // for few rows or no columns look whether this tile or the next has any.
+            constexpr bool kLoadX = TALL && (FA != RB || SRC != 0);
             constexpr int NPH = 2 * PP;               // phases of the step
             constexpr int kReadsA = (A_KC ? 1 : 2) * AB, kReadsB = (B_KC ? 1 : 2);  // LDS reads per pair, per B fragment
             // On entry A buffer 0 and the B registers hold the fragments of the first phase.
@@ -832,6 +926,13 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
                     issue_a_gathered(stage, k0, (of_next ? round + 1u : round) & 1u, of_next ? g_bytes_nxt : g_full, SRC != 2, i0_c, i1_c);
                 } else {
                     issue_a(stage, k0, i0_c, i1_c);
+                }
+            };
+            auto issue_x_part = [&](uint32_t k0) __attribute__((always_inline)) {
+                if constexpr (kLoadX) {
+                    if (FA < RB && !extra_near) return;
+                    if constexpr (GATHER) issue_a_part(k0, std::integral_constant<int, 4>{}, std::integral_constant<int, 5>{});
+                    else issue_x(stage, k0);
                 }
             };
             // kGatherK: the entries for this step's loads were requested two steps ago: by a step of this tile into a register,
@@ -878,7 +979,7 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
                 }
                 return k0;
             };
-            if constexpr (FA == RB) {
+            if constexpr (FA >= RB) {
                 // Full tiles: the barrier comes after five of the eight phases, with the A fragments of the last three phases
                 // already in registers (four A buffers), so that the step's loads go out over three phases instead of one:
                 // eight wavefronts that leave the barrier together otherwise queue 72 loads on the one address path at once.
@@ -888,42 +989,53 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
 #pragma unroll
                 for (int ph = 0; ph < 4; ++ph) {
                     load_a(fa_c, stage, (ph + 2) / PP, (ph + 2) % PP, (ph + 2) & 3);
+                    if (X && ph == 1) load_x(stage, 0);
                     mma(fa_c, ph, ph, ph == 3, stage, 1);
                     if (ph == 3) {
                         __builtin_amdgcn_sched_group_barrier(0x100, kReadsA, 0);
 #pragma unroll
                         for (int j = 0; j < CB; ++j) {
-                            __builtin_amdgcn_sched_group_barrier(0x008, AB, 0);
+                            __builtin_amdgcn_sched_group_barrier(0x008, AB + X, 0);
                             __builtin_amdgcn_sched_group_barrier(0x100, kReadsB, 0);
                         }
                     } else {
                         if (ph == 0) interleave3<0, AB * CB, 2 * kReadsA, 0>();
+                        else if (ph == 1) interleave3<0, AB * CB, kReadsA + X, 0>();
                         else interleave3<0, AB * CB, kReadsA, 0>();
                     }
                     __builtin_amdgcn_sched_barrier(0);
                 }
                 load_a(fa_c, stage, 1, 2, 2);
                 load_a(fa_c, stage, 1, 3, 3);
+                if (X) load_x(stage, 1);
                 mma(fa_c, 0, 0, false, stage, 1);
-                __builtin_amdgcn_sched_group_barrier(0x100, 2 * kReadsA, 0);
+                __builtin_amdgcn_sched_group_barrier(0x100, 2 * kReadsA + X, 0);
                 __builtin_amdgcn_sched_group_barrier(0x008, AB * CB, 0);
                 // every load of step kt+1 has landed and every LDS read of this stage has returned
                 __builtin_amdgcn_s_waitcnt(decltype(wait_c)::value);
                 __builtin_amdgcn_s_barrier();
                 asm volatile("" ::: "memory");
                 const uint32_t k0 = aim_loads();
-                issue_a_part(k0, I0_{}, I3_{});
+                if constexpr (kBFirst) issue_b(stage, k0, I0_{}, I3_{});
+                else issue_a_part(k0, I0_{}, I3_{});
                 mma(fa_c, 1, 1, false, stage, 1);
                 spread_mfma_vmem<0, AB * CB, 3>();
                 __builtin_amdgcn_sched_barrier(0);
-                issue_a_part(k0, I3_{}, IN_{});
-                gk_step_offsets(k0);
-                issue_b(stage, k0, I0_{}, I2_{});
+                if constexpr (kBFirst) {
+                    issue_b(stage, k0, I3_{}, IN_{});
+                    issue_a_part(k0, I0_{}, I2_{});
+                } else {
+                    issue_a_part(k0, I3_{}, IN_{});
+                    gk_step_offsets(k0);
+                    issue_b(stage, k0, I0_{}, I2_{});
+                }
                 mma(fa_c, 2, 2, false, stage, 1);
                 spread_mfma_vmem<0, AB * CB, 3>();
                 __builtin_amdgcn_sched_barrier(0);
                 load_a(fa_c, stage ^ 1, 0, 0, 0);
-                issue_b(stage, k0, I2_{}, IN_{});
+                if constexpr (kBFirst) issue_a_part(k0, I2_{}, IN_{});
+                else issue_b(stage, k0, I2_{}, IN_{});
+                issue_x_part(k0);
                 if constexpr (kPrefetch) asm volatile("" : "+v"(pf_voff));
                 issue_prefetch(kt + kPfDist);
                 gk_step_request();
@@ -932,9 +1044,9 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
 #pragma unroll
                 for (int j = 0; j < CB; ++j) {
 #pragma unroll
-                    for (int i = 0; i < AB; ++i) {
+                    for (int i = 0; i < AB + X; ++i) {
                         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                        if (j * AB + i < 2 + (kPrefetch ? 1 : 0) + (kGatherK ? 1 : 0)) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+                        if (j * (AB + X) + i < 2 + (kLoadX ? 1 : 0) + (kPrefetch ? 1 : 0) + (kGatherK ? 1 : 0)) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
                     }
                     __builtin_amdgcn_sched_group_barrier(0x100, kReadsB, 0);
                 }
@@ -969,6 +1081,7 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
                 issue_a_part(k0, I0_{}, IN_{});
                 gk_step_offsets(k0);
                 issue_b(stage, k0, I0_{}, IN_{});
+                issue_x_part(k0);
                 // the prefetch goes out behind this step's loads (the empty statement orders it: the wait of the next step
                 // counts on it being the newest load)
                 if constexpr (kPrefetch) asm volatile("" : "+v"(pf_voff));
@@ -990,6 +1103,7 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
                         }
                         __builtin_amdgcn_sched_group_barrier(0x100, kReadsB, 0);
                     }
+                    if constexpr (kLoadX) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
                     if constexpr (kPrefetch) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
                     if constexpr (kGatherK) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
                 }
@@ -1019,7 +1133,7 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
             }
         };
         Tile nn{};  // the tile after next
-        const uint32_t tile_rows = Me - m0 < (uint32_t)BM ? Me - m0 : (uint32_t)BM;
+        const uint32_t tile_rows = cur.rows;
         const uint32_t wave_rows = tile_rows > wm * WM ? tile_rows - wm * WM : 0u;
         const bool has_columns = n0 + wn * (kGlu ? WN / 2 : WN) < n_lim;
         const uint32_t row_blocks = has_columns ? uniform((wave_rows + 15u) / 16u) : 0u;  // of 16 rows
@@ -1032,7 +1146,7 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
             const uint8_t* const b_hi[3] = {s_b0 + 16384, s_b1 + 16384, s_a1 + 16384};
             auto issue_thin = [&](int st, uint32_t k0) {
                 if constexpr (GATHER) {
-                    uint32_t v[4];
+                    uint32_t v[kRowLoads];
                     g_offsets(round & 1u, k0, v);
                     buffer_load_lds_quiet(make_rsrc_words(args.A, g_full), v[0], k0 * 2u, lds_address(a_at[st]) + wave * 1024u);
                 } else if constexpr (A_KC) lk_a.issue_quiet_first_rows(lds_address(a_at[st]), k0);
@@ -1110,7 +1224,7 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
                 for (uint32_t i = 0; i < kTileStores; ++i)  // (distinct offsets: identical stores would be merged into one)
                     store_tile16<false>(nowhere, kOutOfRange + i * 16u, uint4{0u, 0u, 0u, 0u});
                 // the first step's loads have landed; the second step's, and the stand-in stores, may be out
-                __builtin_amdgcn_s_waitcnt(waitcnt_imm((int)(kStepLoads + kTileStores), false));
+                __builtin_amdgcn_s_waitcnt(waitcnt_imm((int)(kColdLoads + kTileStores), false));
                 __builtin_amdgcn_s_barrier();
                 asm volatile("" ::: "memory");
             }
@@ -1128,7 +1242,7 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
                 }
                 step(fa_c, WaitFirst{}, SrcEither{}, 0, 0);
                 step(fa_c, WaitStep{}, SrcEither{}, 1, 1);
-                if constexpr (FA == RB) {
+                if constexpr (FA >= RB) {
                     // full tiles: the steps in the middle load from the current tile and the last two from the next, each
                     // with the loaders aimed once, so that the loop body carries no selects
                     if (KT2 > 2u) {
@@ -1154,7 +1268,11 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
                 }
             };
             static_assert(RB == 8, "the versions below are for eight row blocks per wavefront");
-            if (row_blocks > 4) k_loop(std::integral_constant<int, 8>{});
+            if constexpr (TALL) {
+                if (has_extra && has_columns) k_loop(std::integral_constant<int, RB + 1>{});
+            }
+            if (has_extra && has_columns) {}
+            else if (row_blocks > 4) k_loop(std::integral_constant<int, 8>{});
             else if (row_blocks > 2) k_loop(std::integral_constant<int, 4>{});
             else if (row_blocks == 2) k_loop(std::integral_constant<int, 2>{});
             else if (row_blocks == 1) k_loop(std::integral_constant<int, 1>{});
@@ -1188,7 +1306,7 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
         if (EPI == EPI_PLAIN && args.alpha != 1.0f) {
             const float alpha = args.alpha;
 #pragma unroll
-            for (int i = 0; i < RB; ++i) acc[i] *= alpha;
+            for (int i = 0; i < RBX; ++i) acc[i] *= alpha;
         }
         // Tiles with a short reduction write much per flop (a weight gradient over ~500 rows: 8 K steps per 128 KB tile):
         // their stores carry the non-temporal hint (+4 to 5 % there); for long reductions plain stores are faster by 0 to 1 %
@@ -1219,7 +1337,9 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
             else return product;
         };
         // EPI_SWIGLU_BWD: the h values of the eight passes (16 rows each) of this wavefront's sub-tile: [pass][row 0/1][up, gate]
-        u32x4 bwd_h[EPI == EPI_SWIGLU_BWD ? RB : 1][2][2];
+        u32x4 bwd_h[EPI == EPI_SWIGLU_BWD ? RBX : 1][2][2];
+        // first row, inside the group, of this wavefront's row block i
+        auto block_row = [&](int i) -> uint32_t { return i < RB ? m0 + wm * WM + (uint32_t)i * 16u : m0 + (uint32_t)BM + wm * 16u; };
         // byte offset of this lane's piece of row `r` (0 or 1: rows lane / 8 and 8 + lane / 8 of the pass) from the pass's
         // first row and the wavefront's first column, or out of range
         auto bwd_offset = [&](int r, uint32_t cols_valid) -> uint32_t {
@@ -1228,11 +1348,12 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
             return c16 * 8u < cols_valid ? row * (Ne * 4u) + c16 * 16u : kOutOfRange;
         };
         auto bwd_rows = [&](int pass) -> uint32_t {  // rows of the pass inside the group
-            const uint32_t r0 = m0 + wm * WM + (uint32_t)pass * 16u;
+            const uint32_t r0 = block_row(pass);
+            if (pass == RB && !has_extra) return 0u;
             return r0 < Me ? (Me - r0 < 16u ? Me - r0 : 16u) : 0u;
         };
         auto bwd_origin = [&](int pass, uint32_t col0) -> uint64_t {  // element offset of the pass's first row and column
-            return ((uint64_t)cur.row0 + m0 + wm * WM + (uint32_t)pass * 16u) * (2ull * Ne) + col0;
+            return ((uint64_t)cur.row0 + block_row(pass)) * (2ull * Ne) + col0;
         };
         // h is read once and its gradient written once, in whole 128-byte lines: both carry the non-temporal hint, which
         // keeps them from displacing the operand panels in the L2 (+3 % on the Mixtral shape, +2 % large-E, +0.5 % fine-grained)
@@ -1285,9 +1406,8 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
         };
         const uint32_t put_row = el & 15u, put_col = (el >> 4) * 4u;  // this lane's place in a 16 x 16 block
         uint32_t ypack[2][2][2];  // swiglu: the activation of two row blocks, which share one image: [block][column block][2]
-#pragma unroll
-        for (int i = 0; i < RB; ++i) {
-            const uint32_t r0 = m0 + wm * WM + i * 16;  // first output row of this block
+        auto put_block = [&](int i) __attribute__((always_inline)) {
+            const uint32_t r0 = block_row(i);  // first output row of this block
             const uint32_t rows_valid = r0 < Me ? (Me - r0 < 16u ? Me - r0 : 16u) : 0u;
             if constexpr (kSplit) {
                 // the sums as they are: a lane's four consecutive columns of every 16 x 16 block, 64 bytes per row and block
@@ -1330,7 +1450,7 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
 #pragma unroll
                     for (int j = 0; j < CB; ++j) stage_put_quiet<WN * 2>(img, put_row, j * 16 + put_col, w[j]);
                     bwd_finish(i, col0, cols_valid);
-                    if (i + kAhead < RB) bwd_request(i + kAhead, col0, cols_valid);
+                    if (i + kAhead < RBX) bwd_request(i + kAhead, col0, cols_valid);
                 }
             } else {
                 // first the rounded pre-activation (32 "up" columns | 32 "gate" columns per row) of this row block, then,
@@ -1368,11 +1488,12 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
                     stage_flush_split_quiet<HB, 16, WN / 2>(img, args.D + off_d + (uint64_t)r0 * Ne + col0, Ne, rows_valid, cols_valid,
                                                             n_span, el);
                 }
-                if (i & 1) {
-                    const uint32_t row0 = r0 - 16u;  // first row of the pair of blocks
-                    const uint32_t rows_pair = row0 < Me ? (Me - row0 < 32u ? Me - row0 : 32u) : 0u;
+                // (the ninth block goes alone: the second half of its image is past its rows)
+                if ((i & 1) || i == RB) {
+                    const uint32_t row0 = i == RB ? r0 : r0 - 16u;  // first row of the pair of blocks
+                    const uint32_t rows_pair = i == RB ? rows_valid : (row0 < Me ? (Me - row0 < 32u ? Me - row0 : 32u) : 0u);
 #pragma unroll
-                    for (int b = 0; b < 2; ++b)
+                    for (int b = 0; b < (i == RB ? 1 : 2); ++b)
 #pragma unroll
                         for (int jj = 0; jj < 2; ++jj) {
                             uint2 wy;
@@ -1383,6 +1504,11 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
                     stage_flush_quiet<YB, 32>(img, args.ACT + off_d / 2 + (uint64_t)row0 * n_span + col0, n_span, rows_pair, cols_valid, el);
                 }
             }
+        };
+#pragma unroll
+        for (int i = 0; i < RB; ++i) put_block(i);
+        if constexpr (TALL) {
+            if (has_extra) put_block(RB);
         }
 
         // ---- on to the next tile ----
@@ -1400,6 +1526,37 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
         ++round;
     }
 }
+
+template <typename EL, bool A_KC, bool B_KC, int EPI, bool VARY_K, bool BIAS, bool GATHER, bool TALL>
+int launch(const Args& args, hipStream_t st) {
+    int cus = num_compute_units();
+    if (cus <= 0) cus = 256;
+    hipLaunchKernelGGL((ragged_gemm_kernel<EL, A_KC, B_KC, EPI, VARY_K, BIAS, GATHER, TALL>), dim3((uint32_t)cus), dim3(NT), 0, st,
+                       args);
+    return launch_status("grouped_gemm_ragged");
+}
+
+// the forward (NT) kernels by epilogue, bias and gather
+template <typename EL, int EPI, bool TALL>
+int launch_forward_as(const Args& args, hipStream_t st) {
+    const bool bias = args.bias != nullptr, gather = args.row_index != nullptr;
+    if (bias && gather) return launch<EL, true, true, EPI, false, true, true, TALL>(args, st);
+    if (bias) return launch<EL, true, true, EPI, false, true, false, TALL>(args, st);
+    if (gather) return launch<EL, true, true, EPI, false, false, true, TALL>(args, st);
+    return launch<EL, true, true, EPI, false, false, false, TALL>(args, st);
+}
+
+// The launches with varying rows and A's reduction contiguous, for at most kTallGroups groups (grouped_gemm_ragged_tall.hip).
+// epi: EPI_PLAIN, EPI_SWIGLU, EPI_SWIGLU_ACT with B's reduction contiguous and any bias and gather; without them EPI_PLAIN and
+// EPI_SPLIT in both layouts of B, and EPI_SWIGLU_BWD with B stored [reduction, out].
+int launch_tall(const Args& args, int epi, bool b_kc, bool bf16, hipStream_t st);
+
+// The parts of a split reduction (ragged_split.hip)
+struct SplitPlan {
+    uint32_t splits, steps;  // parts and K steps of each (even; the last part takes what is left); splits 1: no split
+};
+SplitPlan plan_split(int64_t R, int64_t E, int64_t N, int64_t K, bool b_kc, bool tall);
+int launch_split_reduce(const Args& args, bool bf16, hipStream_t st);
 
 }  // namespace ragged
 }  // namespace gemm

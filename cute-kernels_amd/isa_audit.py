@@ -2,18 +2,19 @@
 
 Usage: python cute-kernels_amd/isa_audit.py [file.s]
 
-The kernels of csrc/ragged_kernel.h (instantiated in csrc/grouped_gemm_ragged.hip) wait for their operand loads with `s_waitcnt vmcnt(N)` where N is a constant
+The kernels of csrc/ragged_kernel.h wait for their operand loads with `s_waitcnt vmcnt(N)` where N is a constant
 that counts the vector-memory instructions a wavefront has issued after the loads it waits for (loads and stores complete
 in issue order). The constants are derived in the source from the number of loads per K step, the number of stores an
 epilogue issues and whether a prefetch, a bias load or a request for row_index entries follows a step's loads. This script
-compiles the source to assembly (device code only; or reads a file made with `hipcc ... --cuda-device-only -S`) and checks,
+compiles the sources that instantiate them to assembly (device code only; or reads a file made with `hipcc ... --cuda-device-only -S`) and checks,
 for every instantiation of ragged_gemm_kernel, that the instruction stream has the shape those constants assume:
 
  * every wait that is followed by a barrier and the eight operand loads of a K step allows exactly the number of newer
    instructions of a step in the loop (prefetch, request) or of a tile's first step (the epilogue's stores, prefetch, bias);
- * between the two barriers of a loop body of two K steps a wavefront issues the eight loads and exactly those extras;
- * the cold start issues sixteen operand loads, as many stand-in stores as an epilogue issues stores, and waits for all but
-   the eight loads of the second step and the stores;
+ * between the two barriers of a loop body of two K steps a wavefront issues the eight loads and exactly those extras (nine loads in
+   the version for tiles with rows past 256 of the tall kernels);
+ * the cold start issues sixteen operand loads (tall kernels: eighteen), as many stand-in stores as an epilogue issues stores, and
+   waits for all but the loads of the second step and the stores;
  * the three-stage loop of groups of at most 64 rows issues five loads per step and waits for all but five;
  * no instantiation touches scratch memory, and none contains a loop over the distinct values of an operand that the
    hardware wants in scalar registers (what the compiler generates around a vector-memory instruction whose descriptor or
@@ -31,15 +32,15 @@ import sys
 import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-SOURCE = os.path.join(HERE, "csrc", "grouped_gemm_ragged.hip")
+SOURCES = [os.path.join(HERE, "csrc", name) for name in ("grouped_gemm_ragged.hip", "grouped_gemm_ragged_tall.hip")]
 # stores per wavefront and tile: plain, SwiGLU with h, SwiGLU, SwiGLU backward, fp32 sums of a split reduction
 EPI_STORES = {0: 16, 1: 24, 2: 8, 3: 32, 4: 32}
 
 
-def compile_to_assembly(path: str) -> None:
+def compile_to_assembly(source: str, path: str) -> None:
     from build import FLAGS, HIPCC  # the flags the library is built with
 
-    cmd = [HIPCC] + FLAGS + ["--cuda-device-only", "-S", SOURCE, "-o", path]
+    cmd = [HIPCC] + FLAGS + ["--cuda-device-only", "-S", source, "-o", path]
     proc = subprocess.run(cmd, capture_output=True, text=True)
     if proc.returncode != 0:
         raise RuntimeError(proc.stderr[-2000:])
@@ -81,8 +82,8 @@ def audit(asm_path: str) -> int:
     problems = 0
     for a, b in zip(starts[:-1], starts[1:]):
         name = lines[a].split(":")[0]
-        m = re.search(r"ragged_gemm_kernelINS0_(\w+?)ELb(\d)ELb(\d)ELi(\d)ELb(\d)ELb(\d)ELb(\d)E", name)
-        el, a_kc, b_kc, epi, vary_k, bias, gather = m.group(1), *[int(x) for x in m.groups()[1:]]
+        m = re.search(r"ragged_gemm_kernelINS0_(\w+?)ELb(\d)ELb(\d)ELi(\d)ELb(\d)ELb(\d)ELb(\d)ELb(\d)E", name)
+        el, a_kc, b_kc, epi, vary_k, bias, gather, tall = m.group(1), *[int(x) for x in m.groups()[1:]]
         body = lines[a:b]
         end = next((k for k, line in enumerate(body) if "s_endpgm" in line), len(body))
         blocks, waterfalls = tokens(body[:end])
@@ -90,7 +91,7 @@ def audit(asm_path: str) -> int:
         request = 1 if (vary_k and gather) else 0
         stores = EPI_STORES[epi]
         wait_step, wait_first = prefetch + request, stores + prefetch + bias
-        tag = f"{el} A_KC={a_kc} B_KC={b_kc} epilogue={epi} reduction_varies={vary_k} bias={bias} gather={gather}"
+        tag = f"{el} A_KC={a_kc} B_KC={b_kc} epilogue={epi} reduction_varies={vary_k} bias={bias} gather={gather} tall={tall}"
         found = {"step": 0, "first": 0, "body": 0, "cold": 0, "thin": 0}
         gathers_rows = bool(gather and not vary_k)
 
@@ -107,12 +108,12 @@ def audit(asm_path: str) -> int:
             # waits in front of a barrier that the operand loads of a K step follow
             for w, loads in ([] if gathers_rows else re.findall(r"w(\d+),\|(O+)", blk)):
                 n, count = int(w), len(loads)
-                if count == 8:
+                if count in (8, 8 + tall):
                     if n == wait_step:
                         found["step"] += 1
                     elif n == wait_first:
                         found["first"] += 1
-                    elif n == 8 + stores:
+                    elif n == 8 + tall + stores:
                         pass  # (the cold start's wait directly followed by the first step: not a shape the compiler produces)
                     else:
                         fail(f"a step waits for all but {n}, expected {wait_step} or {wait_first}", blk)
@@ -124,18 +125,20 @@ def audit(asm_path: str) -> int:
             # a loop body of two steps in one block: what is issued between its two barriers
             for between in re.findall(r"\|(O{8}[^|]*?)w\d+,\|O{8}", blk):
                 issued = len(re.sub(r"w\d+,", "", between))
-                if issued == 8 + wait_step:
+                if issued in (8 + wait_step, 8 + tall + wait_step):
                     found["body"] += 1
                 else:
-                    fail(f"{issued} instructions between the barriers of two steps, expected {8 + wait_step}", blk)
+                    fail(f"{issued} instructions between the barriers of two steps, expected {8 + wait_step}"
+                         + (f" or {9 + wait_step}" if tall else ""), blk)
             # the cold start: sixteen operand loads (the gathered kinds mix loads of row_index entries in), the stand-in
             # stores, the wait
             cold = None if gathers_rows else re.search(r"((?:[OLp]|w\d+,)*O)(s+)w(\d+),\|", blk)
             if cold and cold.group(1).count("O") >= 16:
                 found["cold"] += 1
-                if cold.group(1).count("O") != 16 or len(cold.group(2)) != stores or int(cold.group(3)) != 8 + stores:
+                loads = 8 + tall
+                if cold.group(1).count("O") != 2 * loads or len(cold.group(2)) != stores or int(cold.group(3)) != loads + stores:
                     fail(f"cold start: {cold.group(1).count('O')} loads, {len(cold.group(2))} stores, wait {cold.group(3)}; "
-                         f"expected 16, {stores}, {8 + stores}", blk)
+                         f"expected {2 * loads}, {stores}, {loads + stores}", blk)
         if gathers_rows:
             if found["body"] == 0:
                 fail(f"expected shapes not found ({found})", "")
@@ -152,11 +155,14 @@ def audit(asm_path: str) -> int:
 def main() -> int:
     if len(sys.argv) > 1:
         return audit(sys.argv[1])
+    problems = 0
+    sys.path.insert(0, HERE)
     with tempfile.TemporaryDirectory() as tmp:
-        path = os.path.join(tmp, "grouped_gemm_ragged.s")
-        sys.path.insert(0, HERE)
-        compile_to_assembly(path)
-        return audit(path)
+        for source in SOURCES:
+            path = os.path.join(tmp, os.path.basename(source) + ".s")
+            compile_to_assembly(source, path)
+            problems += audit(path)
+    return problems
 
 
 if __name__ == "__main__":

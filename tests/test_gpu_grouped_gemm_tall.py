@@ -1,0 +1,166 @@
+"""GPU parity of the tiles of up to 288 rows, which launches of at most 256 groups with varying rows take where that makes fewer
+tiles. The same groups followed by empty ones up to 257 run on tiles of 256 rows: the same bits from every kernel that has both
+forms; the plain product also against a float64 product of integer operands."""
+
+import pytest
+import torch
+
+from fma import _lib
+from fma.modules.moe.cuda_implementation import (
+    gather_rows_cuda,
+    grouped_gemm_gathered_cuda,
+    grouped_gemm_ragged_cuda,
+    grouped_gemm_swiglu_bwd_cuda,
+    grouped_gemm_swiglu_cuda,
+)
+
+from gpu_util import DEV
+
+pytestmark = pytest.mark.gpu
+
+MOST = 256  # groups of a launch on tall tiles
+
+# rows per group around every edge of a tall tile: none or all rows past 256, of one wavefront or both, one to three tiles, the sizes
+# from which on 256-row tiles are as few, between groups of few rows and empty ones
+SIZES = [256, 257, 271, 272, 273, 287, 288, 289, 0, 512, 513, 544, 576, 577, 16, 64, 65, 800, 864, 865, 1152, 1, 300]
+# N, K: whole tiles, an odd number of K steps; partial column tiles (columns of some wavefronts only), a partial K step; one K step
+DIMS = [(512, 192), (264, 584), (40, 64)]
+
+
+def _u32(values):
+    return torch.tensor(values, dtype=torch.int64).to(torch.uint32).to(DEV)
+
+
+def _both(sizes):
+    return [_u32(sizes), _u32(list(sizes) + [0] * (MOST + 1 - len(sizes)))]
+
+
+def _inputs(sizes, N, K, dtype, b_shape):
+    g = torch.Generator(device=DEV).manual_seed(N + K)
+    x = torch.randint(-3, 4, (sum(sizes), K), device=DEV, generator=g).to(dtype)
+    w = torch.randint(-3, 4, (MOST + 1, *b_shape), device=DEV, generator=g).to(dtype)
+    bias = torch.randint(-8, 9, (MOST + 1, N), device=DEV, generator=g).to(dtype)
+    return x, w, bias
+
+
+def _fresh(*shape, dtype):
+    return torch.full(shape, 7.0, dtype=dtype, device=DEV)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("tB", [True, False])
+@pytest.mark.parametrize("N,K", DIMS)
+def test_plain(N, K, tB, dtype):
+    x, w, bias = _inputs(SIZES, N, K, dtype, (N, K) if tB else (K, N))
+    R = x.shape[0]
+    for b in (None, bias) if tB else (None,):
+        results = []
+        for M in _both(SIZES):
+            E = M.numel()
+            out = _fresh(R, N, dtype=dtype)
+            grouped_gemm_ragged_cuda(x, w[:E], out, M, False, 0, N, K, False, tB, None if b is None else b[:E])
+            results.append(out)
+        assert torch.equal(*results)
+        at = 0
+        for e, m in enumerate(SIZES):
+            expect = (x[at : at + m].double() @ (w[e].T if tB else w[e]).double()).to(dtype)
+            if b is not None:
+                expect = (expect.float() + b[e].float()).to(dtype)
+            assert torch.equal(results[0][at : at + m], expect), f"group {e} of {m} rows"
+            at += m
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("with_bias", [False, True])
+@pytest.mark.parametrize("N,K", [(512, 192), (272, 584), (48, 64)])
+def test_swiglu_and_gather(N, K, with_bias, dtype):
+    g = torch.Generator(device=DEV).manual_seed(N + K)
+    R, T, divisor = sum(SIZES), 700, 3
+    x = torch.randn(T, K, device=DEV, generator=g).to(dtype)
+    w = (torch.randn(MOST + 1, N, K, device=DEV, generator=g) * 0.1).to(dtype)
+    bias = torch.randn(MOST + 1, N, device=DEV, generator=g).to(dtype)
+    row_index = torch.randint(0, T * divisor, (R,), device=DEV, generator=g, dtype=torch.int32)
+    row_index[::11] = -3  # rows of zeros
+    xg = torch.zeros(R, K, device=DEV, dtype=dtype)
+    gather_rows_cuda(x, row_index.clamp(min=0), divisor, xg)
+    xg[::11] = 0
+    results = []
+    for M in _both(SIZES):
+        E = M.numel()
+        b = bias[:E].contiguous() if with_bias else None
+        h, act, act_only, plain = (_fresh(R, n, dtype=dtype) for n in (N, N // 2, N // 2, N))
+        gh, gact, gact_only = (_fresh(R, n, dtype=dtype) for n in (N, N // 2, N // 2))
+        grouped_gemm_swiglu_cuda(xg, w[:E], M, h, act, b)
+        grouped_gemm_swiglu_cuda(xg, w[:E], M, None, act_only, b)
+        grouped_gemm_gathered_cuda(x, row_index, divisor, w[:E], b, M, gh, gact)
+        grouped_gemm_gathered_cuda(x, row_index, divisor, w[:E], b, M, None, gact_only)
+        grouped_gemm_gathered_cuda(x, row_index, divisor, w[:E], b, M, plain, None)
+        assert torch.equal(act, act_only) and torch.equal(act, gact) and torch.equal(act, gact_only)
+        assert torch.equal(h, gh) and torch.equal(h, plain)
+        results.append((h, act))
+    assert torch.equal(results[0][0], results[1][0]) and torch.equal(results[0][1], results[1][1])
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("inter,K", [(512, 192), (136, 584), (40, 64)])
+def test_swiglu_backward(inter, K, dtype):
+    g = torch.Generator(device=DEV).manual_seed(inter + K)
+    R = sum(SIZES)
+    dy = torch.randn(R, K, device=DEV, generator=g).to(dtype)
+    w = (torch.randn(MOST + 1, K, inter, device=DEV, generator=g) * 0.1).to(dtype)
+    h = (torch.randn(R, 2 * inter, device=DEV, generator=g) * 2).to(dtype)
+    results = []
+    for M in _both(SIZES):
+        results.append(_fresh(R, 2 * inter, dtype=dtype))
+        grouped_gemm_swiglu_bwd_cuda(dy, w[: M.numel()], h, M, results[-1])
+    assert torch.equal(*results)
+
+
+@pytest.mark.parametrize("tB", [True, False])
+def test_split_reduction(tB):
+    sizes, N, K = [257, 288, 289, 0, 270, 16, 530], 264, 4104
+    x, w, _ = _inputs(sizes, N, K, torch.bfloat16, (N, K) if tB else (K, N))
+    lib, R = _lib.load(), sum(sizes)
+    results = []
+    for M in _both(sizes):
+        E = M.numel()
+        out = _fresh(R, N, dtype=x.dtype)
+        nbytes = lib.fma_grouped_gemm_ragged_workspace_bytes(R, E, N, K, int(tB))
+        workspace = torch.full((max(nbytes // 4, 1),), float("nan"), device=DEV)
+        rc = lib.fma_grouped_gemm_ragged_split(
+            x.data_ptr(), w.data_ptr(), out.data_ptr(), M.data_ptr(), None, E, _lib.FMA_VARY_M, 0, N, K, 0, int(tB), 1.0, R,
+            workspace.data_ptr() if nbytes else None, nbytes, _lib.FMA_BF16, torch.cuda.current_stream().cuda_stream,
+        )  # fmt: skip
+        _lib.check(rc, "fma_grouped_gemm_ragged_split")
+        results.append(out)
+    assert lib.fma_grouped_gemm_ragged_workspace_bytes(R, len(sizes), N, K, int(tB)) > 0  # the tall launch is split
+    assert torch.equal(*results)  # (integers below 2^24: exact in any order)
+
+
+@pytest.mark.parametrize("N,K", [(257, 72), (72, 67)])
+def test_element_wise_tiles(N, K):
+    """sizes whose rows are no multiple of 16 bytes take the element-wise path, a tall tile of it too"""
+    sizes = [257, 288, 289, 530, 3]
+    x, w, _ = _inputs(sizes, N, K, torch.bfloat16, (N, K))
+    out = _fresh(sum(sizes), N, dtype=x.dtype)
+    grouped_gemm_ragged_cuda(x, w[: len(sizes)], out, _u32(sizes), False, 0, N, K, False, True, None)
+    at = 0
+    for e, m in enumerate(sizes):
+        assert torch.equal(out[at : at + m], (x[at : at + m].double() @ w[e].T.double()).bfloat16()), f"group {e}"
+        at += m
+
+
+def test_many_tiles_per_workgroup():
+    """tall and other tiles after each other in every workgroup, 256 groups"""
+    sizes = [(250 + 7 * (e % 11)) if e % 5 else (e % 3) * 40 for e in range(MOST)]
+    N, K = 512, 136
+    x, w, _ = _inputs(sizes, N, K, torch.bfloat16, (N, K))
+    results = []
+    for M in _both(sizes):
+        results.append(_fresh(x.shape[0], N, dtype=x.dtype))
+        grouped_gemm_ragged_cuda(x, w[: M.numel()], results[-1], M, False, 0, N, K, False, True, None)
+    assert torch.equal(*results)
+    at = 0
+    for e, m in enumerate(sizes):
+        assert torch.equal(results[0][at : at + m], (x[at : at + m].double() @ w[e].T.double()).bfloat16()), f"group {e}"
+        at += m
