@@ -69,6 +69,10 @@ SIGNATURES = {
     "fma_router_topk": (_i32, [_p, _p, _i64, _i64, _i64, _i64, _p, _p, _p, _p, _p, _i32, _p]),
     "fma_moe_build_index_from_hist": (_i32, [_p, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p, _p]),
     "fma_router_topk_bwd": (_i32, [_p, _p, _p, _p, _i64, _i64, _i64, _p, _i32, _p]),
+    "fma_router_topk_f32": (_i32, [_p, _p, _i64, _i64, _i64, _i64, _p, _p, _p, _p, _p]),
+    "fma_router_topk_bwd_f32": (_i32, [_p, _p, _p, _p, _i64, _i64, _i64, _p, _p]),
+    "fma_swiglu_experts_f32": (_i32, [_p] * 10 + [_i64] * 5 + [_p] * 6),
+    "fma_swiglu_experts_bwd_f32": (_i32, [_p] * 14 + [_i64] * 5 + [_p] * 8),
     "fma_fused_residual_add_rmsnorm_fwd": (_i32, [_p, _p, _p, _p, _p, _p, _i64, _i64, _f32, _f32, _i32, _p]),
     "fma_fused_residual_add_rmsnorm_bwd_workspace_bytes": (_i64, [_i64, _i64]),
     "fma_fused_residual_add_rmsnorm_bwd": (

@@ -536,6 +536,121 @@ def router_topk_backward_cuda(
     _lib.check(rc, "router_topk_backward_cuda")
 
 
+@hip_op("router_topk_f32_cuda", mutates_args={"logits", "weights", "selected", "token_block_hist"})
+def router_topk_f32_cuda(
+    x: torch.Tensor, gate_weight: torch.Tensor, top_k: int, logits: torch.Tensor, weights: torch.Tensor,
+    selected: torch.Tensor, token_block_hist: torch.Tensor,
+) -> None:  # fmt: skip
+    _lib.require_gpu(x, gate_weight, logits, weights, selected, token_block_hist)
+    T, H = x.shape
+    E = gate_weight.size(0)
+    assert gate_weight.shape == (E, H) and logits.shape == (T, E)
+    assert weights.shape == (T, top_k) and selected.shape == (T, top_k)
+    assert x.dtype == gate_weight.dtype == logits.dtype == weights.dtype == torch.float32 and selected.dtype == torch.int32
+    assert token_block_hist.dtype == torch.uint32 and token_block_hist.shape == ((T + 15) // 16, E)
+    for t in (x, gate_weight, logits, weights, selected, token_block_hist):
+        assert t.is_contiguous()
+    with _lib.on_device(x.device):
+        rc = _lib.load().fma_router_topk_f32(
+            x.data_ptr(), gate_weight.data_ptr(), T, H, E, top_k, logits.data_ptr(), weights.data_ptr(),
+            selected.data_ptr(), token_block_hist.data_ptr(), _lib.current_stream(x.device),
+        )
+    _lib.check(rc, "router_topk_f32_cuda")
+
+
+@hip_op("router_topk_backward_f32_cuda", mutates_args={"logits_grad"})
+def router_topk_backward_f32_cuda(
+    logits: torch.Tensor, selected: torch.Tensor, weights_grad: torch.Tensor | None,
+    logits_output_grad: torch.Tensor | None, logits_grad: torch.Tensor,
+) -> None:  # fmt: skip
+    _lib.require_gpu(logits, selected, weights_grad, logits_output_grad, logits_grad)
+    T, E = logits.shape
+    top_k = selected.size(1)
+    assert selected.shape == (T, top_k) and selected.dtype == torch.int32 and logits_grad.shape == (T, E)
+    assert logits_grad.dtype == logits.dtype == torch.float32
+    assert weights_grad is None or (weights_grad.shape == (T, top_k) and weights_grad.dtype == logits.dtype)
+    assert logits_output_grad is None or (logits_output_grad.shape == (T, E) and logits_output_grad.dtype == logits.dtype)
+    for t in (logits, selected, weights_grad, logits_output_grad, logits_grad):
+        assert t is None or t.is_contiguous()
+    with _lib.on_device(logits.device):
+        rc = _lib.load().fma_router_topk_bwd_f32(
+            logits.data_ptr(), selected.data_ptr(), _lib.ptr(weights_grad), _lib.ptr(logits_output_grad), T, E, top_k,
+            logits_grad.data_ptr(), _lib.current_stream(logits.device),
+        )
+    _lib.check(rc, "router_topk_backward_f32_cuda")
+
+
+def _check_experts_f32(x, gates, weight1, weight2, inv, sizes) -> tuple[int, int, int, int, int]:
+    T, H = x.shape
+    E, N1, _ = weight1.shape
+    k, inter = gates.size(1), N1 // 2
+    assert N1 % 2 == 0 and weight1.shape == (E, N1, H) and weight2.shape == (E, H, inter) and gates.shape == (T, k)
+    assert x.dtype == gates.dtype == weight1.dtype == weight2.dtype == torch.float32
+    assert inv.dtype == torch.int32 and inv.numel() == T * k
+    for t in sizes:
+        assert t.dtype == torch.uint32 and t.numel() == E and t.is_contiguous()
+    return T, k, E, H, inter
+
+
+@hip_op("swiglu_experts_f32_cuda", mutates_args={"xg", "h", "act", "o", "y"})
+def swiglu_experts_f32_cuda(
+    x: torch.Tensor, gates: torch.Tensor, weight1: torch.Tensor, weight2: torch.Tensor, inv: torch.Tensor,
+    M_array: torch.Tensor, N1_array: torch.Tensor, K1_array: torch.Tensor, N2_array: torch.Tensor, K2_array: torch.Tensor,
+    xg: torch.Tensor, h: torch.Tensor, act: torch.Tensor, o: torch.Tensor, y: torch.Tensor,
+) -> None:  # fmt: skip
+    """The experts of an fp32 SwiGLU layer on its routed tokens (fma_swiglu_experts_f32): y = the gated sum of o, the
+    projections' grouped rows xg, h, act and o on the way."""
+    _lib.require_gpu(x, gates, weight1, weight2, inv, M_array, N1_array, K1_array, N2_array, K2_array, xg, h, act, o, y)
+    sizes = (M_array, N1_array, K1_array, N2_array, K2_array)
+    T, k, E, H, inter = _check_experts_f32(x, gates, weight1, weight2, inv, sizes)
+    R = T * k
+    assert xg.shape == o.shape == (R, H) and h.shape == (R, 2 * inter) and act.shape == (R, inter) and y.shape == (T, H)
+    for t in (x, gates, weight1, weight2, inv, xg, h, act, o, y):
+        assert t.is_contiguous()
+    assert xg.dtype == h.dtype == act.dtype == o.dtype == y.dtype == torch.float32
+    with _lib.on_device(x.device):
+        rc = _lib.load().fma_swiglu_experts_f32(
+            x.data_ptr(), inv.data_ptr(), gates.data_ptr(), weight1.data_ptr(), weight2.data_ptr(),
+            *[t.data_ptr() for t in sizes], T, k, E, H, inter,
+            *[t.data_ptr() for t in (xg, h, act, o, y)], _lib.current_stream(x.device),
+        )  # fmt: skip
+    _lib.check(rc, "swiglu_experts_f32_cuda")
+
+
+@hip_op(
+    "swiglu_experts_backward_f32_cuda",
+    mutates_args={"o_grad", "act_grad", "h_grad", "x_grad", "gates_grad", "weight1_grad", "weight2_grad"},
+)
+def swiglu_experts_backward_f32_cuda(
+    y_grad: torch.Tensor, gates: torch.Tensor, weight1: torch.Tensor, weight2: torch.Tensor, inv: torch.Tensor,
+    M_array: torch.Tensor, N1_array: torch.Tensor, K1_array: torch.Tensor, N2_array: torch.Tensor, K2_array: torch.Tensor,
+    xg: torch.Tensor, h: torch.Tensor, act: torch.Tensor, o: torch.Tensor,
+    o_grad: torch.Tensor, act_grad: torch.Tensor, h_grad: torch.Tensor, x_grad: torch.Tensor | None,
+    gates_grad: torch.Tensor | None, weight1_grad: torch.Tensor | None, weight2_grad: torch.Tensor | None,
+) -> None:  # fmt: skip
+    """Backward of swiglu_experts_f32_cuda (fma_swiglu_experts_bwd_f32); o_grad, act_grad and h_grad are scratch memory."""
+    buffers = (o_grad, act_grad, h_grad, x_grad, gates_grad, weight1_grad, weight2_grad)
+    _lib.require_gpu(y_grad, gates, weight1, weight2, inv, M_array, N1_array, K1_array, N2_array, K2_array, xg, h, act, o, *buffers)
+    sizes = (M_array, N1_array, K1_array, N2_array, K2_array)
+    T, k, E, H, inter = _check_experts_f32(y_grad, gates, weight1, weight2, inv, sizes)
+    R = T * k
+    assert xg.shape == o.shape == o_grad.shape == (R, H)
+    assert h.shape == h_grad.shape == (R, 2 * inter) and act.shape == act_grad.shape == (R, inter)
+    for t, like in ((x_grad, y_grad), (gates_grad, gates), (weight1_grad, weight1), (weight2_grad, weight2)):
+        assert t is None or t.shape == like.shape
+    for t in (y_grad, gates, weight1, weight2, inv, xg, h, act, o):
+        assert t.is_contiguous()
+    for t in buffers:
+        assert t is None or (t.is_contiguous() and t.dtype == torch.float32)
+    with _lib.on_device(y_grad.device):
+        rc = _lib.load().fma_swiglu_experts_bwd_f32(
+            y_grad.data_ptr(), inv.data_ptr(), gates.data_ptr(), weight1.data_ptr(), weight2.data_ptr(),
+            *[t.data_ptr() for t in (xg, h, act, o)], *[t.data_ptr() for t in sizes], T, k, E, H, inter,
+            *[_lib.ptr(t) for t in buffers], _lib.current_stream(y_grad.device),
+        )  # fmt: skip
+    _lib.check(rc, "swiglu_experts_backward_f32_cuda")
+
+
 # ---- index construction -----------------------------------------------------------------------------
 
 
@@ -616,6 +731,93 @@ def fused_router_with_histogram(x: torch.Tensor, gate_weight: torch.Tensor, top_
     """fused_router plus the uint32 [ceil(T / 16), E] histogram of the choices per block of 16 tokens, which
     build_routing_index takes (and overwrites)"""
     return _FusedRouter.apply(x, gate_weight, top_k)
+
+
+class _Fp32Router(torch.autograd.Function):
+    """_FusedRouter for fp32 activations. A backward pass that is itself recorded (create_graph) forms the logits' gradient from
+    differentiable operations, as the library calls that this node stands for do."""
+
+    @staticmethod
+    @ensure_contiguous
+    def forward(ctx, x: torch.Tensor, gate_weight: torch.Tensor, top_k: int):
+        T, E = x.size(0), gate_weight.size(0)
+        logits, weights = x.new_empty(T, E), x.new_empty(T, top_k)
+        selected = torch.empty(T, top_k, device=x.device, dtype=torch.int32)
+        token_block_hist = torch.empty((T + 15) // 16, E, device=x.device, dtype=torch.uint32)
+        router_topk_f32_cuda(x, gate_weight, top_k, logits, weights, selected, token_block_hist)
+        ctx.save_for_backward(x, gate_weight, logits, selected)
+        ctx.mark_non_differentiable(selected, token_block_hist)
+        ctx.set_materialize_grads(False)
+        return logits, weights, selected, token_block_hist
+
+    @staticmethod
+    @ensure_contiguous
+    def backward(ctx, logits_output_grad, weights_grad, _, __):
+        x, gate_weight, logits, selected = ctx.saved_tensors
+        if logits_output_grad is None and weights_grad is None:
+            return None, None, None
+        if torch.is_grad_enabled():
+            logits_grad = torch.zeros_like(logits) if logits_output_grad is None else logits_output_grad
+            if weights_grad is not None:
+                columns = selected.long()
+                s = torch.softmax((x @ gate_weight.t()).gather(1, columns), dim=-1)
+                logits_grad = logits_grad.scatter_add(1, columns, s * (weights_grad - (s * weights_grad).sum(-1, keepdim=True)))
+        else:
+            logits_grad = torch.empty_like(logits)
+            router_topk_backward_f32_cuda(logits, selected, weights_grad, logits_output_grad, logits_grad)
+        x_grad = logits_grad @ gate_weight if ctx.needs_input_grad[0] else None
+        gate_weight_grad = logits_grad.t() @ x if ctx.needs_input_grad[1] else None
+        return x_grad, gate_weight_grad, None
+
+
+class _Fp32SwigluExperts(torch.autograd.Function):
+    """The experts of an fp32 SwiGLU layer without biases, from the tokens to the gated sum, as one node: the values of
+    gather_rows, grouped_gemm_experts, swiglu_packed, grouped_gemm_experts and combine, which it runs in one call."""
+
+    @staticmethod
+    @ensure_contiguous
+    def forward(
+        ctx, x: torch.Tensor, gates: torch.Tensor, weight1: torch.Tensor, weight2: torch.Tensor, inv: torch.Tensor,
+        M_array: torch.Tensor, N1_array: torch.Tensor, K1_array: torch.Tensor, N2_array: torch.Tensor,
+        K2_array: torch.Tensor, grad_enabled: bool,
+    ) -> torch.Tensor:  # fmt: skip
+        T, H = x.shape
+        R, inter = T * gates.size(1), weight2.size(2)
+        xg, h, act, o = x.new_empty(R, H), x.new_empty(R, 2 * inter), x.new_empty(R, inter), x.new_empty(R, H)
+        y = torch.empty_like(x)
+        sizes = (M_array, N1_array, K1_array, N2_array, K2_array)
+        swiglu_experts_f32_cuda(x, gates, weight1, weight2, inv, *sizes, xg, h, act, o, y)
+        if grad_enabled and any(ctx.needs_input_grad[:4]):
+            ctx.save_for_backward(gates, weight1, weight2, inv, *sizes, xg, h, act, o)
+        return y
+
+    @staticmethod
+    @ensure_contiguous
+    def backward(ctx, y_grad: torch.Tensor) -> tuple[torch.Tensor | None]:
+        gates, weight1, weight2, inv, *sizes, xg, h, act, o = ctx.saved_tensors
+        needs_x, needs_gates, needs_weight1, needs_weight2 = ctx.needs_input_grad[:4]
+        x_grad = torch.empty_like(y_grad) if needs_x else None
+        gates_grad = torch.empty_like(gates) if needs_gates else None
+        weight1_grad = torch.empty_like(weight1) if needs_weight1 else None
+        weight2_grad = torch.empty_like(weight2) if needs_weight2 else None
+        swiglu_experts_backward_f32_cuda(
+            y_grad, gates, weight1, weight2, inv, *sizes, xg, h, act, o, torch.empty_like(o), torch.empty_like(act),
+            torch.empty_like(h), x_grad, gates_grad, weight1_grad, weight2_grad,
+        )  # fmt: skip
+        return x_grad, gates_grad, weight1_grad, weight2_grad, None, None, None, None, None, None, None
+
+
+def fp32_swiglu_layer(
+    x: torch.Tensor, gate_weight: torch.Tensor, weight1: torch.Tensor, weight2: torch.Tensor, N1_array: torch.Tensor,
+    K1_array: torch.Tensor, N2_array: torch.Tensor, K2_array: torch.Tensor, top_k: int,
+) -> tuple[torch.Tensor, torch.Tensor]:  # fmt: skip
+    """(output, router_logits) of a SwiGLU layer without biases in fp32: router, routing index and experts in one operator each"""
+    logits, gates, selected, token_block_hist = _Fp32Router.apply(x, gate_weight, top_k)
+    M_array, _, _, _, inv = build_routing_index(selected, gate_weight.size(0), token_block_hist)
+    y = _Fp32SwigluExperts.apply(
+        x, gates, weight1, weight2, inv, M_array, N1_array, K1_array, N2_array, K2_array, torch.is_grad_enabled()
+    )
+    return y, logits
 
 
 class _GatherRows(torch.autograd.Function):

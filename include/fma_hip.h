@@ -370,6 +370,29 @@ int fma_router_topk_bwd(const void* logits, const int32_t* selected, const void*
                         const void* d_logits, int64_t T, int64_t E, int64_t top_k, void* d_out, int dtype,
                         void* stream);
 
+/* fma_router_topk and fma_router_topk_bwd for fp32 activations: the same results (no rounding; without counts), H % 4 == 0. */
+int fma_router_topk_f32(const void* x, const void* gate_weight, int64_t T, int64_t H, int64_t E, int64_t top_k, void* logits,
+                        void* weights, int32_t* selected, uint32_t* token_block_hist, void* stream);
+int fma_router_topk_bwd_f32(const void* logits, const int32_t* selected, const void* d_weights, const void* d_logits, int64_t T,
+                            int64_t E, int64_t top_k, void* d_out, void* stream);
+
+/* The expert path of an fp32 SwiGLU layer without biases, enqueued by one call: fma_dispatch_rows (xg [R, H], R = T * k),
+ * fma_grouped_gemm (h [R, 2 I] = xg W1^T), fma_swiglu_forward (act [R, I]; "up" first in h), fma_grouped_gemm (o [R, H] = act W2^T),
+ * fma_combine (y [T, H]). W1 [E, 2 I, H], W2 [E, H, I]; counts: rows per expert, N1 / K1 and N2 / K2: out and in features of the two
+ * projections per expert, all uint32 [E] in device memory. T >= 1.
+ * Replaces MoE._compute_experts (fma/modules/moe/__init__.py:206-290) for such layers. */
+int fma_swiglu_experts_f32(const void* x, const int32_t* inv, const void* gates, const void* W1, const void* W2, const uint32_t* counts,
+                           const uint32_t* N1, const uint32_t* K1, const uint32_t* N2, const uint32_t* K2, int64_t T, int64_t k,
+                           int64_t E, int64_t H, int64_t I, void* xg, void* h, void* act, void* o, void* y, void* stream);
+/* Its backward from dy [T, H] and the buffers of the forward call: fma_combine_bwd, the two input and two weight gradients
+ * (fma_grouped_gemm), fma_swiglu_backward, fma_combine. d_gates [T, k], dW1, dW2 and dx [T, H] may be NULL (not computed);
+ * d_o [R, H], d_act [R, I] and d_h [R, 2 I] are scratch memory. */
+int fma_swiglu_experts_bwd_f32(const void* dy, const int32_t* inv, const void* gates, const void* W1, const void* W2, const void* xg,
+                               const void* h, const void* act, const void* o, const uint32_t* counts, const uint32_t* N1,
+                               const uint32_t* K1, const uint32_t* N2, const uint32_t* K2, int64_t T, int64_t k, int64_t E, int64_t H,
+                               int64_t I, void* d_o, void* d_act, void* d_h, void* dx, void* d_gates, void* dW1, void* dW2,
+                               void* stream);
+
 /* ---- residual add + RMSNorm ------------------------------------------------------------------- */
 
 /* For each of the B rows of H elements, in fp32:
