@@ -4,7 +4,7 @@
 //
 // What bounds it: the weights, read once each, against a handful of rows; the product is a stream of E_active * N * K elements.
 // The tile kernel spends that stream in 256-column tiles (one workgroup per compute unit, two or three K steps in flight, and for
-// one token of the fine-grained shape 88 tiles for 256 compute units). Here the unit of work is ONE wavefront with kRows weight
+// one token of the fine-grained shape 88 tiles for 256 compute units). Here the unit of work is ONE wavefront with 16, 32 or 64 weight
 // rows over the whole reduction:
 //  * no workgroup barrier anywhere: a wavefront fills a private ring of LDS stages by direct global -> LDS loads, each
 //    instruction 8 rows x 128 bytes (whole cache lines), waits with a counted vmcnt and multiplies; 6 such wavefronts (3 of the
@@ -66,6 +66,11 @@ __device__ __forceinline__ uint32_t lds_off(uint32_t row, uint32_t chunk) { retu
 
 template <int ROWS>
 struct Config;
+template <>
+struct Config<16> {  // launches of few units (half_units)
+    static constexpr uint32_t kLds = 24576;
+    static constexpr uint32_t kMaxTokens = 32;
+};
 template <>
 struct Config<32> {  // up to about 16 rows per expert
     static constexpr uint32_t kLds = 24576;
@@ -169,12 +174,19 @@ __device__ __forceinline__ void unit(const Args& a, uint8_t* lds, uint32_t e, ui
     wait_vm<0>();  // the loads past the end write zeros into the ring: they are done before it is used again
 
     // a lane holds row r16, columns 4 q .. 4 q + 3 of each block; rounding points as in the tile kernel's epilogue
+    // (one block with both halves: 8 "up" columns in lanes 0 .. 31, their "gate" in lanes 32 .. 63)
+    constexpr bool kOneBlock = GLU && WB == 1;
 #pragma unroll
     for (int j = 0; j < TB; ++j) {
-        const uint32_t row = (uint32_t)j * 16u + r16;
-        if (row >= rows) continue;
+        float gate[4];
+        if constexpr (kOneBlock) {
 #pragma unroll
-        for (int b = 0; b < (GLU ? WB / 2 : WB); ++b) {
+            for (int x = 0; x < 4; ++x) gate[x] = __shfl_xor(acc[0][j][x], 32, 64);
+        }
+        const uint32_t row = (uint32_t)j * 16u + r16;
+        if (row >= rows || (kOneBlock && q >= 2u)) continue;
+#pragma unroll
+        for (int b = 0; b < (GLU && WB > 1 ? WB / 2 : WB); ++b) {
             const uint32_t c = n0 + (uint32_t)b * 16u + 4u * q;
             if (c >= I) continue;
             float y[4];
@@ -183,7 +195,7 @@ __device__ __forceinline__ void unit(const Args& a, uint8_t* lds, uint32_t e, ui
                 float u = acc[b][j][x];
                 if constexpr (BIAS) u = EL::round(u) + EL::from_bits(a.bias[We + c + x]);
                 if constexpr (GLU) {
-                    float g = acc[WB / 2 + b][j][x];
+                    float g = kOneBlock ? gate[x] : acc[kOneBlock ? 0 : WB / 2 + b][j][x];
                     if constexpr (BIAS) g = EL::round(g) + EL::from_bits(a.bias[We + I + c + x]);
                     u = EL::round(u);
                     g = EL::round(g);
@@ -296,9 +308,24 @@ int launch(Args a, bool glu, int64_t R, int64_t groups, hipStream_t st) {
     else a.bias ? run(thin_gemm_kernel<EL, ROWS, false, true, PASSES>) : run(thin_gemm_kernel<EL, ROWS, false, false, PASSES>);
     return launch_status("grouped_gemm_thin");
 }
+// Units of 16 weight rows where a launch has at most two units of 32 per compute unit, a third of what fits its LDS, and a reduction
+// long enough to stream: twice as many wavefronts, with rings of five stages in flight instead of three. Whole layer of one token,
+// units of 32 -> 16 where the line says so, us: hidden 2048, I 8192, E 8, k 2 (second projection: 128 units) 75.5 -> 66.8, 2 / 4 / 8
+// tokens 93.4 -> 83.8, 116.7 -> 109.7, 141.5 -> 137.2; hidden 2880, I 2880, E 32, k 4 53.3 -> 50.8; hidden 2048, I 768, E 128, k 8 34.6
+// -> 33.5. With up to three units per compute unit and any reduction: hidden 2048, I 1408, E 64 (K 1408) 42.3 -> 43.2, hidden 2880 with
+// two tokens 82.1 -> 84.5.
+bool half_units(const Args& a, bool glu, int64_t groups) {
+    const int64_t cus = num_compute_units() > 0 ? num_compute_units() : 256;
+    const int64_t cols = glu ? a.N / 2 : a.N, per = glu ? 16 : 32;
+    return a.K >= 2048 && groups * ((cols + per - 1) / per) <= 2 * cus;
+}
 // max_rows: as in fma_thin_swiglu_experts, or 0 (not known)
 template <typename EL, int ROWS>
 int launch(const Args& a, bool glu, int64_t R, int64_t groups, int64_t max_rows, hipStream_t st) {
+    if constexpr (ROWS == 32) {
+        if (!a.taken && max_rows >= 1 && max_rows <= Config<16>::kMaxTokens && half_units(a, glu, groups))
+            return launch<EL, 16, ONE_PASS>(a, glu, R, groups, st);
+    }
     if (a.taken) return launch<EL, ROWS, MAY_YIELD>(a, glu, R, groups, st);
     if (max_rows >= 1 && max_rows <= Config<ROWS>::kMaxTokens) return launch<EL, ROWS, ONE_PASS>(a, glu, R, groups, st);
     return launch<EL, ROWS, MANY_PASSES>(a, glu, R, groups, st);

@@ -287,3 +287,27 @@ def test_layer_without_backward_where_the_training_forward_splits_its_reduction(
         y, logits = moe(x, kernel_backend=KernelBackend.cuda)
     assert torch.equal(logits, expect_logits)
     assert float((y.double() - expect.double()).norm() / expect.double().norm()) <= 2.0**-7
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("bias", [False, True])
+@pytest.mark.parametrize(
+    "T,k,E,H,inter",
+    # units of 16 weight rows (reductions from 2048 on): one to 32 rows per expert (both token blocks), partial last units of 8 columns,
+    # partial last steps; in the first projection, in the second, in both
+    [(1, 1, 4, 2056, 24), (3, 2, 8, 2048, 104), (16, 2, 2, 40, 2056), (17, 2, 2, 2120, 2072), (32, 3, 3, 72, 2048)],
+)
+def test_units_of_sixteen_weight_rows(T, k, E, H, inter, bias, dtype):
+    from fma import KernelBackend, MoE, swiglu_packed
+
+    torch.manual_seed(T + inter)
+    moe = MoE(E, k, H, inter, swiglu_packed, True, bias, 0.1).to(dtype).to(DEV)
+    if bias:
+        with torch.no_grad():
+            moe.c_fc.bias.normal_(0, 0.5)
+            moe.c_proj.bias.normal_(0, 0.5)
+    x = torch.randn(T, H, device=DEV).to(dtype)
+    expect = moe(x.clone().requires_grad_(), kernel_backend=KernelBackend.cuda)
+    with torch.no_grad():
+        got = moe(x, kernel_backend=KernelBackend.cuda)
+    assert torch.equal(got[0], expect[0]) and torch.equal(got[1], expect[1])
