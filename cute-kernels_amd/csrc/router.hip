@@ -9,7 +9,7 @@
 // (four 16-byte loads) per step and feeds the four MFMAs of the step from them. A row is then read in 256-byte pieces
 // per wavefront, 1 KB per workgroup. The router weight matrix (E*H elements, at most a few MB) is re-read by every
 // workgroup from the L2.
-#include "router_parts.h"
+#include "router_logits.h"
 
 namespace fmahip {
 namespace {
@@ -356,8 +356,49 @@ __global__ __launch_bounds__(W * kWave) void router_topk_wide_kernel(const Route
     flush_histogram(a, s_hist, W, tok0, tid, kThreadsW);
 }
 
+// Weights, choice and histogram of 16 tokens from logits in memory, keys in registers (NK per lane: ceil(E / 16) or more).
+template <typename EL, int NK>
+__global__ __launch_bounds__(kRouterThreads) void topk_from_logits_kernel(const RouterArgs a) {
+    __shared__ uint32_t s_hist[16 * NK];
+    const int tid = threadIdx.x, c = tid & 15, E = a.E;
+    const int64_t tok0 = (int64_t)blockIdx.x * kTok, token = tok0 + (tid >> 4);
+    clear_histogram(a, s_hist, 1, tid, kRouterThreads);
+    const int64_t from = token < a.T ? token : a.T - 1;  // (real keys; nothing is stored for it)
+    uint32_t keys[NK];
+#pragma unroll
+    for (int i = 0; i < NK; ++i) {
+        const int n = c + 16 * i;
+        keys[i] = n < E ? make_key<EL>(a.logits[from * E + n], n) : 0u;
+    }
+    __syncthreads();
+    topk_softmax_in_registers<EL, NK>(keys, c, token, a, tok0, s_hist);
+    flush_histogram(a, s_hist, 1, tok0, tid, kRouterThreads);
+}
+
+// Few tokens: logits by workgroups of 16 tokens x 16 experts, then their top-k. The kernels below read the router matrix through one
+// compute unit per 32 or 64 tokens, which takes the same time for 130 tokens as for 8192. One launch / these two, us, at 130, 512, 1024
+// and 2048 tokens: E 64, hidden 2048 15.7 / 9.1, 15.9 / 8.7, 15.9 / 9.2, 16.2 / 13.8; E 128, hidden 4096 36.4 / 12.9, 36.8 / 12.7, 37.3 /
+// 19.7, 37.5 / 35.4 (not taken); E 256, hidden 4096 67.3 / 15.3, 67.7 / 21.5, 68.4 / 35.4 (not taken), 68.5 / 65; E 32, hidden 2880 13.4
+// / 9.4, 13.7 / 9.4, 13.8 / 9.4, 15.3 / 10.0, at 4096 15.8 / 17.0 (not taken).
+// The line: at most two rounds of such workgroups (one fits a compute unit), one where the matrix is small (up to 32 experts).
+bool few_tokens(const RouterArgs& a) {
+    const int64_t cus = num_compute_units() > 0 ? num_compute_units() : 256;
+    const int64_t groups = ((a.T + kTok - 1) / kTok) * ((a.E + 15) / 16);
+    return groups <= (a.E > 32 ? 2 : 1) * cus && a.H < (1 << 21);
+}
+template <typename EL, int NK>
+int launch_router_few(const RouterArgs& a, hipStream_t st) {
+    const uint32_t blocks = (uint32_t)((a.T + kTok - 1) / kTok);
+    hipLaunchKernelGGL((router_logits_kernel<EL, false>), dim3(blocks, (uint32_t)((a.E + 15) / 16)), dim3(256), 0, st, a);
+    const int rc = launch_status("router_topk (logits)");
+    if (rc) return rc;
+    hipLaunchKernelGGL((topk_from_logits_kernel<EL, NK>), dim3(blocks), dim3(kRouterThreads), 0, st, a);
+    return launch_status("router_topk (top-k)");
+}
+
 template <typename EL, int NBLK, int EMAX>
 int launch_router_wide(const RouterArgs& a, hipStream_t st) {
+    if (few_tokens(a)) return launch_router_few<EL, EMAX / 16>(a, st);
     // 64 tokens per workgroup share each weight tile four ways; with too few tokens to give every compute unit such a
     // workgroup, 32 tokens per workgroup keep twice as many units busy
     const int64_t cus = num_compute_units() > 0 ? num_compute_units() : 256;

@@ -176,7 +176,8 @@ __device__ __forceinline__ void topk_softmax_tokens(uint32_t* const (&keys)[NR],
 // The same for one token whose keys are in registers: lane c holds the keys of the columns congruent to c mod 16 (0 where there
 // is none), NK = ceil(E / 16) of them.
 template <typename EL, int NK>
-__device__ __forceinline__ void topk_softmax_in_registers(uint32_t (&keys)[NK], int c, int64_t token, const RouterArgs& a) {
+__device__ __forceinline__ void topk_softmax_in_registers(uint32_t (&keys)[NK], int c, int64_t token, const RouterArgs& a,
+                                                          int64_t tok0 = 0, uint32_t* s_hist = nullptr) {
     uint32_t mine[1][kMaxTopK / 16] = {};
     uint32_t first[1] = {0};
     for (int j = 0; j < a.k; ++j) {
@@ -192,7 +193,7 @@ __device__ __forceinline__ void topk_softmax_in_registers(uint32_t (&keys)[NK], 
             if (c == (j & 15) && (j >> 4) == i) mine[0][i] = best;
     }
     const int64_t tokens[1] = {token};
-    softmax_tokens<EL, 1>(mine, first, c, tokens, 0, a, nullptr);
+    softmax_tokens<EL, 1>(mine, first, c, tokens, tok0, a, s_hist);
 }
 
 }  // namespace

@@ -257,3 +257,27 @@ def test_router_rejects_bad_arguments():
     with pytest.raises(RuntimeError, match="dtype"):
         call(x.float(), w.float(), 2)
     call(x[:0], w, 2)  # no tokens: nothing to do
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,E,k", [(520, 17, 3), (2048, 64, 8), (136, 65, 1), (1032, 130, 64), (4096, 256, 8)])
+@pytest.mark.parametrize("rows", [1, 15, 130, 400])
+def test_few_tokens_give_the_bits_of_many(rows, H, E, k, dtype):
+    """a call with few tokens runs as two launches (product, top-k), one with many as one: the same logits, weights, choices, counts"""
+    g = torch.Generator(device=DEV).manual_seed(rows + E)
+    x = torch.randn(16384, H, device=DEV, generator=g).to(dtype)
+    w = (torch.randn(E, H, device=DEV, generator=g) * 0.1).to(dtype)
+    results = []
+    for T in (16384, rows):
+        logits, weights = (torch.empty(T, n, device=DEV, dtype=dtype) for n in (E, k))
+        selected = torch.empty(T, k, device=DEV, dtype=torch.int32)
+        counts = torch.empty(E, device=DEV, dtype=torch.uint32)
+        hist = torch.empty((T + 15) // 16, E, device=DEV, dtype=torch.uint32)
+        router_topk_cuda(x[:T], w, k, logits, weights, selected, counts, hist)
+        results.append((logits[:rows], weights[:rows], selected[:rows]))
+    for many, few in zip(*results):
+        assert torch.equal(many, few)
+    expect = torch.zeros((rows + 15) // 16, E, dtype=torch.int64, device=DEV)
+    block = (torch.arange(rows, device=DEV) // 16)[:, None].expand(rows, k)
+    expect.index_put_((block, selected.long()), torch.ones_like(block), accumulate=True)
+    assert torch.equal(hist.to(torch.int64), expect) and torch.equal(counts.to(torch.int64), expect.sum(0))
