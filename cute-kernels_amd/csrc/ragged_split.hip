@@ -23,16 +23,17 @@ namespace ragged {
 // stay in the last-level cache), and a split has to promise a tenth less than none. Groups of few rows run the three-stage
 // loop, whose steps are shorter, without a split on half-width tiles in the NT layout: NT 4096 x 14336 on 8 groups of 32 rows
 // streams its weights in 176 us as it is and would take 184 us in two parts.
-// Tall tiles (TALL in ragged_kernel.h): a round takes 1.6 to 1.9 us per K step of its tiles, most when every compute unit streams
-// weights of its own, and a partial last round, in parts of its columns, 0.65 to 0.75 of that behind whole rounds and 0.8 to 0.95 alone. The
+// Tall tiles (TALL in ragged_kernel.h): a round takes 1.6 to 2.0 us per K step of its tiles, most when every compute unit is busy and
+// streams weights of its own, and a partial last round, in parts of its columns, 0.65 to 0.75 of that behind whole rounds and 0.8 to 0.95 alone. The
 // tiles of a group follow from the spread of a random routing (a standard deviation of the root of the mean): 8 groups of 256 or
-// 512 rows are 8 or 16 tiles high, not 12 or 20. That ends the split of [8 x 500 rows, 4096 x 14336] (420 us as 256 tiles, 468 us
+// 512 rows are 8 or 16 tiles high, not 12 or 20 (and three parts of 64 tiles of 128 steps, 121 us, are better than four, 123 us and 165
+// us in the sixth of the launches in which an expert is past 288 rows). That ends the split of [8 x 500 rows, 4096 x 14336] (420 us as 256 tiles, 468 us
 // in two parts, 556 us in three parts of 256-row tiles) and of [8 x 2000 rows, 2048 x 8192] (451 us, 563 us).
 // Uneven loads make fewer tiles, which a split helps the more; where they happen to fill the compute units exactly once as they are, the
 // sums are the price. Training steps without -> with splits on 256-row tiles: 2048 tokens, hidden 4096, I 14336, E 8, k 2, evenly
 // 5100 -> 4630 us, all on two experts 3870 -> 3990 us; 4000 tokens, hidden 2048, I 8192: 2775 -> 2627 and 2157 -> 2225 us; 512 and 1021
 // tokens gain either way (2219 -> 1779 and 2727 -> 2478 us, 886 -> 565 us at 256 tokens of the second shape).
-constexpr double kStepUs = 1.45, kTallStepUs = 1.75, kThinStepUs[2] = {1.1, 0.75}, kTileSteps = 6.0, kThinRows = 48.0;
+constexpr double kStepUs = 1.45, kTallStepUs = 1.55, kFullStepUs = 0.4, kThinStepUs[2] = {1.1, 0.75}, kTileSteps = 6.0, kThinRows = 48.0;
 constexpr double kTailCost = 0.7, kLoneTailCost = 0.85, kWeightBytesPerUs = 5.5e6;
 constexpr double kReduceUs = 4.0, kReduceBytesPerUs = 4.5e6, kSplitGain = 0.9;
 constexpr uint32_t kSplitMinSteps = 24;
@@ -48,24 +49,34 @@ SplitPlan plan_split(int64_t R, int64_t E, int64_t N, int64_t K, bool b_kc, bool
     const bool thin = mean <= kThinRows;
     double row_tiles = active * (mean < BM / 2 ? 1.0 : mean / BM + 0.5);
     if (tall) {
-        // about a boundary b of kTallM rows, the share of the groups past it is that of a normal distribution; as a whole number of
-        // tiles, so that one group in a hundred past a boundary does not count for a round
+        // about a boundary b of kTallM rows, the share of the groups past it is that of a normal distribution
         const double b = std::max(1.0, std::floor(mean / kTallM + 0.5));
         const double past = 0.5 * std::erfc((b * kTallM - mean) / std::sqrt(2.0 * mean));
-        row_tiles = std::floor(active * (b + past) + 0.5);
+        row_tiles = active * (b + past);
     }
-    const double tiles = row_tiles * (double)((N + BN - 1) / BN);
-    const bool narrow = thin && b_kc && 2.0 * tiles <= cus;
-    const double step_us = thin ? kThinStepUs[b_kc] : (tall ? kTallStepUs : kStepUs);
+    const double columns = (double)((N + BN - 1) / BN);
     const double weights_us = active * N * K * 2.0 / kWeightBytesPerUs;
-    auto us = [&](uint32_t parts, uint32_t steps) {
+    auto us_of = [&](double tiles, uint32_t parts, uint32_t steps) {
+        const bool narrow = thin && b_kc && 2.0 * tiles <= cus;
         const double units = tiles * parts * (parts == 1 && narrow ? 2.0 : 1.0);
         double rounds = std::ceil(units / cus - 1e-9);
         const double whole = std::floor(units / cus), rest = units - whole * cus;
-        if (tall && !thin && parts == 1 && rest > 0.5 && 2.0 * rest <= cus) rounds = whole + (whole > 0.0 ? kTailCost : kLoneTailCost);
+        double step_us = thin ? kThinStepUs[b_kc] : kStepUs;
+        if (tall && !thin) {
+            const bool in_parts = parts == 1 && rest > 0.5 && 2.0 * rest <= cus;
+            if (in_parts) rounds = whole + (whole > 0.0 ? kTailCost : kLoneTailCost);
+            step_us = kTallStepUs + (in_parts ? kFullStepUs : kFullStepUs * std::min(1.0, units / cus));
+        }
         const double products = rounds * (steps + kTileSteps) * step_us;
         const double sums = parts > 1 ? kReduceUs + (double)R * N * (8.0 * parts + 2.0) / kReduceBytesPerUs : 0.0;
         return std::max(products, weights_us) + sums;
+    };
+    // tall: between the two numbers of row tiles about the expected one, by how likely they are. (What fills the compute units
+    // exactly once is worth little if one group in ten launches spoils it.)
+    const double low = tall ? std::floor(row_tiles) : row_tiles, more = row_tiles - low;
+    auto us = [&](uint32_t parts, uint32_t steps) {
+        const double t = us_of(low * columns, parts, steps);
+        return more > 0.0 ? (1.0 - more) * t + more * us_of((low + 1.0) * columns, parts, steps) : t;
     };
     double best_us = us(1, all) * kSplitGain;
     for (uint32_t parts = 2; parts * kSplitMinSteps <= all && parts <= 32; ++parts) {
