@@ -224,6 +224,9 @@ __global__ __launch_bounds__(kIdxThreads) void index_hist_kernel(const id_t* __r
 
 // counts, inclusive offsets, and hist[c * rows][e] <- first output position of chunk c's slots of expert e.
 // A chunk's histogram is the sum of `rows` consecutive rows of hist (the last chunk may have fewer: nrows in all).
+// (One workgroup; what bounds it is the latency of its loads one after the other. With eight, and four chunks, in flight instead of one,
+// and a prefix over the segments that have chunks only, the index build (both launches) of 8192 tokens takes 30.6 -> 17.6 us on 128
+// experts, 20.9 -> 12.4 on 64, of 4096 tokens on 128 20.1 -> 13.1.)
 __global__ __launch_bounds__(kScanThreads) void index_scan_kernel(uint32_t E, uint32_t nchunks, uint32_t rows,
                                                                   uint32_t nrows, uint32_t* hist,
                                                                   uint32_t* __restrict__ counts,
@@ -247,7 +250,16 @@ __global__ __launch_bounds__(kScanThreads) void index_scan_kernel(uint32_t E, ui
         const uint32_t r_lo = c_lo * rows;
         uint32_t r_hi = c_hi * rows;
         if (r_hi > nrows) r_hi = nrows;
-        for (uint32_t r = r_lo; r < r_hi; ++r) s += hist[(uint64_t)r * E + e];
+        // (eight loads in flight: every thread walks up to nrows / parts rows of its column)
+        uint32_t r = r_lo;
+        for (; r + 8u <= r_hi; r += 8u) {
+            uint32_t v[8];
+#pragma unroll
+            for (uint32_t i = 0; i < 8u; ++i) v[i] = hist[(uint64_t)(r + i) * E + e];
+#pragma unroll
+            for (uint32_t i = 0; i < 8u; ++i) s += v[i];
+        }
+        for (; r < r_hi; ++r) s += hist[(uint64_t)r * E + e];
         s_seg[part * E + e] = s;
     }
     __syncthreads();
@@ -255,7 +267,8 @@ __global__ __launch_bounds__(kScanThreads) void index_scan_kernel(uint32_t E, ui
     // per-expert totals and exclusive prefix over the segments (thread e < E walks its column)
     uint32_t total = 0;
     if (tid < E) {
-        for (uint32_t p = 0; p < parts; ++p) {
+        const uint32_t used = seg ? (nchunks + seg - 1) / seg : 0u;  // segments with chunks
+        for (uint32_t p = 0; p < used; ++p) {
             const uint32_t v = s_seg[p * E + tid];
             s_seg[p * E + tid] = total;
             total += v;
@@ -282,40 +295,34 @@ __global__ __launch_bounds__(kScanThreads) void index_scan_kernel(uint32_t E, ui
 
     if (active) {
         uint32_t running = s_start[e] + s_seg[part * E + e];
-        for (uint32_t c = c_lo; c < c_hi; ++c) {
+        // the sums of a chunk's rows are formed before its first row is overwritten, those of the next four chunks before any of theirs
+        auto rows_of = [&](uint32_t c) -> uint32_t {
             const uint32_t r0 = c * rows;
-            uint32_t r1 = r0 + rows;
-            if (r1 > nrows) r1 = nrows;
+            const uint32_t n = c >= c_hi ? 0u : (nrows - r0 < rows ? nrows - r0 : rows);
             uint32_t v = 0;
-            for (uint32_t r = r0; r < r1; ++r) v += hist[(uint64_t)r * E + e];
-            hist[(uint64_t)r0 * E + e] = running;
-            running += v;
+#pragma unroll 4
+            for (uint32_t r = 0; r < n; ++r) v += hist[(uint64_t)(r0 + r) * E + e];
+            return v;
+        };
+        for (uint32_t c = c_lo; c < c_hi; c += 4u) {
+            const uint32_t v[4] = {rows_of(c), rows_of(c + 1u), rows_of(c + 2u), rows_of(c + 3u)};
+#pragma unroll
+            for (uint32_t i = 0; i < 4u; ++i) {
+                if (c + i < c_hi) hist[(uint64_t)(c + i) * rows * E + e] = running;
+                running += v[i];
+            }
         }
     }
 }
 
 // One wavefront per chunk walks its slots in order; lanes with the same expert id find each other with
 // ballots, the lowest of them advances the expert's cursor, each takes cursor + its rank in the group.
-// A chunk is chunk_slots <= STEPS * 64 consecutive slots; its cursors start at base[c * base_stride + e].
+// A chunk is chunk_slots <= STEPS * 64 consecutive slots; cur: its cursors, one per expert, in LDS.
 template <typename id_t, int STEPS>
-__global__ __launch_bounds__(kIdxThreads) void index_place_kernel(const id_t* __restrict__ ids, int64_t R, uint32_t E,
-                                                                  uint32_t nbits, uint32_t nchunks, uint32_t chunk_slots,
-                                                                  uint64_t base_stride,
-                                                                  const uint32_t* __restrict__ base,
-                                                                  int32_t* __restrict__ perm, int32_t* __restrict__ eid,
-                                                                  int32_t* __restrict__ inv) {
-    extern __shared__ uint32_t lds[];
+__device__ __forceinline__ void place_chunk(const id_t* __restrict__ ids, int64_t R, uint32_t E, uint32_t nbits, uint32_t c,
+                                            uint32_t chunk_slots, uint32_t* cur, int32_t* __restrict__ perm,
+                                            int32_t* __restrict__ eid, int32_t* __restrict__ inv) {
     const uint32_t lane = threadIdx.x & (kWave - 1);
-    const uint32_t wave = threadIdx.x / kWave;
-    uint32_t* cur = lds + wave * E;
-    const uint32_t c = blockIdx.x * kIdxWaves + wave;
-    const bool live = c < nchunks;
-    if (live) {
-        for (uint32_t e = lane; e < E; e += kWave) cur[e] = base[(uint64_t)c * base_stride + e];
-    }
-    __syncthreads();
-    if (!live) return;
-
     const int64_t first = (int64_t)c * chunk_slots;
     const int64_t end = first + chunk_slots < R ? first + chunk_slots : R;  // slots past the chunk read as "no id"
     int32_t id[STEPS];
@@ -344,6 +351,90 @@ __global__ __launch_bounds__(kIdxThreads) void index_place_kernel(const id_t* __
             inv[slot] = pos;
         }
     }
+}
+
+// The cursors of chunk c start at base[c * base_stride + e].
+template <typename id_t, int STEPS>
+__global__ __launch_bounds__(kIdxThreads) void index_place_kernel(const id_t* __restrict__ ids, int64_t R, uint32_t E,
+                                                                  uint32_t nbits, uint32_t nchunks, uint32_t chunk_slots,
+                                                                  uint64_t base_stride,
+                                                                  const uint32_t* __restrict__ base,
+                                                                  int32_t* __restrict__ perm, int32_t* __restrict__ eid,
+                                                                  int32_t* __restrict__ inv) {
+    extern __shared__ uint32_t lds[];
+    const uint32_t lane = threadIdx.x & (kWave - 1);
+    const uint32_t wave = threadIdx.x / kWave;
+    uint32_t* cur = lds + wave * E;
+    const uint32_t c = blockIdx.x * kIdxWaves + wave;
+    const bool live = c < nchunks;
+    if (live) {
+        for (uint32_t e = lane; e < E; e += kWave) cur[e] = base[(uint64_t)c * base_stride + e];
+    }
+    __syncthreads();
+    if (!live) return;
+    place_chunk<id_t, STEPS>(ids, R, E, nbits, c, chunk_slots, cur, perm, eid, inv);
+}
+
+// Scan and placement in one launch, for histograms so small that every workgroup sums all of it (hist[nrows][E], a chunk being `rows`
+// of them): a launch of its own for the scan is bound by latency, its serial sums over rows and segments, 7 to 8 us.
+constexpr uint32_t kFusedExperts = kIdxThreads;  // a thread per expert
+// Index build, us, at 130 / 512 / 1024 / 4096 tokens, two launches -> one: E 8, k 2 8.6 -> 3.7, 10.6 -> 4.8, 10.6 -> 5.1, 10.9 -> 7.7;
+// E 32, k 4 8.2 -> 5.5, 8.4 -> 6.0, 8.6 -> 8.2, at 2048 tokens (4096 words) 9.0 -> 10.3 (not taken); E 64, k 8 7.6 -> 5.9, 8.2 -> 8.3 (2048
+// words), 9.5 -> 10.6 (not taken).
+inline bool fused_scan(uint64_t nrows, uint64_t E) { return E <= kFusedExperts && nrows * E <= (E <= 16 ? 4096u : 2048u); }
+template <int STEPS>
+__global__ __launch_bounds__(kIdxThreads) void index_scan_place_kernel(const int32_t* __restrict__ ids, int64_t R, uint32_t E,
+                                                                       uint32_t nbits, uint32_t nchunks, uint32_t chunk_slots,
+                                                                       uint32_t rows, uint32_t nrows,
+                                                                       const uint32_t* __restrict__ hist,
+                                                                       uint32_t* __restrict__ counts,
+                                                                       uint32_t* __restrict__ offsets, int32_t* __restrict__ perm,
+                                                                       int32_t* __restrict__ eid, int32_t* __restrict__ inv) {
+    __shared__ uint32_t s_total[kFusedExperts];
+    // [w]: first what lies in front of the workgroup (w = 0) and in its chunk w - 1, then the cursors of its chunk w
+    __shared__ uint32_t s_cur[kIdxWaves][kFusedExperts];
+    __shared__ uint32_t s_wave_tot[kIdxWaves];
+    const uint32_t tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
+    s_total[tid] = 0;
+#pragma unroll
+    for (int w = 0; w < kIdxWaves; ++w) s_cur[w][tid] = 0;
+    __syncthreads();
+    // 2^nbits >= E threads per row of the histogram
+    const uint32_t e = tid & ((1u << nbits) - 1u), part = tid >> nbits, parts = (uint32_t)kIdxThreads >> nbits;
+    const uint32_t r0 = blockIdx.x * kIdxWaves * rows;
+    if (e < E) {
+        uint32_t total = 0, in[kIdxWaves] = {};
+#pragma unroll 8
+        for (uint32_t r = part; r < nrows; r += parts) {
+            const uint32_t v = hist[r * E + e];
+            total += v;
+            in[0] += r < r0 ? v : 0u;
+#pragma unroll
+            for (int w = 1; w < kIdxWaves; ++w) in[w] += r >= r0 + (w - 1) * rows && r < r0 + w * rows ? v : 0u;
+        }
+        atomicAdd(&s_total[e], total);
+#pragma unroll
+        for (int w = 0; w < kIdxWaves; ++w) atomicAdd(&s_cur[w][e], in[w]);
+    }
+    __syncthreads();
+    const uint32_t total = s_total[tid];  // (0 past E)
+    uint32_t incl = wave_inclusive_scan<uint32_t>(total);
+    if (lane == kWave - 1) s_wave_tot[wave] = incl;
+    __syncthreads();
+    for (uint32_t w = 0; w < wave; ++w) incl += s_wave_tot[w];
+    if (blockIdx.x == 0 && tid < E) {
+        counts[tid] = total;
+        offsets[tid] = incl;
+    }
+    uint32_t running = incl - total;
+#pragma unroll
+    for (int w = 0; w < kIdxWaves; ++w) {
+        running += s_cur[w][tid];
+        s_cur[w][tid] = running;
+    }
+    __syncthreads();
+    const uint32_t c = blockIdx.x * kIdxWaves + wave;
+    if (c < nchunks) place_chunk<int32_t, STEPS>(ids, R, E, nbits, c, chunk_slots, s_cur[wave], perm, eid, inv);
 }
 
 inline uint32_t index_nchunks(int64_t R) { return (uint32_t)((R + kIdxChunk - 1) / kIdxChunk); }
@@ -401,7 +492,7 @@ int launch_build_index(const void* ids, int id_bytes, int64_t R, int64_t E, uint
 }
 
 // The same sort from histograms the caller already has: hist[r][e] = number of slots of the r-th block of
-// 16 * top_k consecutive slots (16 tokens) that go to expert e. Two launches: scan and placement. A chunk of the
+// 16 * top_k consecutive slots (16 tokens) that go to expert e. Two launches, scan and placement, or one where the histogram is small. A chunk of the
 // placement is `rows` consecutive blocks, about 512 slots.
 int launch_build_index_from_hist(const int32_t* ids, int64_t R, int64_t E, int64_t top_k, uint32_t* counts,
                                  uint32_t* offsets, int32_t* perm, int32_t* eid, int32_t* inv, uint32_t* hist,
@@ -415,6 +506,15 @@ int launch_build_index_from_hist(const int32_t* ids, int64_t R, int64_t E, int64
     const size_t lds_bytes = (size_t)kIdxWaves * E * 4;
     uint32_t nbits = 0;
     while ((1ll << nbits) < E) ++nbits;
+    if (nchunks > 0 && fused_scan(nrows, (uint64_t)E)) {
+        auto run = [&](auto kernel) {
+            hipLaunchKernelGGL(kernel, dim3(blocks), dim3(kIdxThreads), 0, st, ids, R, (uint32_t)E, nbits, nchunks, chunk_slots, rows,
+                               nrows, (const uint32_t*)hist, counts, offsets, perm, eid, inv);
+        };
+        if (chunk_slots <= kIdxSteps * kWave) run(index_scan_place_kernel<kIdxSteps>);
+        else run(index_scan_place_kernel<2 * kIdxSteps>);
+        return launch_status("moe_build_index_from_hist");
+    }
     hipLaunchKernelGGL(index_scan_kernel, dim3(1), dim3(kScanThreads), 0, st, (uint32_t)E, nchunks, rows, nrows, hist,
                        counts, offsets);
     int rc = launch_status("moe_build_index_from_hist(scan)");

@@ -99,8 +99,8 @@ int fma_moe_build_index(const void* ids, int id_bytes, int64_t R, int64_t E, uin
 
 /* fma_moe_build_index for ids that come from fma_router_topk, which has already counted them: token_block_hist
  * ([ceil(T / 16), E] uint32, T = R / top_k) holds, per block of 16 consecutive tokens, the number of choices of every
- * expert, as that call writes it. Two launches (prefix scan, placement) instead of three, no workspace: the histogram
- * itself is the scratch memory and is OVERWRITTEN. ids: int32 [R], every id in [0, E); top_k <= 64 divides R. Same
+ * expert, as that call writes it. Two launches (prefix scan, placement; one where the histogram is small) instead of three, no
+ * workspace: the histogram itself is the scratch memory and is OVERWRITTEN. ids: int32 [R], every id in [0, E); top_k <= 64 divides R. Same
  * outputs, bit for bit, as fma_moe_build_index. Replaces the same reference lines, for the case that the choice and
  * its histogram come out of one kernel (fma/modules/moe/__init__.py:191-217). */
 int fma_moe_build_index_from_hist(const int32_t* ids, int64_t R, int64_t E, int64_t top_k, uint32_t* token_block_hist,

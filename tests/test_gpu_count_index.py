@@ -125,6 +125,25 @@ def test_routing_index_from_token_block_histogram(T, E, k, kind, empty):
         assert np.array_equal(to_np(a), expect[key]), key
 
 
+@pytest.mark.parametrize(
+    "T,E,k",
+    # scan and placement in one launch, at its edges: one expert, one token, 4096 words of histogram for up to 16 experts and 2048 beyond,
+    # one row more than that (two launches), several workgroups with a last short chunk, long chunks, 256 and 257 experts
+    [(40, 1, 1), (1, 2, 1), (8192, 8, 2), (8193, 8, 2), (4096, 16, 3), (1920, 17, 4), (1937, 17, 4), (512, 64, 8), (513, 64, 8),
+     (128, 256, 8), (129, 256, 8), (100, 257, 8), (33, 60, 50), (2048, 16, 16), (2000, 3, 3)],
+)  # fmt: skip
+def test_routing_index_from_small_histograms(T, E, k):
+    selected, _ = make_routing(T, E, k, "uniform", seed=T + E, empty_tail=0)
+    expect = c_oracle.routing_index(selected.numpy(), E)
+    hist = np.zeros(((T + 15) // 16, E), dtype=np.int32)
+    np.add.at(hist, (np.repeat(np.arange(T) // 16, k), selected.numpy().reshape(-1)), 1)
+    got = build_routing_index(
+        selected.to(torch.int32).to(DEV), E, token_block_histogram=torch.from_numpy(hist).to(DEV).view(torch.uint32)
+    )
+    for a, key in zip(got, ("counts", "offsets", "perm", "eid", "inv")):
+        assert np.array_equal(to_np(a), expect[key]), key
+
+
 def test_routing_index_fixture():
     # tests/golden/routing_index_4096.npz: 4096 skewed ids, three empty experts, answers from numpy
     import os
