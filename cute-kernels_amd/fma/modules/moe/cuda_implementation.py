@@ -812,6 +812,9 @@ def fp32_swiglu_layer(
     K1_array: torch.Tensor, N2_array: torch.Tensor, K2_array: torch.Tensor, top_k: int,
 ) -> tuple[torch.Tensor, torch.Tensor]:  # fmt: skip
     """(output, router_logits) of a SwiGLU layer without biases in fp32: router, routing index and experts in one operator each"""
+    # (made contiguous here, where it is recorded: a copy made inside the router's node would be one that its recorded backward
+    # cannot be differentiated through)
+    x, gate_weight = x.contiguous(), gate_weight.contiguous()
     logits, gates, selected, token_block_hist = _Fp32Router.apply(x, gate_weight, top_k)
     M_array, _, _, _, inv = build_routing_index(selected, gate_weight.size(0), token_block_hist)
     y = _Fp32SwigluExperts.apply(

@@ -1,0 +1,67 @@
+"""What the host decides and records about the fp32 SwiGLU layer, on the CPU: the operators are replaced by the same values from torch."""
+
+import pytest
+import torch
+import torch.nn.functional as F
+
+from fma.modules.moe import cuda_implementation as ci
+
+TOL = 1e-5  # fp32 sums of 24 terms of size one
+
+
+def _router_in_torch(x, gate_weight, top_k, logits, weights, selected, token_block_hist):
+    with torch.no_grad():
+        logits.copy_(x @ gate_weight.t())
+        top, chosen = logits.topk(top_k, dim=-1)
+        weights.copy_(top.softmax(-1))
+        selected.copy_(chosen)
+
+
+def _router_backward_in_torch(logits, selected, weights_grad, logits_output_grad, logits_grad):
+    with torch.no_grad():
+        columns = selected.long()
+        s = logits.gather(1, columns).softmax(-1)
+        logits_grad.copy_(torch.zeros_like(logits) if logits_output_grad is None else logits_output_grad)
+        if weights_grad is not None:
+            logits_grad.scatter_add_(1, columns, s * (weights_grad - (s * weights_grad).sum(-1, keepdim=True)))
+
+
+class _GatedSum:
+    """stands for the experts' node: depends on tokens and gates as they do, and is differentiated by autograd"""
+
+    @staticmethod
+    def apply(x, gates, *_):
+        return x * gates.pow(2).sum(-1, keepdim=True)
+
+
+@pytest.mark.parametrize("strided", ["tokens", "gate", "neither"])
+def test_second_derivative_with_strided_arguments(strided, monkeypatch):
+    T, H, E, k = 12, 24, 6, 2
+    torch.manual_seed(0)
+    wide = torch.randn(T, H + 8)
+    x = wide[:, :H] if strided == "tokens" else wide[:, :H].contiguous()
+    w = torch.randn(H, E).t() if strided == "gate" else torch.randn(E, H)
+    assert (x.is_contiguous(), w.is_contiguous()) == (strided != "tokens", strided != "gate")
+    monkeypatch.setattr(ci, "router_topk_f32_cuda", _router_in_torch)
+    monkeypatch.setattr(ci, "router_topk_backward_f32_cuda", _router_backward_in_torch)
+    monkeypatch.setattr(ci, "build_routing_index", lambda *_: (None,) * 5)
+    monkeypatch.setattr(ci, "_Fp32SwigluExperts", _GatedSum)
+
+    def layer(x, w):
+        y, logits = ci.fp32_swiglu_layer(x, w, *[None] * 6, k)
+        return y, logits
+
+    def library(x, w):
+        logits = F.linear(x, w)
+        gates = logits.topk(k, dim=-1).values.softmax(-1)
+        return _GatedSum.apply(x, gates), logits
+
+    results = []
+    for fn in (layer, library):
+        xi, wi = x.detach().requires_grad_(), w.detach().requires_grad_()
+        assert xi.stride() == x.stride() and wi.stride() == w.stride()
+        y, logits = fn(xi, wi)
+        first = torch.autograd.grad(y.sin().sum() + logits.logsumexp(-1).pow(2).sum(), (xi, wi), create_graph=True)
+        results.append([*first, *torch.autograd.grad(sum(g.pow(2).sum() for g in first), (xi, wi))])
+    for got, expect in zip(*results):
+        assert float((got - expect).norm() / expect.norm()) < TOL

@@ -169,3 +169,22 @@ def test_what_takes_the_general_path(case, monkeypatch):
     assert seen and (calls == [] or (case == "autocast" and not torch.is_autocast_enabled("cuda")))
     for a, b in zip(got, expect):
         assert float((a.float() - b).norm() / b.norm()) < (TOL if case != "autocast" else 1e-2)
+
+
+@pytest.mark.parametrize("strided", ["tokens", "gate"])
+def test_second_derivative_of_strided_tokens_and_gate(strided):
+    moe = _layer(8, 2, 64, 32)
+    wide = torch.randn(20, 72, device=DEV)
+    x = wide[:, :64] if strided == "tokens" else wide[:, :64].contiguous()
+    if strided == "gate":
+        moe.gate.weight = torch.nn.Parameter(moe.gate.weight.detach().t().contiguous().t())
+    results = []
+    for fused in (True, False):
+        moe.fuse_swiglu_backward = fused
+        xi = x.detach().requires_grad_()
+        assert xi.is_contiguous() == (strided != "tokens")
+        _, logits = moe(xi, kernel_backend=KernelBackend.cuda)
+        first = torch.autograd.grad(logits.logsumexp(-1).pow(2).sum(), (xi, moe.gate.weight), create_graph=True)
+        results.append([*first, *torch.autograd.grad(sum(g.pow(2).sum() for g in first), (xi, moe.gate.weight))])
+    for a, b in zip(*results):
+        assert float((a - b).norm() / b.norm()) < TOL
