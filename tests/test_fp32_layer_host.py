@@ -3,7 +3,11 @@
 import pytest
 import torch
 import torch.nn.functional as F
+from torch._subclasses.fake_tensor import FakeTensorMode
+from torch.fx.experimental.proxy_tensor import make_fx
+from torch.utils._python_dispatch import TorchDispatchMode
 
+from fma import KernelBackend, MoE, swiglu_packed
 from fma.modules.moe import cuda_implementation as ci
 
 TOL = 1e-5  # fp32 sums of 24 terms of size one
@@ -65,3 +69,38 @@ def test_second_derivative_with_strided_arguments(strided, monkeypatch):
         results.append([*first, *torch.autograd.grad(sum(g.pow(2).sum() for g in first), (xi, wi))])
     for got, expect in zip(*results):
         assert float((got - expect).norm() / expect.norm()) < TOL
+
+
+class _Names(TorchDispatchMode):
+    def __init__(self):
+        super().__init__()
+        self.names = []
+
+    def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+        self.names.append(func.name())
+        return func(*args, **(kwargs or {}))
+
+
+@pytest.mark.parametrize("how", ["fake mode", "make_fx"])
+@pytest.mark.filterwarnings("error")
+def test_tracing_takes_the_general_path(how):
+    """a traced layer is made of the library's router and the operators of the general path, and no address is asked for"""
+    fake = FakeTensorMode(allow_non_fake_inputs=True)
+    with fake, torch.device("cuda"):
+        moe = MoE(8, 2, 64, 32, swiglu_packed, True, False, 0.02)
+        x = torch.randn(20, 64)
+
+    def layer(x):
+        return moe(x, kernel_backend=KernelBackend.cuda)
+
+    if how == "make_fx":
+        with fake:
+            names = [str(n.target) for n in make_fx(layer)(x).graph.nodes]
+        linear, of_layer = "aten.mm.default", "f32_cuda.default"
+    else:
+        with fake, _Names() as seen:
+            layer(x)
+        names, linear, of_layer = seen.names, "aten::mm", "f32_cuda"
+    assert linear in names and not any(n.endswith(of_layer) for n in names), names
+    # outside the mode its tensors are still no tensors with an address
+    assert moe._fp32_operands(x, KernelBackend.cuda) is None
