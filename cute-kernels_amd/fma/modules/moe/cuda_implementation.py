@@ -807,15 +807,36 @@ class _Fp32SwigluExperts(torch.autograd.Function):
         return x_grad, gates_grad, weight1_grad, weight2_grad, None, None, None, None, None, None, None
 
 
+def fp32_router_is_fusable(num_tokens: int, num_experts: int, hidden_size: int, top_k: int) -> bool:
+    """Whether _Fp32Router stands for the library's product, top-k and softmax. It gives 16 tokens one compute unit, through which
+    the router's whole matrix goes, 64 experts at a time (1 us per 64 k of such a pass), and in which the choices are made one after
+    the other (0.25 us each, and 3.5 ns per expert); more compute units make neither shorter. The library takes 30 us and more for
+    top-k, half of that for one choice. Router and index build in a graph, library / kernel, us, at 16, 512 and 8192 tokens:
+    E 64, k 8: hidden 256 33 / 16, 39 / 22, 64 / 29, hidden 1152 33 / 28, 40 / 34, 73 / 54, hidden 2048 33 / 39, 41 / 45, 80 / 76;
+    E 128, k 8: hidden 576 42 / 31, 43 / 38, 101 / 55, hidden 1024 35 / 42, 44 / 50, 106 / 84; E 256, k 8: hidden 256 40 / 35, 48 / 42,
+    159 / 90, hidden 576 43 / 51, 47 / 59, 167 / 129; k 32: E 64, hidden 256 37 / 27, 43 / 32, 73 / 47, E 128, hidden 576 44 / 47, 46 / 55,
+    121 / 85; k 1, E 64: hidden 256 21 / 13, 24 / 18, 29 / 25 (65536 tokens 75 / 85), hidden 1024 20 / 24, 24 / 28, 36 / 47."""
+    passes = (num_experts + 63) // 64 * hidden_size
+    if top_k == 1:
+        return passes <= 256 and num_tokens <= 8192
+    return passes / 64 + top_k * (num_experts + 72) / 288 <= 26
+
+
 def fp32_swiglu_layer(
     x: torch.Tensor, gate_weight: torch.Tensor, weight1: torch.Tensor, weight2: torch.Tensor, N1_array: torch.Tensor,
     K1_array: torch.Tensor, N2_array: torch.Tensor, K2_array: torch.Tensor, top_k: int,
+    routed: tuple[torch.Tensor, torch.Tensor, torch.Tensor] | None = None,
 ) -> tuple[torch.Tensor, torch.Tensor]:  # fmt: skip
-    """(output, router_logits) of a SwiGLU layer without biases in fp32: router, routing index and experts in one operator each"""
-    # (made contiguous here, where it is recorded: a copy made inside the router's node would be one that its recorded backward
-    # cannot be differentiated through)
-    x, gate_weight = x.contiguous(), gate_weight.contiguous()
-    logits, gates, selected, token_block_hist = _Fp32Router.apply(x, gate_weight, top_k)
+    """(output, router_logits) of a SwiGLU layer without biases in fp32: router, routing index and experts in one operator each.
+    routed: logits, weights and choice of a router that the caller has run itself."""
+    token_block_hist = None
+    if routed is None:
+        # (made contiguous here, where it is recorded: a copy made inside the router's node would be one that its recorded
+        # backward cannot be differentiated through)
+        x, gate_weight = x.contiguous(), gate_weight.contiguous()
+        logits, gates, selected, token_block_hist = _Fp32Router.apply(x, gate_weight, top_k)
+    else:
+        logits, gates, selected = routed
     M_array, _, _, _, inv = build_routing_index(selected, gate_weight.size(0), token_block_hist)
     y = _Fp32SwigluExperts.apply(
         x, gates, weight1, weight2, inv, M_array, N1_array, K1_array, N2_array, K2_array, torch.is_grad_enabled()

@@ -188,3 +188,21 @@ def test_second_derivative_of_strided_tokens_and_gate(strided):
         results.append([*first, *torch.autograd.grad(sum(g.pow(2).sum() for g in first), (xi, moe.gate.weight))])
     for a, b in zip(*results):
         assert float((a - b).norm() / b.norm()) < TOL
+
+
+@pytest.mark.parametrize(
+    "E,H,k,fused",
+    [(64, 1152, 8, True), (128, 576, 8, True), (1000, 24, 4, True), (64, 256, 32, True), (64, 256, 1, True), (64, 1664, 2, False), (129, 576, 2, False),
+     (64, 1024, 64, False), (64, 264, 1, False), (8, 2048, 2, False)],
+)  # fmt: skip
+def test_large_routers_are_the_library_s(E, H, k, fused, monkeypatch):
+    moe = _layer(E, k, H, 16)
+    x, dy, dlogits = torch.randn(30, H, device=DEV), torch.randn(30, H, device=DEV), torch.randn(30, E, device=DEV)
+    calls = []
+    for name in ("router_topk_f32_cuda", "swiglu_experts_f32_cuda"):
+        real = getattr(ci, name)
+        monkeypatch.setattr(ci, name, lambda *a, real=real, name=name: (calls.append(name), real(*a))[1])
+    got = _step(moe, x, dy, dlogits)
+    assert calls == ["router_topk_f32_cuda"] * fused + ["swiglu_experts_f32_cuda"]
+    moe.fuse_swiglu_backward = False
+    _close(got, _step(moe, x, dy, dlogits))
