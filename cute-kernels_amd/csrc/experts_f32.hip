@@ -29,8 +29,9 @@ int fma_swiglu_experts_bwd_f32(const void* dy, const int32_t* inv, const void* g
                                void* stream) {
     using namespace fmahip;
     FMA_REQUIRE(T >= 1 && k >= 1 && E >= 1 && H >= 1 && I >= 1, FMA_ERR_BAD_SIZE, "swiglu_experts_bwd_f32: sizes must be positive");
-    FMA_REQUIRE(dy && inv && gates && W1 && W2 && xg && h && act && o && counts && N1 && K1 && N2 && K2 && d_o && d_act && d_h,
+    FMA_REQUIRE(dy && inv && gates && W1 && W2 && xg && h && act && o && counts && N1 && K1 && N2 && K2 && d_o,
                 FMA_ERR_NULL_POINTER, "swiglu_experts_bwd_f32: NULL pointer");
+    FMA_REQUIRE((d_act && d_h) || !(dx || dW1), FMA_ERR_NULL_POINTER, "swiglu_experts_bwd_f32: dx and dW1 need d_act and d_h");
     const int64_t R = T * k;
     const float* const hf = (const float*)h;
     float* const dhf = (float*)d_h;

@@ -599,7 +599,7 @@ def swiglu_experts_f32_cuda(
     xg: torch.Tensor, h: torch.Tensor, act: torch.Tensor, o: torch.Tensor, y: torch.Tensor,
 ) -> None:  # fmt: skip
     """The experts of an fp32 SwiGLU layer on its routed tokens (fma_swiglu_experts_f32): y = the gated sum of o, the
-    projections' grouped rows xg, h, act and o on the way."""
+    projections' grouped rows xg, h, act and o on the way (o may be xg's memory where no backward follows)."""
     _lib.require_gpu(x, gates, weight1, weight2, inv, M_array, N1_array, K1_array, N2_array, K2_array, xg, h, act, o, y)
     sizes = (M_array, N1_array, K1_array, N2_array, K2_array)
     T, k, E, H, inter = _check_experts_f32(x, gates, weight1, weight2, inv, sizes)
@@ -625,18 +625,20 @@ def swiglu_experts_backward_f32_cuda(
     y_grad: torch.Tensor, gates: torch.Tensor, weight1: torch.Tensor, weight2: torch.Tensor, inv: torch.Tensor,
     M_array: torch.Tensor, N1_array: torch.Tensor, K1_array: torch.Tensor, N2_array: torch.Tensor, K2_array: torch.Tensor,
     xg: torch.Tensor, h: torch.Tensor, act: torch.Tensor, o: torch.Tensor,
-    o_grad: torch.Tensor, act_grad: torch.Tensor, h_grad: torch.Tensor, x_grad: torch.Tensor | None,
+    o_grad: torch.Tensor, act_grad: torch.Tensor | None, h_grad: torch.Tensor | None, x_grad: torch.Tensor | None,
     gates_grad: torch.Tensor | None, weight1_grad: torch.Tensor | None, weight2_grad: torch.Tensor | None,
 ) -> None:  # fmt: skip
-    """Backward of swiglu_experts_f32_cuda (fma_swiglu_experts_bwd_f32); o_grad, act_grad and h_grad are scratch memory."""
+    """Backward of swiglu_experts_f32_cuda (fma_swiglu_experts_bwd_f32); o_grad, act_grad and h_grad are scratch memory, the last two
+    needed for the gradients of x and weight1 only."""
     buffers = (o_grad, act_grad, h_grad, x_grad, gates_grad, weight1_grad, weight2_grad)
     _lib.require_gpu(y_grad, gates, weight1, weight2, inv, M_array, N1_array, K1_array, N2_array, K2_array, xg, h, act, o, *buffers)
     sizes = (M_array, N1_array, K1_array, N2_array, K2_array)
     T, k, E, H, inter = _check_experts_f32(y_grad, gates, weight1, weight2, inv, sizes)
     R = T * k
     assert xg.shape == o.shape == o_grad.shape == (R, H)
-    assert h.shape == h_grad.shape == (R, 2 * inter) and act.shape == act_grad.shape == (R, inter)
-    for t, like in ((x_grad, y_grad), (gates_grad, gates), (weight1_grad, weight1), (weight2_grad, weight2)):
+    assert h.shape == (R, 2 * inter) and act.shape == (R, inter)
+    assert (act_grad is not None and h_grad is not None) or (x_grad is None and weight1_grad is None)
+    for t, like in ((act_grad, act), (h_grad, h), (x_grad, y_grad), (gates_grad, gates), (weight1_grad, weight1), (weight2_grad, weight2)):
         assert t is None or t.shape == like.shape
     for t in (y_grad, gates, weight1, weight2, inv, xg, h, act, o):
         assert t.is_contiguous()
@@ -783,11 +785,13 @@ class _Fp32SwigluExperts(torch.autograd.Function):
     ) -> torch.Tensor:  # fmt: skip
         T, H = x.shape
         R, inter = T * gates.size(1), weight2.size(2)
-        xg, h, act, o = x.new_empty(R, H), x.new_empty(R, 2 * inter), x.new_empty(R, inter), x.new_empty(R, H)
+        keeps = grad_enabled and any(ctx.needs_input_grad[:4])
+        xg, h, act = x.new_empty(R, H), x.new_empty(R, 2 * inter), x.new_empty(R, inter)
+        o = x.new_empty(R, H) if keeps else xg  # (nothing reads the grouped tokens any more when o is written)
         y = torch.empty_like(x)
         sizes = (M_array, N1_array, K1_array, N2_array, K2_array)
         swiglu_experts_f32_cuda(x, gates, weight1, weight2, inv, *sizes, xg, h, act, o, y)
-        if grad_enabled and any(ctx.needs_input_grad[:4]):
+        if keeps:
             ctx.save_for_backward(gates, weight1, weight2, inv, *sizes, xg, h, act, o)
         return y
 
@@ -800,9 +804,10 @@ class _Fp32SwigluExperts(torch.autograd.Function):
         gates_grad = torch.empty_like(gates) if needs_gates else None
         weight1_grad = torch.empty_like(weight1) if needs_weight1 else None
         weight2_grad = torch.empty_like(weight2) if needs_weight2 else None
+        act_grad, h_grad = (torch.empty_like(act), torch.empty_like(h)) if needs_x or needs_weight1 else (None, None)
         swiglu_experts_backward_f32_cuda(
-            y_grad, gates, weight1, weight2, inv, *sizes, xg, h, act, o, torch.empty_like(o), torch.empty_like(act),
-            torch.empty_like(h), x_grad, gates_grad, weight1_grad, weight2_grad,
+            y_grad, gates, weight1, weight2, inv, *sizes, xg, h, act, o, torch.empty_like(o), act_grad, h_grad,
+            x_grad, gates_grad, weight1_grad, weight2_grad,
         )  # fmt: skip
         return x_grad, gates_grad, weight1_grad, weight2_grad, None, None, None, None, None, None, None
 

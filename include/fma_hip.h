@@ -379,14 +379,15 @@ int fma_router_topk_bwd_f32(const void* logits, const int32_t* selected, const v
 /* The expert path of an fp32 SwiGLU layer without biases, enqueued by one call: fma_dispatch_rows (xg [R, H], R = T * k),
  * fma_grouped_gemm (h [R, 2 I] = xg W1^T), fma_swiglu_forward (act [R, I]; "up" first in h), fma_grouped_gemm (o [R, H] = act W2^T),
  * fma_combine (y [T, H]). W1 [E, 2 I, H], W2 [E, H, I]; counts: rows per expert, N1 / K1 and N2 / K2: out and in features of the two
- * projections per expert, all uint32 [E] in device memory. T >= 1.
+ * projections per expert, all uint32 [E] in device memory. T >= 1. o may be xg's memory where no backward follows: xg is read by the
+ * first product only.
  * Replaces MoE._compute_experts (fma/modules/moe/__init__.py:206-290) for such layers. */
 int fma_swiglu_experts_f32(const void* x, const int32_t* inv, const void* gates, const void* W1, const void* W2, const uint32_t* counts,
                            const uint32_t* N1, const uint32_t* K1, const uint32_t* N2, const uint32_t* K2, int64_t T, int64_t k,
                            int64_t E, int64_t H, int64_t I, void* xg, void* h, void* act, void* o, void* y, void* stream);
 /* Its backward from dy [T, H] and the buffers of the forward call: fma_combine_bwd, the two input and two weight gradients
  * (fma_grouped_gemm), fma_swiglu_backward, fma_combine. d_gates [T, k], dW1, dW2 and dx [T, H] may be NULL (not computed);
- * d_o [R, H], d_act [R, I] and d_h [R, 2 I] are scratch memory. */
+ * d_o [R, H], d_act [R, I] and d_h [R, 2 I] are scratch memory, the last two needed (not NULL) for dx and dW1 only. */
 int fma_swiglu_experts_bwd_f32(const void* dy, const int32_t* inv, const void* gates, const void* W1, const void* W2, const void* xg,
                                const void* h, const void* act, const void* o, const uint32_t* counts, const uint32_t* N1,
                                const uint32_t* K1, const uint32_t* N2, const uint32_t* K2, int64_t T, int64_t k, int64_t E, int64_t H,

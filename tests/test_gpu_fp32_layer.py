@@ -206,3 +206,49 @@ def test_large_routers_are_the_library_s(E, H, k, fused, monkeypatch):
     assert calls == ["router_topk_f32_cuda"] * fused + ["swiglu_experts_f32_cuda"]
     moe.fuse_swiglu_backward = False
     _close(got, _step(moe, x, dy, dlogits))
+
+
+def _peak(step):
+    step()
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    step()
+    return torch.cuda.max_memory_allocated() - before
+
+
+@pytest.mark.parametrize("T,fused", [(9000, True), (9600, False)])  # 28096 bytes a token
+def test_memory_of_large_passes(T, fused):
+    """past the size where host time matters a pass takes no more memory than the general path; up to it, without a backward, no more
+    than the rows of the tokens, the pre-activation and the activation (and the output) at once"""
+    moe = _layer(8, 2, 512, 1000)
+    x, dy = torch.randn(T, 512, device=DEV), torch.randn(T, 512, device=DEV)
+
+    def infer():
+        with torch.no_grad():
+            moe(x, kernel_backend=KernelBackend.cuda)
+
+    def train():
+        moe.zero_grad(set_to_none=True)
+        moe(x, kernel_backend=KernelBackend.cuda)[0].backward(dy)
+
+    peaks = []
+    for switch in (True, False):
+        moe.fuse_swiglu_backward = switch
+        peaks.append([_peak(infer), _peak(train)])
+    few = 1 << 22  # logits, weights, choices and index
+    assert peaks[0][0] <= T * 4 * (2 * (512 + 3000) + 512) + few
+    if not fused:
+        assert peaks[0] == peaks[1]
+
+
+def test_scratch_of_a_backward_for_the_second_projection_alone(monkeypatch):
+    moe = _layer(8, 2, 64, 32)
+    moe.c_fc.weight.requires_grad_(False)
+    moe.gate.weight.requires_grad_(False)
+    seen = []
+    real = ci.swiglu_experts_backward_f32_cuda
+    monkeypatch.setattr(ci, "swiglu_experts_backward_f32_cuda", lambda *a: (seen.append(a), real(*a))[1])
+    moe(torch.randn(40, 64, device=DEV), kernel_backend=KernelBackend.cuda)[0].sum().backward()
+    ((*_, o_grad, act_grad, h_grad, x_grad, gates_grad, weight1_grad, weight2_grad),) = seen
+    assert act_grad is h_grad is x_grad is weight1_grad is None and o_grad is not None and weight2_grad is not None
