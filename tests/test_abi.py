@@ -6,6 +6,7 @@ import os
 import re
 
 import pytest
+import torch
 
 from fma import _lib
 
@@ -34,6 +35,24 @@ def test_workspace_queries(lib):
     assert lib.fma_continuous_count_workspace_bytes(16 << 20, 64) >= 256 + 64 * 4
     assert lib.fma_moe_build_index_workspace_bytes(1024, 8) == 2 * 8 * 4  # two 512-slot chunks
     assert lib.fma_moe_build_index_workspace_bytes(0, 8) == 8 * 4
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="a size that is accepted wrongly would be launched on host addresses")
+def test_split_workspace_is_what_the_launch_needs(lib):
+    """a byte less than the query says is refused: the query is for the parts that the launch takes, not for those of another kernel"""
+    buf = ctypes.create_string_buffer(4096 + 16)
+    p = (ctypes.addressof(buf) + 15) & ~15
+    split = 0
+    for N, K in ((4096, 14336), (4096, 28672), (2048, 8192), (2048, 16384)):
+        for tB in (0, 1):
+            for R in range(256, 9000, 256):
+                for E in (8, 300):
+                    nbytes = lib.fma_grouped_gemm_ragged_workspace_bytes(R, E, N, K, tB)
+                    if nbytes:
+                        split += 1
+                        args = (p, p, p, p, None, E, _lib.FMA_VARY_M, 0, N, K, 0, tB, 1.0, R, p, nbytes - 1, _lib.FMA_BF16, None)
+                        assert lib.fma_grouped_gemm_ragged_split(*args) == -7, (R, E, N, K, tB)
+    assert split > 50
 
 
 def _err(lib) -> str:
