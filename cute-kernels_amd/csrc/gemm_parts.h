@@ -599,14 +599,17 @@ __device__ __forceinline__ void spread_mfma_vmem() {
     }
 }
 
-// Slow, layout-agnostic path for a group whose contiguous dimensions are not multiples of 8 elements.
-template <typename EL, bool A_KC, bool B_KC, int TM, int TN>
-__device__ void scalar_tile(const uint16_t* Ae, const uint16_t* Be, uint16_t* De, uint32_t Me, uint32_t Ne,
-                            uint32_t Ke, uint32_t m0, uint32_t n0, float alpha, uint32_t nthreads) {
-    for (uint32_t idx = threadIdx.x; idx < (uint32_t)(TM * TN); idx += nthreads) {
-        const uint32_t m = m0 + idx / TN;
-        const uint32_t n = n0 + idx % TN;
-        if (m >= Me || n >= Ne) continue;
+// Slow, layout-agnostic path for a group whose contiguous dimensions are not multiples of 8 elements: the tile's rows m0 .. m_end - 1 and
+// columns n0 .. n_end - 1 (none, if n_end is n0), an element per thread and trip. Bound by the loads of single elements, so a part of a
+// tile takes only the trips of its own columns, us, against every part walking 256 columns from its first one, its neighbours' with them:
+// 8 groups of 280 rows, N 501, K 333, NN (parts of 64 columns) 4582 -> 1121; of 40 rows, NT (half-width tiles) 1074 -> 495.
+template <typename EL, bool A_KC, bool B_KC>
+__device__ void scalar_tile(const uint16_t* Ae, const uint16_t* Be, uint16_t* De, uint32_t Me, uint32_t Ne, uint32_t Ke, uint32_t m0,
+                            uint32_t m_end, uint32_t n0, uint32_t n_end, float alpha, uint32_t nthreads) {
+    const uint32_t cols = n_end - n0, elements = (m_end - m0) * cols;
+    for (uint32_t idx = threadIdx.x; idx < elements; idx += nthreads) {
+        const uint32_t m = m0 + idx / cols;
+        const uint32_t n = n0 + idx % cols;
         float acc = 0.0f;
         for (uint32_t k = 0; k < Ke; ++k) {
             const uint16_t a = A_KC ? Ae[(uint64_t)m * Ke + k] : Ae[(uint64_t)k * Me + m];

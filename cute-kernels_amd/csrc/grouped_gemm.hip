@@ -444,8 +444,8 @@ __global__ __launch_bounds__(NWM* NWN * 64) void grouped_gemm_kernel(const GemmA
         if (!prefetched) {
             if (!cur.fast) {
                 if constexpr (EPI == EPI_PLAIN) {
-                    scalar_tile<EL, A_KC, B_KC, BM, BN>(args.A + cur.off_a, args.B + cur.off_b, args.D + off_d, Me, Ne, Ke, m0, n0,
-                                                args.alpha, NT);
+                    scalar_tile<EL, A_KC, B_KC>(args.A + cur.off_a, args.B + cur.off_b, args.D + off_d, Me, Ne, Ke, m0,
+                                                Me - m0 < (uint32_t)BM ? Me : m0 + BM, n0, n_lim, args.alpha, NT);
                 }
                 cur = lookup(++round);
                 continue;

@@ -772,9 +772,8 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
         if (!streamed) {
             if (!cur.fast) {
                 if constexpr (EPI == EPI_PLAIN && !kGatherK) {  // (the gathered entry point admits only sizes without such tiles)
-                    // (TALL: up to the tile's last row; with A_KC the number of rows is no pitch)
-                    scalar_tile<EL, A_KC, B_KC, TALL ? kTallM : BM, BN>(args.A + cur.off_a, args.B + cur.off_b, args.D + off_d,
-                                                                        TALL ? m0 + cur.rows : Me, Ne, Ke, m0, n0, args.alpha, NT);
+                    scalar_tile<EL, A_KC, B_KC>(args.A + cur.off_a, args.B + cur.off_b, args.D + off_d, Me, Ne, Ke, m0, m0 + cur.rows,
+                                                n0, n_lim, args.alpha, NT);
                 }
                 cur = nxt;
                 nxt = lookup(round + 2);

@@ -137,10 +137,11 @@ def test_split_reduction(tB):
     assert torch.equal(*results)  # (integers below 2^24: exact in any order)
 
 
-@pytest.mark.parametrize("N,K", [(257, 72), (72, 67)])
-def test_element_wise_tiles(N, K):
-    """sizes whose rows are no multiple of 16 bytes take the element-wise path, a tall tile of it too"""
-    sizes = [257, 288, 289, 530, 3]
+@pytest.mark.parametrize("sizes", [[257, 288, 289, 530, 3], [40, 0, 3, 64, 17]])
+@pytest.mark.parametrize("N,K", [(257, 72), (72, 67), (501, 31)])
+def test_element_wise_tiles(N, K, sizes):
+    """sizes whose rows are no multiple of 16 bytes take the element-wise path: tall tiles, tiles in parts of their columns (some past
+    the last column), half-width tiles"""
     x, w, _ = _inputs(sizes, N, K, torch.bfloat16, (N, K))
     out = _fresh(sum(sizes), N, dtype=x.dtype)
     grouped_gemm_ragged_cuda(x, w[: len(sizes)], out, _u32(sizes), False, 0, N, K, False, True, None)
