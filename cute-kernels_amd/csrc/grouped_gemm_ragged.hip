@@ -1,4 +1,5 @@
 // Entry points of the grouped GEMM for launches whose groups differ in one dimension (the kernel: ragged_kernel.h).
+#include <algorithm>
 #include <type_traits>
 
 #include "ragged_kernel.h"
@@ -144,8 +145,16 @@ int launch_ragged_from_arrays(const void* A, const void* B, void* D, const uint3
 extern "C" {
 
 
-int64_t fma_grouped_gemm_ragged_workspace_bytes(int64_t R, int64_t E, int64_t N, int64_t K, int trans_b) {
+int64_t fma_grouped_gemm_ragged_split_bytes(int64_t R, int64_t E, int64_t N, int64_t K, int trans_b) {
     const uint32_t parts = fmahip::gemm::ragged::plan_split(R, E, N, K, trans_b != 0, E <= fmahip::gemm::ragged::kTallGroups).splits;
+    return parts > 1 ? R * N * 4 * (int64_t)parts : 0;
+}
+
+int64_t fma_grouped_gemm_ragged_workspace_bytes(int64_t R, int64_t E, int64_t N, int64_t K, int trans_b) {
+    // (enough for either kernel: callers may pad their groups with empty ones past the number that decides between them)
+    uint32_t parts = 1;
+    for (const bool tall : {false, true})
+        parts = std::max(parts, fmahip::gemm::ragged::plan_split(R, E, N, K, trans_b != 0, tall).splits);
     return parts > 1 ? R * N * 4 * (int64_t)parts : 0;
 }
 

@@ -48,6 +48,7 @@ SIGNATURES = {
     "fma_grouped_gemm": (_i32, [_p, _p, _p, _p, _p, _p, _i64, _i32, _i32, _f32, _i32, _p]),
     "fma_grouped_gemm_ragged": (_i32, [_p, _p, _p, _p, _p, _i64, _i32, _i64, _i64, _i64, _i32, _i32, _f32, _i32, _p]),
     "fma_grouped_gemm_ragged_workspace_bytes": (_i64, [_i64, _i64, _i64, _i64, _i32]),
+    "fma_grouped_gemm_ragged_split_bytes": (_i64, [_i64, _i64, _i64, _i64, _i32]),
     "fma_grouped_gemm_ragged_split": (
         _i32, [_p, _p, _p, _p, _p, _i64, _i32, _i64, _i64, _i64, _i32, _i32, _f32, _i64, _p, _i64, _i32, _p],
     ),

@@ -176,7 +176,7 @@ def grouped_gemm_ragged_cuda(
         # sums of a split reduction, where the launch has too few tiles for the compute units; owned by this call
         nbytes = 0
         if not vary_k and not is_A_transposed and A.numel() >= rows * K:
-            nbytes = lib.fma_grouped_gemm_ragged_workspace_bytes(rows, sizes.numel(), N, K, int(is_B_transposed))
+            nbytes = lib.fma_grouped_gemm_ragged_split_bytes(rows, sizes.numel(), N, K, int(is_B_transposed))
         workspace = None
         if nbytes:
             try:

@@ -221,6 +221,9 @@ int fma_grouped_gemm_ragged(const void* A, const void* B, void* D, const uint32_
  * call; workspace NULL, a workspace query of 0 or another form: exactly fma_grouped_gemm_ragged. Rows past the groups are
  * left as they are. */
 int64_t fma_grouped_gemm_ragged_workspace_bytes(int64_t rows, int64_t E, int64_t N, int64_t K, int trans_b);
+/* The bytes that such a launch takes of its workspace: 0 where it runs unsplit, at most the query above, which is enough for any E
+ * (another kernel takes more than 256 groups, and other launches pay a split on it). */
+int64_t fma_grouped_gemm_ragged_split_bytes(int64_t rows, int64_t E, int64_t N, int64_t K, int trans_b);
 int fma_grouped_gemm_ragged_split(const void* A, const void* B, void* D, const uint32_t* sizes, const void* bias, int64_t E,
                                   int vary, int64_t M, int64_t N, int64_t K, int trans_a, int trans_b, float alpha,
                                   int64_t rows, void* workspace, int64_t workspace_bytes, int dtype, void* stream);

@@ -39,7 +39,7 @@ def test_workspace_queries(lib):
 
 @pytest.mark.skipif(torch.cuda.is_available(), reason="a size that is accepted wrongly would be launched on host addresses")
 def test_split_workspace_is_what_the_launch_needs(lib):
-    """a byte less than the query says is refused: the query is for the parts that the launch takes, not for those of another kernel"""
+    """a byte less than the query of the bytes taken says is refused, and the query of the workspace is never less"""
     buf = ctypes.create_string_buffer(4096 + 16)
     p = (ctypes.addressof(buf) + 15) & ~15
     split = 0
@@ -47,7 +47,8 @@ def test_split_workspace_is_what_the_launch_needs(lib):
         for tB in (0, 1):
             for R in range(256, 9000, 256):
                 for E in (8, 300):
-                    nbytes = lib.fma_grouped_gemm_ragged_workspace_bytes(R, E, N, K, tB)
+                    nbytes = lib.fma_grouped_gemm_ragged_split_bytes(R, E, N, K, tB)
+                    assert nbytes <= lib.fma_grouped_gemm_ragged_workspace_bytes(R, E, N, K, tB)
                     if nbytes:
                         split += 1
                         args = (p, p, p, p, None, E, _lib.FMA_VARY_M, 0, N, K, 0, tB, 1.0, R, p, nbytes - 1, _lib.FMA_BF16, None)
