@@ -896,7 +896,8 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
         // WAIT: the s_waitcnt immediate in front of the barrier. The loads issued after the barrier are those of step
         // kt + 2: of this tile, or, in the last two steps, steps 0 and 1 of the next tile (or nothing).
         // SRC: which tile the loads issued in the step belong to: 0 the current one, 1 the next one (the loaders are aimed
-        // by the caller in both cases), 2 decided here (first steps of a tile, and the versions for tiles with few rows).
+        // by the caller in both cases), 2 decided here (first steps of a tile, and the versions for tiles with few rows), 3 the same
+        // in a step that fetches no rows past 256.
         auto step = [&](auto fa_c, auto wait_c, auto src_c, int stage, uint32_t kt) __attribute__((always_inline)) {
             constexpr int FA = decltype(fa_c)::value;
             constexpr int SRC = decltype(src_c)::value;
@@ -907,9 +908,11 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
             // gradients: 1498 -> 1440 us, hidden 4096, I 14336, E 8, k 2, 4096 tokens); in the NT layout 3 to 6 % slower, and in tiles of
             // few rows up to 6 %.
             constexpr bool kBFirst = X && !B_KC;
-            // The rows past 256 are fetched where the tile has them and in the steps whose loads may be for the next tile; the versions
-            // for few rows or no columns look whether this tile or the next has any.
-            constexpr bool kLoadX = TALL && (FA != RB || SRC != 0);
+            // The rows past 256 are fetched where the tile has them and in the steps whose loads may be for the next tile. The version
+            // for no columns looks whether this tile or the next has any; it has no matrix instructions to place loads between, as
+            // the others have: a branch in front of their ninth load would leave the other eight in a block of their own.
+            constexpr bool kLoadX = TALL && (FA > RB || FA == 0 || SRC == 1 || SRC == 2);
+            constexpr bool kEither = SRC >= 2;
             constexpr int NPH = 2 * PP;               // phases of the step
             constexpr int kReadsA = (A_KC ? 1 : 2) * AB, kReadsB = (B_KC ? 1 : 2);  // LDS reads per pair, per B fragment
             // On entry A buffer 0 and the B registers hold the fragments of the first phase.
@@ -921,15 +924,15 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
             // the A loads [i0, i1) of the step's load slot
             auto issue_a_part = [&](uint32_t k0, auto i0_c, auto i1_c) __attribute__((always_inline)) {
                 if constexpr (GATHER) {
-                    const bool of_next = SRC == 1 || (SRC == 2 && kt + 2u >= KT2);
-                    issue_a_gathered(stage, k0, (of_next ? round + 1u : round) & 1u, of_next ? g_bytes_nxt : g_full, SRC != 2, i0_c, i1_c);
+                    const bool of_next = SRC == 1 || (kEither && kt + 2u >= KT2);
+                    issue_a_gathered(stage, k0, (of_next ? round + 1u : round) & 1u, of_next ? g_bytes_nxt : g_full, !kEither, i0_c, i1_c);
                 } else {
                     issue_a(stage, k0, i0_c, i1_c);
                 }
             };
             auto issue_x_part = [&](uint32_t k0) __attribute__((always_inline)) {
                 if constexpr (kLoadX) {
-                    if (FA < RB && !extra_near) return;
+                    if (FA == 0 && !extra_near) return;
                     if constexpr (GATHER) issue_a_part(k0, std::integral_constant<int, 4>{}, std::integral_constant<int, 5>{});
                     else issue_x(stage, k0);
                 }
@@ -940,7 +943,7 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
             // throughout
             auto gk_step_offsets = [&](uint32_t k0) __attribute__((always_inline)) {
                 if constexpr (kGatherK) {
-                    constexpr bool kFromLds = FA != RB || SRC == 2;
+                    constexpr bool kFromLds = FA != RB || kEither;
                     gk_offsets(k0, lt_b.kdim, kFromLds ? gk_from_lds(stage) : gk_ring[stage], gk_v);
                 }
             };
@@ -953,7 +956,7 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
                     else gk_ring[stage] = gk_request(gk_first(kt + 4u), true);
                 }
             };
-            // what the loads issued in this step fetch: the K offset (returned) and, decided here (SRC == 2), whether the
+            // what the loads issued in this step fetch: the K offset (returned) and, decided here (kEither), whether the
             // loaders aim at the current tile's operands or the next one's
             auto aim_loads = [&]() __attribute__((always_inline)) -> uint32_t {
                 uint32_t k0;
@@ -1232,6 +1235,7 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
             using SrcCur = std::integral_constant<int, 0>;
             using SrcNext = std::integral_constant<int, 1>;
             using SrcEither = std::integral_constant<int, 2>;
+            using SrcEitherLow = std::integral_constant<int, 3>;
             auto k_loop = [&](auto fa_c) {
                 constexpr int FA = decltype(fa_c)::value;
                 load_a(fa_c, 0, 0, 0, 0);
@@ -1260,7 +1264,15 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
                         step(fa_c, WaitStep{}, SrcNext{}, 1, kt + 1);
                     }
                 } else {
-                    for (uint32_t kt = 2; kt < KT2; kt += 2) {
+                    uint32_t kt = 2;
+                    if constexpr (TALL && FA > 0) {
+                        // (a tile of few rows has none past 256: they are fetched for the next one, in the last two steps)
+                        for (; kt + 2u < KT2; kt += 2) {
+                            step(fa_c, WaitStep{}, SrcEitherLow{}, 0, kt);
+                            step(fa_c, WaitStep{}, SrcEitherLow{}, 1, kt + 1);
+                        }
+                    }
+                    for (; kt < KT2; kt += 2) {
                         step(fa_c, WaitStep{}, SrcEither{}, 0, kt);
                         step(fa_c, WaitStep{}, SrcEither{}, 1, kt + 1);
                     }

@@ -11,18 +11,15 @@ for every instantiation of ragged_gemm_kernel, that the instruction stream has t
 
  * every wait that is followed by a barrier and the eight operand loads of a K step allows exactly the number of newer
    instructions of a step in the loop (prefetch, request) or of a tile's first step (the epilogue's stores, prefetch, bias);
- * between the two barriers of a loop body of two K steps a wavefront issues the eight loads and exactly those extras (nine loads in
-   the version for tiles with rows past 256 of the tall kernels);
+ * between the two barriers of a loop body of two K steps a wavefront issues the eight loads and exactly those extras; in the tall
+   kernels both steps of a body issue eight loads or both nine, and there are four bodies with eight: the middle of the K loops for
+   eight, four, two and one row blocks, which fetch no rows past 256 (every other step does);
  * the cold start issues sixteen operand loads (tall kernels: eighteen), as many stand-in stores as an epilogue issues stores, and
    waits for all but the loads of the second step and the stores;
  * the three-stage loop of groups of at most 64 rows issues five loads per step and waits for all but five;
  * no instantiation touches scratch memory, and none contains a loop over the distinct values of an operand that the
    hardware wants in scalar registers (what the compiler generates around a vector-memory instruction whose descriptor or
    scalar offset it cannot prove to be the same in every lane: each costs a dozen instructions and a branch per use).
-
-The kernels that gather the rows of their first operand (forward form) read a row table between a step's barrier and its
-loads, which spreads a step over several basic blocks in ways that differ from version to version of the loop: for them
-only the loop bodies of two steps, the scratch memory and the loops over scalar operands are checked.
 """
 
 import os
@@ -92,8 +89,7 @@ def audit(asm_path: str) -> int:
         stores = EPI_STORES[epi]
         wait_step, wait_first = prefetch + request, stores + prefetch + bias
         tag = f"{el} A_KC={a_kc} B_KC={b_kc} epilogue={epi} reduction_varies={vary_k} bias={bias} gather={gather} tall={tall}"
-        found = {"step": 0, "first": 0, "body": 0, "cold": 0, "thin": 0}
-        gathers_rows = bool(gather and not vary_k)
+        found = {"step": 0, "first": 0, "body": 0, "eight": 0, "cold": 0, "thin": 0}
 
         def fail(what, block):
             nonlocal problems
@@ -106,7 +102,7 @@ def audit(asm_path: str) -> int:
             if "X" in blk:
                 fail("scratch access", blk)
             # waits in front of a barrier that the operand loads of a K step follow
-            for w, loads in ([] if gathers_rows else re.findall(r"w(\d+),\|(O+)", blk)):
+            for w, loads in re.findall(r"w(\d+),\|(O+)", blk):
                 n, count = int(w), len(loads)
                 if count in (8, 8 + tall):
                     if n == wait_step:
@@ -123,7 +119,10 @@ def audit(asm_path: str) -> int:
                     else:
                         fail(f"a three-stage step waits for all but {n}, expected 5", blk)
             # a loop body of two steps in one block: what is issued between its two barriers
-            for between in re.findall(r"\|(O{8}[^|]*?)w\d+,\|O{8}", blk):
+            for between, second in re.findall(r"\|(O{8}[^|]*?)w\d+,\|(O{8,})", blk):
+                if between.count("O") != len(second):
+                    fail(f"{between.count('O')} and {len(second)} operand loads in the two steps of a body", blk)
+                found["eight"] += len(second) == 8
                 issued = len(re.sub(r"w\d+,", "", between))
                 if issued in (8 + wait_step, 8 + tall + wait_step):
                     found["body"] += 1
@@ -132,21 +131,19 @@ def audit(asm_path: str) -> int:
                          + (f" or {9 + wait_step}" if tall else ""), blk)
             # the cold start: sixteen operand loads (the gathered kinds mix loads of row_index entries in), the stand-in
             # stores, the wait
-            cold = None if gathers_rows else re.search(r"((?:[OLp]|w\d+,)*O)(s+)w(\d+),\|", blk)
+            cold = re.search(r"((?:[OLp]|w\d+,)*O)(s+)w(\d+),\|", blk)
             if cold and cold.group(1).count("O") >= 16:
                 found["cold"] += 1
                 loads = 8 + tall
                 if cold.group(1).count("O") != 2 * loads or len(cold.group(2)) != stores or int(cold.group(3)) != loads + stores:
                     fail(f"cold start: {cold.group(1).count('O')} loads, {len(cold.group(2))} stores, wait {cold.group(3)}; "
                          f"expected {2 * loads}, {stores}, {loads + stores}", blk)
-        if gathers_rows:
-            if found["body"] == 0:
-                fail(f"expected shapes not found ({found})", "")
-        else:
-            if found["step"] == 0 or found["first"] == 0 or found["cold"] != 1:
-                fail(f"expected shapes not found ({found})", "")
-            if a_kc and found["thin"] == 0:
-                fail("no three-stage loop found", "")
+        if found["step"] == 0 or found["first"] == 0 or found["cold"] != 1:
+            fail(f"expected shapes not found ({found})", "")
+        if a_kc and found["thin"] == 0:
+            fail("no three-stage loop found", "")
+        if tall and (found["eight"] != 4 or found["body"] == 4):
+            fail(f"{found['eight']} of {found['body']} loop bodies with eight operand loads, expected 4 and some with nine", "")
         print(f"ok  {tag}: steps {found['step']}, first steps {found['first']}, two-step bodies {found['body']}, "
               f"three-stage steps {found['thin']}")
     return problems
