@@ -35,13 +35,14 @@
 //    operands, above all of B (a tile of 8 rows takes 88 % of a full one's time), so what counts is how many tiles stream a
 //    panel of B: experts of 256 or 512 +- 20 rows, as an even routing makes them, take one or two tiles instead of every other one
 //    a nearly empty one more. A group gets as few tiles as 288 rows allow, of which as few as its rows need are tall (a tall
-//    step costs 6 % more loads and 12 % more matrix instructions). Same sums in the same order: same bits. Products of evenly
+//    step costs 6 % more loads and 12 % more matrix instructions), in launches where that saves rounds of tiles (most_rows), by the
+//    sizes in device memory. Same sums in the same order: same bits. Products of evenly
 //    routed layers, 256-row tiles -> tall (us): hidden 4096, I 1536, E 128, k 8, 4096 tokens 984 -> 945, 541 -> 500 (up, down), input
 //    gradients 951 -> 852, 595 -> 522; 8192 tokens 1570 -> 1432, 858 -> 801, 1536 -> 1416, 924 -> 806; hidden 4096, I 14336, E 8,
 //    k 2, 4096 tokens 1600 -> 1510, 1004 -> 749, 1996 -> 1460, 900 -> 842; hidden 2048, I 8192, 1021 tokens 228 -> 159 (up); rows that
 //    leave the number of tiles as it is (94 to 156 an expert) 0.99 to 1.01 of the time.
 //  * The last, partial round of tiles of a tall kernel is cut into 2 or 4 parts of their columns where there are workgroups for them: the
-//    loads of B shrink with the columns, and the round takes 0.65 to 0.75 of a whole one's time. Products of 384 tiles (hidden 2880,
+//    loads of B shrink with the columns, and the round takes 0.8 to 0.9 of a whole one's time. Products of 384 tiles (hidden 2880,
 //    I 2880, E 32, k 4, 2000 tokens) 191 -> 179 us (down), 331 -> 314 us (input gradient); of 320 (hidden 2048, I 8192, E 8, k 2, 5000
 //    tokens) 393 -> 364 us.
 #pragma once
@@ -116,6 +117,18 @@ struct Feed {
 // columns, as many as there are workgroups for.
 __device__ __forceinline__ uint32_t parts_of_tail(uint32_t rest, uint32_t g) {
     return rest * 4u <= g ? 2u : (rest * 2u <= g ? 1u : 0u);
+}
+
+// The time of `units` tiles on `g` workgroups in rounds of 256-row tiles, `tall` of them with rows past 256: such a tile takes a seventh
+// more (8 groups of about 300 rows, 2048 x 8192: 211 us with one or more of them against 244 us), the last, partial round 0.87 of a
+// whole one in parts of its columns and on its own 0.85 (NN, 64 tiles of 2048 x 16384: 394 -> 330 us). In the NT layout a launch of at
+// most half as many tiles as workgroups is never cut.
+template <bool PARTS, bool B_KC>
+__device__ __forceinline__ float rounds_of(uint32_t units, uint32_t tall, uint32_t g) {
+    const uint32_t whole = units / g, rest = units - whole * g;
+    float last = rest ? 1.0f : 0.0f;
+    if (PARTS && rest && parts_of_tail(rest, g)) last = whole ? 0.87f : (B_KC ? 1.0f : 0.85f);
+    return (float)whole + last + 0.14f * (float)((tall + g - 1) / g);
 }
 
 // Names an accumulator value as one 16-register value (no instruction, no ordering).
@@ -234,7 +247,12 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
     constexpr uint32_t kTileN = kGlu ? BN / 2 : BN;  // columns of the tile grid one tile covers
     const uint32_t n_span = kGlu ? Ne / 2 : Ne;      // columns the tile grid runs over
     bool narrow = false;
-    auto row_tiles = [&](uint32_t m) -> uint32_t { return (m + kMostRows - 1) / kMostRows; };
+    uint32_t most_rows = kMostRows;  // rows of a tile of this launch (TALL: decided below)
+    auto row_tiles = [&](uint32_t m) -> uint32_t { return (m + most_rows - 1) / most_rows; };
+    // how many of a group's tiles have rows past 256
+    auto tall_tiles = [&](uint32_t m, uint32_t tiles) -> uint32_t {
+        return m > tiles * (uint32_t)BM ? (m - tiles * (uint32_t)BM + (uint32_t)(kTallM - BM) - 1) / (uint32_t)(kTallM - BM) : 0u;
+    };
     auto tiles_of = [&](uint32_t m) -> uint32_t {
         if (m == 0 || Ne == 0) return 0;
         const uint32_t width = (kCanNarrow && narrow && m <= 64u) ? kTileN / 2 : kTileN;
@@ -267,25 +285,40 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
         __syncthreads();
     }
 
-    if constexpr (kCanNarrow) {
-        // half-width column tiles for groups of at most 64 rows when that fills the workgroups better (grouped_gemm.hip)
-        uint32_t mine_small = 0, mine_other = 0;
-        for (uint32_t e = tid; e < E; e += NT) {
-            const uint32_t m = group_m(e), t = tiles_of(m);
-            if (m <= 64u) mine_small += t;
-            else mine_other += t;
+    if constexpr (TALL || kCanNarrow) {
+        // (every wavefront sums by itself: no barrier, and no atomics, which the compiler makes a loop over the lanes)
+        uint32_t few = 0, sums[3] = {0u, 0u, 0u};  // groups of at most 64 rows; tiles of 256 rows, tiles of up to 288, tall ones of these
+        for (uint32_t e = lane; e < E; e += 64u) {
+            const uint32_t m = group_m(e), tiles = (m + (uint32_t)kTallM - 1) / (uint32_t)kTallM;
+            few += m > 0u && m <= 64u ? 1u : 0u;
+            sums[0] += (m + (uint32_t)BM - 1) / (uint32_t)BM;
+            sums[1] += tiles;
+            sums[2] += tall_tiles(m, tiles);
         }
-        uint32_t* const total = reinterpret_cast<uint32_t*>(s_a0);
-        if (tid < 2) total[tid] = 0;
-        __syncthreads();
-        if (mine_small) atomicAdd(total, mine_small);
-        if (mine_other) atomicAdd(total + 1, mine_other);
-        __syncthreads();
-        const uint32_t t_small = uniform(total[0]), t_other = uniform(total[1]), g = gridDim.x;
-        const uint32_t rounds = (t_small + t_other + g - 1) / g;
-        const uint32_t half_rounds = (2 * t_small + g - 1) / g;
-        narrow = t_other == 0 ? half_rounds * 10u <= 2u * rounds * 9u : (t_small + t_other) * 2u <= g;
-        __syncthreads();
+#pragma unroll
+        for (int d = 32; d > 0; d >>= 1) {
+            few += (uint32_t)__shfl_xor((int)few, d, 64);
+#pragma unroll
+            for (int i = 0; i < 3; ++i) sums[i] += (uint32_t)__shfl_xor((int)sums[i], d, 64);
+        }
+        const uint32_t columns = (n_span + kTileN - 1) / kTileN, g = gridDim.x;
+        if constexpr (TALL) {
+            // Tiles of up to 288 rows where they save more rounds than their longer K steps cost. 256-row tiles / tall ones wherever a
+            // group has more than 256 rows, us, randomly routed: 2048 x 8192, E 8, 300, 600 and 800 rows a group (one round either way:
+            // not taken) 211 / 244, 213 / 239, 207 / 237, 1000 rows (two rounds / one) 391 / 227; 2880 x 2880, E 32, 300 rows (three /
+            // three) 238 / 262, 256 rows 261 / 212; 4096 x 1536, E 128, 256 rows (12 / 9) 559 / 512; 2048 x 1408, E 64, 300 rows 173 / 189.
+            const uint32_t per = columns * (kSplit ? args.splits : 1u);
+            const float low = rounds_of<kTail, B_KC>(uniform(sums[0]) * per, 0u, g);
+            const float high = rounds_of<kTail, B_KC>(uniform(sums[1]) * per, uniform(sums[2]) * per, g);
+            most_rows = uniform(high < low ? (uint32_t)kTallM : (uint32_t)BM);
+        }
+        if constexpr (kCanNarrow) {
+            // half-width column tiles for groups of at most 64 rows when that fills the workgroups better (grouped_gemm.hip)
+            const uint32_t t_small = uniform(few) * columns, t_other = uniform(sums[most_rows == (uint32_t)BM ? 0 : 1]) * columns - t_small;
+            const uint32_t rounds = (t_small + t_other + g - 1) / g;
+            const uint32_t half_rounds = (2 * t_small + g - 1) / g;
+            narrow = t_other == 0 ? half_rounds * 10u <= 2u * rounds * 9u : (t_small + t_other) * 2u <= g;
+        }
     }
 
     // ---- group table, built by wavefront 0: exclusive prefix of tiles over the order above, exclusive prefix of the
@@ -408,7 +441,7 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
         t.pf_r = (local % band) % band_m;
         t.pf_c = nt & 3u;
         // TALL: the first tiles of the group are 288 rows high, as many as its rows need; the others 256
-        const uint32_t past = TALL && t.Me > tiles_m * (uint32_t)BM ? (t.Me - tiles_m * (uint32_t)BM + 31u) / 32u : 0u;
+        const uint32_t past = TALL ? tall_tiles(t.Me, tiles_m) : 0u;
         const uint32_t height = mt < past ? kMostRows : (uint32_t)BM;
         t.m0 = mt * (uint32_t)BM + (mt < past ? mt : past) * (kMostRows - (uint32_t)BM);
         t.rows = t.Me - t.m0 < height ? t.Me - t.m0 : height;
