@@ -9,33 +9,32 @@ namespace gemm {
 namespace ragged {
 
 // ---- split reduction ---------------------------------------------------------------------------------------------
-// A launch with fewer tiles than compute units leaves the others idle for the whole reduction: the second projection of
-// 1021 tokens on 8 experts (2048 x 8192) is 64 tiles of 128 K steps, 229 us. With the reduction in four parts (256 units of
-// 32 steps, fp32 sums to memory and one pass over them) it takes 123 us. More of the same (unsplit -> parts):
-//   NT 2048 x 8192, 8 groups of 128 / 256 / 500 rows         190 -> 94 us (4), 229 -> 123 us (4), 212 -> 153 us (2)
-//   NT 4096 x 14336, 8 groups of 128 / 256 rows              361 -> 230 us (2), 411 -> 285 us (2)
-//   NN 2048 x 16384, 8 groups of 128 / 256 / 500 rows        299 -> 134 us (4), 349 -> 169 us (4), 363 -> 262 us (2)
-//   NN 4096 x 28672, 8 groups of 128 / 256 rows              567 -> 379 us (2), 682 -> 485 us (2)
+// A launch with fewer tiles than compute units leaves the others idle for the whole reduction: the second projection of 800 tokens on
+// 8 experts (2048 x 8192) is 64 tiles of 128 K steps, 239 us. With the reduction in three parts (192 units of 44 steps, fp32 sums to
+// memory and one pass over them) it takes 130 us. More of the same, 8 groups, randomly routed (unsplit -> parts):
+//   NT 2048 x 8192, 150 / 256 / 400 / 512 rows a group       229 -> 124 us (3), 239 -> 143 us (3), 230 -> 165 us (2), 235 -> 180 us (2)
+//   NT 4096 x 14336, 100 / 256 / 600 rows                    382 -> 252 us (2), 411 -> 291 us (2), 678 -> 625 us (2)
+//   NN 2048 x 16384, 150 / 256 / 400 / 512 rows              321 -> 158 us (4), 352 -> 202 us (3), 345 -> 246 us (2), 388 -> 262 us (2)
+//   NN 4096 x 28672, 100 / 256 rows                          576 -> 392 us (4), 701 -> 519 us (4)
 //
 // How many parts: the number with the least predicted time, rounds of tiles times (K steps + a tile's fixed cost) or the
 // weights at the rate they stream, plus the traffic of the sums. The row counts lie in device memory, so the number of tiles
 // is the expected one for evenly loaded groups. Parts have at least kSplitMinSteps steps, the sums at most kSplitMaxBytes (they
-// stay in the last-level cache), and a split has to promise a tenth less than none. Groups of few rows run the three-stage
+// stay in the last-level cache), and a split has to promise a twentieth less than none. Groups of few rows run the three-stage
 // loop, whose steps are shorter, without a split on half-width tiles in the NT layout: NT 4096 x 14336 on 8 groups of 32 rows
 // streams its weights in 176 us as it is and would take 184 us in two parts.
 // Tall tiles (TALL in ragged_kernel.h): a round takes 1.6 to 2.0 us per K step of its tiles, most when every compute unit is busy and
-// streams weights of its own, and a partial last round, in parts of its columns, 0.65 to 0.75 of that behind whole rounds and 0.8 to 0.95 alone. The
-// tiles of a group follow from the spread of a random routing (a standard deviation of the root of the mean): 8 groups of 256 or
-// 512 rows are 8 or 16 tiles high, not 12 or 20 (and three parts of 64 tiles of 128 steps, 121 us, are better than four, 123 us and 165
-// us in the sixth of the launches in which an expert is past 288 rows). That ends the split of [8 x 500 rows, 4096 x 14336] (420 us as 256 tiles, 468 us
-// in two parts, 556 us in three parts of 256-row tiles) and of [8 x 2000 rows, 2048 x 8192] (451 us, 563 us).
-// Uneven loads make fewer tiles, which a split helps the more; where they happen to fill the compute units exactly once as they are, the
-// sums are the price. Training steps without -> with splits on 256-row tiles: 2048 tokens, hidden 4096, I 14336, E 8, k 2, evenly
-// 5100 -> 4630 us, all on two experts 3870 -> 3990 us; 4000 tokens, hidden 2048, I 8192: 2775 -> 2627 and 2157 -> 2225 us; 512 and 1021
-// tokens gain either way (2219 -> 1779 and 2727 -> 2478 us, 886 -> 565 us at 256 tokens of the second shape).
+// streams weights of its own, and a partial last round costs what rounds_of there says. The tiles of a group follow from the spread of a
+// random routing (a standard deviation of the root of the mean): 8 groups of 256 or 512 rows are 8 or 16 tiles high, not 12 or 20. That
+// ends the split of [8 x 512 rows, 4096 x 14336] (440 us, two parts 485).
+// Routings are less even than random ones, too, and what fills the compute units exactly once is worth little if one more row tile spoils
+// it: one launch in five (kUneven) is taken to have one. 8 groups of 200 rows, 2048 x 8192 and 2048 x 16384 in four parts (256 units)
+// take 153 and 173 us, but with odds of the experts as their rank to the -0.7 (9 row tiles) 188 and 256; in three parts 130 and 187, 132 and
+// 193. 4096 x 28672, 256 rows: 487 and 721 us in two parts, 519 and 607 in four. Over 540 launches (six shapes, 24 to 1000 rows a group, three routings)
+// the parts taken cost 0.7 % (random), 2.9 and 3.6 % (two uneven ones) more than the best number would; without the line 0.7, 3.7 and 4.6 %.
 constexpr double kStepUs = 1.45, kTallStepUs = 1.55, kFullStepUs = 0.4, kThinStepUs[2] = {1.1, 0.75}, kTileSteps = 6.0, kThinRows = 48.0;
-constexpr double kTailCost = 0.7, kLoneTailCost = 0.85, kWeightBytesPerUs = 5.5e6;
-constexpr double kReduceUs = 4.0, kReduceBytesPerUs = 4.5e6, kSplitGain = 0.9;
+constexpr double kTailCost = 0.87, kLoneTailCost = 0.85, kUneven = 0.2, kWeightBytesPerUs = 5.5e6;
+constexpr double kReduceUs = 4.0, kReduceBytesPerUs = 4.5e6, kSplitGain[2] = {0.9, 0.95};  // [tall]
 constexpr uint32_t kSplitMinSteps = 24;
 constexpr int64_t kSplitMaxBytes = 256ll << 20;
 SplitPlan plan_split(int64_t R, int64_t E, int64_t N, int64_t K, bool b_kc, bool tall) {
@@ -63,7 +62,7 @@ SplitPlan plan_split(int64_t R, int64_t E, int64_t N, int64_t K, bool b_kc, bool
         const double whole = std::floor(units / cus), rest = units - whole * cus;
         double step_us = thin ? kThinStepUs[b_kc] : kStepUs;
         if (tall && !thin) {
-            const bool in_parts = parts == 1 && rest > 0.5 && 2.0 * rest <= cus;
+            const bool in_parts = parts == 1 && rest > 0.5 && 2.0 * rest <= cus && (whole > 0.0 || !b_kc);
             if (in_parts) rounds = whole + (whole > 0.0 ? kTailCost : kLoneTailCost);
             step_us = kTallStepUs + (in_parts ? kFullStepUs : kFullStepUs * std::min(1.0, units / cus));
         }
@@ -71,14 +70,13 @@ SplitPlan plan_split(int64_t R, int64_t E, int64_t N, int64_t K, bool b_kc, bool
         const double sums = parts > 1 ? kReduceUs + (double)R * N * (8.0 * parts + 2.0) / kReduceBytesPerUs : 0.0;
         return std::max(products, weights_us) + sums;
     };
-    // tall: between the two numbers of row tiles about the expected one, by how likely they are. (What fills the compute units
-    // exactly once is worth little if one group in ten launches spoils it.)
-    const double low = tall ? std::floor(row_tiles) : row_tiles, more = row_tiles - low;
+    // tall: between the two numbers of row tiles about the expected one, by how likely they are
+    const double low = tall ? std::floor(row_tiles) : row_tiles, more = tall && !thin ? std::max(row_tiles - low, kUneven) : row_tiles - low;
     auto us = [&](uint32_t parts, uint32_t steps) {
         const double t = us_of(low * columns, parts, steps);
         return more > 0.0 ? (1.0 - more) * t + more * us_of((low + 1.0) * columns, parts, steps) : t;
     };
-    double best_us = us(1, all) * kSplitGain;
+    double best_us = us(1, all) * kSplitGain[tall];
     for (uint32_t parts = 2; parts * kSplitMinSteps <= all && parts <= 32; ++parts) {
         const uint32_t steps = ((all + parts - 1) / parts + 1u) & ~1u;
         const uint32_t used = (all + steps - 1) / steps;

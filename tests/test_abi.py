@@ -56,6 +56,18 @@ def test_split_workspace_is_what_the_launch_needs(lib):
     assert split > 50
 
 
+@pytest.mark.parametrize("rows,N,K,tB,parts", [
+    (150, 2048, 8192, 1, 3), (200, 2048, 8192, 1, 3), (256, 2048, 8192, 1, 3), (512, 2048, 8192, 1, 2), (600, 2048, 8192, 1, 1),
+    (256, 4096, 14336, 1, 2), (400, 4096, 14336, 1, 1), (512, 4096, 14336, 1, 1), (600, 4096, 14336, 1, 2),
+    (150, 2048, 16384, 0, 4), (256, 2048, 16384, 0, 3), (256, 4096, 28672, 0, 4), (600, 4096, 28672, 0, 2),
+])  # fmt: skip
+@pytest.mark.skipif(torch.cuda.is_available(), reason="the plan is for 256 compute units where there is no device to ask")
+def test_parts_of_a_split(lib, rows, N, K, tB, parts):
+    """the best number of parts for 8 randomly routed groups, or one within 10 % of it that uneven routing does not spoil"""
+    nbytes = lib.fma_grouped_gemm_ragged_split_bytes(8 * rows, 8, N, K, tB)
+    assert nbytes == (8 * rows * N * 4 * parts if parts > 1 else 0)
+
+
 def _err(lib) -> str:
     return lib.fma_last_error_string().decode()
 
