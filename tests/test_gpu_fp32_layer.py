@@ -154,8 +154,12 @@ def test_what_takes_the_general_path(case, monkeypatch):
         own = moe.c_fc.cuda_forward
         moe.c_fc.cuda_forward = lambda **kw: (seen.append(1), own(**kw))[1]
     elif case == "autocast":
-        context = torch.autocast("cuda", enabled=True, dtype=torch.float32)
+        context = torch.autocast("cuda", dtype=torch.bfloat16)
         seen.append(1)
+        moe.fuse_swiglu_backward = False
+        with context:
+            expect = moe(x, kernel_backend=KernelBackend.cuda)
+        moe.fuse_swiglu_backward = True
     elif case == "misaligned":
         x = torch.cat([x.new_zeros(1), x.reshape(-1)])[1:].view(20, 64)
         seen.append(1)
@@ -166,9 +170,9 @@ def test_what_takes_the_general_path(case, monkeypatch):
         moe.gate.weight = torch.nn.Parameter(_layer(8, 2, 64, 32).gate.weight.detach().clone())
     with context:
         got = moe(x, kernel_backend=KernelBackend.cuda)
-    assert seen and (calls == [] or (case == "autocast" and not torch.is_autocast_enabled("cuda")))
+    assert seen and calls == []
     for a, b in zip(got, expect):
-        assert float((a.float() - b).norm() / b.norm()) < (TOL if case != "autocast" else 1e-2)
+        assert a.dtype == b.dtype and float((a.float() - b.float()).norm() / b.float().norm()) < TOL
 
 
 @pytest.mark.parametrize("strided", ["tokens", "gate"])
