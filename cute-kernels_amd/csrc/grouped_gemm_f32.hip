@@ -22,6 +22,7 @@ namespace fmahip {
 namespace gemm_f32 {
 namespace {
 
+typedef __attribute__((ext_vector_type(4))) float f32x4;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 
 constexpr int kThreads = 256;
@@ -222,9 +223,10 @@ __device__ __forceinline__ void run(const Args& args, const Table& table, float*
                     const uint32_t n = n0 + wn * (S / 2) + j * 32 + q * 8 + (lane >> 5) * 4;
                     float* dst = De + (uint64_t)m * Ne + n;
                     if (n + 3 < Ne && (reinterpret_cast<uintptr_t>(dst) & 15u) == 0) {
-                        float4 v = {alpha * acc[i][j][q * 4 + 0], alpha * acc[i][j][q * 4 + 1], alpha * acc[i][j][q * 4 + 2],
-                                    alpha * acc[i][j][q * 4 + 3]};
-                        *reinterpret_cast<float4*>(dst) = v;
+                        // (one value of a vector type: of four floats the compiler sank the last one's store into the other branch's,
+                        // a 12- and a 4-byte store for each of these)
+                        *reinterpret_cast<f32x4*>(dst) = f32x4{alpha * acc[i][j][q * 4 + 0], alpha * acc[i][j][q * 4 + 1],
+                                                               alpha * acc[i][j][q * 4 + 2], alpha * acc[i][j][q * 4 + 3]};
                     } else {
 #pragma unroll
                         for (int x = 0; x < 4; ++x)

@@ -20,6 +20,9 @@ for every instantiation of ragged_gemm_kernel, that the instruction stream has t
  * no instantiation touches scratch memory, and none contains a loop over the distinct values of an operand that the
    hardware wants in scalar registers (what the compiler generates around a vector-memory instruction whose descriptor or
    scalar offset it cannot prove to be the same in every lane: each costs a dozen instructions and a branch per use).
+
+The kernels of csrc/grouped_gemm_f32.hip store four results as 16 bytes: none of their stores may be of 12 bytes, which is what the
+compiler makes of four separate values next to an element-wise branch, with a store of the fourth shared by both.
 """
 
 import os
@@ -149,6 +152,16 @@ def audit(asm_path: str) -> int:
     return problems
 
 
+def audit_f32(asm_path: str) -> int:
+    text = open(asm_path).read()
+    whole, cut = len(re.findall(r"\bglobal_store_dwordx4\b", text)), len(re.findall(r"\bglobal_store_dwordx3\b", text))
+    if whole == 0 or cut:
+        print(f"PROBLEM fp32 products: {whole} stores of 16 bytes, {cut} of 12")
+        return 1
+    print(f"ok  fp32 products: {whole} stores of 16 bytes")
+    return 0
+
+
 def main() -> int:
     if len(sys.argv) > 1:
         return audit(sys.argv[1])
@@ -159,6 +172,9 @@ def main() -> int:
             path = os.path.join(tmp, os.path.basename(source) + ".s")
             compile_to_assembly(source, path)
             problems += audit(path)
+        path = os.path.join(tmp, "f32.s")
+        compile_to_assembly(os.path.join(HERE, "csrc", "grouped_gemm_f32.hip"), path)
+        problems += audit_f32(path)
     return problems
 
 
