@@ -250,20 +250,29 @@ __global__ __launch_bounds__(kThreads) void grouped_gemm_f32_kernel(const Args a
         const uint32_t lane = threadIdx.x;
         auto tiles_of = [](uint64_t M, uint64_t N, uint32_t S) { return (uint32_t)(((M + S - 1) / S) * ((N + S - 1) / S)); };
         uint32_t n_large = 0, n_small = 0;
+        float k_sum = 0.0f;  // of the large tiles' reductions
         for (uint32_t e = lane; e < args.E; e += 64) {
-            n_large += tiles_of(args.M_arr[e], args.N_arr[e], Large::S);
+            const uint32_t t = tiles_of(args.M_arr[e], args.N_arr[e], Large::S);
+            n_large += t;
+            k_sum += (float)t * (float)args.K_arr[e];
             n_small += tiles_of(args.M_arr[e], args.N_arr[e], Small::S);
         }
 #pragma unroll
         for (int d = 32; d > 0; d >>= 1) {
             n_large += (uint32_t)__shfl_xor((int)n_large, d, 64);
             n_small += (uint32_t)__shfl_xor((int)n_small, d, 64);
+            k_sum += __shfl_xor(k_sum, d, 64);
         }
-        // The compute unit with the most tiles ends last; a small tile counts as a quarter of a large one and a fifth more: 256 large
-        // tiles, one per compute unit, beat 1024 small ones by 5 to 20 % (39 against 41 us, 19 against 23), 272 lose by a quarter (347
-        // against 256 us).
-        const uint64_t cus = gridDim.x / 2u;
-        const bool small = (n_small + cus - 1) / cus * 6u < (n_large + cus - 1) / cus * 20u;
+        // The compute unit with the most tiles ends last. A large tile takes as long as 48 more k of its reduction on top of that, a small
+        // one a little less than a third, and of the fixed part not much less than a half: 256 large tiles, one per compute unit, beat 1024
+        // small ones by 5 to 20 % over long reductions (39 against 41 us, 19 against 23), 272 lose by a quarter (347 against 256 us); over 7 to
+        // 30 rows weight gradients [576, 576] of 8, 64 and 100 experts take 12, 41 and 57 us on large tiles and 14, 63 and 97 on
+        // small ones. Over 420 products of all kinds (1 to 200 groups, reductions of 1 to 4096) the tiles taken cost 0.4 % more than the
+        // better ones; a third whatever the reduction cost 1.5 %, and up to 1.6 times what large tiles alone had.
+        // (every workgroup forms the same sums in the same order: all of them choose alike)
+        const uint32_t cus = gridDim.x / 2u;
+        const float k_mean = k_sum / (float)(n_large > 0u ? n_large : 1u);
+        const bool small = (float)((n_small + cus - 1) / cus) * (20.0f + 0.31f * k_mean) < (float)((n_large + cus - 1) / cus) * (48.0f + k_mean);
         uint32_t tiles = 0;
         uint64_t oa = 0, ob = 0, od = 0;
         for (uint32_t base = 0; base < args.E; base += 64) {

@@ -20,6 +20,9 @@ SIZES = [
     ([64, 65, 1, 127], [64, 63, 129, 1], [32, 33, 31, 64]),
     ([3, 128], [5, 192], [7, 100]),
     ([1], [1], [1]),
+    # 384 large tiles, 1536 small ones: large over few k, small over many
+    ([767] * 16, [511] * 16, [6] * 15 + [1]),
+    ([767] * 16, [511] * 16, [300] * 15 + [299]),
 ]
 
 
