@@ -15,7 +15,7 @@ namespace ragged {
 //   NT 2048 x 8192, 150 / 256 / 400 / 512 rows a group       229 -> 124 us (3), 239 -> 143 us (3), 230 -> 165 us (2), 235 -> 180 us (2)
 //   NT 4096 x 14336, 100 / 256 / 600 rows                    382 -> 252 us (2), 411 -> 291 us (2), 678 -> 625 us (2)
 //   NN 2048 x 16384, 150 / 256 / 400 / 512 rows              321 -> 158 us (4), 352 -> 202 us (3), 345 -> 246 us (2), 388 -> 262 us (2)
-//   NN 4096 x 28672, 100 / 256 rows                          576 -> 392 us (4), 701 -> 519 us (4)
+//   NN 4096 x 28672, 100 / 256 rows                          576 -> 375 us (2), 701 -> 519 us (4)
 //
 // How many parts: the number with the least predicted time, rounds of tiles times (K steps + a tile's fixed cost) or the
 // weights at the rate they stream, plus the traffic of the sums. The row counts lie in device memory, so the number of tiles
@@ -28,10 +28,11 @@ namespace ragged {
 // random routing (a standard deviation of the root of the mean): 8 groups of 256 or 512 rows are 8 or 16 tiles high, not 12 or 20. That
 // ends the split of [8 x 512 rows, 4096 x 14336] (440 us, two parts 485).
 // Routings are less even than random ones, too, and what fills the compute units exactly once is worth little if one more row tile spoils
-// it: one launch in five (kUneven) is taken to have one. 8 groups of 200 rows, 2048 x 8192 and 2048 x 16384 in four parts (256 units)
-// take 153 and 173 us, but with odds of the experts as their rank to the -0.7 (9 row tiles) 188 and 256; in three parts 130 and 187, 132 and
-// 193. 4096 x 28672, 256 rows: 487 and 721 us in two parts, 519 and 607 in four. Over 540 launches (six shapes, 24 to 1000 rows a group, three routings)
-// the parts taken cost 0.7 % (random), 2.9 and 3.6 % (two uneven ones) more than the best number would; without the line 0.7, 3.7 and 4.6 %.
+// it: where a group of 2.5 times the mean rows has a second tile, one launch in five (kUneven) is taken to have one. 8 groups of 200 rows,
+// 2048 x 8192 and 2048 x 16384 in four parts (256 units) take 153 and 173 us, but with odds of the experts as their rank to the -0.7 (9 row
+// tiles) 188 and 256; in three parts 130 and 187, 132 and 193. 4096 x 28672, 256 rows: 487 and 721 us in two parts, 519 and 607 in four. Over
+// 1380 launches (seven shapes, 24 to 1000 rows a group, three routings) the parts taken cost 2.1 % (random), 4.0 and 4.6 % (two uneven ones)
+// more than the best number would; without the line 2.0, 5.3 and 5.9 %.
 constexpr double kStepUs = 1.45, kTallStepUs = 1.55, kFullStepUs = 0.4, kThinStepUs[2] = {1.1, 0.75}, kTileSteps = 6.0, kThinRows = 48.0;
 constexpr double kTailCost = 0.87, kLoneTailCost = 0.85, kUneven = 0.2, kWeightBytesPerUs = 5.5e6;
 constexpr double kReduceUs = 4.0, kReduceBytesPerUs = 4.5e6, kSplitGain[2] = {0.9, 0.95};  // [tall]
@@ -71,7 +72,8 @@ SplitPlan plan_split(int64_t R, int64_t E, int64_t N, int64_t K, bool b_kc, bool
         return std::max(products, weights_us) + sums;
     };
     // tall: between the two numbers of row tiles about the expected one, by how likely they are
-    const double low = tall ? std::floor(row_tiles) : row_tiles, more = tall && !thin ? std::max(row_tiles - low, kUneven) : row_tiles - low;
+    const double low = tall ? std::floor(row_tiles) : row_tiles, uneven = tall && !thin && mean * 2.5 > kTallM ? kUneven : 0.0;
+    const double more = std::max(row_tiles - low, uneven);
     auto us = [&](uint32_t parts, uint32_t steps) {
         const double t = us_of(low * columns, parts, steps);
         return more > 0.0 ? (1.0 - more) * t + more * us_of((low + 1.0) * columns, parts, steps) : t;

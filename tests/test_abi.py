@@ -58,8 +58,8 @@ def test_split_workspace_is_what_the_launch_needs(lib):
 
 @pytest.mark.parametrize("rows,N,K,tB,parts", [
     (150, 2048, 8192, 1, 3), (200, 2048, 8192, 1, 3), (256, 2048, 8192, 1, 3), (512, 2048, 8192, 1, 2), (600, 2048, 8192, 1, 1),
-    (256, 4096, 14336, 1, 2), (400, 4096, 14336, 1, 1), (512, 4096, 14336, 1, 1), (600, 4096, 14336, 1, 2),
-    (150, 2048, 16384, 0, 4), (256, 2048, 16384, 0, 3), (256, 4096, 28672, 0, 4), (600, 4096, 28672, 0, 2),
+    (70, 4096, 14336, 1, 2), (256, 4096, 14336, 1, 2), (400, 4096, 14336, 1, 1), (512, 4096, 14336, 1, 1), (600, 4096, 14336, 1, 2),
+    (150, 2048, 16384, 0, 4), (256, 2048, 16384, 0, 3), (100, 4096, 28672, 0, 2), (256, 4096, 28672, 0, 4), (600, 4096, 28672, 0, 2),
 ])  # fmt: skip
 @pytest.mark.skipif(torch.cuda.is_available(), reason="the plan is for 256 compute units where there is no device to ask")
 def test_parts_of_a_split(lib, rows, N, K, tB, parts):
