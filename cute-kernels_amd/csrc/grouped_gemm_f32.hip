@@ -11,7 +11,7 @@
 // Workgroups are persistent and find their tiles in a per-workgroup prefix table of the groups' tile counts, like the
 // 16-bit kernel.
 // Against 128 x 128 tiles alone, fetched and staged element by element (us; layer of hidden 256, I 512, E 8, k 2, 512 tokens): up 30 ->
-// 17, down 50 -> 18, input gradients 102 -> 38 and 31 -> 14, weight gradients 23 -> 16 and 22 -> 12; hidden 2048, I 4096, 4096 tokens
+// 17, down 50 -> 18, input gradients 102 -> 38 and 31 -> 13, weight gradients 23 -> 16 and 22 -> 11; hidden 2048, I 4096, 4096 tokens
 // (large tiles): 2660 -> 2377, 1521 -> 1379, 3415 -> 3030, 1533 -> 1398, 2680 -> 2669, 1346 -> 1339 (116 TFLOP/s).
 #include <type_traits>
 

@@ -1,8 +1,8 @@
 // The router of an fp32 layer in one pass: logits = x @ Wg^T on the fp32 matrix instruction, top-k, softmax over the k kept logits and
 // the choices counted per 16 tokens; and the backward of the top-k and softmax. fp32 layers are small, so both are bound by latency:
 // what counts is that the product, the selection (two launches in ATen), the softmax and, in the backward, its gradient, the scatter
-// and the sum with the logits' own gradient are one launch each. At 512 tokens, hidden 256, E 8, k 2: 8.2 us
-// against 27 us of the four launches that stood there, and 3.6 us against 14 us of four.
+// and the sum with the logits' own gradient are one launch each. At 512 tokens, hidden 256, E 8, k 2: 8.1 us
+// against 27 us of the four launches that stood there, and 4.4 us against 14 us of four.
 // A workgroup takes 16 tokens; its four wavefronts share the reduction (16 k per step: a lane loads four consecutive k of one token and
 // of one expert per 16 experts, and feeds the four instructions of the step from them) and their partial sums are added in a fixed
 // order through LDS. Sixteen lanes then select and weigh the choices of a token.
