@@ -175,6 +175,13 @@ def test_what_takes_the_general_path(case, monkeypatch):
         assert a.dtype == b.dtype and float((a.float() - b.float()).norm() / b.float().norm()) < TOL
 
 
+@pytest.mark.parametrize("H,inter", [(64, 36), (60, 64), (64, 33), (12, 16)])
+def test_sizes_that_are_no_multiples_of_eight_are_refused(H, inter):
+    moe = _layer(4, 2, H, inter)
+    with pytest.raises(AssertionError):
+        moe(torch.randn(20, H, device=DEV), kernel_backend=KernelBackend.cuda)
+
+
 @pytest.mark.parametrize("strided", ["tokens", "gate"])
 def test_second_derivative_of_strided_tokens_and_gate(strided):
     moe = _layer(8, 2, 64, 32)
