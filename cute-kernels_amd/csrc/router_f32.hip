@@ -19,6 +19,7 @@ struct F32RouterArgs {
     const float* w;        // [E, H]
     float* logits;         // [T, E]
     float* weights;        // [T, k]
+    float* kept;           // [T, k] or null: the chosen logits
     int32_t* selected;     // [T, k]
     uint32_t* hist;        // [ceil(T / 16), E] or null
     int64_t T;
@@ -128,6 +129,11 @@ __global__ __launch_bounds__(kThreads) void router_topk_f32_kernel(const F32Rout
                 col[i] = chosen;
             }
     }
+    if (a.kept && token < a.T) {
+#pragma unroll
+        for (int i = 0; i < kMaxTopK / 16; ++i)
+            if (c + 16 * i < a.k) a.kept[token * a.k + c + 16 * i] = val[i];
+    }
     float sum = 0.f;
 #pragma unroll
     for (int i = 0; i < kMaxTopK / 16; ++i) {
@@ -160,7 +166,7 @@ __device__ __forceinline__ double row16_sum(double v) {
 
 // d_out[t, :] = d_logits[t, :] (zeros if absent), and at the k chosen columns s_j (dw_j - sum_i s_i dw_i) more. 16 lanes per token.
 // (s_j and the difference in double: the gradients of a token's choices nearly cancel in it, and these are k values per token)
-__global__ __launch_bounds__(kThreads) void router_topk_bwd_f32_kernel(const float* __restrict__ logits,
+__global__ __launch_bounds__(kThreads) void router_topk_bwd_f32_kernel(const float* __restrict__ kept,
                                                                        const int32_t* __restrict__ selected,
                                                                        const float* __restrict__ d_weights,
                                                                        const float* __restrict__ d_logits, int64_t T, int E, int k,
@@ -171,10 +177,9 @@ __global__ __launch_bounds__(kThreads) void router_topk_bwd_f32_kernel(const flo
     const int64_t t = (int64_t)blockIdx.x * kTok + tok;
     const bool live = t < T;
     const int64_t tt = live ? t : T - 1;
-    auto inside = [&](int col) { return col < 0 ? 0 : (col < E ? col : E - 1); };  // a corrupt index must not become a wild read
     double s[kMaxTopK / 16], dw[kMaxTopK / 16], sum = 0.0;
     int sel[kMaxTopK / 16];
-    const float vmax = logits[tt * E + inside(selected[tt * k])];  // the first choice is the largest kept logit
+    const float vmax = kept[tt * k];  // the first choice is the largest kept logit
 #pragma unroll
     for (int i = 0; i < kMaxTopK / 16; ++i) {
         const int j = c + 16 * i;
@@ -182,7 +187,7 @@ __global__ __launch_bounds__(kThreads) void router_topk_bwd_f32_kernel(const flo
         s[i] = dw[i] = 0.0;
         if (j < k) {
             sel[i] = selected[tt * k + j];
-            s[i] = (double)expf(logits[tt * E + inside(sel[i])] - vmax);
+            s[i] = (double)expf(kept[tt * k + j] - vmax);
             dw[i] = d_weights ? (double)d_weights[tt * k + j] : 0.0;
             sum += s[i];
         }
@@ -230,7 +235,7 @@ int check_f32(const char* what, int64_t T, int64_t E, int64_t k) {
 extern "C" {
 
 int fma_router_topk_f32(const void* x, const void* gate_weight, int64_t T, int64_t H, int64_t E, int64_t top_k, void* logits,
-                        void* weights, int32_t* selected, uint32_t* token_block_hist, void* stream) {
+                        void* weights, int32_t* selected, uint32_t* token_block_hist, void* kept, void* stream) {
     using namespace fmahip;
     const int rc = check_f32("router_topk_f32", T, E, top_k);
     if (rc) return rc;
@@ -245,6 +250,7 @@ int fma_router_topk_f32(const void* x, const void* gate_weight, int64_t T, int64
     a.logits = (float*)logits;
     a.weights = (float*)weights;
     a.selected = selected;
+    a.kept = (float*)kept;
     a.hist = token_block_hist;
     a.T = T;
     a.H = (int32_t)H;
@@ -256,15 +262,15 @@ int fma_router_topk_f32(const void* x, const void* gate_weight, int64_t T, int64
     return launch_status("router_topk_f32");
 }
 
-int fma_router_topk_bwd_f32(const void* logits, const int32_t* selected, const void* d_weights, const void* d_logits, int64_t T,
+int fma_router_topk_bwd_f32(const void* kept, const int32_t* selected, const void* d_weights, const void* d_logits, int64_t T,
                             int64_t E, int64_t top_k, void* d_out, void* stream) {
     using namespace fmahip;
     const int rc = check_f32("router_topk_bwd_f32", T, E, top_k);
     if (rc) return rc;
     if (T == 0) return FMA_OK;
-    FMA_REQUIRE(logits && selected && d_out, FMA_ERR_NULL_POINTER, "router_topk_bwd_f32: NULL pointer");
+    FMA_REQUIRE(kept && selected && d_out, FMA_ERR_NULL_POINTER, "router_topk_bwd_f32: NULL pointer");
     hipLaunchKernelGGL(router_topk_bwd_f32_kernel, dim3((uint32_t)((T + kTok - 1) / kTok)), dim3(kThreads), 0, (hipStream_t)stream,
-                       (const float*)logits, selected, (const float*)d_weights, (const float*)d_logits, T, (int)E, (int)top_k,
+                       (const float*)kept, selected, (const float*)d_weights, (const float*)d_logits, T, (int)E, (int)top_k,
                        (float*)d_out);
     return launch_status("router_topk_bwd_f32");
 }

@@ -70,7 +70,7 @@ SIGNATURES = {
     "fma_router_topk": (_i32, [_p, _p, _i64, _i64, _i64, _i64, _p, _p, _p, _p, _p, _i32, _p]),
     "fma_moe_build_index_from_hist": (_i32, [_p, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p, _p]),
     "fma_router_topk_bwd": (_i32, [_p, _p, _p, _p, _i64, _i64, _i64, _p, _i32, _p]),
-    "fma_router_topk_f32": (_i32, [_p, _p, _i64, _i64, _i64, _i64, _p, _p, _p, _p, _p]),
+    "fma_router_topk_f32": (_i32, [_p, _p, _i64, _i64, _i64, _i64, _p, _p, _p, _p, _p, _p]),
     "fma_router_topk_bwd_f32": (_i32, [_p, _p, _p, _p, _i64, _i64, _i64, _p, _p]),
     "fma_swiglu_experts_f32": (_i32, [_p] * 10 + [_i64] * 5 + [_p] * 6),
     "fma_swiglu_experts_bwd_f32": (_i32, [_p] * 14 + [_i64] * 5 + [_p] * 8),

@@ -536,16 +536,17 @@ def router_topk_backward_cuda(
     _lib.check(rc, "router_topk_backward_cuda")
 
 
-@hip_op("router_topk_f32_cuda", mutates_args={"logits", "weights", "selected", "token_block_hist"})
+@hip_op("router_topk_f32_cuda", mutates_args={"logits", "weights", "selected", "token_block_hist", "kept"})
 def router_topk_f32_cuda(
     x: torch.Tensor, gate_weight: torch.Tensor, top_k: int, logits: torch.Tensor, weights: torch.Tensor,
-    selected: torch.Tensor, token_block_hist: torch.Tensor,
+    selected: torch.Tensor, token_block_hist: torch.Tensor, kept: torch.Tensor | None = None,
 ) -> None:  # fmt: skip
-    _lib.require_gpu(x, gate_weight, logits, weights, selected, token_block_hist)
+    _lib.require_gpu(x, gate_weight, logits, weights, selected, token_block_hist, kept)
     T, H = x.shape
     E = gate_weight.size(0)
     assert gate_weight.shape == (E, H) and logits.shape == (T, E)
     assert weights.shape == (T, top_k) and selected.shape == (T, top_k)
+    assert kept is None or (kept.shape == (T, top_k) and kept.dtype == torch.float32 and kept.is_contiguous())
     assert x.dtype == gate_weight.dtype == logits.dtype == weights.dtype == torch.float32 and selected.dtype == torch.int32
     assert token_block_hist.dtype == torch.uint32 and token_block_hist.shape == ((T + 15) // 16, E)
     for t in (x, gate_weight, logits, weights, selected, token_block_hist):
@@ -553,29 +554,29 @@ def router_topk_f32_cuda(
     with _lib.on_device(x.device):
         rc = _lib.load().fma_router_topk_f32(
             x.data_ptr(), gate_weight.data_ptr(), T, H, E, top_k, logits.data_ptr(), weights.data_ptr(),
-            selected.data_ptr(), token_block_hist.data_ptr(), _lib.current_stream(x.device),
+            selected.data_ptr(), token_block_hist.data_ptr(), _lib.ptr(kept), _lib.current_stream(x.device),
         )
     _lib.check(rc, "router_topk_f32_cuda")
 
 
 @hip_op("router_topk_backward_f32_cuda", mutates_args={"logits_grad"})
 def router_topk_backward_f32_cuda(
-    logits: torch.Tensor, selected: torch.Tensor, weights_grad: torch.Tensor | None,
+    kept: torch.Tensor, selected: torch.Tensor, weights_grad: torch.Tensor | None,
     logits_output_grad: torch.Tensor | None, logits_grad: torch.Tensor,
 ) -> None:  # fmt: skip
-    _lib.require_gpu(logits, selected, weights_grad, logits_output_grad, logits_grad)
-    T, E = logits.shape
+    _lib.require_gpu(kept, selected, weights_grad, logits_output_grad, logits_grad)
+    T, E = logits_grad.shape
     top_k = selected.size(1)
-    assert selected.shape == (T, top_k) and selected.dtype == torch.int32 and logits_grad.shape == (T, E)
-    assert logits_grad.dtype == logits.dtype == torch.float32
-    assert weights_grad is None or (weights_grad.shape == (T, top_k) and weights_grad.dtype == logits.dtype)
-    assert logits_output_grad is None or (logits_output_grad.shape == (T, E) and logits_output_grad.dtype == logits.dtype)
-    for t in (logits, selected, weights_grad, logits_output_grad, logits_grad):
+    assert kept.shape == selected.shape == (T, top_k) and selected.dtype == torch.int32
+    assert logits_grad.dtype == kept.dtype == torch.float32
+    assert weights_grad is None or (weights_grad.shape == (T, top_k) and weights_grad.dtype == kept.dtype)
+    assert logits_output_grad is None or (logits_output_grad.shape == (T, E) and logits_output_grad.dtype == kept.dtype)
+    for t in (kept, selected, weights_grad, logits_output_grad, logits_grad):
         assert t is None or t.is_contiguous()
-    with _lib.on_device(logits.device):
+    with _lib.on_device(kept.device):
         rc = _lib.load().fma_router_topk_bwd_f32(
-            logits.data_ptr(), selected.data_ptr(), _lib.ptr(weights_grad), _lib.ptr(logits_output_grad), T, E, top_k,
-            logits_grad.data_ptr(), _lib.current_stream(logits.device),
+            kept.data_ptr(), selected.data_ptr(), _lib.ptr(weights_grad), _lib.ptr(logits_output_grad), T, E, top_k,
+            logits_grad.data_ptr(), _lib.current_stream(kept.device),
         )
     _lib.check(rc, "router_topk_backward_f32_cuda")
 
@@ -735,19 +736,26 @@ def fused_router_with_histogram(x: torch.Tensor, gate_weight: torch.Tensor, top_
     return _FusedRouter.apply(x, gate_weight, top_k)
 
 
+def _is_batched(t: torch.Tensor | None) -> bool:
+    """several gradients at once: is_grads_batched, and a backward pass under vmap"""
+    functorch = torch._C._functorch
+    return t is not None and (functorch.is_legacy_batchedtensor(t) or functorch.is_batchedtensor(t))
+
+
 class _Fp32Router(torch.autograd.Function):
-    """_FusedRouter for fp32 activations. A backward pass that is itself recorded (create_graph) forms the logits' gradient from
-    differentiable operations, as the library calls that this node stands for do."""
+    """_FusedRouter for fp32 activations. A backward pass that is itself recorded (create_graph) or runs for several gradients at
+    once forms the logits' gradient from library operations, as the calls that this node stands for do. Saved are the chosen logits,
+    not all of them: the layer returns those, and its caller may change them in place."""
 
     @staticmethod
     @ensure_contiguous
     def forward(ctx, x: torch.Tensor, gate_weight: torch.Tensor, top_k: int):
         T, E = x.size(0), gate_weight.size(0)
-        logits, weights = x.new_empty(T, E), x.new_empty(T, top_k)
+        logits, weights, kept = x.new_empty(T, E), x.new_empty(T, top_k), x.new_empty(T, top_k)
         selected = torch.empty(T, top_k, device=x.device, dtype=torch.int32)
         token_block_hist = torch.empty((T + 15) // 16, E, device=x.device, dtype=torch.uint32)
-        router_topk_f32_cuda(x, gate_weight, top_k, logits, weights, selected, token_block_hist)
-        ctx.save_for_backward(x, gate_weight, logits, selected)
+        router_topk_f32_cuda(x, gate_weight, top_k, logits, weights, selected, token_block_hist, kept)
+        ctx.save_for_backward(x, gate_weight, kept, selected)
         ctx.mark_non_differentiable(selected, token_block_hist)
         ctx.set_materialize_grads(False)
         return logits, weights, selected, token_block_hist
@@ -755,18 +763,19 @@ class _Fp32Router(torch.autograd.Function):
     @staticmethod
     @ensure_contiguous
     def backward(ctx, logits_output_grad, weights_grad, _, __):
-        x, gate_weight, logits, selected = ctx.saved_tensors
+        x, gate_weight, kept, selected = ctx.saved_tensors
         if logits_output_grad is None and weights_grad is None:
             return None, None, None
-        if torch.is_grad_enabled():
-            logits_grad = torch.zeros_like(logits) if logits_output_grad is None else logits_output_grad
+        shape = (x.size(0), gate_weight.size(0))
+        if torch.is_grad_enabled() or _is_batched(logits_output_grad) or _is_batched(weights_grad):
+            logits_grad = x.new_zeros(shape) if logits_output_grad is None else logits_output_grad
             if weights_grad is not None:
                 columns = selected.long()
                 s = torch.softmax((x @ gate_weight.t()).gather(1, columns), dim=-1)
                 logits_grad = logits_grad.scatter_add(1, columns, s * (weights_grad - (s * weights_grad).sum(-1, keepdim=True)))
         else:
-            logits_grad = torch.empty_like(logits)
-            router_topk_backward_f32_cuda(logits, selected, weights_grad, logits_output_grad, logits_grad)
+            logits_grad = x.new_empty(shape)
+            router_topk_backward_f32_cuda(kept, selected, weights_grad, logits_output_grad, logits_grad)
         x_grad = logits_grad @ gate_weight if ctx.needs_input_grad[0] else None
         gate_weight_grad = logits_grad.t() @ x if ctx.needs_input_grad[1] else None
         return x_grad, gate_weight_grad, None

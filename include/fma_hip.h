@@ -373,10 +373,11 @@ int fma_router_topk_bwd(const void* logits, const int32_t* selected, const void*
                         const void* d_logits, int64_t T, int64_t E, int64_t top_k, void* d_out, int dtype,
                         void* stream);
 
-/* fma_router_topk and fma_router_topk_bwd for fp32 activations: the same results (no rounding; without counts), H % 4 == 0. */
+/* fma_router_topk and fma_router_topk_bwd for fp32 activations: the same results (no rounding; without counts), H % 4 == 0.
+ * kept [T, top_k], or NULL: the chosen logits, which the backward reads in place of [T, E] (a caller may change its logits). */
 int fma_router_topk_f32(const void* x, const void* gate_weight, int64_t T, int64_t H, int64_t E, int64_t top_k, void* logits,
-                        void* weights, int32_t* selected, uint32_t* token_block_hist, void* stream);
-int fma_router_topk_bwd_f32(const void* logits, const int32_t* selected, const void* d_weights, const void* d_logits, int64_t T,
+                        void* weights, int32_t* selected, uint32_t* token_block_hist, void* kept, void* stream);
+int fma_router_topk_bwd_f32(const void* kept, const int32_t* selected, const void* d_weights, const void* d_logits, int64_t T,
                             int64_t E, int64_t top_k, void* d_out, void* stream);
 
 /* The expert path of an fp32 SwiGLU layer without biases, enqueued by one call: fma_dispatch_rows (xg [R, H], R = T * k),

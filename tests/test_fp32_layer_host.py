@@ -13,19 +13,20 @@ from fma.modules.moe import cuda_implementation as ci
 TOL = 1e-5  # fp32 sums of 24 terms of size one
 
 
-def _router_in_torch(x, gate_weight, top_k, logits, weights, selected, token_block_hist):
+def _router_in_torch(x, gate_weight, top_k, logits, weights, selected, token_block_hist, kept):
     with torch.no_grad():
         logits.copy_(x @ gate_weight.t())
         top, chosen = logits.topk(top_k, dim=-1)
         weights.copy_(top.softmax(-1))
         selected.copy_(chosen)
+        kept.copy_(top)
 
 
-def _router_backward_in_torch(logits, selected, weights_grad, logits_output_grad, logits_grad):
+def _router_backward_in_torch(kept, selected, weights_grad, logits_output_grad, logits_grad):
     with torch.no_grad():
         columns = selected.long()
-        s = logits.gather(1, columns).softmax(-1)
-        logits_grad.copy_(torch.zeros_like(logits) if logits_output_grad is None else logits_output_grad)
+        s = kept.softmax(-1)
+        logits_grad.copy_(torch.zeros_like(logits_grad) if logits_output_grad is None else logits_output_grad)
         if weights_grad is not None:
             logits_grad.scatter_add_(1, columns, s * (weights_grad - (s * weights_grad).sum(-1, keepdim=True)))
 
@@ -69,6 +70,30 @@ def test_second_derivative_with_strided_arguments(strided, monkeypatch):
         results.append([*first, *torch.autograd.grad(sum(g.pow(2).sum() for g in first), (xi, wi))])
     for got, expect in zip(*results):
         assert float((got - expect).norm() / expect.norm()) < TOL
+
+
+@pytest.mark.parametrize("how", ["logits changed in place", "is_grads_batched", "vmap"])
+def test_what_the_library_calls_allow(how, monkeypatch):
+    T, H, E, k = 12, 24, 6, 2
+    torch.manual_seed(0)
+    x, w, v = torch.randn(T, H, requires_grad=True), torch.randn(E, H), torch.randn(3, T, E)
+    monkeypatch.setattr(ci, "router_topk_f32_cuda", _router_in_torch)
+    monkeypatch.setattr(ci, "router_topk_backward_f32_cuda", _router_backward_in_torch)
+    results = []
+    for node in (True, False):
+        if node:
+            logits, gates = ci._Fp32Router.apply(x, w, k)[:2]
+        else:
+            logits = F.linear(x, w)
+            gates = logits.topk(k, dim=-1).values.softmax(-1)
+        if how == "logits changed in place":
+            logits.mul_(2.0)
+            results.append(torch.autograd.grad(gates.sin().sum() + logits.pow(2).sum(), x)[0])
+        elif how == "is_grads_batched":
+            results.append(torch.autograd.grad(logits, x, v, is_grads_batched=True)[0])
+        else:
+            results.append(torch.vmap(lambda g: torch.autograd.grad(logits, x, g)[0])(v))
+    assert float((results[0] - results[1]).norm() / results[1].norm()) < TOL
 
 
 class _Names(TorchDispatchMode):
