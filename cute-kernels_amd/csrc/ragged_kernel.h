@@ -19,7 +19,18 @@
 //    compute unit's one address path, no wait for first operands, no barrier.
 //  * The epilogue's stores stay outstanding across the start of the next tile: they are issued after that tile's first
 //    loads, and loads and stores of a wavefront complete in issue order, so the first K step waits for "all but the
-//    stores and the newest prefetch" (an exact count) and the second for everything, two K steps after the stores went out.
+//    stores and its own newest loads" (an exact count) and the second for everything older than its own loads.
+//  * A K step has two barriers. Behind the first, in the middle of its fifth phase, the step's LDS stage is free (all its fragments have been
+//    read) and the loads of step kt + 2 begin; the second, in the middle of the eighth, is where step kt + 1 has to have landed, and
+//    leaves the four loads behind the first outstanding. One barrier for both, as there was, waits for every load in flight, so that
+//    once a step nothing is on its way and the latency of an L2 miss is paid in full; a compute unit has no more than 32 KB of
+//    misses in flight (60 GB/s from HBM for one alone, 114 from the last-level cache, with 32 KB as with 128), so what the stream needs
+//    is to be continuous. Products, one barrier and an L2 prefetch of the lines shared -> two
+//    barriers and none, us: hidden 4096, I 1536, E 128, 512 rows an expert 1415 -> 1332, 789 -> 756 (up, down), input gradients 1397 ->
+//    1350, weight gradients 1735 -> 1694, 902 -> 866; 256 rows 901 -> 840, 479 -> 449 (up with the activation 889 -> 800); 128 rows 807 ->
+//    734 (up); hidden 2048, I 1408, E 64, 4096 rows 2360 -> 2296, 1242 -> 1198, input gradient 2284 -> 2236; hidden 4096, I 14336, E 8,
+//    4096 rows 5640 -> 5650, 2981 -> 2862, input gradient of the first projection 5920 -> 5867 (there the matrix instructions' power is the
+//    bound: all-zero operands 4657 -> 4310, 5107 -> 4620).
 //  * A K loop always runs an even number of steps (a step of zeros is appended to an odd reduction length), so every tile
 //    starts in LDS stage 0 and the loop body stays two straight-line steps.
 //  * Tiles that break the pattern (groups of at most 64 rows on their three-stage loop, groups without reduction, groups
@@ -53,7 +64,6 @@ namespace fmahip {
 namespace gemm {
 namespace ragged {
 
-constexpr uint32_t kPfDist = 4;     // K steps between a line's prefetch and the step that loads it
 constexpr int kBwdAhead = 2;        // passes of the SwiGLU-gradient epilogue whose h values are requested ahead
 constexpr uint32_t kStreamOutSteps = 16;  // weight-gradient tiles of at most this many K steps store with the non-temporal hint
 
@@ -162,7 +172,6 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
     __shared__ __attribute__((aligned(TALL ? 1024 : 16))) uint8_t s_x0[TALL ? kExtraBytes : 16];
     __shared__ __attribute__((aligned(TALL ? 1024 : 16))) uint8_t s_x1[TALL ? kExtraBytes : 16];
     __shared__ __attribute__((aligned(1024))) uint8_t s_stage[NW * kStageBytes];
-    __shared__ uint32_t s_pf[64];  // where the dwords fetched by the L2 prefetch end up (never read)
     // BIAS: per wavefront, the bias values of its own 64 columns (plain) or 32 "up" | 32 "gate" columns
     constexpr int kBiasBytes = 128;
     __shared__ __attribute__((aligned(256))) uint8_t s_bias[BIAS ? NW * kBiasBytes : 16];
@@ -392,7 +401,6 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
         uint32_t e;                      // the group
         uint32_t row0;                   // first packed row (reduction row, if the reduction varies) of the group
         uint64_t off_a, off_b, off_d;
-        uint32_t pf_r, pf_c;  // position of the tile in its XCD's 8 x 4 block of tiles (row, column)
         uint32_t ks, part;    // kSplit: first K element of the tile's part of the reduction, and which part
     };
     auto lookup = [&](uint32_t round) -> Tile {
@@ -438,8 +446,6 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
         const uint32_t band_m = tiles_m - first_m < (uint32_t)kGroupM ? tiles_m - first_m : (uint32_t)kGroupM;
         const uint32_t mt = first_m + (local % band) % band_m;
         const uint32_t nt = (local % band) / band_m;
-        t.pf_r = (local % band) % band_m;
-        t.pf_c = nt & 3u;
         // TALL: the first tiles of the group are 288 rows high, as many as its rows need; the others 256
         const uint32_t past = TALL ? tall_tiles(t.Me, tiles_m) : 0u;
         const uint32_t height = mt < past ? kMostRows : (uint32_t)BM;
@@ -528,12 +534,24 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
         }
     };
     // points a loader object at a feed (what depends on lane and wavefront only stays as the last setup left it)
-    auto aim_a = [&](const Feed<A_KC>& f, uint32_t v) {
+    // (kSplit: the same in every lane, which the compiler does not see in the NT kernels: without this it wraps every load in a loop
+    // over the distinct descriptors it fears)
+    auto same = [](auto f) __attribute__((always_inline)) {
+        if constexpr (kSplit) {
+            f.base0 = reinterpret_cast<const uint16_t*>(uniform((uint64_t)(uintptr_t)f.base0));
+            f.extent = uniform(f.extent);
+            f.ldb = uniform(f.ldb);
+        }
+        return f;
+    };
+    auto aim_a = [&](const Feed<A_KC>& any, uint32_t v) {
         if constexpr (GATHER) return;
+        const Feed<A_KC> f = same(any);
         if constexpr (A_KC) { lk_a.base0 = f.base0; lk_a.bytes = f.extent; lk_a.ldb = f.ldb; lk_a.kdim = f.ldb / 2u; lk_a.voff = v; }
         else { lt_a.base = f.base0; lt_a.kdim = f.extent; lt_a.ldb = f.ldb; lt_a.col_bytes = f.col_bytes; lt_a.voff = v; }
     };
-    auto aim_b = [&](const Feed<B_KC>& f, uint32_t v) {
+    auto aim_b = [&](const Feed<B_KC>& any, uint32_t v) {
+        const Feed<B_KC> f = same(any);
         if constexpr (B_KC) { lk_b.base0 = f.base0; lk_b.base1 = f.base1; lk_b.bytes = f.extent; lk_b.ldb = f.ldb; lk_b.kdim = f.ldb / 2u; lk_b.voff = v; }
         else { lt_b.base = f.base0; lt_b.kdim = f.extent; lt_b.ldb = f.ldb; lt_b.col_bytes = f.col_bytes; lt_b.voff = v; }
     };
@@ -603,7 +621,7 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
     // either way, so the LDS image, the fragment reads and the order of the sums are those of the packed kernel.
     // The eight entries are one vector load per wavefront and step (lane l: entry l % 8; a position past the end of
     // row_index reads as 0), issued two steps ahead of the loads that use them, behind the step's own loads: a step's loads
-    // for K step kt + 2 go out with the entries requested in step kt - 2, which the wait of step kt - 1 has seen arrive
+    // for K step kt + 2 go out with the entries requested in step kt - 2, which the second barrier of step kt has seen arrive
     // (loads complete in issue order). Inside a tile the entries travel in a register (gk_ring[s]: requested in the latest
     // step that ran in LDS stage s). Across a tile boundary they travel through LDS (s_gk, a direct-to-LDS load read back
     // in assembly): a register loaded in one tile and used in the next makes the compiler, which cannot count the
@@ -648,69 +666,6 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
             const uint32_t odd = (uint32_t)__builtin_amdgcn_readlane((int)off, 2 * i + 1);
             v[i] = (gk_half ? odd : even) + (gk_chunk ^ (128u * ((uint32_t)i & 1u)));
         }
-    };
-
-    // ---- L2 prefetch by designated workgroups (grouped_gemm.hip): one 4-byte load per shared line, kPfDist steps ahead ----
-    constexpr bool kPrefetch = A_KC == B_KC;
-    uint32_t pf_voff = kOutOfRange;
-    const uint16_t* pf_base = nullptr;
-    uint32_t pf_bytes = 0, pf_ldb = 0, pf_col_bytes = 0, pf_kdim = 0, pf_steps = 0, pf_k0 = 0;
-    const bool pf_is_b = (wave & 1u) != 0;
-    const bool pf_t = pf_is_b ? !B_KC : !A_KC;
-    auto setup_prefetch = [&](const Tile& t) {
-        if constexpr (!kPrefetch) return;
-        const uint32_t p = wave >> 1;
-        pf_steps = k_steps(t);
-        if constexpr (kSplit) pf_k0 = t.ks;
-        if (!pf_is_b) {
-            // (TALL: lanes 16 and 17 take the rows past 256; those past the tile are out of the descriptor's range or no row)
-            constexpr uint32_t kLanes = TALL ? 18u : 16u;
-            const uint32_t i = lane < 16u ? p * 16u + lane : 64u + p * 2u + (lane - 16u);
-            if constexpr (GATHER) {
-                const uint32_t n = lds_read1_quiet(lds_address(reinterpret_cast<const uint8_t*>(s_rows)) + (round & 1u) * (kMostRows * 4u) +
-                                                   (lane < kLanes ? 4u * i + t.pf_c : 0u) * 4u);
-                pf_base = args.A; pf_bytes = g_full;
-                const uint32_t src = lane < kLanes && 4u * i + t.pf_c < t.rows ? g_source_row(n) : 0xffffffffu;
-                pf_voff = src < args.a_rows ? src * g_ldb : kOutOfRange;
-            } else if constexpr (A_KC) {
-                pf_base = fa_cur.base0; pf_bytes = fa_cur.extent;
-                pf_voff = lane < kLanes ? (4u * i + t.pf_c) * (t.Ke * 2u) : kOutOfRange;
-            } else {
-                pf_base = fa_cur.base0; pf_ldb = fa_cur.ldb; pf_col_bytes = fa_cur.col_bytes; pf_kdim = t.Ke;
-                pf_voff = lane < 16u ? i * fa_cur.ldb + t.pf_c * 128u : kOutOfRange;
-            }
-        } else {
-            if constexpr (B_KC) {
-                pf_bytes = fb_cur.extent;
-                if constexpr (kGlu) {
-                    pf_base = (p >> 1) ? fb_cur.base1 : fb_cur.base0;
-                    pf_voff = lane < 8u ? (8u * ((p & 1u) * 8u + lane) + t.pf_r) * (t.Ke * 2u) : kOutOfRange;
-                } else {
-                    pf_base = fb_cur.base0;
-                    pf_voff = lane < 8u ? (8u * (p * 8u + lane) + t.pf_r) * (t.Ke * 2u) : kOutOfRange;
-                }
-            } else {
-                pf_base = fb_cur.base0; pf_ldb = fb_cur.ldb; pf_col_bytes = fb_cur.col_bytes; pf_kdim = t.Ke;
-                // (gathered reduction rows: no prefetch of B, the instruction fetches nothing)
-                pf_voff = (!kGatherK && lane < 8u) ? (2u * (p * 8u + lane) + (t.pf_r >> 2)) * fb_cur.ldb + (t.pf_r & 3u) * 128u : kOutOfRange;
-            }
-        }
-    };
-    // requests this wavefront's lines of K step `kstep` of the current tile (nothing past its last step)
-    auto issue_prefetch = [&](uint32_t kstep) {
-        if constexpr (!kPrefetch) return;
-        const uint32_t k0 = kstep * (uint32_t)BK + pf_k0;
-        const bool inside = kstep < pf_steps;
-        const uint32_t rows = k0 >= pf_kdim ? 0u : (pf_kdim - k0 < (uint32_t)BK ? pf_kdim - k0 : (uint32_t)BK);
-        const uint16_t* base = pf_t ? pf_base + (uint64_t)k0 * (pf_ldb / 2u) : pf_base;
-        uint32_t bytes = !inside ? 0u : (pf_t ? (rows ? rows * pf_ldb - pf_col_bytes : 0u) : pf_bytes);
-        if constexpr (GATHER) {
-            // (the same in every lane, which the compiler does not see in these kernels: without this it wraps the load
-            // in a loop over the distinct descriptors it fears)
-            base = reinterpret_cast<const uint16_t*>(uniform((uint64_t)(uintptr_t)base));
-            bytes = uniform(bytes);
-        }
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(make_rsrc(base, bytes), (lds_void*)s_pf, 4, pf_voff, pf_t ? 0u : k0 * 2u, 0, 0);
     };
 
     constexpr int kLoads = 32 / NW;                // load instructions per wavefront, operand and K step
@@ -823,7 +778,6 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
         }
-        setup_prefetch(cur);
         const uint32_t KT = k_steps(cur);
         const uint32_t KT2 = (KT + 1u) & ~1u;  // steps of the K loop: an odd count gets a step of zeros
         const bool thin = is_thin(cur);
@@ -906,27 +860,27 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
             if constexpr (B_KC) fb[j] = __builtin_bit_cast(typename EL::frag, read_kc_frag(tb + b_off[j] + kc_slice[ks]));
             else fb[j] = __builtin_bit_cast(typename EL::frag, read_tr_frag(tb + b_off[j] + ks * kSliceT));
         };
-        // pair `pair` from A buffer abuf times the B fragments; reload: each B fragment is then read anew from slice
-        // next_ks of stage next_stage
-        auto mma = [&](auto fa_c, int pair, int abuf, bool reload, int next_stage, int next_ks) __attribute__((always_inline)) {
+        // pair `pair` from A buffer abuf times the B fragments j0 .. j1 - 1; reload: each B fragment is then read anew from slice
+        // next_ks of stage next_stage; reload or nine: the ninth row block joins
+        auto mma = [&](auto fa_c, int pair, int abuf, bool reload, int next_stage, int next_ks, int j0 = 0, int j1 = CB, bool nine = false) __attribute__((always_inline)) {
             constexpr int FA = decltype(fa_c)::value;
             constexpr int AB = FA < 2 ? FA : 2;
             if constexpr (FA > 0) {
 #pragma unroll
-                for (int j = 0; j < CB; ++j) {
+                for (int j = j0; j < j1; ++j) {
 #pragma unroll
                     for (int i = 0; i < AB; ++i)
                         mfma_block(acc[pair * 2 + i], j, fb[j], fa[abuf][i]);
                     if constexpr (FA > RB) {
-                        if (reload) mfma_block(acc[RB], j, fb[j], fx);
+                        if (reload || nine) mfma_block(acc[RB], j, fb[j], fx);
                     }
                     if (reload) load_b(next_stage, next_ks, j);
                 }
             }
         };
 
-        // ---- one K step (see grouped_gemm.hip for the placement of barrier, waits and loads) ----
-        // WAIT: the s_waitcnt immediate in front of the barrier. The loads issued after the barrier are those of step
+        // ---- one K step ----
+        // WAIT: the s_waitcnt immediate in front of the second barrier. The loads issued after the first barrier are those of step
         // kt + 2: of this tile, or, in the last two steps, steps 0 and 1 of the next tile (or nothing).
         // SRC: which tile the loads issued in the step belong to: 0 the current one, 1 the next one (the loaders are aimed
         // by the caller in both cases), 2 decided here (first steps of a tile, and the versions for tiles with few rows), 3 the same
@@ -937,10 +891,6 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
             constexpr int AB = FA < 2 ? FA : 2;       // row blocks per phase
             constexpr int PP = FA >= RB ? RB / 2 : (FA >= 2 ? FA / 2 : 1);  // phases per k slice
             constexpr int X = FA > RB ? 1 : 0;        // the ninth row block
-            // The loads of B in front of those of A: in tall tiles of the NN layout, which has no L2 prefetch, 1 to 4 % faster (input
-            // gradients: 1498 -> 1440 us, hidden 4096, I 14336, E 8, k 2, 4096 tokens); in the NT layout 3 to 6 % slower, and in tiles of
-            // few rows up to 6 %.
-            constexpr bool kBFirst = X && !B_KC;
             // The rows past 256 are fetched where the tile has them and in the steps whose loads may be for the next tile. The version
             // for no columns looks whether this tile or the next has any; it has no matrix instructions to place loads between, as
             // the others have: a branch in front of their ninth load would leave the other eight in a block of their own.
@@ -950,10 +900,10 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
             constexpr int kReadsA = (A_KC ? 1 : 2) * AB, kReadsB = (B_KC ? 1 : 2);  // LDS reads per pair, per B fragment
             // On entry A buffer 0 and the B registers hold the fragments of the first phase.
             typedef std::integral_constant<int, 0> I0_;
-            typedef std::integral_constant<int, 2> I2_;
+            typedef std::integral_constant<int, 1> I1_;
             typedef std::integral_constant<int, 3> I3_;
             typedef std::integral_constant<int, kLoads> IN_;
-            static_assert(kLoads == 4, "the split of a step's loads over three phases is written for four per operand");
+            static_assert(kLoads == 4, "a step's loads are placed for four per operand");
             // the A loads [i0, i1) of the step's load slot
             auto issue_a_part = [&](uint32_t k0, auto i0_c, auto i1_c) __attribute__((always_inline)) {
                 if constexpr (GATHER) {
@@ -969,6 +919,29 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
                     if constexpr (GATHER) issue_a_part(k0, std::integral_constant<int, 4>{}, std::integral_constant<int, 5>{});
                     else issue_x(stage, k0);
                 }
+            };
+            // The operand whose loads go out behind the first barrier, and the other one, behind the second: B and A (A first: the input
+            // gradients 2 to 6 % slower, 512 rows an expert and up; the rest within 1 %, both ways). Gathered reduction rows: A and B,
+            // whose entries of row_index have landed at the second barrier only.
+            auto issue_first = [&](uint32_t k0, auto i0_c, auto i1_c) __attribute__((always_inline)) {
+                if constexpr (kGatherK) issue_a_part(k0, i0_c, i1_c);
+                else issue_b(stage, k0, i0_c, i1_c);
+            };
+            auto issue_second = [&](uint32_t k0) __attribute__((always_inline)) {
+                if constexpr (kGatherK) issue_b(stage, k0, I0_{}, IN_{});
+                else issue_a_part(k0, I0_{}, IN_{});
+            };
+            // first barrier: every LDS read of this stage has returned, in every wavefront; the loads of step kt + 2 may fill it
+            auto free_stage = [&]() __attribute__((always_inline)) {
+                __builtin_amdgcn_s_waitcnt(waitcnt_imm(63, true));
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+            };
+            // second barrier: every load of step kt + 1 has landed
+            auto next_landed = [&]() __attribute__((always_inline)) {
+                __builtin_amdgcn_s_waitcnt(decltype(wait_c)::value);
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
             };
             // kGatherK: the entries for this step's loads were requested two steps ago: by a step of this tile into a register,
             // or, for a tile's first two steps (SRC == 2 in a full tile), by the tile before or the cold start into LDS; the
@@ -1015,9 +988,11 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
                 return k0;
             };
             if constexpr (FA >= RB) {
-                // Full tiles: the barrier comes after five of the eight phases, with the A fragments of the last three phases
-                // already in registers (four A buffers), so that the step's loads go out over three phases instead of one:
-                // eight wavefronts that leave the barrier together otherwise queue 72 loads on the one address path at once.
+                // Full tiles: the first barrier comes after four and a half of the eight phases, with the A fragments of the last
+                // three phases already in registers (four A buffers), and the loads go out a few a phase: eight wavefronts that leave a
+                // barrier together otherwise queue 72 loads on the one address path at once. Both barriers lie in the middle of a
+                // phase, where the reads they wait for have had half a phase to return and the matrix instructions behind them need
+                // nothing from LDS (at the phases' ends, and 2 + 2 loads: 0 to 5 % slower on large tiles, 1 % faster on a few others).
                 // A fragments are read two phases ahead (phase p's pair sits in buffer p % 4): phase 0 reads those of phases 1
                 // (the step before could not: they are behind its barrier) and 2, phase 4 those of 6 and 7 first thing
                 load_a(fa_c, stage, 0, 1, 1);
@@ -1043,45 +1018,42 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
                 load_a(fa_c, stage, 1, 2, 2);
                 load_a(fa_c, stage, 1, 3, 3);
                 if (X) load_x(stage, 1);
-                mma(fa_c, 0, 0, false, stage, 1);
+                mma(fa_c, 0, 0, false, stage, 1, 0, CB / 2);
                 __builtin_amdgcn_sched_group_barrier(0x100, 2 * kReadsA + X, 0);
-                __builtin_amdgcn_sched_group_barrier(0x008, AB * CB, 0);
-                // every load of step kt+1 has landed and every LDS read of this stage has returned
-                __builtin_amdgcn_s_waitcnt(decltype(wait_c)::value);
-                __builtin_amdgcn_s_barrier();
-                asm volatile("" ::: "memory");
+                __builtin_amdgcn_sched_group_barrier(0x008, AB * CB / 2, 0);
+                __builtin_amdgcn_sched_barrier(0);
+                free_stage();
                 const uint32_t k0 = aim_loads();
-                if constexpr (kBFirst) issue_b(stage, k0, I0_{}, I3_{});
-                else issue_a_part(k0, I0_{}, I3_{});
+                issue_first(k0, I0_{}, I1_{});
+                mma(fa_c, 0, 0, false, stage, 1, CB / 2, CB);
+                spread_mfma_vmem<0, AB * CB / 2, 1>();
+                __builtin_amdgcn_sched_barrier(0);
+                issue_first(k0, I1_{}, I3_{});
                 mma(fa_c, 1, 1, false, stage, 1);
-                spread_mfma_vmem<0, AB * CB, 3>();
+                spread_mfma_vmem<0, AB * CB, 2>();
                 __builtin_amdgcn_sched_barrier(0);
-                if constexpr (kBFirst) {
-                    issue_b(stage, k0, I3_{}, IN_{});
-                    issue_a_part(k0, I0_{}, I2_{});
-                } else {
-                    issue_a_part(k0, I3_{}, IN_{});
-                    gk_step_offsets(k0);
-                    issue_b(stage, k0, I0_{}, I2_{});
-                }
+                issue_first(k0, I3_{}, IN_{});
                 mma(fa_c, 2, 2, false, stage, 1);
-                spread_mfma_vmem<0, AB * CB, 3>();
+                spread_mfma_vmem<0, AB * CB, 1>();
                 __builtin_amdgcn_sched_barrier(0);
+                mma(fa_c, 3, 3, false, stage ^ 1, 0, 0, CB / 2, true);
+                __builtin_amdgcn_sched_barrier(0);
+                next_landed();
                 load_a(fa_c, stage ^ 1, 0, 0, 0);
-                if constexpr (kBFirst) issue_a_part(k0, I2_{}, IN_{});
-                else issue_b(stage, k0, I2_{}, IN_{});
+                load_b(stage ^ 1, 0, 0);
+                load_b(stage ^ 1, 0, 1);
+                gk_step_offsets(k0);
+                issue_second(k0);
                 issue_x_part(k0);
-                if constexpr (kPrefetch) asm volatile("" : "+v"(pf_voff));
-                issue_prefetch(kt + kPfDist);
                 gk_step_request();
-                mma(fa_c, 3, 3, true, stage ^ 1, 0);
-                __builtin_amdgcn_sched_group_barrier(0x100, kReadsA, 0);
+                mma(fa_c, 3, 3, true, stage ^ 1, 0, CB / 2, CB);
+                __builtin_amdgcn_sched_group_barrier(0x100, kReadsA + 2 * kReadsB, 0);
 #pragma unroll
-                for (int j = 0; j < CB; ++j) {
+                for (int j = 0; j < CB / 2; ++j) {
 #pragma unroll
                     for (int i = 0; i < AB + X; ++i) {
                         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                        if (j * (AB + X) + i < 2 + (kLoadX ? 1 : 0) + (kPrefetch ? 1 : 0) + (kGatherK ? 1 : 0)) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+                        if (j * (AB + X) + i < kLoads + (kLoadX ? 1 : 0) + (kGatherK ? 1 : 0)) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
                     }
                     __builtin_amdgcn_sched_group_barrier(0x100, kReadsB, 0);
                 }
@@ -1107,51 +1079,40 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
                         __builtin_amdgcn_sched_barrier(0);
                     }
                 }
-                // every load of step kt+1 has landed and every LDS read of this stage has returned
-                __builtin_amdgcn_s_waitcnt(decltype(wait_c)::value);
-                __builtin_amdgcn_s_barrier();
-                asm volatile("" ::: "memory");
-                load_a(fa_c, stage ^ 1, 0, 0, 0);
+                free_stage();
                 const uint32_t k0 = aim_loads();
-                issue_a_part(k0, I0_{}, IN_{});
+                issue_first(k0, I0_{}, IN_{});
+                next_landed();
+                load_a(fa_c, stage ^ 1, 0, 0, 0);
                 gk_step_offsets(k0);
-                issue_b(stage, k0, I0_{}, IN_{});
+                issue_second(k0);
                 issue_x_part(k0);
-                // the prefetch goes out behind this step's loads (the empty statement orders it: the wait of the next step
-                // counts on it being the newest load)
-                if constexpr (kPrefetch) asm volatile("" : "+v"(pf_voff));
-                issue_prefetch(kt + kPfDist);
                 gk_step_request();
                 mma(fa_c, PP - 1, 1, true, stage ^ 1, 0);
                 if constexpr (FA > 0) {
-                    // the A reads; per column block its matrix instructions, each followed by its share of the step's loads,
-                    // and the read of the block's next fragment; the prefetch last
-                    constexpr int kLoadsPer = (int)kStepLoads / (AB * CB);
-                    static_assert(kLoadsPer * AB * CB == (int)kStepLoads, "the loads divide evenly over the matrix instructions");
+                    // the A reads; per column block its matrix instructions, followed by a load, and the read of the block's next
+                    // fragment
                     __builtin_amdgcn_sched_group_barrier(0x100, kReadsA, 0);
 #pragma unroll
                     for (int j = 0; j < CB; ++j) {
-#pragma unroll
-                        for (int i = 0; i < AB; ++i) {
-                            __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-                            __builtin_amdgcn_sched_group_barrier(0x020, kLoadsPer, 0);
-                        }
+                        __builtin_amdgcn_sched_group_barrier(0x008, AB, 0);
+                        __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
                         __builtin_amdgcn_sched_group_barrier(0x100, kReadsB, 0);
                     }
                     if constexpr (kLoadX) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
-                    if constexpr (kPrefetch) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
                     if constexpr (kGatherK) __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
                 }
             }
         };
-        // waits of a step: all but the newest load when that is the previous step's prefetch; in a tile's first step the
-        // stores of the previous epilogue (or the cold start's stand-ins) and the one load of the bias values are newer
-        // than the loads waited for as well
+        // What the second barrier of a step waits for: all but the four loads behind the first barrier; in a tile's first step the
+        // stores of the previous epilogue (or the cold start's stand-ins) and the one load of the bias values are newer than the
+        // loads waited for as well, from the second on they are older.
         // (kGatherK: and the request for row_index entries that follows every step's loads. In a tile's first step that
-        // request, like the prefetch of the same step, is older than the stores, and a cold start issues none behind the
-        // loads waited for: the count stays the one of the cold start, which only waits for more in a streamed tile)
-        using WaitStep = std::integral_constant<int, waitcnt_imm((kPrefetch ? 1 : 0) + (kGatherK ? 1 : 0), true)>;
-        using WaitFirst = std::integral_constant<int, waitcnt_imm((int)kTileStores + (kPrefetch ? 1 : 0) + (BIAS ? 1 : 0), true)>;
+        // request is older than the stores, and a cold start issues none behind the loads waited for: the count stays the one of
+        // the cold start, which only waits for more in a streamed tile. A step forms the offsets of its gathered loads behind its second
+        // barrier, from the request before the last one, which that wait has seen arrive.)
+        using WaitStep = std::integral_constant<int, waitcnt_imm(kLoads + (kGatherK ? 1 : 0), false)>;
+        using WaitFirst = std::integral_constant<int, waitcnt_imm(kLoads + (int)kTileStores + (BIAS ? 1 : 0), false)>;
 
         // BIAS: the bias values of this wavefront's columns of the tile into its 128 bytes of LDS: one load by 32 lanes
         // (every wavefront issues it, so that all count the same loads), complete (loads and stores complete in issue
@@ -1264,7 +1225,6 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
                 asm volatile("" ::: "memory");
             }
             issue_bias();
-            issue_prefetch(kPfDist - 1);
             using SrcCur = std::integral_constant<int, 0>;
             using SrcNext = std::integral_constant<int, 1>;
             using SrcEither = std::integral_constant<int, 2>;

@@ -5,15 +5,16 @@ Usage: python cute-kernels_amd/isa_audit.py [file.s]
 The kernels of csrc/ragged_kernel.h wait for their operand loads with `s_waitcnt vmcnt(N)` where N is a constant
 that counts the vector-memory instructions a wavefront has issued after the loads it waits for (loads and stores complete
 in issue order). The constants are derived in the source from the number of loads per K step, the number of stores an
-epilogue issues and whether a prefetch, a bias load or a request for row_index entries follows a step's loads. This script
+epilogue issues and whether a bias load or a request for row_index entries follows a step's loads. This script
 compiles the sources that instantiate them to assembly (device code only; or reads a file made with `hipcc ... --cuda-device-only -S`) and checks,
 for every instantiation of ragged_gemm_kernel, that the instruction stream has the shape those constants assume:
 
- * every wait that is followed by a barrier and the eight operand loads of a K step allows exactly the number of newer
-   instructions of a step in the loop (prefetch, request) or of a tile's first step (the epilogue's stores, prefetch, bias);
- * between the two barriers of a loop body of two K steps a wavefront issues the eight loads and exactly those extras; in the tall
-   kernels both steps of a body issue eight loads or both nine, and there are four bodies with eight: the middle of the K loops for
-   eight, four, two and one row blocks, which fetch no rows past 256 (every other step does);
+ * a K step issues four operand loads behind its first barrier, then the wait and the second barrier, then four more (tall kernels: four
+   or five) and the request, if the kernel has one, and nothing else up to the next step's first barrier;
+ * that wait allows exactly the four loads, the request of a step in the loop, or in a tile's first step the epilogue's stores and the
+   bias load;
+ * in the tall kernels both steps of a loop body of two issue the same number of loads, and there are four bodies with eight: the middle of
+   the K loops for eight, four, two and one row blocks, which fetch no rows past 256 (every other step does);
  * the cold start issues sixteen operand loads (tall kernels: eighteen), as many stand-in stores as an epilogue issues stores, and
    waits for all but the loads of the second step and the stores;
  * the three-stage loop of groups of at most 64 rows issues five loads per step and waits for all but five;
@@ -63,7 +64,7 @@ def tokens(lines):
         elif s.startswith("buffer_load_dwordx4") and " lds" in s:
             cur.append("O")  # sixteen bytes per lane into LDS: an operand load
         elif s.startswith("buffer_load_dword ") and " lds" in s:
-            cur.append("p")  # four bytes per lane into LDS: prefetch, bias, row table, row_index request across a tile boundary
+            cur.append("p")  # four bytes per lane into LDS: bias, row table, row_index request across a tile boundary
         elif s.startswith("buffer_load") or s.startswith("global_load"):
             cur.append("L")  # a load into registers
         elif s.startswith("buffer_store") or s.startswith("global_store"):
@@ -87,10 +88,9 @@ def audit(asm_path: str) -> int:
         body = lines[a:b]
         end = next((k for k, line in enumerate(body) if "s_endpgm" in line), len(body))
         blocks, waterfalls = tokens(body[:end])
-        prefetch = 1 if a_kc == b_kc else 0
         request = 1 if (vary_k and gather) else 0
         stores = EPI_STORES[epi]
-        wait_step, wait_first = prefetch + request, stores + prefetch + bias
+        wait_step, wait_first = 4 + request, 4 + stores + bias
         tag = f"{el} A_KC={a_kc} B_KC={b_kc} epilogue={epi} reduction_varies={vary_k} bias={bias} gather={gather} tall={tall}"
         found = {"step": 0, "first": 0, "body": 0, "eight": 0, "cold": 0, "thin": 0}
 
@@ -104,34 +104,37 @@ def audit(asm_path: str) -> int:
         for blk in blocks:
             if "X" in blk:
                 fail("scratch access", blk)
-            # waits in front of a barrier that the operand loads of a K step follow
+            # the steps: in front of the second barrier four operand loads since the first
+            for before, w, after in re.findall(r"\|([OLp]+|(?:[OLp]|w\d+,)*?)w(\d+),\|((?:[OLp]|w\d+,)*)", blk):
+                n, count = int(w), before.count("O")
+                if count != 4:
+                    continue
+                if len(re.sub(r"w\d+,", "", before)) != 4:
+                    fail(f"{before} between the barriers of a step, expected four operand loads", blk)
+                if n == wait_step:
+                    found["step"] += 1
+                elif n == wait_first:
+                    found["first"] += 1
+                else:
+                    fail(f"a step waits for all but {n}, expected {wait_step} or {wait_first}", blk)
+                behind = after.count("O")
+                if behind not in (4, 4 + tall):
+                    fail(f"{behind} operand loads behind the second barrier", blk)
+            # the three-stage loop
             for w, loads in re.findall(r"w(\d+),\|(O+)", blk):
-                n, count = int(w), len(loads)
-                if count in (8, 8 + tall):
-                    if n == wait_step:
-                        found["step"] += 1
-                    elif n == wait_first:
-                        found["first"] += 1
-                    elif n == 8 + tall + stores:
-                        pass  # (the cold start's wait directly followed by the first step: not a shape the compiler produces)
-                    else:
-                        fail(f"a step waits for all but {n}, expected {wait_step} or {wait_first}", blk)
-                elif count == 5:
-                    if n == 5:
-                        found["thin"] += 1
-                    else:
-                        fail(f"a three-stage step waits for all but {n}, expected 5", blk)
-            # a loop body of two steps in one block: what is issued between its two barriers
-            for between, second in re.findall(r"\|(O{8}[^|]*?)w\d+,\|(O{8,})", blk):
-                if between.count("O") != len(second):
-                    fail(f"{between.count('O')} and {len(second)} operand loads in the two steps of a body", blk)
-                found["eight"] += len(second) == 8
+                if len(loads) == 5 and int(w) == 5 and "|OOOOw" not in blk:
+                    found["thin"] += 1
+            # a loop body of two steps in one block: what is issued from the first step's second barrier to the second step's first
+            # barrier, and behind the second step's second barrier
+            for between, second in re.findall(r"\|O{4}w\d+,\|([^|]*)\|O{4}w\d+,\|((?:[OLp]|w\d+,)*)", blk):
+                if between.count("O") != second.count("O"):
+                    fail(f"{between.count('O')} and {second.count('O')} operand loads in the second halves of a body's steps", blk)
+                found["eight"] += second.count("O") == 4
                 issued = len(re.sub(r"w\d+,", "", between))
-                if issued in (8 + wait_step, 8 + tall + wait_step):
+                if issued in (4 + request, 4 + tall + request):
                     found["body"] += 1
                 else:
-                    fail(f"{issued} instructions between the barriers of two steps, expected {8 + wait_step}"
-                         + (f" or {9 + wait_step}" if tall else ""), blk)
+                    fail(f"{issued} instructions between two steps, expected {4 + request}" + (f" or {5 + request}" if tall else ""), blk)
             # the cold start: sixteen operand loads (the gathered kinds mix loads of row_index entries in), the stand-in
             # stores, the wait
             cold = re.search(r"((?:[OLp]|w\d+,)*O)(s+)w(\d+),\|", blk)
