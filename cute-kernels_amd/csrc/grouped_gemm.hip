@@ -575,7 +575,7 @@ __global__ __launch_bounds__(NWM* NWN * 64) void grouped_gemm_kernel(const GemmA
             const uint8_t* const b_lo[3] = {s_b0, s_b1, s_a0 + 16384};
             const uint8_t* const b_hi[3] = {s_b0 + 16384, s_b1 + 16384, s_a1 + 16384};
             auto issue_thin = [&](int st, uint32_t k0) {
-                if constexpr (A_KC) lk_a.issue_quiet_first_rows(lds_address(a_at[st]), k0);
+                if constexpr (A_KC) lk_a.template issue_quiet_first_rows<1>(lds_address(a_at[st]), k0);
                 if constexpr (B_KC) lk_b.issue_quiet_halves(lds_address(b_lo[st]), lds_address(b_hi[st]), k0);
                 else lt_b.issue_quiet_halves(lds_address(b_lo[st]), lds_address(b_hi[st]), k0);
             };

@@ -33,7 +33,7 @@
 //    bound: all-zero operands 4657 -> 4310, 5107 -> 4620).
 //  * A K loop always runs an even number of steps (a step of zeros is appended to an odd reduction length), so every tile
 //    starts in LDS stage 0 and the loop body stays two straight-line steps.
-//  * Tiles that break the pattern (groups of at most 64 rows on their three-stage loop, groups without reduction, groups
+//  * Tiles that break the pattern (groups of few rows on their three-stage loop, groups without reduction, groups
 //    that need the element-wise path) start cold: the tile before them lets its last two load slots fetch nothing and
 //    drains, and they issue their first loads themselves, followed by as many stores outside every buffer as an epilogue
 //    issues, so that the waits of the K loop are the same constants in both cases.
@@ -74,6 +74,15 @@ constexpr int kTallM = 288;                  // rows of a tall tile: 256, and on
 constexpr uint32_t kTallGroups = 256;        // groups a launch of the tall kernels may have (their table is that much shorter)
 constexpr int kRowLoads = 5;                 // loads of A rows per wavefront and K step of a tall tile (otherwise four)
 constexpr int kExtraBytes = (kTallM - BM) * kRowBytes;  // LDS of the rows past 256, per stage
+// The three-stage K loop: groups of at most 64 rows, and without a bias of at most kShortRows where the reduction has kShortSteps K steps
+// and more (with one, isa_audit.py finds loops around the loads of the kernels that have both). Such a group has one row tile, whose panels
+// of B no other workgroup reads: a stream of the weights, with one more K step in flight than two stages hold and with the non-temporal
+// hint (a compute unit streams from HBM at 6.2 TB/s / 256 without, 6.9 with it). What it pays is that its tiles start cold, which short
+// reductions feel. Two stages, plain loads -> this, us: [128 x 96 rows, 3072 x 4096] 705 -> 638, its input gradient 545 -> 534; [8 x 96,
+// 28672 x 4096] 434 -> 408, [8 x 96, 4096 x 14336] 270 -> 261, [8 x 100, 16384 x 2048] 140 -> 137; 24 K steps, [128 x 128, 4096 x 1536], 371
+// -> 378 (hence the line); at 48 rows the hint alone 638 -> 619, gradient 526 -> 509. The hint on all tiles: 4 to 17 % slower where
+// row tiles share a panel, and 1 to 2 % at 200 to 256 rows on 128 experts.
+constexpr uint32_t kShortRows = 128, kShortSteps = 32;
 constexpr int kStageBytes = 2048;            // epilogue staging per wavefront: 16 rows of 128 bytes or 32 rows of 64
 
 struct Args {
@@ -486,8 +495,11 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
         const uint32_t left = all - t.part * args.split_steps;
         return left < args.split_steps ? left : args.split_steps;
     };
-    // groups of at most 64 rows run a K loop of their own with a third LDS stage (grouped_gemm.hip); they start cold
-    auto is_thin = [&](const Tile& t) { return A_KC && t.Me <= 64u && k_steps(t) >= 3u; };
+    // groups of few rows run a K loop of their own with a third LDS stage; they start cold
+    auto is_thin = [&](const Tile& t) {
+        if constexpr (BIAS) return A_KC && t.Me <= 64u && k_steps(t) >= 3u;
+        return A_KC && t.Me <= kShortRows && k_steps(t) >= (t.Me <= 64u ? 3u : kShortSteps);
+    };
     // a tile whose first two K steps can be fetched by the tile before it, and which can fetch the next tile's
     // (gathered reduction rows: their indices are fetched two K steps ahead of the loads, four ahead of the step itself,
     // which looks at most one tile ahead if every tile in the stream has four steps)
@@ -1134,18 +1146,21 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
         const bool has_columns = n0 + wn * (kGlu ? WN / 2 : WN) < n_lim;
         const uint32_t row_blocks = has_columns ? uniform((wave_rows + 15u) / 16u) : 0u;  // of 16 rows
         if (thin) {
-            // three LDS stages in the space a tile of at most 64 rows leaves unused (grouped_gemm.hip); cold start
-            constexpr uint32_t kThinLoads = 1 + kLoads;
-            static_assert(kThinLoads == 5, "the waits below are written for five loads per step");
-            const uint8_t* const a_at[3] = {s_a0, s_a1, s_a0 + 8192};
+            // three LDS stages in the space that a tile of at most 64 rows leaves unused, or of at most 128 rows and the epilogue's
+            // staging buffer; cold start
+            constexpr int kThinA = BIAS ? 1 : 2;  // loads of A per wavefront and step, 64 rows each
+            constexpr uint32_t kThinLoads = kThinA + kLoads;
+            const uint8_t* const a_at[3] = {s_a0, s_a1, kThinA == 1 ? s_a0 + 8192 : s_stage};
             const uint8_t* const b_lo[3] = {s_b0, s_b1, s_a0 + 16384};
             const uint8_t* const b_hi[3] = {s_b0 + 16384, s_b1 + 16384, s_a1 + 16384};
             auto issue_thin = [&](int st, uint32_t k0) {
                 if constexpr (GATHER) {
                     uint32_t v[kRowLoads];
                     g_offsets(round & 1u, k0, v);
-                    buffer_load_lds_quiet(make_rsrc_words(args.A, g_full), v[0], k0 * 2u, lds_address(a_at[st]) + wave * 1024u);
-                } else if constexpr (A_KC) lk_a.issue_quiet_first_rows(lds_address(a_at[st]), k0);
+#pragma unroll
+                    for (int i = 0; i < kThinA; ++i)
+                        buffer_load_lds_quiet(make_rsrc_words(args.A, g_full), v[i], k0 * 2u, lds_address(a_at[st]) + (uint32_t)(i * NW) * 1024u + wave * 1024u);
+                } else if constexpr (A_KC) lk_a.template issue_quiet_first_rows<kThinA>(lds_address(a_at[st]), k0);
                 if constexpr (B_KC) lk_b.issue_quiet_halves(lds_address(b_lo[st]), lds_address(b_hi[st]), k0);
                 else lt_b.issue_quiet_halves(lds_address(b_lo[st]), lds_address(b_hi[st]), k0);
             };
@@ -1197,7 +1212,11 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
                 if (kt < KT) thin_step(0, kt);
                 if (kt + 1 < KT) thin_step(1, kt + 1);
             };
-            if (row_blocks > 2) thin_loop(std::integral_constant<int, 4>{});
+            if constexpr (kThinA > 1) {
+                if (row_blocks > 4) thin_loop(std::integral_constant<int, 8>{});
+            }
+            if (kThinA > 1 && row_blocks > 4) {}
+            else if (row_blocks > 2) thin_loop(std::integral_constant<int, 4>{});
             else if (row_blocks == 2) thin_loop(std::integral_constant<int, 2>{});
             else if (row_blocks == 1) thin_loop(std::integral_constant<int, 1>{});
             else thin_loop(std::integral_constant<int, 0>{});

@@ -17,7 +17,7 @@ for every instantiation of ragged_gemm_kernel, that the instruction stream has t
    the K loops for eight, four, two and one row blocks, which fetch no rows past 256 (every other step does);
  * the cold start issues sixteen operand loads (tall kernels: eighteen), as many stand-in stores as an epilogue issues stores, and
    waits for all but the loads of the second step and the stores;
- * the three-stage loop of groups of at most 64 rows issues five loads per step and waits for all but five;
+ * the three-stage loop of groups of few rows issues five loads per step with a bias and otherwise six, and waits for all but as many;
  * no instantiation touches scratch memory, and none contains a loop over the distinct values of an operand that the
    hardware wants in scalar registers (what the compiler generates around a vector-memory instruction whose descriptor or
    scalar offset it cannot prove to be the same in every lane: each costs a dozen instructions and a branch per use).
@@ -122,7 +122,7 @@ def audit(asm_path: str) -> int:
                     fail(f"{behind} operand loads behind the second barrier", blk)
             # the three-stage loop
             for w, loads in re.findall(r"w(\d+),\|(O+)", blk):
-                if len(loads) == 5 and int(w) == 5 and "|OOOOw" not in blk:
+                if len(loads) in (5, 6) and int(w) == len(loads) and "|OOOOw" not in blk:
                     found["thin"] += 1
             # a loop body of two steps in one block: what is issued from the first step's second barrier to the second step's first
             # barrier, and behind the second step's second barrier

@@ -169,3 +169,33 @@ def test_many_tiles_per_workgroup():
     for e, m in enumerate(sizes):
         assert torch.equal(results[0][at : at + m], (x[at : at + m].double() @ w[e].T.double()).bfloat16()), f"group {e}"
         at += m
+
+
+@pytest.mark.parametrize("K", [1984, 2040, 2048, 2120])  # 31 K steps: two LDS stages from 65 rows on; 32 (the last partial or whole), 34
+@pytest.mark.parametrize("tB", [True, False])
+def test_groups_around_the_three_stage_loop(tB, K):
+    """groups on either side of 64 and 128 rows, after each other in every workgroup: packed, gathered and with the activation, against
+    a float64 product of integer operands (|sum| <= 9 K < 2^24: exact in fp32)"""
+    sizes = [64, 65, 128, 129, 1, 100, 0, 127, 300, 63, 80, 256, 112, 16, 113, 96] * 3
+    N = 520
+    x, w, bias = _inputs(sizes, N, K, torch.bfloat16, (N, K) if tB else (K, N))
+    E, R = len(sizes), sum(sizes)
+    w, bias = w[:E], bias[:E].contiguous()
+    out = _fresh(R, N, dtype=x.dtype)
+    grouped_gemm_ragged_cuda(x, w, out, _u32(sizes), False, 0, N, K, False, tB, None)
+    at = 0
+    for e, m in enumerate(sizes):
+        assert torch.equal(out[at : at + m], (x[at : at + m].double() @ (w[e].T if tB else w[e]).double()).bfloat16()), f"group {e} of {m} rows"
+        at += m
+    if not tB:
+        return
+    row_index = torch.randperm(R, device=DEV).int()
+    packed = torch.empty_like(x)
+    gather_rows_cuda(x, row_index, 1, packed)
+    h, act, gh, gact, gact_only = (_fresh(R, n, dtype=x.dtype) for n in (N - 8, (N - 8) // 2, N - 8, (N - 8) // 2, (N - 8) // 2))
+    w, bias = w[:, : N - 8].contiguous(), bias[:, : N - 8].contiguous()
+    grouped_gemm_ragged_cuda(packed, w, h, _u32(sizes), False, 0, N - 8, K, False, True, bias)
+    grouped_gemm_gathered_cuda(x, row_index, 1, w, bias, _u32(sizes), gh, gact)
+    grouped_gemm_gathered_cuda(x, row_index, 1, w, bias, _u32(sizes), None, gact_only)
+    grouped_gemm_swiglu_cuda(packed, w, _u32(sizes), None, act, bias)
+    assert torch.equal(h, gh) and torch.equal(act, gact) and torch.equal(act, gact_only)
