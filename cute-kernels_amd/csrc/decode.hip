@@ -10,10 +10,23 @@
 //  * topk_index_kernel: ONE workgroup turns the logits of up to 1024 (token, choice) slots into weights, choice, counts, offsets
 //    and both permutations: keys stay in registers, choices, histograms and ranks in LDS. It replaces the top-k tail of the router, the
 //    scan and the placement.
+//  * One token with up to eight choices needs no index: its two products choose their experts from the logits, and the second one
+//    combines (thin_experts.hip).
 #include "gemm_parts.h"
 #include "router_logits.h"
 
 namespace fmahip {
+namespace gemm {
+namespace thin {
+// thin_experts.hip
+int check(const char* who, const void* x, int64_t x_rows, const int32_t* row_index, int32_t divisor, const void* W,
+          const void* out, const uint32_t* counts, const uint32_t* offsets, int64_t R, int64_t E, int64_t N, int64_t K, int swiglu,
+          int dtype);
+bool takes_one_token(int64_t T, int64_t top_k);
+int one_token(const void* x, const void* logits, const void* W1, const void* bias1, const void* W2, const void* bias2, void* act, void* y,
+              int64_t E, int64_t H, int64_t I, int64_t top_k, int dtype, hipStream_t st);
+}  // namespace thin
+}  // namespace gemm
 namespace {
 
 constexpr int kIndexThreads = 1024;
@@ -91,11 +104,16 @@ __global__ __launch_bounds__(kIndexThreads) void topk_index_kernel(RouterArgs a,
 }
 
 template <typename EL>
-int launch_router_index(const RouterArgs& a, uint32_t* counts, uint32_t* offsets, int32_t* perm, int32_t* inv, hipStream_t st) {
+int launch_router_logits(const RouterArgs& a, hipStream_t st) {
     const dim3 grid((uint32_t)((a.T + kTok - 1) / kTok), (uint32_t)((a.E + 15) / 16));
     if (a.E <= 16) hipLaunchKernelGGL((router_logits_kernel<EL, true>), grid, dim3(256), 0, st, a);
     else hipLaunchKernelGGL((router_logits_kernel<EL, false>), grid, dim3(256), 0, st, a);
-    int rc = launch_status("router_topk_index (logits)");
+    return launch_status("router_topk_index (logits)");
+}
+
+template <typename EL>
+int launch_router_index(const RouterArgs& a, uint32_t* counts, uint32_t* offsets, int32_t* perm, int32_t* inv, hipStream_t st) {
+    const int rc = launch_router_logits<EL>(a, st);
     if (rc) return rc;
     uint32_t nbits = 0;
     while ((1u << nbits) < (uint32_t)a.E) ++nbits;
@@ -112,6 +130,34 @@ int launch_router_index(const RouterArgs& a, uint32_t* counts, uint32_t* offsets
 
 int64_t round_up(int64_t n) { return (n + 255) / 256 * 256; }
 
+int check_router(const char* who, const void* x, const void* gate_weight, int64_t T, int64_t H, int64_t E, int64_t top_k, void* logits,
+                 int dtype) {
+    FMA_REQUIRE(dtype == FMA_BF16 || dtype == FMA_F16, FMA_ERR_BAD_DTYPE, "%s: dtype must be FMA_BF16 or FMA_F16 (got %d)", who, dtype);
+    FMA_REQUIRE(E >= 1 && E <= FMA_MAX_DECODE_EXPERTS, FMA_ERR_TOO_MANY_EXPERTS, "%s: E must be in [1, %d] (got %lld)", who,
+                FMA_MAX_DECODE_EXPERTS, (long long)E);
+    FMA_REQUIRE(top_k >= 1 && top_k <= E && top_k <= FMA_MAX_ROUTER_TOP_K, FMA_ERR_BAD_SIZE,
+                "%s: top_k must be in [1, min(E, %d)] (got %lld)", who, FMA_MAX_ROUTER_TOP_K, (long long)top_k);
+    FMA_REQUIRE(T >= 1 && T <= FMA_MAX_DECODE_ROWS && T * top_k <= FMA_MAX_DECODE_ROWS, FMA_ERR_BAD_SIZE,
+                "%s: T * top_k must be in [1, %d] (T=%lld, top_k=%lld)", who, FMA_MAX_DECODE_ROWS, (long long)T, (long long)top_k);
+    FMA_REQUIRE(H >= 8 && H % 8 == 0 && H < (1 << 21), FMA_ERR_BAD_SIZE, "%s: H must be a multiple of 8 in [8, 2^21) (got %lld)",
+                who, (long long)H);
+    FMA_REQUIRE(x && gate_weight && logits, FMA_ERR_NULL_POINTER, "%s: NULL pointer", who);
+    FMA_REQUIRE(aligned16(x) && aligned16(gate_weight), FMA_ERR_MISALIGNED, "%s: x and gate_weight must be 16-byte aligned", who);
+    return FMA_OK;
+}
+
+RouterArgs router_args(const void* x, const void* gate_weight, int64_t T, int64_t H, int64_t E, int64_t top_k, void* logits) {
+    RouterArgs a{};
+    a.x = (const uint16_t*)x;
+    a.w = (const uint16_t*)gate_weight;
+    a.logits = (uint16_t*)logits;
+    a.T = T;
+    a.H = (int32_t)H;
+    a.E = (int32_t)E;
+    a.k = (int32_t)top_k;
+    return a;
+}
+
 }  // namespace
 }  // namespace fmahip
 
@@ -122,27 +168,11 @@ int fma_router_topk_index(const void* x, const void* gate_weight, int64_t T, int
                           void* stream) {
     using namespace fmahip;
     const char* who = "router_topk_index";
-    FMA_REQUIRE(dtype == FMA_BF16 || dtype == FMA_F16, FMA_ERR_BAD_DTYPE, "%s: dtype must be FMA_BF16 or FMA_F16 (got %d)", who, dtype);
-    FMA_REQUIRE(E >= 1 && E <= FMA_MAX_DECODE_EXPERTS, FMA_ERR_TOO_MANY_EXPERTS, "%s: E must be in [1, %d] (got %lld)", who,
-                FMA_MAX_DECODE_EXPERTS, (long long)E);
-    FMA_REQUIRE(top_k >= 1 && top_k <= E && top_k <= FMA_MAX_ROUTER_TOP_K, FMA_ERR_BAD_SIZE,
-                "%s: top_k must be in [1, min(E, %d)] (got %lld)", who, FMA_MAX_ROUTER_TOP_K, (long long)top_k);
-    FMA_REQUIRE(T >= 1 && T <= FMA_MAX_DECODE_ROWS && T * top_k <= FMA_MAX_DECODE_ROWS, FMA_ERR_BAD_SIZE,
-                "%s: T * top_k must be in [1, %d] (T=%lld, top_k=%lld)", who, FMA_MAX_DECODE_ROWS, (long long)T, (long long)top_k);
-    FMA_REQUIRE(H >= 8 && H % 8 == 0 && H < (1 << 21), FMA_ERR_BAD_SIZE, "%s: H must be a multiple of 8 in [8, 2^21) (got %lld)",
-                who, (long long)H);
-    FMA_REQUIRE(x && gate_weight && logits && weights && counts && offsets && perm && inv, FMA_ERR_NULL_POINTER,
-                "%s: NULL pointer", who);
-    FMA_REQUIRE(aligned16(x) && aligned16(gate_weight), FMA_ERR_MISALIGNED, "%s: x and gate_weight must be 16-byte aligned", who);
-    RouterArgs a{};
-    a.x = (const uint16_t*)x;
-    a.w = (const uint16_t*)gate_weight;
-    a.logits = (uint16_t*)logits;
+    const int rc = check_router(who, x, gate_weight, T, H, E, top_k, logits, dtype);
+    if (rc) return rc;
+    FMA_REQUIRE(weights && counts && offsets && perm && inv, FMA_ERR_NULL_POINTER, "%s: NULL pointer", who);
+    RouterArgs a = router_args(x, gate_weight, T, H, E, top_k, logits);
     a.weights = (uint16_t*)weights;
-    a.T = T;
-    a.H = (int32_t)H;
-    a.E = (int32_t)E;
-    a.k = (int32_t)top_k;
     hipStream_t st = (hipStream_t)stream;
     return dtype == FMA_BF16 ? launch_router_index<RouterBf16>(a, counts, offsets, perm, inv, st)
                              : launch_router_index<RouterF16>(a, counts, offsets, perm, inv, st);
@@ -179,7 +209,21 @@ int fma_moe_decode(const void* x, const void* gate_weight, const void* W1, const
     const int64_t experts_bytes = fma_thin_swiglu_experts_workspace_bytes(R, I);
     void* experts = take(experts_bytes);
     void* out = take(2 * R * H);
-    int rc = fma_router_topk_index(x, gate_weight, T, H, E, top_k, logits, weights, counts, offsets, perm, inv, dtype, stream);
+    int rc;
+    if (gemm::thin::takes_one_token(T, top_k)) {
+        const char* who = "moe_decode";
+        hipStream_t st = (hipStream_t)stream;
+        rc = check_router(who, x, gate_weight, T, H, E, top_k, logits, dtype);
+        if (!rc) rc = gemm::thin::check(who, x, T, perm, 1, W1, experts, counts, offsets, R, E, 2 * I, H, 1, dtype);
+        if (!rc) rc = gemm::thin::check(who, experts, R, nullptr, 1, W2, out, counts, offsets, R, E, H, I, 0, dtype);
+        if (rc) return rc;
+        FMA_REQUIRE(y, FMA_ERR_NULL_POINTER, "moe_decode: NULL pointer");
+        FMA_REQUIRE((reinterpret_cast<uintptr_t>(y) & 1u) == 0, FMA_ERR_MISALIGNED, "moe_decode: y not aligned to the element size");
+        const RouterArgs a = router_args(x, gate_weight, T, H, E, top_k, logits);
+        rc = dtype == FMA_BF16 ? launch_router_logits<RouterBf16>(a, st) : launch_router_logits<RouterF16>(a, st);
+        return rc ? rc : gemm::thin::one_token(x, logits, W1, bias1, W2, bias2, experts, y, E, H, I, top_k, dtype, st);
+    }
+    rc = fma_router_topk_index(x, gate_weight, T, H, E, top_k, logits, weights, counts, offsets, perm, inv, dtype, stream);
     if (rc) return rc;
     // (a token's choices are distinct: no expert has more than T rows)
     rc = fma_thin_swiglu_experts(x, T, perm, (int32_t)top_k, W1, bias1, W2, bias2, out, counts, offsets, R, T, E, H, I, experts,

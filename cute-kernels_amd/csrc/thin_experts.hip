@@ -30,6 +30,7 @@
 // With the hint the last two take 269 and 215 us; with the smaller token blocks of a short last pass, which then runs ahead of the
 // others, 48 tokens of the third take 286 instead of 230 us.
 #include "gemm_parts.h"
+#include "router_parts.h"
 
 namespace fmahip {
 namespace gemm {
@@ -339,6 +340,165 @@ namespace fmahip {
 namespace gemm {
 namespace thin {
 
+// ---- one token -------------------------------------------------------------------------------------------------
+// A step of one token is bound by its launches: of 41 us (hidden 2048, I 1408, E 64, k 8) the weights need 24, and router logits, top-k
+// and index, two products and combine are five kernels that each fill and drain the chip. Each choice is a group of its own here, in the
+// order of the choice, so no index is needed: every wavefront of the products reads the top-k off the logits by itself (about as long as
+// looking its expert up in the counts took), and the second product's workgroup holds the same 8 columns of all choices, a wavefront
+// for two of them, whose rounded results it combines through LDS. Three launches, the same bits. Whole layer, replayed from a graph, us: hidden 2048, I 1408,
+// E 64, k 8 39.9 -> 33.0; I 1024 33.7 -> 26.8; hidden 2048, I 768, E 128, k 8 31.4 -> 26.1; hidden 4096, I 1536, E 128, k 8 69.4 -> 62.4; hidden
+// 2880, I 2880, E 32, k 4 49.2 -> 44.9; hidden 2048, I 8192, E 8, k 2 65.5 -> 58.9; hidden 4096, I 14336, E 8, k 2 137.5 -> 130.9. With 16
+// columns and a wavefront per choice in a workgroup of the second product (128 workgroups for 2048 columns) the first takes 37.8.
+constexpr uint32_t kMostChoices = 8;  // two per wavefront of a workgroup of the second product
+
+// The first `rounds` choices of the one token, choice j in lane j of every sixteen; NK = ceil(E / 16) and more keys per lane
+template <typename RT, int NK>
+__device__ __forceinline__ uint32_t choices(const uint16_t* logits, uint32_t E, uint32_t rounds, uint32_t lane) {
+    const uint32_t c = lane & 15u;
+    uint32_t keys[NK], mine = 0;
+#pragma unroll
+    for (int i = 0; i < NK; ++i) {
+        const uint32_t n = c + 16u * i;
+        keys[i] = n < E ? make_key<RT>(logits[n], (int)n) : 0u;
+    }
+    for (uint32_t j = 0; j < rounds; ++j) {
+        uint32_t best = keys[0];
+#pragma unroll
+        for (int i = 1; i < NK; ++i) best = max(best, keys[i]);
+        best = row16_max(best);  // top_k <= E: a real key, and no two keys are equal
+#pragma unroll
+        for (int i = 0; i < NK; ++i) keys[i] = keys[i] == best ? 0u : keys[i];
+        if (c == j) mine = best;
+    }
+    return mine;
+}
+__device__ __forceinline__ uint32_t expert_of_choice(uint32_t mine, uint32_t j) {
+    return uniform((uint32_t)key_column((uint32_t)__builtin_amdgcn_readlane((int)mine, (int)j)));
+}
+
+// row j of a.out: the activation of the token's first projection by the expert of choice j
+template <typename EL, typename RT, int ROWS, int NK, bool BIAS>
+__global__ __launch_bounds__(64) void one_token_up_kernel(Args a, const uint16_t* __restrict__ logits) {
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[Config<ROWS>::kLds];
+    const uint32_t j = blockIdx.x / a.units, u = blockIdx.x - j * a.units;
+    const uint32_t e = expert_of_choice(choices<RT, NK>(logits, a.E, j + 1u, threadIdx.x), j);
+    a.out += (uint64_t)j * (a.N / 2);
+    unit<EL, ROWS, true, BIAS, 1, true>(a, lds, e, 0u, 1u, u * (ROWS / 2));
+}
+
+// Columns n0 .. n0 + 7 of the second projection for two choices, rows `x` and the one behind it (rows: how many of them exist), by the experts
+// e0 and e1: the sixteen weight rows of a matrix instruction are eight of each expert, and of its sixteen by sixteen results the two
+// blocks of eight that belong together are used. Results, rounded, to s_o[0] and s_o[1].
+template <typename EL, bool BIAS, int STAGES>
+__device__ __forceinline__ void pair_unit(const Args& a, uint8_t* lds, const uint16_t* x, uint32_t rows, uint32_t e0, uint32_t e1, uint32_t n0,
+                                          uint16_t (*s_o)[8]) {
+    using frag = typename EL::frag;
+    constexpr uint32_t kStage = 24 * kKB;  // sixteen weight rows and eight of x
+    constexpr int kIPS = 3;
+    static_assert(kIPS * (STAGES - 1) < 64, "vmcnt holds six bits");
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t K2 = a.K * 2u, lr = lane >> 3, lp = lane & 7u;
+    const uint32_t n_rows = a.N - n0 < 8u ? a.N - n0 : 8u;
+    // descriptors end with the rows that exist: the rest arrives as zeros
+    const u32x4 rw0 = make_rsrc_words(a.W + ((uint64_t)e0 * a.N + n0) * a.K, n_rows * K2);
+    const u32x4 rw1 = make_rsrc_words(a.W + ((uint64_t)e1 * a.N + n0) * a.K, rows > 1u ? n_rows * K2 : 0u);
+    const u32x4 rx = make_rsrc_words(x, rows * K2);
+    const uint32_t lds0 = lds_address(lds), nsteps = (K2 + kKB - 1) / kKB;
+    auto issue = [&](uint32_t s, uint32_t slot) {
+        const uint32_t kb = s * kKB;
+#pragma unroll
+        for (uint32_t i = 0; i < 3u; ++i) {
+            const uint32_t chunk = lp ^ flip(i * kRPI + lr);
+            const uint32_t v = kb + chunk * 16u < K2 ? lr * K2 + chunk * 16u : kOutOfRange;
+            if (i < 2u) load_lds<true>(i ? rw1 : rw0, v, kb, lds0 + slot * kStage + i * 1024u);
+            else load_lds<false>(rx, v, kb, lds0 + slot * kStage + 2048u);
+        }
+    };
+    f32x4 acc = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (uint32_t d = 0; d + 1 < (uint32_t)STAGES; ++d) issue(d, d);
+    const uint32_t r16 = lane & 15u, q = lane >> 4;
+    uint32_t slot = 0, fill = STAGES - 1;
+    for (uint32_t s = 0; s < nsteps; ++s) {
+        wait_lds();  // the stage filled here was read in the previous iteration
+        issue(s + STAGES - 1, fill);
+        fill = fill == STAGES - 1 ? 0u : fill + 1u;
+        wait_vm<kIPS*(STAGES - 1)>();
+        const uint8_t* stage = lds + slot * kStage;
+        slot = slot == STAGES - 1 ? 0u : slot + 1u;
+#pragma unroll
+        for (uint32_t sl = 0; sl < 2u; ++sl) {
+            const frag w = __builtin_bit_cast(frag, read_kc_frag(stage + lds_off(r16, sl * 4u + q)));
+            const frag t = __builtin_bit_cast(frag, read_kc_frag(stage + lds_off(16u + (r16 & 7u), sl * 4u + q)));
+            acc = EL::mfma16(w, t, acc);
+        }
+    }
+    wait_vm<0>();
+    // a lane holds row r16 of x, weight rows 4 q .. 4 q + 3: row 0 with the first expert's, row 1 with the second's
+    const uint32_t c = 4u * (q & 1u);
+    if (r16 == q >> 1 && r16 < rows && n0 + c < a.N) {
+        float y[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            y[i] = acc[i];
+            if constexpr (BIAS) y[i] = EL::round(y[i]) + EL::from_bits(a.bias[(uint64_t)(r16 ? e1 : e0) * a.N + n0 + c + i]);
+        }
+        *reinterpret_cast<uint2*>(s_o[r16] + c) = uint2{EL::pack2(y[0], y[1]), EL::pack2(y[2], y[3])};
+    }
+}
+
+// KW: wavefronts of a workgroup, at least one per two choices (a.units of them)
+template <typename EL, typename RT, int NK, int KW, bool BIAS>
+__global__ __launch_bounds__(64 * KW) void one_token_down_kernel(Args a, const uint16_t* __restrict__ logits) {
+    constexpr int kStages = KW > 2 ? 6 : (KW > 1 ? 12 : 16);  // two and more workgroups fit the LDS of a compute unit
+    constexpr uint32_t kRing = kStages * 24 * kKB;
+    __shared__ __attribute__((aligned(1024))) uint8_t lds[KW * kRing];
+    __shared__ __attribute__((aligned(16))) uint16_t s_o[2 * KW][8];
+    __shared__ float s_gate[2 * KW];
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, p = uniform(tid >> 6), k = a.units, j = 2u * p;
+    const uint32_t n0 = blockIdx.x * 8u, rows = k - j < 2u ? k - j : 2u;
+    const uint32_t mine = choices<RT, NK>(logits, a.E, p == 0u ? k : j + rows, lane);
+    if (p == 0u) {
+        // the weights, with the sums of softmax_tokens (router_parts.h)
+        const float vmax = key_value<RT>((uint32_t)__builtin_amdgcn_readlane((int)mine, 0));
+        const float ex = (lane & 15u) < k ? expf(key_value<RT>(mine) - vmax) : 0.f;
+        const float sum = row16_sum(ex);
+        if (lane < k) s_gate[lane] = RT::from_bits(RT::bits(ex / sum));
+    }
+    pair_unit<EL, BIAS, kStages>(a, lds + p * kRing, a.x + (uint64_t)j * a.K, rows, expert_of_choice(mine, j),
+                                 expert_of_choice(mine, j + rows - 1u), n0, s_o + j);
+    __syncthreads();
+    if (tid < 8u && n0 + tid < a.N) {
+        float acc = 0.f;
+        for (uint32_t i = 0; i < k; ++i) acc = fmaf(s_gate[i], RT::from_bits(s_o[i][tid]), acc);
+        a.out[n0 + tid] = RT::bits(acc);
+    }
+}
+
+template <typename EL, typename RT, int NK, bool BIAS1, bool BIAS2>
+int launch_one_token(Args up, Args down, const uint16_t* logits, uint32_t k, hipStream_t st) {
+    const uint32_t I = up.N / 2;
+    const bool half = half_units(up, true, k);
+    up.units = (I + (half ? 7u : 15u)) / (half ? 8u : 16u);
+    if (half) hipLaunchKernelGGL((one_token_up_kernel<EL, RT, 16, NK, BIAS1>), dim3(k * up.units), dim3(64), 0, st, up, logits);
+    else hipLaunchKernelGGL((one_token_up_kernel<EL, RT, 32, NK, BIAS1>), dim3(k * up.units), dim3(64), 0, st, up, logits);
+    const int rc = launch_status("moe_decode (one token, up)");
+    if (rc) return rc;
+    down.units = k;
+    const dim3 grid((down.N + 7u) / 8u), block(64u * ((k + 1u) / 2u));
+    if (k <= 2) hipLaunchKernelGGL((one_token_down_kernel<EL, RT, NK, 1, BIAS2>), grid, block, 0, st, down, logits);
+    else if (k <= 4) hipLaunchKernelGGL((one_token_down_kernel<EL, RT, NK, 2, BIAS2>), grid, block, 0, st, down, logits);
+    else hipLaunchKernelGGL((one_token_down_kernel<EL, RT, NK, 4, BIAS2>), grid, block, 0, st, down, logits);
+    return launch_status("moe_decode (one token, down)");
+}
+template <typename EL, typename RT, int NK>
+int launch_one_token(const Args& up, const Args& down, const uint16_t* logits, uint32_t k, hipStream_t st) {
+    if (up.bias) return down.bias ? launch_one_token<EL, RT, NK, true, true>(up, down, logits, k, st)
+                                  : launch_one_token<EL, RT, NK, true, false>(up, down, logits, k, st);
+    return down.bias ? launch_one_token<EL, RT, NK, false, true>(up, down, logits, k, st)
+                     : launch_one_token<EL, RT, NK, false, false>(up, down, logits, k, st);
+}
+
 // Up to 16 rows per expert on average 32 weight rows per wavefront, beyond that 64. Up / down projection, E 8, k 2, hidden
 // 4096, I 14336: 16 rows (64 tokens) 317 / 154 us against 322 / 150 us, 32 rows 466 / 227 against 334 / 167 us; the shape
 // with E 128 at 6 rows 506 / 244 against 531 / 250 us, E 64 at one row 16.8 / 9.3 against 18.6 / 11.6 us.
@@ -392,6 +552,31 @@ int product(const void* x, int64_t x_rows, const int32_t* row_index, int32_t div
     const bool w = wide(R, E), glu = swiglu != 0;
     if (dtype == FMA_BF16) return w ? launch<ElemBf16, 64>(a, glu, R, groups, max_rows, st) : launch<ElemBf16, 32>(a, glu, R, groups, max_rows, st);
     return w ? launch<ElemF16, 64>(a, glu, R, groups, max_rows, st) : launch<ElemF16, 32>(a, glu, R, groups, max_rows, st);
+}
+
+// The expert path of one token (decode.hip): act [top_k, I] is scratch, y [H] the layer's output. E up to FMA_MAX_DECODE_EXPERTS.
+bool takes_one_token(int64_t T, int64_t top_k) { return T == 1 && top_k <= (int64_t)kMostChoices; }
+int one_token(const void* x, const void* logits, const void* W1, const void* bias1, const void* W2, const void* bias2, void* act, void* y,
+              int64_t E, int64_t H, int64_t I, int64_t top_k, int dtype, hipStream_t st) {
+    Args up{}, down{};
+    up.x = (const uint16_t*)x;
+    up.W = (const uint16_t*)W1;
+    up.bias = (const uint16_t*)bias1;
+    up.out = (uint16_t*)act;
+    up.N = (uint32_t)(2 * I);
+    up.K = (uint32_t)H;
+    down.x = (const uint16_t*)act;
+    down.W = (const uint16_t*)W2;
+    down.bias = (const uint16_t*)bias2;
+    down.out = (uint16_t*)y;
+    down.N = (uint32_t)H;
+    down.K = (uint32_t)I;
+    up.E = down.E = (uint32_t)E;
+    up.divisor = down.divisor = 1;
+    const uint16_t* l = (const uint16_t*)logits;
+    const uint32_t k = (uint32_t)top_k;
+    if (dtype == FMA_BF16) return E <= 64 ? launch_one_token<ElemBf16, RouterBf16, 4>(up, down, l, k, st) : launch_one_token<ElemBf16, RouterBf16, 16>(up, down, l, k, st);
+    return E <= 64 ? launch_one_token<ElemF16, RouterF16, 4>(up, down, l, k, st) : launch_one_token<ElemF16, RouterF16, 16>(up, down, l, k, st);
 }
 
 }  // namespace thin

@@ -298,7 +298,8 @@ int fma_router_topk_index(const void* x, const void* gate_weight, int64_t T, int
                           int dtype, void* stream);
 
 /* MoE.forward (fma/modules/moe/__init__.py:165-298) of a SwiGLU layer for a few tokens without a backward, enqueued by one
- * call: fma_router_topk_index, fma_thin_swiglu_experts, fma_combine. W1 [E, 2 I, H], W2 [E, H, I], biases
+ * call: fma_router_topk_index, fma_thin_swiglu_experts, fma_combine, or for one token and top_k <= 8 three kernels with the same
+ * results (the logits, both products, the second with the combine). W1 [E, 2 I, H], W2 [E, H, I], biases
  * [E, 2 I] / [E, H] or NULL; y [T, H] and logits [T, E] are written. The limits of fma_router_topk_index; the workspace needs no
  * initialisation. */
 int64_t fma_moe_decode_workspace_bytes(int64_t T, int64_t H, int64_t I, int64_t E, int64_t top_k);
