@@ -53,7 +53,7 @@ def _headers() -> list[str]:
 # the operands have landed. Their kernels must use no scratch memory; the build checks the compiler's resource report.
 NO_SCRATCH_SOURCES = {"grouped_gemm.hip": "grouped_gemm_kernel", "grouped_gemm_ragged.hip": "ragged_gemm_kernel",
                       "grouped_gemm_ragged_tall.hip": "ragged_gemm_kernel",
-                      "thin_experts.hip": "thin_gemm_kernel|one_token", "decode.hip": "router_logits_kernel", "router.hip": "router_logits_kernel"}
+                      "thin_experts.hip": "thin_gemm_kernel|one_token", "decode.hip": "router_logits_kernel", "router.hip": "router_logits"}
 
 
 def _check_no_scratch(src: str, report: str, kernel_pattern: str) -> None:

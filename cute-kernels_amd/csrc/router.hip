@@ -375,6 +375,78 @@ __global__ __launch_bounds__(kRouterThreads) void topk_from_logits_kernel(const 
     flush_histogram(a, s_hist, 1, tok0, tid, kRouterThreads);
 }
 
+// Logits of 64 tokens x 32 experts per workgroup, a wavefront per 16 tokens. The kernels that also choose read the router matrix through one
+// compute unit per 32 or 64 tokens, and are bound by that stream until there are several such workgroups per compute unit; here the
+// tokens and the matrix both come as direct global -> LDS loads of 256 bytes a row, five steps in flight, from the L2 for the most part (the
+// workgroups of one XCD are neighbours: the experts of the same tokens). The same sums in the same order, the same bits.
+constexpr int kTileToks = 64, kTileExps = 32, kTileStages = 6;
+template <typename EL>
+__global__ __launch_bounds__(256) void router_logits_tile_kernel(const RouterArgs a, uint32_t columns) {
+    using frag = typename EL::frag;
+    constexpr int kRows = kTileToks + kTileExps, kWaveLoads = kRows / 16;  // a load: four rows of 256 bytes
+    constexpr uint32_t kStage = kRows * kRowBytes;
+    __shared__ __attribute__((aligned(1024))) uint8_t s_ring[kTileStages][kStage];
+    const uint32_t lane = threadIdx.x & 63u, wave = gemm::uniform(threadIdx.x >> 6);
+    // workgroups go to the eight XCDs in turn: a run of neighbouring tiles each
+    const uint32_t per_xcd = gridDim.x / 8u, even = per_xcd * 8u;
+    const uint32_t tile = blockIdx.x < even ? (blockIdx.x % 8u) * per_xcd + blockIdx.x / 8u : blockIdx.x;
+    const uint32_t tok0 = tile / columns * kTileToks, e0 = tile % columns * kTileExps;
+    const uint32_t H2 = (uint32_t)a.H * 2u;
+    const uint32_t toks = (uint32_t)a.T - tok0 < (uint32_t)kTileToks ? (uint32_t)a.T - tok0 : (uint32_t)kTileToks;
+    const uint32_t exps = (uint32_t)a.E - e0 < (uint32_t)kTileExps ? (uint32_t)a.E - e0 : (uint32_t)kTileExps;
+    // rows past the end are out of the descriptors' range and arrive as zeros, and so do the chunks past the end of a row
+    const gemm::u32x4 rx = gemm::make_rsrc_words(a.x + (uint64_t)tok0 * a.H, toks * H2);
+    const gemm::u32x4 rw = gemm::make_rsrc_words(a.w + (uint64_t)e0 * a.H, exps * H2);
+    const uint32_t lr = lane >> 4, lp = lane & 15u;
+    const uint32_t nsteps = (H2 + kRowBytes - 1) / kRowBytes;
+    const uint32_t ring0 = gemm::lds_address(s_ring[0]);
+    auto issue = [&](uint32_t step, uint32_t stage) {
+        const uint32_t kb = step * kRowBytes;
+#pragma unroll
+        for (uint32_t i = 0; i < (uint32_t)kWaveLoads; ++i) {
+            const uint32_t row = (i * 4u + wave) * 4u;  // rows 0 .. 63: tokens, then experts
+            const bool x = i < (uint32_t)kTileToks / 16u;
+            const uint32_t chunk = lp ^ ((row + lr) & 15u);
+            const uint32_t v = kb + chunk * 16u < H2 ? lr * H2 + chunk * 16u : gemm::kOutOfRange;
+            gemm::load_lds<false>(x ? rx : rw, v, (x ? row : row - kTileToks) * H2 + kb, ring0 + stage * kStage + row * kRowBytes);
+        }
+    };
+    f32x4 acc[kTileExps / 16];
+#pragma unroll
+    for (int b = 0; b < kTileExps / 16; ++b) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const uint32_t r = lane & 15u, q = lane >> 4;
+#pragma unroll
+    for (uint32_t d = 0; d + 1 < (uint32_t)kTileStages; ++d) issue(d, d);  // (steps past the end fetch nothing)
+    uint32_t slot = 0, fill = kTileStages - 1;
+    for (uint32_t step = 0; step < nsteps; ++step) {
+        gemm::wait_vm<kWaveLoads*(kTileStages - 2)>();  // this step has landed; the others may be out
+        __syncthreads();                                // ... in every wavefront, and the stage filled next has been read
+        issue(step + kTileStages - 1, fill);
+        fill = fill == kTileStages - 1 ? 0u : fill + 1u;
+        const uint8_t* stage = s_ring[slot];
+        slot = slot == kTileStages - 1 ? 0u : slot + 1u;
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) {
+            const frag xf = load_frag<frag>(reinterpret_cast<const uint16_t*>(stage + chunk_off(wave * 16u + r, q * 4u + j)));
+#pragma unroll
+            for (int b = 0; b < kTileExps / 16; ++b) {
+                const frag wf = load_frag<frag>(reinterpret_cast<const uint16_t*>(stage + chunk_off(kTileToks + b * 16u + r, q * 4u + j)));
+                acc[b] = EL::mfma(xf, wf, acc[b]);
+            }
+        }
+        gemm::wait_lds();
+    }
+    gemm::wait_vm<0>();
+    // a lane holds tokens 4 q .. 4 q + 3 of expert r of each block
+#pragma unroll
+    for (int b = 0; b < kTileExps / 16; ++b)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t tok = wave * 16u + q * 4u + i, n = e0 + b * 16u + r;
+            if (tok < toks && n < (uint32_t)a.E) a.logits[(uint64_t)(tok0 + tok) * a.E + n] = EL::bits(acc[b][i]);
+        }
+}
+
 // Few tokens: logits by workgroups of 16 tokens x 16 experts, then their top-k. The kernels below read the router matrix through one
 // compute unit per 32 or 64 tokens, which takes the same time for 130 tokens as for 8192. One launch / these two, us, at 130, 512, 1024
 // and 2048 tokens: E 64, hidden 2048 15.7 / 9.1, 15.9 / 8.7, 15.9 / 9.2, 16.2 / 13.8; E 128, hidden 4096 36.4 / 12.9, 36.8 / 12.7, 37.3 /
@@ -386,10 +458,26 @@ bool few_tokens(const RouterArgs& a) {
     const int64_t groups = ((a.T + kTok - 1) / kTok) * ((a.E + 15) / 16);
     return groups <= (a.E > 32 ? 2 : 1) * cus && a.H < (1 << 21);
 }
+// More tokens: up to two rounds of tiles, and from 32 tokens per compute unit on where one column of tiles is all of the matrix. One launch /
+// tiles and top-k, us: E 128, hidden 4096, 2048, 4096, 8192 and 16384 tokens 37.7 / 20.2, 37.9 / 21.1, 40.1 / 37.7, 54.4 / 77.7 (not taken); E 64,
+// hidden 2048, 3000, 8192, 16384 and 32768 tokens 16.3 / 12.9, 17.9 / 14.5, 25.3 / 25.7, 46.1 / 53.9 (not taken); E 256, hidden 4096, 2048, 4096 and
+// 8192 tokens 68.0 / 23.2, 68.9 / 37.7, 71.5 / 68.8 (not taken); E 32, hidden 2880, 8192, 16384 and 32768 tokens 17.5 / 16.2, 32.5 / 25.2, 55.4 /
+// 43.8; E 20, hidden 4096, 3000 tokens 16.6 / 18.7 (not taken), 8192 24.3 / 20.3.
+bool some_tokens(const RouterArgs& a) {
+    const int64_t cus = num_compute_units() > 0 ? num_compute_units() : 256;
+    const int64_t tiles = ((a.T + kTileToks - 1) / kTileToks) * ((a.E + kTileExps - 1) / kTileExps);
+    return tiles <= 2 * cus && (a.E > kTileExps || a.T >= 32 * cus) && a.H < (1 << 21);
+}
 template <typename EL, int NK>
-int launch_router_few(const RouterArgs& a, hipStream_t st) {
+int launch_router_logits_first(const RouterArgs& a, bool few, hipStream_t st) {
     const uint32_t blocks = (uint32_t)((a.T + kTok - 1) / kTok);
-    hipLaunchKernelGGL((router_logits_kernel<EL, false>), dim3(blocks, (uint32_t)((a.E + 15) / 16)), dim3(256), 0, st, a);
+    if (few) {
+        hipLaunchKernelGGL((router_logits_kernel<EL, false>), dim3(blocks, (uint32_t)((a.E + 15) / 16)), dim3(256), 0, st, a);
+    } else {
+        const uint32_t columns = (uint32_t)((a.E + kTileExps - 1) / kTileExps);
+        const uint32_t tiles = (uint32_t)((a.T + kTileToks - 1) / kTileToks) * columns;
+        hipLaunchKernelGGL((router_logits_tile_kernel<EL>), dim3(tiles), dim3(256), 0, st, a, columns);
+    }
     const int rc = launch_status("router_topk (logits)");
     if (rc) return rc;
     hipLaunchKernelGGL((topk_from_logits_kernel<EL, NK>), dim3(blocks), dim3(kRouterThreads), 0, st, a);
@@ -398,7 +486,8 @@ int launch_router_few(const RouterArgs& a, hipStream_t st) {
 
 template <typename EL, int NBLK, int EMAX>
 int launch_router_wide(const RouterArgs& a, hipStream_t st) {
-    if (few_tokens(a)) return launch_router_few<EL, EMAX / 16>(a, st);
+    const bool few = few_tokens(a);
+    if (few || some_tokens(a)) return launch_router_logits_first<EL, EMAX / 16>(a, few, st);
     // 64 tokens per workgroup share each weight tile four ways; with too few tokens to give every compute unit such a
     // workgroup, 32 tokens per workgroup keep twice as many units busy
     const int64_t cus = num_compute_units() > 0 ? num_compute_units() : 256;

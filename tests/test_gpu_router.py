@@ -281,3 +281,21 @@ def test_few_tokens_give_the_bits_of_many(rows, H, E, k, dtype):
     block = (torch.arange(rows, device=DEV) // 16)[:, None].expand(rows, k)
     expect.index_put_((block, selected.long()), torch.ones_like(block), accumulate=True)
     assert torch.equal(hist.to(torch.int64), expect) and torch.equal(counts.to(torch.int64), expect.sum(0))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("H,E,k", [(520, 17, 3), (2048, 64, 8), (136, 65, 1), (1032, 130, 64), (1000, 100, 4), (4096, 256, 8), (8, 33, 2)])
+def test_tiles_give_the_bits_of_many(H, E, k, dtype):
+    """numbers of tokens whose logits come from tiles of 64 tokens x 32 experts, ragged and whole, against the launch of all of them with
+    40000 tokens, which one kernel computes"""
+    g = torch.Generator(device=DEV).manual_seed(E)
+    x = torch.randn(40000, H, device=DEV, generator=g).to(dtype)
+    w = (torch.randn(E, H, device=DEV, generator=g) / H**0.5).to(dtype)
+    many = _run_forward(x, w, k)
+    for rows in (2049, 4096, 8191, 8256):
+        hist = _block_hist_buffer(rows, E)
+        got = _run_forward(x[:rows].contiguous(), w, k, block_hist=hist)
+        for a, b in zip(got[:3], many[:3]):
+            assert torch.equal(a, b[:rows])
+        counts = torch.bincount(got[2].flatten().long(), minlength=E)
+        assert torch.equal(got[3].view(torch.int32).long(), counts) and torch.equal(hist.view(torch.int32).long().sum(0), counts)
