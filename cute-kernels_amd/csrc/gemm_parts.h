@@ -91,20 +91,13 @@ __device__ __forceinline__ u32x4 uniform(u32x4 x) {
 // issued this way, partly while the previous tile's epilogue is still running, and waited for with an exact count.
 // (s_nop 2: the scalar operands may come from a v_readfirstlane right in front of the assembly, and a vector-memory
 // instruction must not read such a register within five wait states; the compiler does not check assembly for that.)
-template <bool STREAM = false>
 __device__ __forceinline__ void buffer_load_lds_quiet(u32x4 rsrc, uint32_t voff, uint32_t soff, uint32_t lds_addr) {
     // M0 is put back afterwards: the compiler keeps its own values in it and does not honour a clobber of it
     uint32_t saved_m0;
-    if constexpr (STREAM)
-        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %4\n\ts_nop 2\n\tbuffer_load_dwordx4 %1, %2, %3 offen nt lds\n\t"
-                     "s_mov_b32 m0, %0"
-                     : "=&s"(saved_m0)
-                     : "v"(voff), "s"(uniform(rsrc)), "s"(uniform(soff)), "s"(uniform(lds_addr)));
-    else
-        asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %4\n\ts_nop 2\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds\n\t"
-                     "s_mov_b32 m0, %0"
-                     : "=&s"(saved_m0)
-                     : "v"(voff), "s"(uniform(rsrc)), "s"(uniform(soff)), "s"(uniform(lds_addr)));
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %4\n\ts_nop 2\n\tbuffer_load_dwordx4 %1, %2, %3 offen lds\n\t"
+                 "s_mov_b32 m0, %0"
+                 : "=&s"(saved_m0)
+                 : "v"(voff), "s"(uniform(rsrc)), "s"(uniform(soff)), "s"(uniform(lds_addr)));
 }
 // The same load as a compiler fence, for kernels that read what it fills with ordinary LDS reads: nothing moves across it, and the
 // wait for it is wait_vm. STREAM: with the non-temporal hint.
@@ -483,8 +476,7 @@ struct LoaderK {
         for (int i = 0; i < N; ++i)
             buffer_load_lds_quiet(make_rsrc_words(base0, bytes), v, k0 * 2u + (uint32_t)i * kRowsPerInst * ldb, lds_base + (uint32_t)(i * NW) * 1024u + wave * 1024u);
     }
-    // the NI loads with the first half of the tile's 1 KB pieces going to lds_lo and the second half to lds_hi (non-temporal: of a panel
-    // that one workgroup reads)
+    // the NI loads with the first half of the tile's 1 KB pieces going to lds_lo and the second half to lds_hi
     __device__ __forceinline__ void issue_quiet_halves(uint32_t lds_lo, uint32_t lds_hi, uint32_t k0) const {
         uint32_t v = voff;
         if (k0 + BK > kdim && k0 + chunk * 8u >= kdim) v = kOutOfRange;
@@ -495,7 +487,7 @@ struct LoaderK {
             const bool second = SPLIT && i >= NI / 2;
             const uint32_t row = (uint32_t)(second ? i - NI / 2 : i) * kRowsPerInst;
             const uint32_t lds = (i < NI / 2 ? lds_lo + (uint32_t)(i * NW) * 1024u : lds_hi + (uint32_t)((i - NI / 2) * NW) * 1024u) + wave * 1024u;
-            buffer_load_lds_quiet<true>(second ? r1 : r0, v, k0 * 2u + row * ldb, lds);
+            buffer_load_lds_quiet(second ? r1 : r0, v, k0 * 2u + row * ldb, lds);
         }
     }
 };
@@ -551,14 +543,14 @@ struct LoaderT {
             buffer_load_lds_quiet(r, voff, (uint32_t)(i * NW + wave) * 2u * ldb, lds0 + (uint32_t)(i * NW) * 1024u);
         }
     }
-    // the NI loads with k rows 0..31 of the step going to lds_lo and k rows 32..63 to lds_hi (non-temporal, as in LoaderK)
+    // the NI loads with k rows 0..31 of the step going to lds_lo and k rows 32..63 to lds_hi
     __device__ __forceinline__ void issue_quiet_halves(uint32_t lds_lo, uint32_t lds_hi, uint32_t k0) const {
         const uint32_t rows = k0 >= kdim ? 0u : (kdim - k0 < (uint32_t)BK ? kdim - k0 : (uint32_t)BK);
         const u32x4 r = make_rsrc_words(base + (uint64_t)k0 * (ldb / 2u), rows ? rows * ldb - col_bytes : 0u);
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
             const uint32_t lds = (i < NI / 2 ? lds_lo + (uint32_t)(i * NW) * 1024u : lds_hi + (uint32_t)((i - NI / 2) * NW) * 1024u) + wave * 1024u;
-            buffer_load_lds_quiet<true>(r, voff, (uint32_t)(i * NW + wave) * 2u * ldb, lds);
+            buffer_load_lds_quiet(r, voff, (uint32_t)(i * NW + wave) * 2u * ldb, lds);
         }
     }
 };

@@ -76,12 +76,14 @@ constexpr int kRowLoads = 5;                 // loads of A rows per wavefront an
 constexpr int kExtraBytes = (kTallM - BM) * kRowBytes;  // LDS of the rows past 256, per stage
 // The three-stage K loop: groups of at most 64 rows, and without a bias of at most kShortRows where the reduction has kShortSteps K steps
 // and more (with one, isa_audit.py finds loops around the loads of the kernels that have both). Such a group has one row tile, whose panels
-// of B no other workgroup reads: a stream of the weights, with one more K step in flight than two stages hold and with the non-temporal
-// hint (a compute unit streams from HBM at 6.2 TB/s / 256 without, 6.9 with it). What it pays is that its tiles start cold, which short
-// reductions feel. Two stages, plain loads -> this, us: [128 x 96 rows, 3072 x 4096] 705 -> 638, its input gradient 545 -> 534; [8 x 96,
-// 28672 x 4096] 434 -> 408, [8 x 96, 4096 x 14336] 270 -> 261, [8 x 100, 16384 x 2048] 140 -> 137; 24 K steps, [128 x 128, 4096 x 1536], 371
-// -> 378 (hence the line); at 48 rows the hint alone 638 -> 619, gradient 526 -> 509. The hint on all tiles: 4 to 17 % slower where
-// row tiles share a panel, and 1 to 2 % at 200 to 256 rows on 128 experts.
+// of B no other workgroup reads: a stream of the weights, with one more K step in flight than two stages hold. What it pays is that its
+// tiles start cold, which short reductions feel. Two stages with one barrier a step -> this, us: [128 x 96 rows, 3072 x 4096] 766 -> 671, its
+// input gradient 627 -> 578; [128 x 128 rows] 682 -> 620 and 645 -> 592; [8 x 96, 28672 x 4096] 490 -> 423, [8 x 100, 2048 x 8192] 82.7 -> 75.7,
+// [64 x 100, 512 x 2048] 44.5 -> 41.3; 24 K steps, [128 x 128, 4096 x 1536], two stages 371, this 378 (hence the line). Groups of up to 64
+// rows, which ran it before: 0 to 1 %, or 0.4 us, more per launch (a larger kernel, and a second load of rows that are not there).
+// B with the non-temporal hint: weights from memory 3 to 5 % faster ([128 x 48, 3072 x 4096] 638 -> 619), weights that the last-level cache
+// holds from the pass before up to 37 % slower ([8 x 48, 4096 x 2048] 27 -> 35, [16 x 40, 2048 x 2048] 27 -> 37); on all tiles 4 to 17 % slower
+// where row tiles share a panel. Not taken.
 constexpr uint32_t kShortRows = 128, kShortSteps = 32;
 constexpr int kStageBytes = 2048;            // epilogue staging per wavefront: 16 rows of 128 bytes or 32 rows of 64
 
