@@ -618,8 +618,9 @@ __global__ __launch_bounds__(NWM* NWN * 64) void grouped_gemm_kernel(const GemmA
                     }
                     // all but the newest five loads: step kt+1 has landed (step kt+2 may still be on its way); past the
                     // barrier every wavefront has finished reading this stage, which then takes the loads of step kt+3
-                    // (zero-filling ones past the end of K, so that the count stays the same)
-                    __builtin_amdgcn_s_waitcnt(0x0f75);
+                    // (zero-filling ones past the end of K, so that the count stays the same). lgkmcnt(0): the compiler moves
+                    // matrix instructions, and the waits for their fragments with them, past the barrier
+                    __builtin_amdgcn_s_waitcnt(0x0075);
                     __builtin_amdgcn_s_barrier();
                     asm volatile("" ::: "memory");
                     issue_thin(st, (kt + 3) * BK);
@@ -636,7 +637,7 @@ __global__ __launch_bounds__(NWM* NWN * 64) void grouped_gemm_kernel(const GemmA
             if (row_blocks == 2) thin_loop(std::integral_constant<int, 2>{});
             else if (row_blocks == 1) thin_loop(std::integral_constant<int, 1>{});
             else thin_loop(std::integral_constant<int, 0>{});
-            __builtin_amdgcn_s_waitcnt(0x0f70);
+            __builtin_amdgcn_s_waitcnt(0x0070);
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
         } else if (KT > 0) {
@@ -667,8 +668,9 @@ __global__ __launch_bounds__(NWM* NWN * 64) void grouped_gemm_kernel(const GemmA
             else if (row_blocks == 2) k_loop(std::integral_constant<int, 2>{});
             else if (row_blocks == 1) k_loop(std::integral_constant<int, 1>{});
             else k_loop(std::integral_constant<int, 0>{});
-            // the zero-fill loads issued past the end of K must have landed before the stages are reused below
-            __builtin_amdgcn_s_waitcnt(0x0f70);
+            // the zero-fill loads issued past the end of K must have landed, and every LDS read returned, before the stages are
+            // reused below
+            __builtin_amdgcn_s_waitcnt(0x0070);
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
         }

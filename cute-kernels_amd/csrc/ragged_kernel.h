@@ -1170,7 +1170,7 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
             const uint32_t k_first = kSplit ? cur.ks : 0u;
             issue_thin(0, k_first);
             issue_thin(1, k_first + BK);
-            __builtin_amdgcn_s_waitcnt(waitcnt_imm((int)kThinLoads, false));
+            __builtin_amdgcn_s_waitcnt(waitcnt_imm((int)kThinLoads, true));
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
             issue_thin(2, k_first + 2 * BK);
@@ -1200,7 +1200,9 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
                                 for (int j = 0; j < CB; ++j) mfma_block(acc[i], j, tb[j], ta[i]);
                         }
                     }
-                    __builtin_amdgcn_s_waitcnt(waitcnt_imm((int)kThinLoads, false));
+                    // (and every LDS read of this stage has returned: the compiler moves matrix instructions, and the waits for their
+                    // fragments with them, past the barrier, behind which the other wavefronts' loads fill the stage again)
+                    __builtin_amdgcn_s_waitcnt(waitcnt_imm((int)kThinLoads, true));
                     __builtin_amdgcn_s_barrier();
                     asm volatile("" ::: "memory");
                     issue_thin(st, k_first + (kt + 3) * BK);
@@ -1222,7 +1224,7 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
             else if (row_blocks == 2) thin_loop(std::integral_constant<int, 2>{});
             else if (row_blocks == 1) thin_loop(std::integral_constant<int, 1>{});
             else thin_loop(std::integral_constant<int, 0>{});
-            __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, false));
+            __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, true));
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
         } else if (KT > 0) {
@@ -1305,7 +1307,7 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
             if (!stream_next) {
                 // nothing rides behind this tile: its last two load slots zero-filled the stages; they must have landed,
                 // and every wavefront must be past its last read, before anyone starts cold
-                __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, false));
+                __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, true));
                 __builtin_amdgcn_s_barrier();
                 asm volatile("" ::: "memory");
             }

@@ -22,6 +22,10 @@ for every instantiation of ragged_gemm_kernel, that the instruction stream has t
    hardware wants in scalar registers (what the compiler generates around a vector-memory instruction whose descriptor or
    scalar offset it cannot prove to be the same in every lane: each costs a dozen instructions and a branch per use).
 
+For these kernels and those of csrc/grouped_gemm.hip it checks as well that a wavefront reaches every barrier with all of its LDS
+reads returned. Behind a barrier the other wavefronts' loads may fill the stage that was read, and the compiler is free to move a matrix
+instruction, and with it the wait for its fragments, past the barrier: only a wait of its own in front of the barrier keeps the reads there.
+
 The kernels of csrc/grouped_gemm_f32.hip store four results as 16 bytes: none of their stores may be of 12 bytes, which is what the
 compiler makes of four separate values next to an element-wise branch, with a store of the fourth shared by both.
 """
@@ -33,7 +37,8 @@ import sys
 import tempfile
 
 HERE = os.path.dirname(os.path.abspath(__file__))
-SOURCES = [os.path.join(HERE, "csrc", name) for name in ("grouped_gemm_ragged.hip", "grouped_gemm_ragged_tall.hip")]
+CSRC = os.path.join(HERE, "csrc")
+SOURCES = [os.path.join(CSRC, name) for name in ("grouped_gemm_ragged.hip", "grouped_gemm_ragged_tall.hip")]
 # stores per wavefront and tile: plain, SwiGLU with h, SwiGLU, SwiGLU backward, fp32 sums of a split reduction
 EPI_STORES = {0: 16, 1: 24, 2: 8, 3: 32, 4: 32}
 
@@ -155,6 +160,61 @@ def audit(asm_path: str) -> int:
     return problems
 
 
+def reads_out_at_barriers(body):
+    """How many barriers of a kernel (its instructions, without comments) some path reaches with LDS operations outstanding: of every
+    block the most that are out where it begins, over all its predecessors, until nothing changes."""
+    labels, starts = {}, {0}
+    for i, s in enumerate(body):
+        m = re.match(r"^(\.LBB\d+_\d+):", s)
+        if m:
+            labels[m.group(1)] = i
+            starts.add(i)
+        elif s.startswith(("s_cbranch", "s_branch", "s_endpgm")) and i + 1 < len(body):
+            starts.add(i + 1)
+    starts = sorted(starts)
+    end_of = dict(zip(starts, starts[1:] + [len(body)]))
+    most, todo, flagged = {0: 0}, [0], set()
+    while todo:
+        start = todo.pop()
+        out, end = most[start], end_of[start]
+        for i in range(start, end):
+            s = body[i]
+            if s.startswith("ds_"):
+                out += 1
+            elif s.startswith("s_waitcnt"):
+                m = re.search(r"lgkmcnt\((\d+)\)", s)
+                out = min(out, int(m.group(1))) if m else out
+            elif s.startswith("s_barrier") and out:
+                flagged.add(i)
+        out = min(out, 16)  # (the counter's range)
+        last = body[end - 1]
+        to = [labels[last.split()[-1]]] if last.startswith(("s_cbranch", "s_branch")) else []
+        if not last.startswith(("s_branch", "s_endpgm")) and end < len(body):
+            to.append(end)
+        for t in to:
+            if out > most.get(t, -1):
+                most[t] = out
+                todo.append(t)
+    return len(flagged)
+
+
+def audit_barriers(asm_path: str) -> int:
+    """Every grouped-GEMM kernel of a listing: no barrier with LDS reads outstanding."""
+    lines = open(asm_path).read().split("\n")
+    starts = [i for i, line in enumerate(lines) if re.match(r"^_ZN6fmahip4gemm\w*(ragged|grouped)_gemm_kernel\w*:", line)]
+    if not starts:
+        raise RuntimeError("no grouped-GEMM kernel in " + asm_path)
+    problems = 0
+    for a in starts:
+        end = next(i for i in range(a, len(lines)) if lines[i].startswith(".Lfunc_end"))
+        out = reads_out_at_barriers([line.split(";")[0].strip() for line in lines[a:end]])
+        if out:
+            problems += 1
+            print(f"PROBLEM {lines[a].split(':')[0]}: {out} barriers with LDS reads outstanding")
+    print(f"{os.path.basename(asm_path)}: LDS reads at the barriers of {len(starts)} kernels, {problems} with some outstanding")
+    return problems
+
+
 def audit_f32(asm_path: str) -> int:
     text = open(asm_path).read()
     whole, cut = len(re.findall(r"\bglobal_store_dwordx4\b", text)), len(re.findall(r"\bglobal_store_dwordx3\b", text))
@@ -167,16 +227,19 @@ def audit_f32(asm_path: str) -> int:
 
 def main() -> int:
     if len(sys.argv) > 1:
-        return audit(sys.argv[1])
+        return audit(sys.argv[1]) + audit_barriers(sys.argv[1])
     problems = 0
     sys.path.insert(0, HERE)
     with tempfile.TemporaryDirectory() as tmp:
         for source in SOURCES:
             path = os.path.join(tmp, os.path.basename(source) + ".s")
             compile_to_assembly(source, path)
-            problems += audit(path)
+            problems += audit(path) + audit_barriers(path)
+        path = os.path.join(tmp, "grouped_gemm.hip.s")
+        compile_to_assembly(os.path.join(CSRC, "grouped_gemm.hip"), path)
+        problems += audit_barriers(path)
         path = os.path.join(tmp, "f32.s")
-        compile_to_assembly(os.path.join(HERE, "csrc", "grouped_gemm_f32.hip"), path)
+        compile_to_assembly(os.path.join(CSRC, "grouped_gemm_f32.hip"), path)
         problems += audit_f32(path)
     return problems
 
