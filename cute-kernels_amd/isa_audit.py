@@ -13,11 +13,13 @@ for every instantiation of ragged_gemm_kernel, that the instruction stream has t
    or five) and the request, if the kernel has one, and nothing else up to the next step's first barrier;
  * that wait allows exactly the four loads, the request of a step in the loop, or in a tile's first step the epilogue's stores and the
    bias load;
- * in the tall kernels both steps of a loop body of two issue the same number of loads, and there are four bodies with eight: the middle of
-   the K loops for eight, four, two and one row blocks, which fetch no rows past 256 (every other step does);
+ * in the tall kernels both steps of a loop body of two issue the same number of loads, and there are eight steps with eight: the middle
+   of the K loops for eight, four, two and one row blocks, which fetch no rows past 256 (every other step does);
  * the cold start issues sixteen operand loads (tall kernels: eighteen), as many stand-in stores as an epilogue issues stores, and
    waits for all but the loads of the second step and the stores;
  * the three-stage loop of groups of few rows issues five loads per step with a bias and otherwise six, and waits for all but as many;
+ * there are exactly as many of each as the source has, and of the waits for everything in front of a barrier, and no operand load is
+   outside of them;
  * no instantiation touches scratch memory, and none contains a loop over the distinct values of an operand that the
    hardware wants in scalar registers (what the compiler generates around a vector-memory instruction whose descriptor or
    scalar offset it cannot prove to be the same in every lane: each costs a dozen instructions and a branch per use).
@@ -79,85 +81,108 @@ def tokens(lines):
     return [b for b in "".join(cur).split(" ") if b], waterfalls
 
 
-def audit(asm_path: str) -> int:
-    lines = open(asm_path).read().split("\n")
-    starts = [i for i, line in enumerate(lines) if re.match(r"^_ZN6fmahip4gemm6ragged18ragged_gemm_kernel.*:", line)]
-    if not starts:
-        raise RuntimeError("no ragged_gemm_kernel in " + asm_path)
-    starts.append(len(lines))
-    problems = 0
-    for a, b in zip(starts[:-1], starts[1:]):
-        name = lines[a].split(":")[0]
-        m = re.search(r"ragged_gemm_kernelINS0_(\w+?)ELb(\d)ELb(\d)ELi(\d)ELb(\d)ELb(\d)ELb(\d)ELb(\d)E", name)
-        el, a_kc, b_kc, epi, vary_k, bias, gather, tall = m.group(1), *[int(x) for x in m.groups()[1:]]
-        body = lines[a:b]
-        end = next((k for k, line in enumerate(body) if "s_endpgm" in line), len(body))
-        blocks, waterfalls = tokens(body[:end])
-        request = 1 if (vary_k and gather) else 0
-        stores = EPI_STORES[epi]
-        wait_step, wait_first = 4 + request, 4 + stores + bias
-        tag = f"{el} A_KC={a_kc} B_KC={b_kc} epilogue={epi} reduction_varies={vary_k} bias={bias} gather={gather} tall={tall}"
-        found = {"step": 0, "first": 0, "body": 0, "eight": 0, "cold": 0, "thin": 0}
+# a K step: the loads behind its first barrier, the wait, the loads behind its second one and the request; waits that the compiler added
+# in front of the counted one only wait for more
+STEP = re.compile(r"\|(O*)(?:w\d+,)*w(\d+),\|(O*)([Lp]?)")
+COLD = re.compile(r"((?:[OLp]|w\d+,)*O)(s+)w(\d+),\|")
 
-        def fail(what, block):
-            nonlocal problems
-            problems += 1
-            print(f"PROBLEM {tag}: {what}: {block[:120]}")
 
-        if waterfalls:
-            fail(f"{waterfalls} loops over the distinct values of a scalar operand", "")
-        for blk in blocks:
-            if "X" in blk:
-                fail("scratch access", blk)
-            # the steps: in front of the second barrier four operand loads since the first
-            for before, w, after in re.findall(r"\|([OLp]+|(?:[OLp]|w\d+,)*?)w(\d+),\|((?:[OLp]|w\d+,)*)", blk):
-                n, count = int(w), before.count("O")
-                if count != 4:
-                    continue
-                if len(re.sub(r"w\d+,", "", before)) != 4:
-                    fail(f"{before} between the barriers of a step, expected four operand loads", blk)
-                if n == wait_step:
-                    found["step"] += 1
-                elif n == wait_first:
-                    found["first"] += 1
-                else:
-                    fail(f"a step waits for all but {n}, expected {wait_step} or {wait_first}", blk)
-                behind = after.count("O")
-                if behind not in (4, 4 + tall):
-                    fail(f"{behind} operand loads behind the second barrier", blk)
-            # the three-stage loop
-            for w, loads in re.findall(r"w(\d+),\|(O+)", blk):
-                if len(loads) in (5, 6) and int(w) == len(loads) and "|OOOOw" not in blk:
-                    found["thin"] += 1
-            # a loop body of two steps in one block: what is issued from the first step's second barrier to the second step's first
-            # barrier, and behind the second step's second barrier
-            for between, second in re.findall(r"\|O{4}w\d+,\|([^|]*)\|O{4}w\d+,\|((?:[OLp]|w\d+,)*)", blk):
-                if between.count("O") != second.count("O"):
-                    fail(f"{between.count('O')} and {second.count('O')} operand loads in the second halves of a body's steps", blk)
-                found["eight"] += second.count("O") == 4
-                issued = len(re.sub(r"w\d+,", "", between))
-                if issued in (4 + request, 4 + tall + request):
-                    found["body"] += 1
-                else:
-                    fail(f"{issued} instructions between two steps, expected {4 + request}" + (f" or {5 + request}" if tall else ""), blk)
-            # the cold start: sixteen operand loads (the gathered kinds mix loads of row_index entries in), the stand-in
-            # stores, the wait
-            cold = re.search(r"((?:[OLp]|w\d+,)*O)(s+)w(\d+),\|", blk)
-            if cold and cold.group(1).count("O") >= 16:
-                found["cold"] += 1
-                loads = 8 + tall
-                if cold.group(1).count("O") != 2 * loads or len(cold.group(2)) != stores or int(cold.group(3)) != loads + stores:
-                    fail(f"cold start: {cold.group(1).count('O')} loads, {len(cold.group(2))} stores, wait {cold.group(3)}; "
-                         f"expected {2 * loads}, {stores}, {loads + stores}", blk)
-        if found["step"] == 0 or found["first"] == 0 or found["cold"] != 1:
-            fail(f"expected shapes not found ({found})", "")
-        if a_kc and found["thin"] == 0:
-            fail("no three-stage loop found", "")
-        if tall and (found["eight"] != 4 or found["body"] == 4):
-            fail(f"{found['eight']} of {found['body']} loop bodies with eight operand loads, expected 4 and some with nine", "")
-        print(f"ok  {tag}: steps {found['step']}, first steps {found['first']}, two-step bodies {found['body']}, "
-              f"three-stage steps {found['thin']}")
+def audit_kernel(name: str, body) -> list:
+    """The problems of one instantiation of ragged_gemm_kernel. Every operand load has to belong to one of the four shapes (K step,
+    step and start of the three-stage loop, cold start), and there has to be the exact number of each."""
+    m = re.search(r"ragged_gemm_kernelINS0_(\w+?)ELb(\d)ELb(\d)ELi(\d)ELb(\d)ELb(\d)ELb(\d)ELb(\d)E", name)
+    el, a_kc, b_kc, epi, vary_k, bias, gather, tall = m.group(1), *[int(x) for x in m.groups()[1:]]
+    blocks, waterfalls = tokens(body)
+    request = 1 if (vary_k and gather) else 0
+    stores = EPI_STORES[epi]
+    wait_step, wait_first = 4 + request, 4 + stores + bias
+    thin = 5 if bias else 6
+    tag = f"{el} A_KC={a_kc} B_KC={b_kc} epilogue={epi} reduction_varies={vary_k} bias={bias} gather={gather} tall={tall}"
+    found = {"steps": 0, "first steps": 0, "steps of eight loads": 0, "cold starts": 0, "three-stage steps": 0, "three-stage starts": 0,
+             "drains": 0}  # fmt: skip
+    # The versions of the K loop have their first step, and behind it the second one and a body of two; those of full tiles two steps more, for
+    # the loads of the next tile, and so have those of tiles of few rows in the tall kernels. Three-stage: a body of three and two more.
+    # Drains (a wait for everything and a barrier): behind the kernel's first load, which fetches nothing, a tile that nothing streams behind,
+    # the three-stage loop, and in front of a gathered tile's cold start.
+    expected = {"steps": 28 if tall else 17, "first steps": 6 if tall else 5, "steps of eight loads": 8 if tall else 22, "cold starts": 1,
+                "three-stage steps": a_kc * 5 * (4 if bias else 5), "three-stage starts": a_kc,
+                "drains": 2 + a_kc + (gather and not vary_k)}  # fmt: skip
+    problems = []
+
+    def fail(what, block=""):
+        problems.append(f"{tag}: {what}: {block[:120]}")
+
+    if waterfalls:
+        fail(f"{waterfalls} loops over the distinct values of a scalar operand")
+    for blk in blocks:
+        if "X" in blk:
+            fail("scratch access", blk)
+        if "O" not in blk:
+            found["drains"] += len(re.findall(r"w0,\|", blk))
+            continue
+        cold = COLD.search(blk)
+        if cold:
+            loads = 8 + tall
+            if cold.group(1).count("O") != 2 * loads or len(cold.group(2)) != stores or int(cold.group(3)) != loads + stores:
+                fail(f"cold start: {cold.group(1).count('O')} loads, {len(cold.group(2))} stores, wait {cold.group(3)}; "
+                     f"expected {2 * loads}, {stores}, {loads + stores}", blk)
+            found["cold starts"] += 1
+        elif re.match(r"(?:w\d+,)*\|O{1,4}w", blk):
+            # steps, and nothing else that counts
+            seconds = []
+            for first, wait, second, asked in STEP.findall(blk):
+                if len(first) != 4:
+                    fail(f"{len(first)} operand loads between the barriers of a step, expected 4", blk)
+                if int(wait) not in (wait_step, wait_first):
+                    fail(f"a step waits for all but {wait}, expected {wait_step} or {wait_first}", blk)
+                if len(second) not in (4, 4 + tall) or len(asked) != request:
+                    fail(f"{second + asked} behind the second barrier, expected {4} or {4 + tall} operand loads and {request} requests", blk)
+                found["first steps" if int(wait) == wait_first else "steps"] += 1
+                found["steps of eight loads"] += len(second) == 4
+                seconds.append(len(second))
+            if len(set(seconds)) != 1:
+                fail(f"steps of {seconds} loads behind the second barrier in one body", blk)
+            if not re.fullmatch(r"(?:w\d+,)*#+(?:w\d+,)*", STEP.sub("#", blk)):
+                fail("more than K steps in a block of K steps", blk)
+        else:
+            # the start of the three-stage loop with the loads of two steps in front, or a step or a body of it
+            shape = re.match(r"(O*)((?:w\d+,\|O+)+)(?:w\d+,)*$", blk)
+            if not shape or len(shape.group(1)) not in (0, 2 * thin):
+                fail("operand loads of no known shape", blk)
+                continue
+            runs = re.findall(r"w(\d+),\|(O+)", shape.group(2))
+            for wait, loads in runs:
+                if len(loads) != thin or int(wait) != thin:
+                    fail(f"a three-stage step of {len(loads)} loads waits for all but {wait}, expected {thin}", blk)
+            start = 1 if shape.group(1) else 0
+            found["three-stage starts"] += start
+            found["three-stage steps"] += len(runs) - start
+    for what, n in expected.items():
+        if found[what] != n:
+            fail(f"{found[what]} {what}, expected {n}")
+    if not problems:
+        print(f"ok  {tag}: " + ", ".join(f"{n} {what}" for what, n in found.items()))
     return problems
+
+
+def kernels(asm_path: str, pattern: str):
+    """(name, lines) of the functions of a listing whose names match"""
+    lines = open(asm_path).read().split("\n")
+    found = [i for i, line in enumerate(lines) if re.match(rf"^{pattern}\w*:", line)]
+    if not found:
+        raise RuntimeError(f"no {pattern} in {asm_path}")
+    for a in found:
+        end = next(i for i in range(a, len(lines)) if lines[i].startswith(".Lfunc_end"))
+        yield lines[a].split(":")[0], [line.split(";")[0] for line in lines[a:end]]
+
+
+def audit(asm_path: str) -> int:
+    problems = []
+    for name, body in kernels(asm_path, r"_ZN6fmahip4gemm6ragged18ragged_gemm_kernel"):
+        problems += audit_kernel(name, body)
+    for p in problems:
+        print("PROBLEM " + p)
+    return len(problems)
 
 
 def reads_out_at_barriers(body):
@@ -200,18 +225,14 @@ def reads_out_at_barriers(body):
 
 def audit_barriers(asm_path: str) -> int:
     """Every grouped-GEMM kernel of a listing: no barrier with LDS reads outstanding."""
-    lines = open(asm_path).read().split("\n")
-    starts = [i for i, line in enumerate(lines) if re.match(r"^_ZN6fmahip4gemm\w*(ragged|grouped)_gemm_kernel\w*:", line)]
-    if not starts:
-        raise RuntimeError("no grouped-GEMM kernel in " + asm_path)
-    problems = 0
-    for a in starts:
-        end = next(i for i in range(a, len(lines)) if lines[i].startswith(".Lfunc_end"))
-        out = reads_out_at_barriers([line.split(";")[0].strip() for line in lines[a:end]])
+    problems, seen = 0, 0
+    for name, body in kernels(asm_path, r"_ZN6fmahip4gemm\w*(?:ragged|grouped)_gemm_kernel"):
+        seen += 1
+        out = reads_out_at_barriers([line.strip() for line in body])
         if out:
             problems += 1
-            print(f"PROBLEM {lines[a].split(':')[0]}: {out} barriers with LDS reads outstanding")
-    print(f"{os.path.basename(asm_path)}: LDS reads at the barriers of {len(starts)} kernels, {problems} with some outstanding")
+            print(f"PROBLEM {name}: {out} barriers with LDS reads outstanding")
+    print(f"{os.path.basename(asm_path)}: LDS reads at the barriers of {seen} kernels, {problems} with some outstanding")
     return problems
 
 
