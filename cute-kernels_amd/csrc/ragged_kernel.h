@@ -80,7 +80,8 @@ constexpr int kExtraBytes = (kTallM - BM) * kRowBytes;  // LDS of the rows past 
 // tiles start cold, which short reductions feel. Two stages with one barrier a step -> this, us: [128 x 96 rows, 3072 x 4096] 766 -> 671, its
 // input gradient 627 -> 578; [128 x 128 rows] 682 -> 620 and 645 -> 592; [8 x 96, 28672 x 4096] 490 -> 423, [8 x 100, 2048 x 8192] 82.7 -> 75.7,
 // [64 x 100, 512 x 2048] 44.5 -> 41.3; 24 K steps, [128 x 128, 4096 x 1536], two stages 371, this 378 (hence the line). Groups of up to 64
-// rows, which ran it before: 0 to 1 %, or 0.4 us, more per launch (a larger kernel, and a second load of rows that are not there).
+// rows fetch 64 rows of A a step and not 128: with one loop for all, SwiGLU gradients of [64 x 32 rows, 1408 x 2048] took 91.8 us instead
+// of 89.5, of [16 x 32, 1024 x 2048] 29.0 instead of 27.8, the input gradient [64 x 32, 1408 x 2048] 75.0 instead of 73.2, the rest up to 1 % more.
 // B with the non-temporal hint: weights from memory 3 to 5 % faster ([128 x 48, 3072 x 4096] 638 -> 619), weights that the last-level cache
 // holds from the pass before up to 37 % slower ([8 x 48, 4096 x 2048] 27 -> 35, [16 x 40, 2048 x 2048] 27 -> 37); on all tiles 4 to 17 % slower
 // where row tiles share a panel. Not taken.
@@ -1150,12 +1151,12 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
         if (thin) {
             // three LDS stages in the space that a tile of at most 64 rows leaves unused, or of at most 128 rows and the epilogue's
             // staging buffer; cold start
-            constexpr int kThinA = BIAS ? 1 : 2;  // loads of A per wavefront and step, 64 rows each
-            constexpr uint32_t kThinLoads = kThinA + kLoads;
-            const uint8_t* const a_at[3] = {s_a0, s_a1, kThinA == 1 ? s_a0 + 8192 : s_stage};
+            constexpr int kMostA = BIAS ? 1 : 2;  // loads of A per wavefront and step, 64 rows each: one up to 64 rows
+            const uint8_t* const a_at[3] = {s_a0, s_a1, kMostA == 1 ? s_a0 + 8192 : s_stage};
             const uint8_t* const b_lo[3] = {s_b0, s_b1, s_a0 + 16384};
             const uint8_t* const b_hi[3] = {s_b0 + 16384, s_b1 + 16384, s_a1 + 16384};
-            auto issue_thin = [&](int st, uint32_t k0) {
+            auto issue_thin = [&](auto a_loads_c, int st, uint32_t k0) __attribute__((always_inline)) {
+                constexpr int kThinA = decltype(a_loads_c)::value;
                 if constexpr (GATHER) {
                     uint32_t v[kRowLoads];
                     g_offsets(round & 1u, k0, v);
@@ -1168,13 +1169,15 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
             };
             issue_bias();
             const uint32_t k_first = kSplit ? cur.ks : 0u;
-            issue_thin(0, k_first);
-            issue_thin(1, k_first + BK);
-            __builtin_amdgcn_s_waitcnt(waitcnt_imm((int)kThinLoads, true));
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-            issue_thin(2, k_first + 2 * BK);
-            auto thin_loop = [&](auto fa_c) {
+            auto thin_start = [&](auto a_loads_c) __attribute__((always_inline)) {
+                issue_thin(a_loads_c, 0, k_first);
+                issue_thin(a_loads_c, 1, k_first + BK);
+                __builtin_amdgcn_s_waitcnt(waitcnt_imm(decltype(a_loads_c)::value + kLoads, true));
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                issue_thin(a_loads_c, 2, k_first + 2 * BK);
+            };
+            auto thin_loop = [&](auto a_loads_c, auto fa_c) __attribute__((always_inline)) {
                 constexpr int FA = decltype(fa_c)::value;
                 auto thin_step = [&](int st, uint32_t kt) {
                     if constexpr (FA > 0) {
@@ -1202,10 +1205,10 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
                     }
                     // (and every LDS read of this stage has returned: the compiler moves matrix instructions, and the waits for their
                     // fragments with them, past the barrier, behind which the other wavefronts' loads fill the stage again)
-                    __builtin_amdgcn_s_waitcnt(waitcnt_imm((int)kThinLoads, true));
+                    __builtin_amdgcn_s_waitcnt(waitcnt_imm(decltype(a_loads_c)::value + kLoads, true));
                     __builtin_amdgcn_s_barrier();
                     asm volatile("" ::: "memory");
-                    issue_thin(st, k_first + (kt + 3) * BK);
+                    issue_thin(a_loads_c, st, k_first + (kt + 3) * BK);
                 };
                 uint32_t kt = 0;
                 for (; kt + 2 < KT; kt += 3) {
@@ -1216,14 +1219,20 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
                 if (kt < KT) thin_step(0, kt);
                 if (kt + 1 < KT) thin_step(1, kt + 1);
             };
-            if constexpr (kThinA > 1) {
-                if (row_blocks > 4) thin_loop(std::integral_constant<int, 8>{});
+            using One = std::integral_constant<int, 1>;
+            using Most = std::integral_constant<int, kMostA>;
+            // (more than 64 rows: more than four row blocks, all of one row of wavefronts)
+            if (kMostA > 1 && Me > 64u) {
+                thin_start(Most{});
+                if (row_blocks > 0) thin_loop(Most{}, std::integral_constant<int, 4 * kMostA>{});
+                else thin_loop(Most{}, std::integral_constant<int, 0>{});
+            } else {
+                thin_start(One{});
+                if (row_blocks > 2) thin_loop(One{}, std::integral_constant<int, 4>{});
+                else if (row_blocks == 2) thin_loop(One{}, std::integral_constant<int, 2>{});
+                else if (row_blocks == 1) thin_loop(One{}, std::integral_constant<int, 1>{});
+                else thin_loop(One{}, std::integral_constant<int, 0>{});
             }
-            if (kThinA > 1 && row_blocks > 4) {}
-            else if (row_blocks > 2) thin_loop(std::integral_constant<int, 4>{});
-            else if (row_blocks == 2) thin_loop(std::integral_constant<int, 2>{});
-            else if (row_blocks == 1) thin_loop(std::integral_constant<int, 1>{});
-            else thin_loop(std::integral_constant<int, 0>{});
             __builtin_amdgcn_s_waitcnt(waitcnt_imm(0, true));
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");

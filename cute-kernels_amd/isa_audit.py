@@ -17,7 +17,8 @@ for every instantiation of ragged_gemm_kernel, that the instruction stream has t
    of the K loops for eight, four, two and one row blocks, which fetch no rows past 256 (every other step does);
  * the cold start issues sixteen operand loads (tall kernels: eighteen), as many stand-in stores as an epilogue issues stores, and
    waits for all but the loads of the second step and the stores;
- * the three-stage loop of groups of few rows issues five loads per step with a bias and otherwise six, and waits for all but as many;
+ * the three-stage loop of groups of few rows issues five loads per step, and without a bias a second one six, and waits for all but as
+   many;
  * there are exactly as many of each as the source has, and of the waits for everything in front of a barrier, and no operand load is
    outside of them;
  * no instantiation touches scratch memory, and none contains a loop over the distinct values of an operand that the
@@ -81,9 +82,9 @@ def tokens(lines):
     return [b for b in "".join(cur).split(" ") if b], waterfalls
 
 
-# a K step: the loads behind its first barrier, the wait, the loads behind its second one and the request; waits that the compiler added
-# in front of the counted one only wait for more
-STEP = re.compile(r"\|(O*)(?:w\d+,)*w(\d+),\|(O*)([Lp]?)")
+# a K step: the loads behind its first barrier, the wait, the loads behind its second one and the request; waits that the compiler adds
+# beside the counted one only wait for more
+STEP = re.compile(r"\|(O*)(?:w\d+,)*w(\d+),\|(?:w\d+,)*(O*)([Lp]?)")
 COLD = re.compile(r"((?:[OLp]|w\d+,)*O)(s+)w(\d+),\|")
 
 
@@ -96,17 +97,17 @@ def audit_kernel(name: str, body) -> list:
     request = 1 if (vary_k and gather) else 0
     stores = EPI_STORES[epi]
     wait_step, wait_first = 4 + request, 4 + stores + bias
-    thin = 5 if bias else 6
     tag = f"{el} A_KC={a_kc} B_KC={b_kc} epilogue={epi} reduction_varies={vary_k} bias={bias} gather={gather} tall={tall}"
-    found = {"steps": 0, "first steps": 0, "steps of eight loads": 0, "cold starts": 0, "three-stage steps": 0, "three-stage starts": 0,
-             "drains": 0}  # fmt: skip
+    found = {"steps": 0, "first steps": 0, "steps of eight loads": 0, "cold starts": 0, "three-stage steps of 5": 0,
+             "three-stage steps of 6": 0, "three-stage starts": 0, "drains": 0}  # fmt: skip
     # The versions of the K loop have their first step, and behind it the second one and a body of two; those of full tiles two steps more, for
-    # the loads of the next tile, and so have those of tiles of few rows in the tall kernels. Three-stage: a body of three and two more.
+    # the loads of the next tile, and so have those of tiles of few rows in the tall kernels. Three-stage: a body of three and
+    # two more, for four versions of up to 64 rows and two of up to 128.
     # Drains (a wait for everything and a barrier): behind the kernel's first load, which fetches nothing, a tile that nothing streams behind,
     # the three-stage loop, and in front of a gathered tile's cold start.
     expected = {"steps": 28 if tall else 17, "first steps": 6 if tall else 5, "steps of eight loads": 8 if tall else 22, "cold starts": 1,
-                "three-stage steps": a_kc * 5 * (4 if bias else 5), "three-stage starts": a_kc,
-                "drains": 2 + a_kc + (gather and not vary_k)}  # fmt: skip
+                "three-stage steps of 5": a_kc * 5 * 4, "three-stage steps of 6": 0 if bias else a_kc * 5 * 2,
+                "three-stage starts": a_kc * (1 if bias else 2), "drains": 2 + a_kc + (gather and not vary_k)}  # fmt: skip
     problems = []
 
     def fail(what, block=""):
@@ -147,16 +148,17 @@ def audit_kernel(name: str, body) -> list:
         else:
             # the start of the three-stage loop with the loads of two steps in front, or a step or a body of it
             shape = re.match(r"(O*)((?:w\d+,\|O+)+)(?:w\d+,)*$", blk)
-            if not shape or len(shape.group(1)) not in (0, 2 * thin):
+            runs = re.findall(r"w(\d+),\|(O+)", shape.group(2)) if shape else []
+            thin = len(runs[0][1]) if runs else 0
+            if thin not in (5, 6) or len(shape.group(1)) not in (0, 2 * thin):
                 fail("operand loads of no known shape", blk)
                 continue
-            runs = re.findall(r"w(\d+),\|(O+)", shape.group(2))
             for wait, loads in runs:
                 if len(loads) != thin or int(wait) != thin:
                     fail(f"a three-stage step of {len(loads)} loads waits for all but {wait}, expected {thin}", blk)
             start = 1 if shape.group(1) else 0
             found["three-stage starts"] += start
-            found["three-stage steps"] += len(runs) - start
+            found[f"three-stage steps of {thin}"] += len(runs) - start
     for what, n in expected.items():
         if found[what] != n:
             fail(f"{found[what]} {what}, expected {n}")
