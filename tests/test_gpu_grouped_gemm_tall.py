@@ -13,6 +13,7 @@ from fma.modules.moe.cuda_implementation import (
     grouped_gemm_swiglu_bwd_cuda,
     grouped_gemm_swiglu_cuda,
 )
+from fma.ops.swiglu.cuda_implementation import swiglu_backward_cuda, swiglu_forward_cuda
 
 from gpu_util import DEV
 
@@ -174,8 +175,8 @@ def test_many_tiles_per_workgroup():
 @pytest.mark.parametrize("K", [1984, 2040, 2048, 2120])  # 31 K steps: two LDS stages from 65 rows on; 32 (the last partial or whole), 34
 @pytest.mark.parametrize("tB", [True, False])
 def test_groups_around_the_three_stage_loop(tB, K):
-    """groups on either side of 64 and 128 rows, after each other in every workgroup: packed, gathered and with the activation, against
-    a float64 product of integer operands (|sum| <= 9 K < 2^24: exact in fp32)"""
+    """groups on either side of 64 and 128 rows, after each other in every workgroup: packed, against a float64 product of integer
+    operands (|sum| <= 9 K < 2^24: exact in fp32); gathered and with the activation, with a bias (the loop ends at 64 rows there)"""
     sizes = [64, 65, 128, 129, 1, 100, 0, 127, 300, 63, 80, 256, 112, 16, 113, 96] * 3
     N = 520
     x, w, bias = _inputs(sizes, N, K, torch.bfloat16, (N, K) if tB else (K, N))
@@ -199,3 +200,52 @@ def test_groups_around_the_three_stage_loop(tB, K):
     grouped_gemm_gathered_cuda(x, row_index, 1, w, bias, _u32(sizes), None, gact_only)
     grouped_gemm_swiglu_cuda(packed, w, _u32(sizes), None, act, bias)
     assert torch.equal(h, gh) and torch.equal(act, gact) and torch.equal(act, gact_only)
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float16])
+@pytest.mark.parametrize("K", [1984, 2040, 2048, 2120])  # 31 K steps: two LDS stages from 65 rows on; 32 (the last partial or whole), 34
+@pytest.mark.parametrize("groups", [48, MOST + 1])  # the kernels of both forms
+def test_every_kernel_with_the_three_stage_loop(groups, K, dtype):
+    """groups on either side of 64 and 128 rows, after each other in every workgroup, through every kernel that has the loop: packed and
+    gathered, with and without a bias (with one it ends at 64 rows), the activation and its gradient, both layouts. Against a float64
+    product of operands that are whole numbers over 64 (|sum| <= 9 K / 64, a multiple of 1 / 64: exact in fp32) and, behind it, the
+    activation's own kernels."""
+    sizes = [64, 65, 128, 129, 1, 100, 0, 127, 300, 63, 80, 256, 112, 16, 113, 96] * 3
+    sizes += [0] * (groups - len(sizes))
+    N, R = 528, sum(sizes)
+    x, w, bias = _inputs(sizes, N, K, dtype, (N, K))
+    w, bias, M = w[:groups] / 64, bias[:groups].contiguous(), _u32(sizes)
+    wt = w.transpose(1, 2).contiguous()
+    product = torch.cat([part.double() @ w[e].T.double() for e, part in enumerate(x.split(sizes))]).to(dtype)
+    row_index = torch.randperm(R, device=DEV).int()
+    tokens = torch.empty_like(x)
+    tokens[row_index.long()] = x
+
+    out = _fresh(R, N, dtype=dtype)
+    grouped_gemm_ragged_cuda(x, wt, out, M, False, 0, N, K, False, False, None)
+    assert torch.equal(out, product), "NN"
+    for b in (None, bias):
+        want = product if b is None else (product.float() + b.repeat_interleave(torch.tensor(sizes, device=DEV), 0).float()).to(dtype)
+        up, gate = want.chunk(2, dim=-1)
+        act_want = torch.empty(R, N // 2, dtype=dtype, device=DEV)
+        swiglu_forward_cuda(gate=gate, up=up, output=act_want, BLOCK_SIZE=1024)
+        h, gh, gh2 = (_fresh(R, N, dtype=dtype) for _ in range(3))
+        act, act_only, gact, gact_only = (_fresh(R, N // 2, dtype=dtype) for _ in range(4))
+        grouped_gemm_ragged_cuda(x, w, h, M, False, 0, N, K, False, True, b)
+        assert torch.equal(h, want), "NT"
+        grouped_gemm_gathered_cuda(tokens, row_index, 1, w, b, M, gh, None)
+        assert torch.equal(gh, want), "NT, gathered"
+        h.fill_(7.0)
+        grouped_gemm_swiglu_cuda(x, w, M, h, act, b)
+        grouped_gemm_swiglu_cuda(x, w, M, None, act_only, b)
+        assert torch.equal(h, want) and torch.equal(act, act_want) and torch.equal(act_only, act_want), "activation"
+        grouped_gemm_gathered_cuda(tokens, row_index, 1, w, b, M, gh2, gact)
+        grouped_gemm_gathered_cuda(tokens, row_index, 1, w, b, M, None, gact_only)
+        assert torch.equal(gh2, want) and torch.equal(gact, act_want) and torch.equal(gact_only, act_want), "activation, gathered"
+
+    pre = torch.randn(R, 2 * N, device=DEV, generator=torch.Generator(device=DEV).manual_seed(K)).to(dtype)
+    got, expect = _fresh(R, 2 * N, dtype=dtype), _fresh(R, 2 * N, dtype=dtype)
+    (up, gate), (up_grad, gate_grad) = pre.chunk(2, dim=-1), expect.chunk(2, dim=-1)
+    swiglu_backward_cuda(gate=gate, up=up, output_grad=product, gate_grad=gate_grad, up_grad=up_grad, BLOCK_SIZE=1024)
+    grouped_gemm_swiglu_bwd_cuda(x, wt, pre, M, got)
+    assert torch.equal(got, expect), "gradient of the activation"
