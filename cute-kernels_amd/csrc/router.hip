@@ -462,18 +462,21 @@ bool few_tokens(const RouterArgs& a) {
 // size, and a top-k that runs on more of the chip, which grows with top_k; what they cost is a launch and the logits' way through memory.
 // One launch / tiles and top-k, us; "no": not taken.
 //  * One column of tiles, from 32 tokens per compute unit on: E 32, hidden 2880, top_k 8, 8192 tokens 18.2 / 15.7, 16384 25.3 / 21.5, 32768 40.5 /
-//    37.4; E 20, hidden 4096, 3000 tokens 16.6 / 18.7 (no); hidden 512, top_k 1, 16384 tokens 8.8 / 7.9, hidden 256 7.0 / 7.3 (no), hidden
-//    64, top_k 4 7.3 / 7.5 (no), with 9000 tokens 7.3 / 6.8. The second round for short rows only as far as it pays: hidden 512, top_k 4, 28000 tokens 13.5 / 12.2, 32768
-//    14.0 / 14.8 (no), with top_k 8 15.6 / 14.4; hidden 256 and 20000 tokens, top_k 4 9.1 / 9.6 (no), top_k 8 10.9 / 10.6; hidden 1024, top_k 1, 32768 tokens 17.8 / 19.1 (no), hidden 2880 37.7 / 35.4.
-//  * The first round of two columns: E 64, hidden 2048, top_k 8, 8192 tokens 16.9 / 14.0, hidden 64, top_k 3 7.5 / 7.1, top_k 2 7.0 / 7.3 (no), with
-//    3000 tokens 6.8 / 6.5; of more:
-//    E 128, hidden 4096, 4096 tokens 37.4 / 20.0, hidden 64, top_k 1 8.1 / 7.4.
+//    37.4; E 20, hidden 4096, 3000 tokens 16.6 / 18.7 (no); hidden 512, top_k 1, 16384 tokens 8.8 / 7.9, hidden 256 7.0 / 7.3 (no), hidden 64,
+//    top_k 4 7.3 / 7.5 (no), with 9000 tokens 7.3 / 6.8. The second round for short rows only as far as it pays: hidden 512, top_k 4, 28000 tokens
+//    13.5 / 12.2, 32768 14.0 / 14.8 (no), with top_k 8 15.6 / 14.4; hidden 256 and 20000 tokens, top_k 4 9.1 / 9.6 (no), top_k 8 10.9 / 10.6;
+//    hidden 1024, top_k 1, 32768 tokens 17.8 / 19.1 (no), hidden 2880 37.7 / 35.4.
+//  * The first round of two columns: E 64, hidden 2048, top_k 8, 8192 tokens 16.9 / 14.0, hidden 64, top_k 3 7.5 / 7.1, top_k 2 7.0 / 7.3 (no),
+//    with 3000 tokens 6.8 / 6.5; of more: E 128, hidden 4096, 4096 tokens 37.4 / 20.0, hidden 64, top_k 1 8.1 / 7.4.
 //  * The second round of two columns: E 64, hidden 2048, 14000 tokens, top_k 8 22.7 / 21.8, top_k 4 21.0 / 21.0 (no), top_k 1 20.2 / 20.5 (no);
-//    hidden 64, top_k 6 9.3 / 9.6 (no); E 48, hidden 512, top_k 8 12.4 / 12.0, E 40 20.9 / 21.0 (no), E 33 21.1 / 21.6 (no); with a 64-token workgroup of the one launch for every
-//    compute unit, 16384 tokens, 21.5 / 22.6 (no), hidden 4096 31.8 / 34.1 (no), E 33 20.1 / 23.1 (no).
-//  * The second round of more: E 128, hidden 4096, 8192 tokens, top_k 8 38.0 / 34.0; hidden 2048, top_k 1 21.5 / 21.4; E 100, hidden 512, top_k 3 12.3 /
-//    12.2, top_k 2 11.8 / 12.1 (no); hidden 64, top_k 4 10.4 / 10.4 (no); where the one launch has a second round itself, E 72, hidden 1024, 10000
-//    tokens, top_k 1 24.9 / 13.8, or two passes over x, E 256, hidden 4096, 4000 tokens 61.6 / 34.3, always.
+//    hidden 64, top_k 6 9.3 / 9.6 (no); E 48, hidden 512, top_k 8 12.4 / 12.0, E 40 20.9 / 21.0 (no), E 33 21.1 / 21.6 (no); with a 64-token
+//    workgroup of the one launch for every compute unit, 16384 tokens, 21.5 / 22.6 (no), hidden 4096 31.8 / 34.1 (no), E 33 20.1 / 23.1 (no),
+//    hidden 512 12.9 / 12.3.
+//  * The second round of more: E 128, hidden 4096, 8192 tokens, top_k 8 38.0 / 34.0; hidden 2048, top_k 1 21.5 / 21.4; E 100, hidden 512, top_k 3
+//    12.3 / 12.2, top_k 2 11.8 / 12.1 (no); hidden 64, top_k 4 10.4 / 10.4 (no); where the one launch has a second round itself, E 72, hidden 1024,
+//    10000 tokens, top_k 1 24.9 / 13.8, or two passes over x, E 256, hidden 4096, 4000 tokens 61.6 / 34.3, always.
+// Over 316 launches (E 17 to 256, hidden 64 to 8192, 1100 to 32768 tokens, top_k 1 to 64) the side taken is never slower than the other by more
+// than a run repeats to (2 %, of launches under 10 us 0.4 us).
 bool some_tokens(const RouterArgs& a) {
     const int64_t cus = num_compute_units() > 0 ? num_compute_units() : 256;
     const int64_t columns = (a.E + kTileExps - 1) / kTileExps, tiles = ((a.T + kTileToks - 1) / kTileToks) * columns;
@@ -486,7 +489,7 @@ bool some_tokens(const RouterArgs& a) {
         return a.T >= 32 * cus && saved >= 4 + full && pays;
     }
     if (!second) return columns > 2 || saved >= 2 + full;
-    if (columns == 2) return a.E > 40 && a.k >= 6 && saved >= 8 && (a.T + 63) / 64 < cus;
+    if (columns == 2) return a.E > 40 && a.k >= 6 && saved >= 8 && (a.H <= 512 || (a.T + 63) / 64 < cus);
     return a.E > 128 || a.T > 32 * cus || a.H >= 1024 || (a.k >= 3 && saved >= 5);
 }
 template <typename EL, int NK>
