@@ -16,7 +16,8 @@
 //    first two K steps of the NEXT tile (the loaders of both tiles are kept, a scalar select picks one per step), so that
 //    when a tile's K loop ends the next tile's first step is already in LDS and its second on the way. The tile boundary
 //    is then the epilogue alone: no loader set-up, no burst of 16 loads per wavefront competing with the 16 stores for the
-//    compute unit's one address path, no wait for first operands, no barrier.
+//    compute unit's one address path, no wait for first operands, no barrier. (Nothing more is requested while it lasts, from the
+//    last step's loads to where the next tile's first step has freed its stage.)
 //  * The epilogue's stores stay outstanding across the start of the next tile: they are issued after that tile's first
 //    loads, and loads and stores of a wavefront complete in issue order, so the first K step waits for "all but the
 //    stores and its own newest loads" (an exact count) and the second for everything older than its own loads.
@@ -30,7 +31,9 @@
 //    1350, weight gradients 1735 -> 1694, 902 -> 866; 256 rows 901 -> 840, 479 -> 449 (up with the activation 889 -> 800); 128 rows 807 ->
 //    734 (up); hidden 2048, I 1408, E 64, 4096 rows 2360 -> 2296, 1242 -> 1198, input gradient 2284 -> 2236; hidden 4096, I 14336, E 8,
 //    4096 rows 5640 -> 5650, 2981 -> 2862, input gradient of the first projection 5920 -> 5867 (there the matrix instructions' power is the
-//    bound: all-zero operands 4657 -> 4310, 5107 -> 4620).
+//    bound: all-zero operands 4657 -> 4310, 5107 -> 4620). What it costs: launches of a tile or two per workgroup 0.3 us (input gradient
+//    [8 x 256 rows, 4096 x 64] 13.7 -> 14.0), gathered weight gradients over few rows, whose second loads wait for the index behind the
+//    second barrier, 1.5 to 2.7 % ([8 x 128 rows, 2048 x 2048] 25.7 -> 26.3, [128 x 128, 3072 x 4096] 845 -> 865; [128 x 512] 1655 -> 1633).
 //  * A K loop always runs an even number of steps (a step of zeros is appended to an odd reduction length), so every tile
 //    starts in LDS stage 0 and the loop body stays two straight-line steps.
 //  * Tiles that break the pattern (groups of few rows on their three-stage loop, groups without reduction, groups
@@ -75,14 +78,15 @@ constexpr uint32_t kTallGroups = 256;        // groups a launch of the tall kern
 constexpr int kRowLoads = 5;                 // loads of A rows per wavefront and K step of a tall tile (otherwise four)
 constexpr int kExtraBytes = (kTallM - BM) * kRowBytes;  // LDS of the rows past 256, per stage
 // The three-stage K loop: groups of at most 64 rows, and without a bias of at most kShortRows where the reduction has kShortSteps K steps
-// and more (with one, isa_audit.py finds loops around the loads of the kernels that have both). Such a group has one row tile, whose panels
-// of B no other workgroup reads: a stream of the weights, with one more K step in flight than two stages hold. What it pays is that its
-// tiles start cold, which short reductions feel. Two stages with one barrier a step -> this, us: [128 x 96 rows, 3072 x 4096] 766 -> 671, its
-// input gradient 627 -> 578; [128 x 128 rows] 682 -> 620 and 645 -> 592; [8 x 96, 28672 x 4096] 490 -> 423, [8 x 100, 2048 x 8192] 82.7 -> 75.7,
-// [64 x 100, 512 x 2048] 44.5 -> 41.3; 24 K steps, [128 x 128, 4096 x 1536], two stages 371, this 378 (hence the line). Groups of up to 64
-// rows fetch 64 rows of A a step and not 128: with one loop for all, SwiGLU gradients of [64 x 32 rows, 1408 x 2048] took 91.8 us instead
-// of 89.5, of [16 x 32, 1024 x 2048] 29.0 instead of 27.8, the input gradient [64 x 32, 1408 x 2048] 75.0 instead of 73.2, the rest up to 1 % more.
-// B with the non-temporal hint: weights from memory 3 to 5 % faster ([128 x 48, 3072 x 4096] 638 -> 619), weights that the last-level cache
+// and more (with a bias and both forms of the loop the plain kernel of tall tiles runs out of registers). Such a group has one row tile, whose
+// panels of B no other workgroup reads: a stream of the weights, with one more K step in flight than two stages hold. What it pays is that
+// its tiles start cold, which short reductions feel. Groups of 65 to 128 rows, two stages / three, us: [8 x 96 rows, 28672 x 4096] 429 / 407, [8 x 100,
+// 2048 x 2048] 38.2 / 36.8, input gradient [16 x 100, 2048 x 2048] 33.4 / 32.1, SwiGLU gradient [64 x 96, 1408 x 2048] 102.2 / 100.7, [64 x 96, 2816 x
+// 2048] gathered 189 / 190, [128 x 96, 3072 x 4096] 683 / 658 (which repeats to 4 %). Below the line: 24 steps [128 x 128, 4096 x 1536] 367 / 372,
+// [8 x 100, 2048 x 1536] 31.9 / 30.6; 16 steps, SwiGLU gradient [64 x 96, 1408 x 1024] 59.9 / 62.0; 8 steps [128 x 96, 3072 x 512] 109 / 112. Groups of up to
+// 64 rows fetch 64 rows of A a step and not 128: with one form of the loop for all, SwiGLU gradients of [64 x 32 rows, 1408 x 2048] took 91.8 us
+// instead of 89.5, of [16 x 32, 1024 x 2048] 29.0 instead of 27.8, the input gradient [64 x 32, 1408 x 2048] 75.0 instead of 73.2, the rest up to 1 %
+// more. B with the non-temporal hint: weights from memory 3 to 5 % faster ([128 x 48, 3072 x 4096] 638 -> 619), weights that the last-level cache
 // holds from the pass before up to 37 % slower ([8 x 48, 4096 x 2048] 27 -> 35, [16 x 40, 2048 x 2048] 27 -> 37); on all tiles 4 to 17 % slower
 // where row tiles share a panel. Not taken.
 constexpr uint32_t kShortRows = 128, kShortSteps = 32;
@@ -142,9 +146,11 @@ __device__ __forceinline__ uint32_t parts_of_tail(uint32_t rest, uint32_t g) {
 }
 
 // The time of `units` tiles on `g` workgroups in rounds of 256-row tiles, `tall` of them with rows past 256: such a tile takes a seventh
-// more (8 groups of about 300 rows, 2048 x 8192: 211 us with one or more of them against 244 us), the last, partial round 0.87 of a
-// whole one in parts of its columns and on its own 0.85 (NN, 64 tiles of 2048 x 16384: 394 -> 330 us). In the NT layout a launch of at
-// most half as many tiles as workgroups is never cut.
+// more (8 groups of about 300 rows, 2048 x 8192: 165 us, with one or more of them 186), the last, partial round 0.87 of a
+// whole one in parts of its columns and on its own 0.85 (NN, 64 tiles of 2048 x 16384: 345 -> 278 us, 327 -> 279). In the NT layout a launch of at
+// most half as many tiles as workgroups is never cut. Over 118 launches (twelve shapes, 200 to 2048 rows a group, randomly routed) the height taken
+// costs 0.6 % more than the better of the two; 256 rows always 5.7 %, 288 wherever a group has more than 256 rows 2.2 %. Without parts of the
+// last round they take 0.8 % longer.
 template <bool PARTS, bool B_KC>
 __device__ __forceinline__ float rounds_of(uint32_t units, uint32_t tall, uint32_t g) {
     const uint32_t whole = units / g, rest = units - whole * g;
@@ -326,8 +332,8 @@ __global__ __launch_bounds__(NT) void ragged_gemm_kernel(const Args args) {
         if constexpr (TALL) {
             // Tiles of up to 288 rows where they save more rounds than their longer K steps cost. 256-row tiles / tall ones wherever a
             // group has more than 256 rows, us, randomly routed: 2048 x 8192, E 8, 300, 600 and 800 rows a group (one round either way:
-            // not taken) 211 / 244, 213 / 239, 207 / 237, 1000 rows (two rounds / one) 391 / 227; 2880 x 2880, E 32, 300 rows (three /
-            // three) 238 / 262, 256 rows 261 / 212; 4096 x 1536, E 128, 256 rows (12 / 9) 559 / 512; 2048 x 1408, E 64, 300 rows 173 / 189.
+            // not taken) 165 / 186, 171 / 196, 181 / 208, 1024 rows (two rounds / one) 309 / 205; 2880 x 2880, E 32, 300 rows (three /
+            // three) 179 / 204, 256 rows 194 / 159; 4096 x 1536, E 128, 256 rows (12 / 9) 516 / 479; 2048 x 1408, E 64, 300 rows 135 / 146.
             const uint32_t per = columns * (kSplit ? args.splits : 1u);
             const float low = rounds_of<kTail, B_KC>(uniform(sums[0]) * per, 0u, g);
             const float high = rounds_of<kTail, B_KC>(uniform(sums[1]) * per, uniform(sums[2]) * per, g);

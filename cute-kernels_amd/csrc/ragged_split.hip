@@ -10,29 +10,31 @@ namespace ragged {
 
 // ---- split reduction ---------------------------------------------------------------------------------------------
 // A launch with fewer tiles than compute units leaves the others idle for the whole reduction: the second projection of 800 tokens on
-// 8 experts (2048 x 8192) is 64 tiles of 128 K steps, 239 us. With the reduction in three parts (192 units of 44 steps, fp32 sums to
-// memory and one pass over them) it takes 130 us. More of the same, 8 groups, randomly routed (unsplit -> parts):
-//   NT 2048 x 8192, 150 / 256 / 400 / 512 rows a group       229 -> 124 us (3), 239 -> 143 us (3), 230 -> 165 us (2), 235 -> 180 us (2)
-//   NT 4096 x 14336, 100 / 256 / 600 rows                    382 -> 252 us (2), 411 -> 291 us (2), 678 -> 625 us (2)
-//   NN 2048 x 16384, 150 / 256 / 400 / 512 rows              321 -> 158 us (4), 352 -> 202 us (3), 345 -> 246 us (2), 388 -> 262 us (2)
-//   NN 4096 x 28672, 100 / 256 rows                          576 -> 375 us (2), 701 -> 519 us (4)
+// 8 experts (2048 x 8192) is 64 tiles of 128 K steps, 184 us. With the reduction in three parts (192 units of 44 steps, fp32 sums to
+// memory and one pass over them) it takes 94 us. More of the same, 8 groups, randomly routed (unsplit -> parts):
+//   NT 2048 x 8192, 150 / 256 / 400 / 512 rows a group       157 -> 86 us (3), 172 -> 106 us (3), 175 -> 121 us (2), 193 -> 149 us (2)
+//   NT 4096 x 14336, 100 / 200 / 600 rows                    265 -> 191 us (2), 330 -> 227 us (2), 605 -> 571 us (2)
+//   NN 2048 x 16384, 150 / 256 / 400 / 512 rows              234 -> 129 us (4), 276 -> 175 us (3), 291 -> 214 us (2), 332 -> 247 us (2)
+//   NN 4096 x 28672, 100 / 256 rows                          380 -> 320 us (2), 619 -> 440 us (4)
 //
 // How many parts: the number with the least predicted time, rounds of tiles times (K steps + a tile's fixed cost) or the
 // weights at the rate they stream, plus the traffic of the sums. The row counts lie in device memory, so the number of tiles
 // is the expected one for evenly loaded groups. Parts have at least kSplitMinSteps steps, the sums at most kSplitMaxBytes (they
 // stay in the last-level cache), and a split has to promise a twentieth less than none. Groups of few rows run the three-stage
-// loop, whose steps are shorter, without a split on half-width tiles in the NT layout: NT 4096 x 14336 on 8 groups of 32 rows
-// streams its weights in 176 us as it is and would take 184 us in two parts.
+// loop, whose steps are shorter, without a split on half-width tiles in the NT layout: NT 4096 x 14336 on 8 groups of 24 rows
+// streams its weights in 175 us as it is and would take 197 us in two parts.
 // Tall tiles (TALL in ragged_kernel.h): a round takes 1.6 to 2.0 us per K step of its tiles, most when every compute unit is busy and
 // streams weights of its own, and a partial last round costs what rounds_of there says. The tiles of a group follow from the spread of a
 // random routing (a standard deviation of the root of the mean): 8 groups of 256 or 512 rows are 8 or 16 tiles high, not 12 or 20. That
-// ends the split of [8 x 512 rows, 4096 x 14336] (440 us, two parts 485).
+// ends the split of [8 x 512 rows, 4096 x 14336] (370 us, two parts 432).
 // Routings are less even than random ones, too, and what fills the compute units exactly once is worth little if one more row tile spoils
 // it: where a group of 2.5 times the mean rows has a second tile, one launch in five (kUneven) is taken to have one. 8 groups of 200 rows,
-// 2048 x 8192 and 2048 x 16384 in four parts (256 units) take 153 and 173 us, but with odds of the experts as their rank to the -0.7 (9 row
-// tiles) 188 and 256; in three parts 130 and 187, 132 and 193. 4096 x 28672, 256 rows: 487 and 721 us in two parts, 519 and 607 in four. Over
-// 1380 launches (seven shapes, 24 to 1000 rows a group, three routings) the parts taken cost 2.1 % (random), 4.0 and 4.6 % (two uneven ones)
-// more than the best number would; without the line 2.0, 5.3 and 5.9 %.
+// 2048 x 8192 and 2048 x 16384 in four parts (256 units) take 101 and 146 us, but with odds of the experts as their rank to the -0.7 (9 row
+// tiles) 135 and 216; in three parts 93 and 157, 88 and 149. Over 210 launches (seven shapes of 4 to 32 groups, 24 to 1000 rows a group,
+// a random and such an uneven routing, one draw of each) the parts taken cost 1.6 % (random) and 6.4 % (uneven) more than the best number
+// would; without the line 1.4 and 9.2 %. A fifth more or less of any constant moves that by less than 1 and 3 %, as another draw does. What the
+// constants miss: with few rows the half-width tiles of no split take 0.6 us a step, the whole ones of parts 1.15, so that 8 groups of 24 or 48
+// rows, NT 2048 x 8192, run in three parts (69 and 72 us) and not in four (58 and 60).
 constexpr double kStepUs = 1.45, kTallStepUs = 1.55, kFullStepUs = 0.4, kThinStepUs[2] = {1.1, 0.75}, kTileSteps = 6.0, kThinRows = 48.0;
 constexpr double kTailCost = 0.87, kLoneTailCost = 0.85, kUneven = 0.2, kWeightBytesPerUs = 5.5e6;
 constexpr double kReduceUs = 4.0, kReduceBytesPerUs = 4.5e6, kSplitGain[2] = {0.9, 0.95};  // [tall]
