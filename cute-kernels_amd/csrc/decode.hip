@@ -14,19 +14,9 @@
 //    combines (thin_experts.hip).
 #include "gemm_parts.h"
 #include "router_logits.h"
+#include "thin_experts.h"
 
 namespace fmahip {
-namespace gemm {
-namespace thin {
-// thin_experts.hip
-int check(const char* who, const void* x, int64_t x_rows, const int32_t* row_index, int32_t divisor, const void* W,
-          const void* out, const uint32_t* counts, const uint32_t* offsets, int64_t R, int64_t E, int64_t N, int64_t K, int swiglu,
-          int dtype);
-bool takes_one_token(int64_t T, int64_t top_k);
-int one_token(const void* x, const void* logits, const void* W1, const void* bias1, const void* W2, const void* bias2, void* act, void* y,
-              int64_t E, int64_t H, int64_t I, int64_t top_k, int dtype, hipStream_t st);
-}  // namespace thin
-}  // namespace gemm
 namespace {
 
 constexpr int kIndexThreads = 1024;

@@ -31,6 +31,7 @@
 // others, 48 tokens of the third take 286 instead of 230 us.
 #include "gemm_parts.h"
 #include "router_parts.h"
+#include "thin_experts.h"
 
 namespace fmahip {
 namespace gemm {
@@ -554,7 +555,7 @@ int product(const void* x, int64_t x_rows, const int32_t* row_index, int32_t div
     return w ? launch<ElemF16, 64>(a, glu, R, groups, max_rows, st) : launch<ElemF16, 32>(a, glu, R, groups, max_rows, st);
 }
 
-// The expert path of one token (decode.hip): act [top_k, I] is scratch, y [H] the layer's output. E up to FMA_MAX_DECODE_EXPERTS.
+// The expert path of one token (decode.hip)
 bool takes_one_token(int64_t T, int64_t top_k) { return T == 1 && top_k <= (int64_t)kMostChoices; }
 int one_token(const void* x, const void* logits, const void* W1, const void* bias1, const void* W2, const void* bias2, void* act, void* y,
               int64_t E, int64_t H, int64_t I, int64_t top_k, int dtype, hipStream_t st) {
