@@ -175,8 +175,8 @@ def test_many_tiles_per_workgroup():
 @pytest.mark.parametrize("K", [1984, 2040, 2048, 2120])  # 31 K steps: two LDS stages from 65 rows on; 32 (the last partial or whole), 34
 @pytest.mark.parametrize("tB", [True, False])
 def test_groups_around_the_three_stage_loop(tB, K):
-    """groups on either side of 64 and 128 rows, after each other in every workgroup: packed, against a float64 product of integer
-    operands (|sum| <= 9 K < 2^24: exact in fp32); gathered and with the activation, with a bias (the loop ends at 64 rows there)"""
+    """groups on either side of 64 and 128 rows, after each other in every workgroup: packed, gathered and with the activation, against
+    a float64 product of integer operands (|sum| <= 9 K < 2^24: exact in fp32)"""
     sizes = [64, 65, 128, 129, 1, 100, 0, 127, 300, 63, 80, 256, 112, 16, 113, 96] * 3
     N = 520
     x, w, bias = _inputs(sizes, N, K, torch.bfloat16, (N, K) if tB else (K, N))
